@@ -971,6 +971,8 @@ int cav_upload_atoms(cav_ctx *c, int n, const int *id, const int *type, const in
   c->gcap = 7 * n;  // at most seven images per owned atom
   c->h_id.assign(id, id + n);
   c->h_type.assign(type, type + n);
+  c->type_count.assign(c->nt, 0);
+  for (int i = 0; i < n; ++i) ++c->type_count[type[i]];
   c->h_mol.assign(n, -1);
   if (mol) c->h_mol.assign(mol, mol + n);
   const size_t tot = (size_t)n + c->gcap;
@@ -1523,10 +1525,7 @@ int cav_energy(cav_ctx *c, double *e_lj, double *e_r, double *e_k)
   if (!c->setup_done) return fail(c, CAV_ERR_STATE, "cav_setup must run first");
   (void)hipSetDevice(c->device);
   CAV_TRY(refresh_params(c));
-  if (e_k) {
-    if (!c->ek_on) return fail(c, CAV_ERR_STATE, "no Ewald_k");
-    CAV_TRY(launch_energy_k(c, e_k));
-  }
+  if (e_k && !c->ek_on) return fail(c, CAV_ERR_STATE, "no Ewald_k");
   if (e_r || e_lj) {
     if (!c->nl_on) return fail(c, CAV_ERR_STATE, "no neighbour list");
     // the cell walk needs cells of the current positions and ghosts
@@ -1535,12 +1534,19 @@ int cav_energy(cav_ctx *c, double *e_lj, double *e_r, double *e_k)
   if (e_r) {
     if (!c->er_on) return fail(c, CAV_ERR_STATE, "no Ewald_r");
     if (!c->build_cells) return fail(c, CAV_ERR_STATE, "Ewald_r energy walks the cell list: needs build_cell_list");
-    CAV_TRY(launch_energy_r(c, e_r));
+    CAV_TRY(launch_energy_r(c));
   }
   if (e_lj) {
     if (!c->lj_on) return fail(c, CAV_ERR_STATE, "no lj_cell_list");
-    CAV_TRY(launch_energy_lj(c, e_lj));
+    CAV_TRY(launch_energy_lj(c));
   }
+  // one read-back for every term: [1] LJ, [2] real space, [3] lattice, [8..10] dipole
+  double v[12];
+  CAV_HIP(hipMemcpyAsync(v, c->scal, sizeof(v), hipMemcpyDeviceToHost, c->stream));
+  CAV_HIP(hipStreamSynchronize(c->stream));
+  if (e_k) *e_k = energy_k(c, v);
+  if (e_r) *e_r = 0.5 * v[2] * c->er_ke;  // energy.cpp:50 and potential.cpp:85
+  if (e_lj) *e_lj = v[1];
   return CAV_OK;
 }
 

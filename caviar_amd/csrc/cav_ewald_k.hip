@@ -1932,24 +1932,18 @@ int ewald_k_field(cav_ctx *c, double *out4)
 
 // E_k = 1/2 C sum W |S|^2 + self (+ dipole), valid after a force evaluation at
 // the same positions (the reference's S(k) coupling, energy.cpp:61-116).
-int launch_energy_k(cav_ctx *c, double *e)
+double energy_k(const cav_ctx *c, const double *v)
 {
-  double v[12];
-  CAV_HIP(hipMemcpyAsync(v, c->scal, sizeof(double) * 12, hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
   double q2 = 0;
-  for (int i = 0; i < c->n; ++i) {
-    const double qq = c->charge[c->h_type[i]];
-    q2 += qq * qq;
-  }
+  const int nt = std::min(c->nt, (int)c->type_count.size());
+  for (int t = 0; t < nt; ++t) q2 += c->type_count[t] * c->charge[t] * c->charge[t];
   const double self = -CAV_PIS_INV * c->ek_alpha * q2 * c->ek_ke;
   double ek = 0.5 * CAV_4PI * c->ek_ke * c->ek.lxyz_inv * v[3] + self;
   if (c->dipole) {
     const double d2 = v[8] * v[8] + v[9] * v[9] + v[10] * v[10];
     ek += 0.5 * c->ek.dip_coef * d2;
   }
-  *e = ek;
-  return CAV_OK;
+  return ek;
 }
 
 // Point queries: tables for the points, then the force pass with q = 1 into a

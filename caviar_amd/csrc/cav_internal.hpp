@@ -169,6 +169,7 @@ struct cav_ctx {
   // atoms
   int n = 0, gcap = 0;
   std::vector<int> h_id, h_type, h_mol;
+  std::vector<int> type_count;  // owned atoms of each type
 
   // device arrays: positions/type/id/mol/charge over owned + ghost capacity
   double *x = nullptr, *y = nullptr, *z = nullptr;
@@ -414,9 +415,9 @@ const char *plan_k_lattice(EwaldKPlan &p, int kx, int ky, int kz, int precision,
 void split_scales(double qmax, double qsum, double wmax, double *sA, double *sB);
 int ewald_k_alloc(cav_ctx *c);
 int ewald_k_autotune(cav_ctx *c);
-int launch_energy_r(cav_ctx *c, double *e);
-int launch_energy_lj(cav_ctx *c, double *e);
-int launch_energy_k(cav_ctx *c, double *e);
+int launch_energy_r(cav_ctx *c);   // into scal[2]
+int launch_energy_lj(cav_ctx *c);  // into scal[1]
+double energy_k(const cav_ctx *c, const double *scal);  // from the scalars of the last evaluation
 int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot);
 int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *pot);
 int reduce_partials(cav_ctx *c, int count, int slot, bool add = false);

@@ -929,6 +929,7 @@ struct CellArgs {
   int n;
   const double *x, *y, *z, *q;
   const int *type, *bin_of, *st_off, *st, *start, *items;
+  const double4 *cpos;  // (x, y, z, index and slot) in bin order
   double lox, loy, loz, cinv;
   int nbx, nby, nbz;
 };
@@ -958,6 +959,7 @@ static CellArgs cell_args(cav_ctx *c)
   a.st = c->d_st;
   a.start = c->bin_start;
   a.items = c->bin_items;
+  a.cpos = c->cpos;
   a.lox = c->lo[0];
   a.loy = c->lo[1];
   a.loz = c->lo[2];
@@ -1014,78 +1016,89 @@ int launch_lj_cellwalk(cav_ctx *c)
   return CAV_OK;
 }
 
+// The cell walk's candidates: the 27-cell stencil of cell b flattened in order
+// (each cell in bin order).  Lanes 0..ns-1 load their cell's range at once; the
+// running offsets go to the wave's LDS (s_base, s_off).  Returns their number.
+__device__ __forceinline__ int walk_ranges(const CellArgs &c, int b, int *s_base, int *s_off)
+{
+  const int lane = threadIdx.x & 63;
+  const int sb = c.st_off[b], ns = c.st_off[b + 1] - sb;  // 1..27 cells
+  int cb = 0, cn = 0;
+  if (lane < ns) {
+    const int cell = c.st[sb + lane];
+    cb = c.start[cell];
+    cn = c.start[cell + 1] - cb;
+  }
+  int incl = cn;
+  for (int o = 1; o < 32; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  if (lane < ns) {
+    s_base[lane] = cb;
+    s_off[lane + 1] = incl;
+  }
+  if (lane == 0) s_off[0] = 0;
+  return __shfl(incl, ns - 1, 64);
+}
+
+// Candidate g of the flattened stencil as (x, y, z, q); `cell` walks forward
+// with g (start at 0, ascending g).
+__device__ __forceinline__ double4 walk_cand(const CellArgs &c, const int *s_base, const int *s_off,
+                                             int g, int &cell)
+{
+  while (s_off[cell + 1] <= g) ++cell;
+  double4 v = c.cpos[s_base[cell] + g - s_off[cell]];
+  v.w = c.q[(int)(__double_as_longlong(v.w) & 0xffffffffll)];  // low word: the atom
+  return v;
+}
+
 // Electrostatic_ewald_r::potential/field at a point (electrostatic_ewald_r/
 // potential.cpp:30-86, field.cpp:31-96): every owned or ghost atom in the 27
 // cells around the point's bin, no cutoff, exact-zero separation skipped.
-__device__ void point_r_eval(const CellArgs &c, double px, double py, double pz, double alpha,
-                             double *field, double *pot)
+// One wave per point, its lanes over the candidates, summed by a fixed shuffle
+// tree.  The FP64 erfc and exp bound it; with one lane per point a lane walked
+// all of its candidates by itself and a launch held np / 64 waves: 1000 points
+// among 100 ions took 818 us, now 14 us.
+__global__ __launch_bounds__(kBlock) void k_point_r(CellArgs c, int np, const double *pts,
+                                                    double alpha, double ke, double *field,
+                                                    double *pot)
 {
-  const int b = cell_of(c, px, py, pz);
+  __shared__ int s_base_[kBlock / 64][32], s_off_[kBlock / 64][33];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int p = blockIdx.x * (kBlock / 64) + wv;
+  if (p >= np) return;
+  const double px = pts[3 * p], py = pts[3 * p + 1], pz = pts[3 * p + 2];
+  int *s_base = s_base_[wv], *s_off = s_off_[wv];
+  const int total = walk_ranges(c, cell_of(c, px, py, pz), s_base, s_off);
+  __syncwarp();
   const double a2 = alpha * alpha;
   double phi = 0, ex = 0, ey = 0, ez = 0;
-  for (int s = c.st_off[b]; s < c.st_off[b + 1]; ++s) {
-    const int cell = c.st[s];
-    for (int t = c.start[cell]; t < c.start[cell + 1]; ++t) {
-      const int j = c.items[t];
-      const double dx = px - c.x[j], dy = py - c.y[j], dz = pz - c.z[j];
-      if (dx == 0 && dy == 0 && dz == 0) continue;
-      const double d2 = dx * dx + dy * dy + dz * dz, dn = sqrt(d2);
-      const double ec = erfc(alpha * dn) / dn;
-      const double qj = c.q[j];
-      phi += qj * ec;
-      const double sr = (2 * alpha * CAV_PIS_INV * exp(-a2 * d2) + ec) / d2;
-      ex += qj * sr * dx;
-      ey += qj * sr * dy;
-      ez += qj * sr * dz;
-    }
+  int cell = 0;
+  for (int g = lane; g < total; g += 64) {
+    const double4 v = walk_cand(c, s_base, s_off, g, cell);
+    const double dx = px - v.x, dy = py - v.y, dz = pz - v.z;
+    if (dx == 0 && dy == 0 && dz == 0) continue;
+    const double d2 = dx * dx + dy * dy + dz * dz, dn = sqrt(d2);
+    const double ec = erfc(alpha * dn) / dn;
+    phi += v.w * ec;
+    const double sr = (2 * alpha * CAV_PIS_INV * exp(-a2 * d2) + ec) / d2;
+    ex += v.w * sr * dx;
+    ey += v.w * sr * dy;
+    ez += v.w * sr * dz;
   }
-  *pot = phi;
-  field[0] = ex;
-  field[1] = ey;
-  field[2] = ez;
-}
-
-__global__ void k_energy_r(CellArgs c, double alpha, double *part)
-{
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  double e = 0;
-  if (i < c.n) {
-    double f[3], phi;
-    point_r_eval(c, c.x[i], c.y[i], c.z[i], alpha, f, &phi);
-    e = c.q[i] * phi;
+  for (int o = 32; o > 0; o >>= 1) {
+    phi += __shfl_xor(phi, o, 64);
+    ex += __shfl_xor(ex, o, 64);
+    ey += __shfl_xor(ey, o, 64);
+    ez += __shfl_xor(ez, o, 64);
   }
-  __shared__ double red[kBlock];
-  red[threadIdx.x] = e;
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
+  if (lane == 0) {
+    pot[p] = phi * ke;
+    field[3 * p] = ex * ke;
+    field[3 * p + 1] = ey * ke;
+    field[3 * p + 2] = ez * ke;
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-int launch_energy_r(cav_ctx *c, double *e)
-{
-  k_energy_r<<<grid_for(c->n), kBlock, 0, c->stream>>>(cell_args(c), c->er_alpha, c->part);
-  CAV_TRY(reduce_partials(c, grid_for(c->n), 2));
-  double v;
-  CAV_HIP(hipMemcpyAsync(&v, c->scal + 2, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
-  *e = 0.5 * v * c->er_ke;  // energy.cpp:50 and potential.cpp:85
-  return CAV_OK;
-}
-
-__global__ void k_point_r(CellArgs c, int np, const double *pts, double alpha, double ke,
-                          double *field, double *pot)
-{
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= np) return;
-  double f[3], phi;
-  point_r_eval(c, pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], alpha, f, &phi);
-  pot[p] = phi * ke;
-  field[3 * p] = f[0] * ke;
-  field[3 * p + 1] = f[1] * ke;
-  field[3 * p + 2] = f[2] * ke;
 }
 
 int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot)
@@ -1093,8 +1106,9 @@ int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *
   double *d;
   CAV_HIP(hipMalloc(&d, sizeof(double) * 7 * (size_t)(np > 0 ? np : 1)));
   CAV_HIP(hipMemcpyAsync(d, pts, sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
-  k_point_r<<<grid_for(np), kBlock, 0, c->stream>>>(cell_args(c), np, d, c->er_alpha, c->er_ke,
-                                                    d + 3 * np, d + 6 * np);
+  if (np > 0)
+    k_point_r<<<(np + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, c->stream>>>(
+        cell_args(c), np, d, c->er_alpha, c->er_ke, d + 3 * np, d + 6 * np);
   CAV_HIP(hipGetLastError());
   if (field)
     CAV_HIP(hipMemcpyAsync(field, d + 3 * np, sizeof(double) * 3 * np, hipMemcpyDeviceToHost,
@@ -1106,50 +1120,137 @@ int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *
   return CAV_OK;
 }
 
+// Stencil candidates staged per pass of the real-space energy (16 KB of LDS).
+constexpr int kWalkCand = 512;
+
+// Electrostatic_ewald_r::energy (electrostatic_ewald_r/energy.cpp:30-51): the
+// potential of the cell walk at every owned atom times its charge.  One
+// workgroup per cell: its stencil's candidates (x, y, z, q) are staged in LDS
+// once for the cell's owned atoms, which the four waves take in turn, lanes
+// over the candidates.  The FP64 erfc of every (atom, candidate) bounds it
+// (about 500 an atom at rho = 0.3); one lane per atom, each walking its
+// stencil through scattered loads, took 3395 us at N = 100003, now 395 us.
+__global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, double alpha, double *part)
+{
+  __shared__ double4 cand[kWalkCand];
+  __shared__ int s_base[32], s_off[33];
+  __shared__ double red[kBlock / 64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int b = blockIdx.x;
+  const int s0 = c.start[b], e0 = c.start[b + 1];
+  int no = 0;  // owned atoms come first in a sorted bin
+  for (int t = s0; t < e0; t += 64)
+    no += __popcll(__ballot(t + lane < e0 && c.items[t + lane] < c.n));
+  double e = 0;
+  if (no > 0) {
+    // every wave forms the ranges (the values are the same)
+    const int total = walk_ranges(c, b, s_base, s_off);
+    __syncthreads();
+    for (int m0 = 0; m0 < total; m0 += kWalkCand) {
+      const int m = min(kWalkCand, total - m0);
+      int cell = 0;
+      for (int t = threadIdx.x; t < m; t += kBlock)
+        cand[t] = walk_cand(c, s_base, s_off, m0 + t, cell);
+      __syncthreads();
+      for (int o = wv; o < no; o += kBlock / 64) {
+        const int i = c.items[s0 + o];
+        const double xi = c.x[i], yi = c.y[i], zi = c.z[i];
+        double phi = 0;
+        for (int t = lane; t < m; t += 64) {
+          const double4 v = cand[t];
+          const double dx = xi - v.x, dy = yi - v.y, dz = zi - v.z;
+          if (dx == 0 && dy == 0 && dz == 0) continue;
+          const double dn = sqrt(dx * dx + dy * dy + dz * dz);
+          phi += v.w * (erfc(alpha * dn) / dn);
+        }
+        e += c.q[i] * phi;
+      }
+      __syncthreads();
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+  if (lane == 0) red[wv] = e;
+  __syncthreads();
+  if (threadIdx.x == 0) part[b] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// Leaves twice the energy over k_electrostatic in scal[2] (energy.cpp:50 and
+// potential.cpp:85).
+int launch_energy_r(cav_ctx *c)
+{
+  if (c->nbins > c->npart) return fail(c, CAV_ERR_STATE, "partial-sum buffer smaller than the cell grid");
+  k_energy_r<<<c->nbins, kBlock, 0, c->stream>>>(cell_args(c), c->er_alpha, c->part);
+  CAV_HIP(hipGetLastError());
+  return reduce_partials(c, c->nbins, 2);
+}
+
 // Shifted-force LJ energy over the full rows: each (i,j) entry carries half of
 // U(r) = 4e[(s/r)^12 - (s/r)^6] + r^2 cshift/2 - (same at rc); every pair is
 // seen from both ends (owned pairs twice in the full rows, periodic pairs once
-// from each owned end through its ghost image).
-__global__ void k_energy_lj(PairArgs a, const double *u12, const double *u6, const double *uc,
-                            double *part)
+// from each owned end through its ghost image).  kLPA lanes per atom and the
+// packed (x, y, z, q), (type, id), as the pair kernel, four entries' loads
+// issued together; the rows are read as the list build wrote them (`items`:
+// bin-order slots to be looked up there, or null for atom indices).  Gather
+// latency bounds it: 242 us at N = 100003 with one lane per atom, and 52 us
+// to fill the index rows first; now 74 us, no fill.
+__global__ __launch_bounds__(kBlock) void k_energy_lj(PairArgs a, const int *rows, const int *items,
+                                                      const double *u12, const double *u6,
+                                                      const double *uc, double *part)
 {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const long gid = (long)blockIdx.x * kBlock + threadIdx.x;
+  const int t = (int)(gid / kLPA), sub = (int)(gid % kLPA);
   double e = 0;
-  if (i < a.n) {
-    const double xi = a.x[i], yi = a.y[i], zi = a.z[i];
-    const int ti = a.type[i];
-    for (int k = 0; k < a.nn[i]; ++k) {
-      const int j = a.nl[(long)i * a.cap + k];
-      const double dx = a.x[j] - xi, dy = a.y[j] - yi, dz = a.z[j] - zi;
-      const double r2 = dot_rn_p(dx, dy, dz);
-      if (r2 > a.lj_rc2) continue;
-      const int tj = a.type[j];
-      const int p = (j < a.n && j < i) ? tj * a.nt + ti : ti * a.nt + tj;
-      const double ri2 = 1.0 / r2, ri6 = ri2 * ri2 * ri2;
-      e += 0.5 * (u12[p] * ri6 * ri6 - u6[p] * ri6 + 0.5 * a.cshift[p] * r2 - uc[p]);
+  if (t < a.n) {
+    const int i = a.order[t];
+    const double4 pi = a.xq[i];
+    const int ti = a.tid[i].x, cnt = a.nn[i];
+    const int *row = rows + (long)i * a.cap;
+    constexpr int U = 4;
+    for (int k0 = sub; k0 < cnt; k0 += U * kLPA) {
+      int j[U], tj[U];
+      double4 pj[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) j[u] = k0 + u * kLPA < cnt ? row[k0 + u * kLPA] : -1;
+      if (items) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) j[u] = j[u] < 0 ? -1 : items[j[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int jj = j[u] < 0 ? i : j[u];
+        pj[u] = a.xq[jj];
+        tj[u] = a.tid[jj].x;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const double r2 = dot_rn_p(pj[u].x - pi.x, pj[u].y - pi.y, pj[u].z - pi.z);
+        if (j[u] < 0 || r2 > a.lj_rc2) continue;
+        const int p = (j[u] < a.n && j[u] < i) ? tj[u] * a.nt + ti : ti * a.nt + tj[u];
+        const double ri2 = 1.0 / r2, ri6 = ri2 * ri2 * ri2;
+        e += 0.5 * (u12[p] * ri6 * ri6 - u6[p] * ri6 + 0.5 * a.cshift[p] * r2 - uc[p]);
+      }
     }
   }
-  __shared__ double red[kBlock];
-  red[threadIdx.x] = e;
+  __shared__ double red[kBlock / 64];
+  for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
   __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-int launch_energy_lj(cav_ctx *c, double *e)
+// Leaves the energy in scal[1].
+int launch_energy_lj(cav_ctx *c)
 {
-  CAV_TRY(launch_nl_fill(c));
-  const int nt2 = c->nt * c->nt;
-  PairArgs a = pair_args(c);
-  k_energy_lj<<<grid_for(c->n), kBlock, 0, c->stream>>>(a, c->d_eps + 3 * nt2, c->d_eps + 4 * nt2,
-                                                        c->d_eps + 5 * nt2, c->part);
-  CAV_TRY(reduce_partials(c, grid_for(c->n), 1));
-  CAV_HIP(hipMemcpyAsync(e, c->scal + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
-  return CAV_OK;
+  const bool slots = sorted_rows(c);
+  if (!slots) CAV_TRY(launch_nl_fill(c));
+  CAV_TRY(launch_pack(c));
+  const int nt2 = c->nt * c->nt, g = pair_grid(c);
+  if (g > c->npart) return fail(c, CAV_ERR_STATE, "partial-sum buffer smaller than the pair grid");
+  k_energy_lj<<<g, kBlock, 0, c->stream>>>(pair_args(c), slots ? c->nlb : c->nl,
+                                           slots ? c->litems : nullptr, c->d_eps + 3 * nt2,
+                                           c->d_eps + 4 * nt2, c->d_eps + 5 * nt2, c->part);
+  CAV_HIP(hipGetLastError());
+  return reduce_partials(c, g, 1);
 }
 
 
