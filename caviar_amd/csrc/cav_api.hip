@@ -238,7 +238,7 @@ static void free_all(cav_ctx *c)
                   c->d_W,     c->kacc,      c->order,    c->ord_blk,  c->xq,
                   c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos, c->sk_sum,
                   c->binpos,  c->xqs,    c->tids,       c->nll,    c->nlb,    c->lstart, c->litems,
-                  c->ekx,     c->eky,    c->ekz,        c->part_k};
+                  c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_flags) (void)hipHostFree(c->h_flags);

@@ -457,6 +457,9 @@ struct FArgs {
   double c0, kxs, kys, kzs;  // C = 4 pi ke / V; 2 pi / l per axis
   double *ax, *ay, *az;
   double *out4;  // optional per-atom (fx, fy, fz, phi) without charge/mass
+  double *part;  // row splits: [slab * splits + split][4][n] sums, or nullptr
+  int rb_per;    // row blocks per split (blockIdx.y)
+  int slab;      // K slab of this launch
   // batched: per workgroup (first atom, end atom, -, replica), the replicas'
   // constants, and the operand stride (bytes) between replicas
   const int4 *items;
@@ -464,6 +467,14 @@ struct FArgs {
   long bm_stride;
 };
 
+// FP32 / FP64 force pass.  The matrix cores bound it where the chip is full
+// (N = 65536, kmax 12, FP64: 237 us = 40 TF/s of the 72.7 a large matrix
+// product reaches here; 268 us before).  The operand of the next row block
+// goes through registers: with direct-to-LDS copies in flight the compiler
+// waits for them before every LDS read, so nothing overlapped.  The phase
+// factors' loads are issued before the products, which cover their latency.
+// Small systems split the row blocks over blockIdx.y (force_splits), each
+// split writing its own sums.
 template <typename T, int KS, int NT>
 __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
 {
@@ -508,26 +519,56 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
     }
   }
   T fx[NT][4], fy[NT][4], fz[NT][4], ph[NT][4];
+  // records of the lane's atoms in the epilogue (atoms past the end read the
+  // last one; their sums are never written)
+  const Cx<T> *rec[NT][4];
 #pragma unroll
   for (int tau = 0; tau < NT; ++tau)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) fx[tau][e] = fy[tau][e] = fz[tau][e] = ph[tau][e] = 0;
+    for (int e = 0; e < 4; ++e) {
+      fx[tau][e] = fy[tau][e] = fz[tau][e] = ph[tau][e] = 0;
+      const long atom = base + tau * 16 + mfma_row<T>(lk, e);
+      rec[tau][e] = tab + (atom < a.n ? atom : a.n - 1) * a.TS;
+    }
 
   constexpr int VW = 16 / (int)sizeof(T);  // values per 16-byte vector
   typedef T Tvw __attribute__((ext_vector_type(VW)));
   const int nrb = a.Rpad >> 4;
+  const int rb0 = blockIdx.y * a.rb_per, rb1 = min(nrb, rb0 + a.rb_per);
   const int nks = a.nks;  // K-steps in use (<= KS)
-  const int blk_bytes = blk_elems * (int)sizeof(T);
-  // the operand of row block rb streams into LDS while rb-1 is multiplied
-  copy_to_lds_async(bm, smem_raw, blk_bytes, wave, nwaves, lane);
-  __builtin_amdgcn_s_waitcnt(0);
+  const int blk_vec = blk_elems / VW;  // 16-byte pieces of a row block's operand
+  // pieces per thread for the longest fragment stride of KS K-steps
+  constexpr int KSPM = (KS + VW - 1) / VW * VW + VW;
+  constexpr int PER = (4 * 64 * KSPM / VW + 64 * kWavesF - 1) / (64 * kWavesF);
+  const u4v *src = reinterpret_cast<const u4v *>(bm) + (size_t)rb0 * blk_vec;
+  u4v *dst = reinterpret_cast<u4v *>(smem_raw);
+  for (int idx = threadIdx.x; idx < blk_vec; idx += 64 * kWavesF) dst[idx] = src[idx];
   __syncthreads();
-  for (int rb = 0; rb < nrb; ++rb) {
-    const int cur = rb & 1;
-    if (rb + 1 < nrb)
-      copy_to_lds_async(bm + (size_t)(rb + 1) * blk_bytes,
-                        smem_raw + (cur ^ 1) * blk_bytes, blk_bytes, wave, nwaves,
-                        lane);
+  // lattice row of the lane, r = rb*16 + l%16 = nxi nY + nyi; rows past R have
+  // zero operands and read the phase factors of row 0, so they add nothing
+  int nxi = (rb0 * 16 + lr) / a.nY, nyi = (rb0 * 16 + lr) % a.nY;
+  for (int rb = rb0; rb < rb1; ++rb) {
+    const int cur = (rb - rb0) & 1;
+    const bool more = rb + 1 < rb1;
+    u4v pf[PER];
+    if (more) {
+      src += blk_vec;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int idx = threadIdx.x + k * (64 * kWavesF);
+        if (idx < blk_vec) pf[k] = src[idx];
+      }
+    }
+    const bool rin = rb * 16 + lr < a.R;
+    const int rx = rin ? nxi : 0, ry = rin ? nyi : 0;
+    Cx<T> X[NT][4], Y[NT][4];
+#pragma unroll
+    for (int tau = 0; tau < NT; ++tau)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        X[tau][e] = rec[tau][e][rx];
+        Y[tau][e] = rec[tau][e][offY + ry];
+      }
     V acc[4][NT];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -554,29 +595,34 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
       }
     }
     // epilogue: lane holds rows r = rb*16 + l%16 for atoms mfma_row(l/16, e) of each tile
-    const int r = rb * 16 + lr;
-    if (r < a.R) {
-      const int nxi = r / a.nY, nyi = r - (r / a.nY) * a.nY;
-      const T wx = (T)nxi, wy = (T)(nyi - a.ky);
+    const T wx = (T)rx, wy = (T)(ry - a.ky);
 #pragma unroll
-      for (int tau = 0; tau < NT; ++tau)
+    for (int tau = 0; tau < NT; ++tau)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const long atom = base + tau * 16 + mfma_row<T>(lk, e);
-          if (atom >= a.n) continue;
-          const Cx<T> X = tab[atom * a.TS + nxi], Y = tab[atom * a.TS + offY + nyi];
-          const T pr = X.re * Y.re - X.im * Y.im;
-          const T pi = X.re * Y.im + X.im * Y.re;
-          const T ur = acc[0][tau][e], ui = acc[1][tau][e];
-          const T uzr = acc[2][tau][e], uzi = acc[3][tau][e];
-          const T h = pr * ui + pi * ur;
-          fx[tau][e] += wx * h;
-          fy[tau][e] += wy * h;
-          fz[tau][e] += pr * uzi + pi * uzr;
-          ph[tau][e] += pr * ur - pi * ui;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const T pr = X[tau][e].re * Y[tau][e].re - X[tau][e].im * Y[tau][e].im;
+        const T pi = X[tau][e].re * Y[tau][e].im + X[tau][e].im * Y[tau][e].re;
+        const T ur = acc[0][tau][e], ui = acc[1][tau][e];
+        const T uzr = acc[2][tau][e], uzi = acc[3][tau][e];
+        const T h = pr * ui + pi * ur;
+        fx[tau][e] += wx * h;
+        fy[tau][e] += wy * h;
+        fz[tau][e] += pr * uzi + pi * uzr;
+        ph[tau][e] += pr * ur - pi * ui;
+      }
+    nyi += 16;
+    while (nyi >= a.nY) {
+      nyi -= a.nY;
+      ++nxi;
     }
-    __builtin_amdgcn_s_waitcnt(0);
+    if (more) {
+      u4v *nxt = dst + (cur ^ 1) * blk_vec;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int idx = threadIdx.x + k * (64 * kWavesF);
+        if (idx < blk_vec) nxt[idx] = pf[k];
+      }
+    }
     __syncthreads();
   }
   // reduce over the 16 lanes that share l/16 (they hold different rows)
@@ -595,7 +641,13 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
       const long atom = base + tau * 16 + mfma_row<T>(lk, e);
       if (lr == 0 && atom < a.n) {
         const double gx = a.c0 * a.kxs * vx, gy = a.c0 * a.kys * vy, gz = a.c0 * a.kzs * vz;
-        if (a.out4 && a.out4_add) {
+        if (a.part) {
+          double *p = a.part + ((long)a.slab * gridDim.y + blockIdx.y) * 4 * a.n + atom;
+          p[0] = gx;
+          p[a.n] = gy;
+          p[2L * a.n] = gz;
+          p[3L * a.n] = a.c0 * vp;
+        } else if (a.out4 && a.out4_add) {
           a.out4[4 * atom + 0] += gx;
           a.out4[4 * atom + 1] += gy;
           a.out4[4 * atom + 2] += gz;
@@ -613,6 +665,52 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
         }
       }
     }
+}
+
+// The row splits' sums of a force pass ([part][4][n], the split form without
+// the potential), added in order, one thread per (atom, component blockIdx.y):
+// into out4, or into the accelerations times q (nullptr where the sums carry
+// the charge) and 1/m.
+__global__ void k_kforce_sum(int n, int nparts, const double *part, const double *q,
+                             const double *minv, const int *type, double *ax, double *ay,
+                             double *az, double *out4)
+{
+  const int i = blockIdx.x * kBlock + threadIdx.x, d = blockIdx.y;
+  if (i >= n) return;
+  const double *p = part + (long)d * n + i;
+  double v = 0;
+#pragma unroll 8
+  for (int s = 0; s < nparts; ++s) v += p[(long)s * 4 * n];
+  if (out4) {
+    out4[4L * i + d] = v;
+  } else {
+    double *a = d == 0 ? ax : (d == 1 ? ay : az);
+    a[i] += v * (q ? q[i] * minv[type[i]] : minv[type[i]]);
+  }
+}
+
+// Row splits of a force pass of g workgroups and nrb row blocks.  A workgroup
+// takes a CU to itself, so g of them run in ceil(g / 256) rounds of nrb row
+// blocks (and about kForceSetup row blocks' time for its fragments and first
+// operand), and below 256, or just past a multiple of it, CUs idle: more,
+// shorter workgroups are taken where that model saves more than the summing
+// launch costs.
+// Measured: 8000 atoms, kmax 8, FP64 (63 workgroups of 10 row blocks) 42 ->
+// 19 + 4 us; 100 atoms, kmax 25 (one workgroup of 83) 595 -> 40 + 13 us;
+// 30011 atoms, kmax 10, split form (118 of 15) 35 -> 25 + 4 us; 65536 and
+// more atoms fill the chip and stay unsplit.
+constexpr int kForceSetup = 2, kForceSplitMax = 64;
+
+static int force_splits(int g, int nrb)
+{
+  auto cost = [&](int ns) {
+    const long rounds = ((long)g * ns + 255) / 256;
+    return rounds * ((nrb + ns - 1) / ns + kForceSetup);
+  };
+  int best = 1;
+  for (int ns = 2; ns <= nrb && ns <= kForceSplitMax; ++ns)
+    if (cost(ns) + 1 < cost(best)) best = ns;
+  return best;
 }
 
 
@@ -969,6 +1067,8 @@ struct FArgsH {
   const int *type;
   double c0, kxs, kys, kzs;  // c0 includes 1/(sA sB): X carries q sA, the operand sB
   double *ax, *ay, *az;
+  double *part;       // row splits, as FArgs (without the potential)
+  int rb_per;
   const int4 *items;  // batched, as FArgs
   const RepDev *rep;
   long bm_stride;
@@ -1074,20 +1174,21 @@ __global__ __launch_bounds__(64 * W) void k_kforce_h(FArgsH a)
   // lattice row of the lane, r = rb*16 + l%16 = nxi nY + nyi, kept incrementally;
   // rows past R have zero operands (U = 0) and read the phase factors of row 0
   // (finite), so they add exactly nothing
-  int nxi = lr / a.nY, nyi = lr % a.nY;
-
   const int nrb = a.Rpad >> 4;
-  copy_to_lds_async(bm, smem_raw + xy_bytes, blk_bytes, wave, nwaves, lane);
+  const int rb0 = blockIdx.y * a.rb_per, rb1 = min(nrb, rb0 + a.rb_per);
+  int nxi = (rb0 * 16 + lr) / a.nY, nyi = (rb0 * 16 + lr) % a.nY;
+
+  copy_to_lds_async(bm + (size_t)rb0 * blk_bytes, smem_raw + xy_bytes, blk_bytes, wave, nwaves, lane);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  for (int rb = 0; rb < nrb; ++rb) {
-    const int cur = rb & 1;
+  for (int rb = rb0; rb < rb1; ++rb) {
+    const int cur = (rb - rb0) & 1;
     // The next row block's operand (CH = 512 NK pieces of 16 B) is fetched
     // into registers here and stored to the other LDS buffer after this block
     // is consumed: with no LDS write in flight, reads of the current block
     // need no wait on the prefetch.
     constexpr int CH = split_blk_bytes(NK) / 16, PER = (CH + 64 * W - 1) / (64 * W);
-    const bool more = rb + 1 < nrb;
+    const bool more = rb + 1 < rb1;
     u4v pf[PER];
     if (more) {
       const u4v *src = reinterpret_cast<const u4v *>(bm + (size_t)(rb + 1) * blk_bytes);
@@ -1193,6 +1294,13 @@ __global__ __launch_bounds__(64 * W) void k_kforce_h(FArgsH a)
       const long atom = base + tau * 16 + 4 * lk + e;
       if (lr == 0 && atom < a.n) {
         const double gx = a.c0 * a.kxs * vx, gy = a.c0 * a.kys * vy, gz = a.c0 * a.kzs * vz;
+        if (a.part) {
+          double *p = a.part + (long)blockIdx.y * 4 * a.n + atom;
+          p[0] = gx;
+          p[a.n] = gy;
+          p[2L * a.n] = gz;
+          continue;
+        }
         // the phase factors carry the atom's charge (times sA, removed in c0)
         const double m = a.minv[a.type[atom]];
         a.ax[atom] += gx * m;
@@ -1439,6 +1547,31 @@ static int s_chunk(const cav_ctx *c, int ntarget)
   return (int)per;
 }
 
+// The row splits' sums: at least `count` doubles in c->kf_part.
+static int force_parts(cav_ctx *c, size_t count)
+{
+  if (count <= c->kf_cap) return CAV_OK;
+  if (c->kf_part) (void)hipFree(c->kf_part);
+  c->kf_part = nullptr;
+  c->kf_cap = 0;
+  CAV_HIP(hipMalloc(&c->kf_part, sizeof(double) * count));
+  c->kf_cap = count;
+  return CAV_OK;
+}
+
+// Splits of a force pass of npts points in workgroups of `wg`, as the passes
+// below take them: row blocks per split and splits with work.
+static int force_layout(const EwaldKPlan &p, long npts, int wg, int *rb_per)
+{
+  const int nrb = p.Rpad / 16, ns = force_splits((int)((npts + wg - 1) / wg), nrb);
+  *rb_per = (nrb + ns - 1) / ns;
+  return (nrb + *rb_per - 1) / *rb_per;
+}
+
+// Atom tiles per force-pass wave: two in FP32 (operand reuse), one in FP64
+// (keeps the kernel at 2+ waves per SIMD).
+template <typename T> constexpr int kforce_nt() { return sizeof(T) == 8 ? 1 : 2; }
+
 int ewald_k_alloc(cav_ctx *c)
 {
   const EwaldKPlan &p = c->ek;
@@ -1480,6 +1613,12 @@ int ewald_k_alloc(cav_ctx *c)
     const size_t bh_elems = (size_t)(p.Rpad / 16) * (split_blk_bytes(c->nkh) / 2);
     CAV_HIP(hipMalloc(&c->bmat_h, bh_elems * sizeof(_Float16)));
     k_zero_t<_Float16><<<grid_for(bh_elems), kBlock, 0, c->stream>>>(bh_elems, (_Float16 *)c->bmat_h);
+  }
+  {  // the force passes' row splits: the FP32 / FP64 tiles and the split form's
+    int per, ns = p.nslab * force_layout(p, c->n, 16 * kWavesF * (tsz == 8 ? 1 : 2), &per);
+    if (c->precision == CAV_MIXED)
+      ns = std::max(ns, force_layout(p, c->n, 16 * c->tune_fnt * c->tune_fw, &per));
+    if (ns > 1) CAV_TRY(force_parts(c, (size_t)ns * 4 * c->n));
   }
   if (c->d_W) (void)hipFree(c->d_W);
   CAV_HIP(hipMalloc(&c->d_W, sizeof(double) * (size_t)p.R * p.nZ));
@@ -1527,15 +1666,12 @@ static void launch_sk_rt(hipStream_t st, SArgs a, dim3 lgrid, size_t smem, int S
   }
 }
 
-// Atom tiles per force-pass wave: two in FP32 (operand reuse), one in FP64
-// (keeps the kernel at 2+ waves per SIMD).
-template <typename T> constexpr int kforce_nt() { return sizeof(T) == 8 ? 1 : 2; }
-
 // The force pass, one launch per K slab (one for nz axes of up to 128 kappa);
 // `a.bm` is the first slab's operand, the others follow it.
 template <typename T>
-static void launch_kforce_t(hipStream_t st, FArgs a, const EwaldKPlan &p, int g)
+static void launch_kforce_t(hipStream_t st, FArgs a, const EwaldKPlan &p, int groups, int splits)
 {
+  const dim3 g(groups, splits);
   constexpr int NT = kforce_nt<T>();
   const size_t smem = 2 * (size_t)4 * 64 * a.KSP * sizeof(T);
   const int KS = p.KSS, nks = p.KZ / 4;
@@ -1544,6 +1680,7 @@ static void launch_kforce_t(hipStream_t st, FArgs a, const EwaldKPlan &p, int g)
     a.s0 = sl * p.KSS;
     a.nks = std::min(p.KSS, nks - a.s0);
     a.out4_add = sl > 0;
+    a.slab = sl;
     a.bm = bm0 + sl * slab_elems(p) * sizeof(T);
     if (KS <= 8) {
       allow_smem(k_kforce<T, 8, NT>, smem);
@@ -1645,7 +1782,17 @@ static int kforce(cav_ctx *c, int npts, const void *tab, double *out4)
   f.bm_stride = 0;
   timer_begin(c, c->t_force);
   constexpr int NT = kforce_nt<T>();
-  launch_kforce_t<T>(c->stream, f, p, (npts + 16 * NT * kWavesF - 1) / (16 * NT * kWavesF));
+  const int g = (npts + 16 * NT * kWavesF - 1) / (16 * NT * kWavesF);
+  const int used = force_layout(p, npts, 16 * NT * kWavesF, &f.rb_per);
+  f.part = nullptr;
+  if (used > 1) {
+    CAV_TRY(force_parts(c, (size_t)p.nslab * used * 4 * npts));
+    f.part = c->kf_part;
+  }
+  launch_kforce_t<T>(c->stream, f, p, g, used);
+  if (used > 1)
+    k_kforce_sum<<<dim3(grid_for(npts), out4 ? 4 : 3), kBlock, 0, c->stream>>>(
+        npts, p.nslab * used, f.part, f.q, f.minv, f.type, f.ax, f.ay, f.az, out4);
   timer_end(c, c->t_force);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -1763,8 +1910,10 @@ static bool split_fits(const EwaldKPlan &p, int nkh, int nt, int w)
 }
 
 template <int NT, int W>
-static void launch_kforce_h(hipStream_t st, const FArgsH &f, int nkh, int g, size_t smem)
+static void launch_kforce_h(hipStream_t st, const FArgsH &f, int nkh, int groups, int splits,
+                            size_t smem)
 {
+  const dim3 g(groups, splits);
   switch (nkh) {
   case 1: allow_smem(k_kforce_h<1, NT, W>, smem); k_kforce_h<1, NT, W><<<g, 64 * W, smem, st>>>(f); break;
   case 2: allow_smem(k_kforce_h<2, NT, W>, smem); k_kforce_h<2, NT, W><<<g, 64 * W, smem, st>>>(f); break;
@@ -1806,17 +1955,26 @@ static int kforce_h(cav_ctx *c)
   const int NT = c->tune_fnt, W = c->tune_fw;
   const int g = (c->n + 16 * NT * W - 1) / (16 * NT * W);
   const size_t smem = split_force_lds(c);
+  const int used = force_layout(p, c->n, 16 * NT * W, &f.rb_per);
+  f.part = nullptr;
+  if (used > 1) {
+    CAV_TRY(force_parts(c, (size_t)used * 4 * c->n));
+    f.part = c->kf_part;
+  }
   timer_begin(c, c->t_force);
   if (W == 16) {
     if (NT == 1)
-      launch_kforce_h<1, 16>(c->stream, f, c->nkh, g, smem);
+      launch_kforce_h<1, 16>(c->stream, f, c->nkh, g, used, smem);
     else
-      launch_kforce_h<2, 16>(c->stream, f, c->nkh, g, smem);
+      launch_kforce_h<2, 16>(c->stream, f, c->nkh, g, used, smem);
   } else if (NT == 1) {
-    launch_kforce_h<1, kWavesF>(c->stream, f, c->nkh, g, smem);
+    launch_kforce_h<1, kWavesF>(c->stream, f, c->nkh, g, used, smem);
   } else {
-    launch_kforce_h<2, kWavesF>(c->stream, f, c->nkh, g, smem);
+    launch_kforce_h<2, kWavesF>(c->stream, f, c->nkh, g, used, smem);
   }
+  if (used > 1)
+    k_kforce_sum<<<dim3(grid_for(c->n), 3), kBlock, 0, c->stream>>>(
+        c->n, used, f.part, nullptr, f.minv, f.type, f.ax, f.ay, f.az, nullptr);
   timer_end(c, c->t_force);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -2311,7 +2469,9 @@ static int batch_ewald_k_t(cav_batch *b)
     f.items = b->f_items;
     f.rep = b->d_rep;
     f.bm_stride = b->bm_stride * (long)sizeof(T);
-    launch_kforce_t<T>(b->stream, f, p, b->n_fitems);
+    f.part = nullptr;
+    f.rb_per = p.Rpad / 16;
+    launch_kforce_t<T>(b->stream, f, p, b->n_fitems, 1);
   } else {
     FArgsH f;
     f.n = 0;
@@ -2337,10 +2497,12 @@ static int batch_ewald_k_t(cav_batch *b)
     f.rep = b->d_rep;
     f.bm_stride = b->bmh_stride * (long)sizeof(_Float16);
     f.inv_sb = 1.0 / b->sB / b->sA;
+    f.part = nullptr;
+    f.rb_per = p.Rpad / 16;
     if (b->f_nt == 1)
-      launch_kforce_h<1, kWavesF>(b->stream, f, b->nkh, b->n_fitems, split_force_lds_p(p, b->nkh, 1));
+      launch_kforce_h<1, kWavesF>(b->stream, f, b->nkh, b->n_fitems, 1, split_force_lds_p(p, b->nkh, 1));
     else
-      launch_kforce_h<2, kWavesF>(b->stream, f, b->nkh, b->n_fitems, split_force_lds_p(p, b->nkh, 2));
+      launch_kforce_h<2, kWavesF>(b->stream, f, b->nkh, b->n_fitems, 1, split_force_lds_p(p, b->nkh, 2));
   }
   BAT_HIP(hipGetLastError());
   return CAV_OK;
@@ -2395,7 +2557,9 @@ static int batch_field_t(cav_batch *b, double *out4)
   f.items = b->f_items;
   f.rep = b->d_rep;
   f.bm_stride = b->bm_stride * (long)sizeof(T);
-  launch_kforce_t<T>(b->stream, f, p, b->n_fitems);
+  f.part = nullptr;
+  f.rb_per = p.Rpad / 16;
+  launch_kforce_t<T>(b->stream, f, p, b->n_fitems, 1);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }

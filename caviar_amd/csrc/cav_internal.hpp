@@ -257,6 +257,8 @@ struct cav_ctx {
   bool nlb_built = false, nlb_pending = false;
   bool tuned = false;
   double *d_W = nullptr;     // [Rpad][nZ]
+  double *kf_part = nullptr; // row splits' sums of the force pass
+  size_t kf_cap = 0;
   double *kacc = nullptr;    // per-atom k-space (fx, fy, fz, phi) scratch for point queries
 
   bool setup_done = false;

@@ -41,3 +41,29 @@ def test_cell_walk_energies_and_points(gpu, n, rho, coef, pair_kernel):
         fo, po = o.point_r(pts)
         assert F.rel_err(f, fo) <= 1e-12
         assert F.rel_err(p, po) <= 1e-12
+
+
+@pytest.mark.parametrize("n,k", [(1, (1, 1, 1)), (127, (2, 3, 4)), (129, (9, 9, 9)), (300, (25, 25, 25)),
+                                 (900, (3, 3, 40)), (4100, (6, 6, 6))])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_force_pass_row_splits(gpu, n, k, precision):
+    """Lattice forces and point fields where the row blocks of the force pass
+    are split over workgroups (few atoms, long lattices, two K slabs), against
+    the oracle.  Mixed: 32-bit sums, 1e-5 of the force RMS."""
+    print(f"[case] force splits n={n} k={k} {precision}", flush=True)
+    s = configs.ions(n=n, rho=0.3 if n > 1 else 0.01, kmax=1, seed=n, with_lj=False, with_r=False)
+    s.neighbor = None
+    s.ewald_k.kx_max, s.ewald_k.ky_max, s.ewald_k.kz_max = k
+    o = Oracle(s)
+    o.setup()
+    e = Engine(s, precision=precision)
+    e.setup()
+    tol = 1e-12 if precision == "fp64" else 1e-5
+    a = o.get("acc")
+    if n > 1:
+        assert F.rel_err(e.get("acc"), a) <= tol
+    pts = np.random.default_rng(1).uniform(s.lower, s.upper, (131, 3))
+    f, p = e.point_field("k", pts)
+    fo, po = o.point_k(pts)
+    assert F.rel_err(f, fo) <= tol
+    assert F.rel_err(p, po) <= tol
