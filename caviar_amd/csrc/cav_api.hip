@@ -49,114 +49,59 @@ static void timer_harvest(Timer &t)
 
 // ------------------------------------------------------- integration kernels --
 
-// integrate_velocity_verlet drift (md_simulator.cpp:584-594) with the PBC wrap
-// of exchange_owned fused in (domain.cpp:418-468).  Every operation is
-// rounded as the reference's expression is: r += (v*dt + ((0.5*a)*dt)*dt).
-// snap (or nullptr): the step snapshot of the owned positions, velocities and
-// accelerations before the drift ([x | y | z | vx | vy | vz | ax | ay | az],
-// n each), written from the values the drift reads anyway.
-__global__ void k_drift(int n, double dt, const double *lo, const double *hi, const double *L,
-                        int bx, int by, int bz, double *x, double *y, double *z, const double *vx,
-                        const double *vy, const double *vz, const double *ax, const double *ay,
-                        const double *az, double *aox, double *aoy, double *aoz, int *flags,
-                        double *snap)
+// The end of a velocity-Verlet step: v += (0.5*dt) * (a + a_old)
+// (md_simulator.cpp:610-617); JOIN: first a += ek, the k-space accelerations of
+// a concurrent Ewald_k (the single addition the in-order schedule makes).
+// Workgroup 0 also sums the pair kernel's virial partials (nvir of them, as
+// k_reduce_part does) and, for steps queued without a host check between
+// them, closes the step's flags: a failed one stops those behind it.  Both
+// were launches of their own, 3-7 us each.
+template <bool JOIN>
+__global__ __launch_bounds__(kBlock) void k_kick(int n, double hdt, double *vx, double *vy,
+                                                 double *vz, double *ax, double *ay, double *az,
+                                                 const double *ekx, const double *eky,
+                                                 const double *ekz, const double *aox,
+                                                 const double *aoy, const double *aoz,
+                                                 const double *part, int nvir, double *virial,
+                                                 int *flags, int queued)
 {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const double a[3] = {ax[i], ay[i], az[i]};
-  if (isnan(a[0]) || isnan(a[1]) || isnan(a[2])) flags[F_NAN] = 1;
-  const double v[3] = {vx[i], vy[i], vz[i]};
-  double *p[3] = {x + i, y + i, z + i};
-  if (snap) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      snap[(long)d * n + i] = *p[d];
-      snap[(long)(3 + d) * n + i] = v[d];
-      snap[(long)(6 + d) * n + i] = a[d];
+  if (i < n) {
+    double a[3] = {ax[i], ay[i], az[i]};
+    if constexpr (JOIN) {
+      a[0] = xadd(a[0], ekx[i]);
+      a[1] = xadd(a[1], eky[i]);
+      a[2] = xadd(a[2], ekz[i]);
+      ax[i] = a[0];
+      ay[i] = a[1];
+      az[i] = a[2];
+    }
+    vx[i] = xadd(vx[i], xmul(hdt, xadd(a[0], aox[i])));
+    vy[i] = xadd(vy[i], xmul(hdt, xadd(a[1], aoy[i])));
+    vz[i] = xadd(vz[i], xmul(hdt, xadd(a[2], aoz[i])));
+  }
+  if (blockIdx.x != 0) return;
+  if (nvir > 0) {
+    __shared__ double red[kBlock];
+    double s = 0;
+    for (int k = threadIdx.x; k < nvir; k += kBlock) s += part[k];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+      if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *virial = red[0];
+  }
+  if (queued && threadIdx.x == 0 && !flags[F_STOP]) {
+    if (flags[F_NAN] || flags[F_OVERFLOW]) {
+      flags[F_STOP] = 1;
+    } else {
+      flags[F_WRAPPED] = 0;
+      flags[F_REBUILD] = 0;
+      flags[F_STEPS] += 1;
     }
   }
-  const int b[3] = {bx, by, bz};
-  bool wrapped = false;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double h = xmul(xmul(xmul(0.5, a[d]), dt), dt);
-    double r = xadd(*p[d], xadd(xmul(v[d], dt), h));
-    if (b[d] == 1) {
-      if (r < lo[d]) {
-        r = xadd(r, L[d]);
-        wrapped = true;
-      } else if (r > hi[d]) {
-        r = xsub(r, L[d]);
-        wrapped = true;
-      }
-    }
-    *p[d] = r;
-  }
-  aox[i] = a[0];
-  aoy[i] = a[1];
-  aoz[i] = a[2];
-  if (wrapped) {
-    flags[F_WRAPPED] = 1;
-    flags[F_REBUILD] = 1;
-  }
-}
-
-// exchange_owned_single_md_domain alone (setup and recalculate).
-__global__ void k_wrap(int n, const double *lo, const double *hi, const double *L, int bx, int by,
-                       int bz, double *x, double *y, double *z, int *flags)
-{
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  double *p[3] = {x + i, y + i, z + i};
-  const int b[3] = {bx, by, bz};
-  bool wrapped = false;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    if (b[d] != 1) continue;
-    double r = *p[d];
-    if (r < lo[d]) {
-      r = xadd(r, L[d]);
-      wrapped = true;
-    } else if (r > hi[d]) {
-      r = xsub(r, L[d]);
-      wrapped = true;
-    }
-    *p[d] = r;
-  }
-  if (wrapped) {
-    flags[F_WRAPPED] = 1;
-    flags[F_REBUILD] = 1;
-  }
-}
-
-// v += (0.5*dt) * (a + a_old)  (md_simulator.cpp:610-617)
-__global__ void k_kick(int n, double hdt, double *vx, double *vy, double *vz, const double *ax,
-                       const double *ay, const double *az, const double *aox, const double *aoy,
-                       const double *aoz)
-{
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  vx[i] = xadd(vx[i], xmul(hdt, xadd(ax[i], aox[i])));
-  vy[i] = xadd(vy[i], xmul(hdt, xadd(ay[i], aoy[i])));
-  vz[i] = xadd(vz[i], xmul(hdt, xadd(az[i], aoz[i])));
-}
-
-// The kick after a concurrent Ewald_k: first a += ek (the k-space
-// accelerations, the single addition the in-order schedule makes), then the kick.
-__global__ void k_kick_join(int n, double hdt, double *vx, double *vy, double *vz, double *ax,
-                            double *ay, double *az, const double *ekx, const double *eky,
-                            const double *ekz, const double *aox, const double *aoy,
-                            const double *aoz)
-{
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const double a[3] = {xadd(ax[i], ekx[i]), xadd(ay[i], eky[i]), xadd(az[i], ekz[i])};
-  ax[i] = a[0];
-  ay[i] = a[1];
-  az[i] = a[2];
-  vx[i] = xadd(vx[i], xmul(hdt, xadd(a[0], aox[i])));
-  vy[i] = xadd(vy[i], xmul(hdt, xadd(a[1], aoy[i])));
-  vz[i] = xadd(vz[i], xmul(hdt, xadd(a[2], aoz[i])));
 }
 
 // a += e per component, one rounded addition (the concurrent Ewald_k's join).
@@ -170,10 +115,13 @@ __global__ void k_add3(int n, double *ax, double *ay, double *az, const double *
   az[i] = xadd(az[i], ez[i]);
 }
 
-__global__ void k_begin_step(int *flags)
+// force: the list is rebuilt whatever the displacements
+__global__ void k_begin_step(int *flags, int force)
 {
   flags[F_WRAPPED] = 0;
-  flags[F_REBUILD] = flags[F_FORCE];
+  flags[F_REBUILD] = force || flags[F_FORCE] ? 1 : 0;
+  flags[F_STOP] = 0;
+  flags[F_STEPS] = 0;
   flags[F_FORCE] = 0;
   flags[F_NAN] = 0;
   flags[F_OVERFLOW] = 0;
@@ -238,14 +186,12 @@ static void free_all(cav_ctx *c)
                   c->d_W,     c->kacc,      c->order,    c->ord_blk,  c->xq,
                   c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos, c->sk_sum,
                   c->binpos,  c->xqs,    c->tids,       c->nll,    c->nlb,    c->lstart, c->litems,
-                  c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part};
+                  c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part,
+                  c->cell_cnt, c->bucket};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_flags) (void)hipHostFree(c->h_flags);
 }
-
-// box arrays on the device (lo, hi, L) live in the scalar buffer tail
-static const int kBoxSlot = 16;
 
 static int upload_params(cav_ctx *c)
 {
@@ -429,14 +375,6 @@ static int sync_flags(cav_ctx *c)
   return CAV_OK;
 }
 
-static int box_dev(cav_ctx *c, const double **lo, const double **hi, const double **L)
-{
-  *lo = c->scal + kBoxSlot;
-  *hi = c->scal + kBoxSlot + 3;
-  *L = c->scal + kBoxSlot + 6;
-  return CAV_OK;
-}
-
 // New parameter values (same structure) set after setup: upload them, refresh
 // the per-atom charges of owned atoms and of the current ghosts (a force call
 // without a new exchange reads the ghosts' charges: the reference reads
@@ -501,8 +439,9 @@ static int ewald_k_join(cav_ctx *c)
 
 // The force phase: reset acceleration + every enabled field (md_simulator.cpp:370-373).
 // `kspace` false leaves Ewald_k to the concurrent side stream.
-static int forces(cav_ctx *c, bool kspace = true);
-static int neighbor_phase(cav_ctx *c, bool forced);
+static int forces(cav_ctx *c, bool kspace = true, bool packed = false, bool sum_virial = true);
+enum class Rebuild { forced, test, decided };
+static int neighbor_phase(cav_ctx *c, Rebuild how, bool fused);
 
 // The autotuner's unit of work: the Ewald_k passes as cav_step runs them,
 // i.e. on the side stream concurrently with a list build and the pair kernel
@@ -512,16 +451,18 @@ int cav::tuning_phase(cav_ctx *c)
 {
   if (!(c->overlap && c->n > 0)) return launch_ewald_k(c);
   CAV_TRY(ewald_k_fork(c));
-  CAV_TRY(neighbor_phase(c, true));
+  CAV_TRY(neighbor_phase(c, Rebuild::forced, false));
   CAV_TRY(forces(c, false));
   return ewald_k_join(c);
 }
 int forces_all(cav_ctx *c) { return forces(c); }
-static int forces(cav_ctx *c, bool kspace)
+// packed: the gathers' copies are current; sum_virial: false leaves the pair
+// kernel's virial partials to the kick.
+static int forces(cav_ctx *c, bool kspace, bool packed, bool sum_virial)
 {
   const bool pair = (c->lj_on && !c->lj_cellwalk) || c->er_on;
   if (pair)
-    CAV_TRY(launch_pairs(c, true, true, false));
+    CAV_TRY(launch_pairs(c, true, true, false, packed, sum_virial));
   else
     CAV_TRY(launch_zero_acc(c));
   if (c->lj_on && c->lj_cellwalk) CAV_TRY(launch_lj_cellwalk(c));
@@ -531,27 +472,31 @@ static int forces(cav_ctx *c, bool kspace)
   return CAV_OK;
 }
 
-// Neighbour phase for one step: ghosts already made; rebuild decision, cells,
-// list, old positions.  `forced` requests an unconditional rebuild.
-static int neighbor_phase(cav_ctx *c, bool forced)
+// Neighbour phase: ghosts already made; rebuild decision, cells, list, old
+// positions.  `how`: an unconditional rebuild, the rebuild test first, or a
+// decision already taken with the ghosts.  `fused`: launch_move and
+// launch_ghosts have just run and left the cells' counts and buckets.
+static int neighbor_phase(cav_ctx *c, Rebuild how, bool fused)
 {
   if (!c->nl_on) return CAV_OK;
-  if (forced) {
+  if (how == Rebuild::forced)
     k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_REBUILD, 1);
-  } else {
+  else if (how == Rebuild::test)
     CAV_TRY(launch_rebuild_check(c));
-  }
   timer_begin(c, c->t_nb);
   // cells are needed on rebuild steps, and every step by the LJ cell walk
-  CAV_TRY(launch_bins(c, !c->lj_cellwalk, true));
+  if (fused)
+    CAV_TRY(launch_cells(c));
+  else
+    CAV_TRY(launch_bins(c, !c->lj_cellwalk, true));
   timer_end(c, c->t_nb);
   timer_begin(c, c->t_list);
   CAV_TRY(launch_list(c, true));
-  if (forced) {  // the build is known to run
+  if (how == Rebuild::forced) {  // the build is known to run
     c->nll_built = c->nll_pending;
     c->nlb_built = c->nlb_pending;
   }
-  CAV_TRY(launch_save_old(c, true));
+  if (!fused) CAV_TRY(launch_save_old(c, true));
   timer_end(c, c->t_list);
   return CAV_OK;
 }
@@ -1070,14 +1015,20 @@ int cav_upload(cav_ctx *c, int which, const double *in)
   return CAV_OK;
 }
 
-static int wrap_and_ghosts(cav_ctx *c)
+// exchange_owned and exchange_ghost, the list (rebuilt or by the test), and
+// the forces of the current positions.
+static int evaluate(cav_ctx *c, bool rebuild)
 {
-  const double *lo, *hi, *L;
-  box_dev(c, &lo, &hi, &L);
-  k_wrap<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, lo, hi, L, c->bc[0], c->bc[1], c->bc[2],
-                                                   c->x, c->y, c->z, c->flags);
-  CAV_HIP(hipGetLastError());
-  return launch_ghosts(c);
+  const bool fused = fused_cells(c);
+  k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, rebuild ? 1 : 0);
+  CAV_TRY(launch_move(c, false, 0, true));
+  CAV_TRY(launch_ghosts(c, true));
+  CAV_TRY(neighbor_phase(c, Rebuild::decided, fused));
+  if (rebuild) {  // the build is known to run
+    c->nll_built = c->nll_pending;
+    c->nlb_built = c->nlb_pending;
+  }
+  return forces(c, true, fused);
 }
 
 int cav_setup(cav_ctx *c)
@@ -1089,16 +1040,9 @@ int cav_setup(cav_ctx *c)
     return fail(c, CAV_ERR_STATE, "lj_cell_list / lj / ewald_r / short_range need a neighborlist");
   if (c->lj_on && !c->build_cells) return fail(c, CAV_ERR_STATE, "lj_cell_list needs build_cell_list");
   (void)hipSetDevice(c->device);
-  // box on the device (lo, hi, L)
-  double box[9];
-  for (int d = 0; d < 3; ++d) {
-    box[d] = c->lo[d];
-    box[3 + d] = c->hi[d];
-    box[6 + d] = c->L[d];
-  }
-  CAV_HIP(hipMemcpy(c->scal + kBoxSlot, box, sizeof(box), hipMemcpyHostToDevice));
   CAV_TRY(upload_params(c));
   CAV_TRY(neighbor_init(c));
+  CAV_TRY(cells_alloc(c));
   // LJ over the list needs rc_lj <= the list's own cutoff (the skin guarantee of
   // the rebuild test); otherwise it walks the cells every step like the reference.
   c->lj_cellwalk = c->lj_on && (c->lj_rc > c->nl_cutoff || c->all_atom_test);
@@ -1145,10 +1089,7 @@ int cav_setup(cav_ctx *c)
   k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_NGHOST_OLD, -1);
   for (int attempt = 0; attempt < 4; ++attempt) {
     if (attempt) CAV_TRY(elc_rewind(c));  // the retried evaluation is the same one
-    k_begin_step<<<1, 1, 0, c->stream>>>(c->flags);
-    CAV_TRY(wrap_and_ghosts(c));
-    CAV_TRY(neighbor_phase(c, true));
-    CAV_TRY(forces(c));
+    CAV_TRY(evaluate(c, true));
     CAV_TRY(sync_flags(c));
     bool redo = false;
     CAV_TRY(check_capacity(c, &redo));
@@ -1162,65 +1103,116 @@ int cav_setup(cav_ctx *c)
   return CAV_OK;
 }
 
+// The launches of one step at Md_simulator::current_step `ts`.  queued: no
+// host check follows (see run_queued).
+static int issue_step(cav_ctx *c, double dt, long ts, bool queued)
+{
+  const bool fused = fused_cells(c);
+  // the step snapshot (restored on NaN or overflow) is written by the drift
+  timer_begin(c, c->t_int);
+  CAV_TRY(launch_move(c, true, dt, true));
+  timer_end(c, c->t_int);
+  const bool side = c->overlap && c->ek_on && c->n > 0;
+  if (side) CAV_TRY(ewald_k_fork(c));
+  CAV_TRY(launch_ghosts(c, true));
+  CAV_TRY(neighbor_phase(c, Rebuild::decided, fused));
+  // the virial partials keep until the kick unless a later field writes its
+  // own into the same buffer
+  const bool pair = (c->lj_on && !c->lj_cellwalk) || c->er_on;
+  const bool late = pair && !c->ljl_on && !c->sr_on && !c->elc_on && !c->dipole &&
+                    (side || !c->ek_on) && !cell_staged(c);
+  CAV_TRY(forces(c, !side, fused, !late));
+  bool join = side;
+  if (side) {
+    CAV_TRY(ewald_k_join(c));
+    if (c->dipole || c->elc_on) {
+      // a = ((a_sr + a_k) + a_dip) + a_elc, as in order: add, dipole, slab
+      // correction, then the kick
+      k_add3<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->ax, c->ay, c->az, c->ekx, c->eky,
+                                                       c->ekz);
+      if (c->dipole) CAV_TRY(launch_dipole(c));
+      if (c->elc_on) CAV_TRY(launch_elc(c));
+      join = false;
+    }
+  }
+  const int nvir = late ? pair_blocks(c) : 0;
+  const auto kick = join ? k_kick<true> : k_kick<false>;
+  kick<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, 0.5 * dt, c->vx, c->vy, c->vz, c->ax, c->ay,
+                                                 c->az, c->ekx, c->eky, c->ekz, c->aox, c->aoy,
+                                                 c->aoz, c->part, nvir, c->scal, c->flags,
+                                                 queued ? 1 : 0);
+  CAV_HIP(hipGetLastError());
+  return thermo_end_of_step(c, ts);
+}
+
+// The state back to the start of the step that failed.
+static int step_back(cav_ctx *c)
+{
+  CAV_TRY(snapshot(c, false));
+  return elc_rewind(c);
+}
+
+// Steps without a host check after each: a step that meets a NaN or a full
+// list sets F_STOP at its end, after which no drift of the steps queued behind
+// it moves anything or touches the snapshot; the host finds how many steps
+// completed, goes back to the start of the failed one and takes it up again
+// (a larger list) or reports it.  Waiting for the flags after every step left
+// the GPU idle for about 15 us a step.
+constexpr int kQueuedSteps = 64;
+
+static int run_queued(cav_ctx *c, double dt, int nsteps)
+{
+  int attempts = 0;
+  for (int done = 0; done < nsteps;) {
+    const int q = std::min(nsteps - done, kQueuedSteps);
+    k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, attempts > 0 ? 1 : 0);
+    for (int s = 0; s < q; ++s) CAV_TRY(issue_step(c, dt, c->step_index + s, true));
+    CAV_TRY(sync_flags(c));
+    const int ok = c->h_flags[F_STEPS];
+    done += ok;
+    c->step_index += ok;
+    if (!c->h_flags[F_STOP]) {
+      attempts = 0;
+      continue;
+    }
+    attempts = ok > 0 ? 1 : attempts + 1;
+    CAV_TRY(step_back(c));
+    k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_STOP, 0);
+    if (c->h_flags[F_NAN]) {
+      CAV_HIP(hipStreamSynchronize(c->stream));
+      return fail(c, CAV_ERR_NAN, "NaN acceleration before the drift");
+    }
+    bool redo = false;
+    CAV_TRY(check_capacity(c, &redo));
+    if (attempts >= 4) return fail(c, CAV_ERR_CAPACITY, "Verlet list capacity could not be met");
+  }
+  return CAV_OK;
+}
+
 int cav_step(cav_ctx *c, double dt, int nsteps)
 {
   if (!c) return CAV_ERR_ARG;
   if (!c->setup_done) return fail(c, CAV_ERR_STATE, "cav_setup must run before cav_step");
   (void)hipSetDevice(c->device);
   CAV_TRY(refresh_params(c));
-  const double *lo, *hi, *L;
-  box_dev(c, &lo, &hi, &L);
+  // per-kernel timings, the slab correction's one-evaluation memory and a list
+  // without slots (another pair kernel was in use) need a look after each step
+  if (fused_cells(c) && c->nlb_built && !c->timing && !c->elc_on) return run_queued(c, dt, nsteps);
   for (int s = 0; s < nsteps; ++s) {
     bool redo = true;
     for (int attempt = 0; redo && attempt < 4; ++attempt) {
-      // the step snapshot (restored on NaN or overflow) is written by the drift
-      k_begin_step<<<1, 1, 0, c->stream>>>(c->flags);
-      timer_begin(c, c->t_int);
-      k_drift<<<grid_for(c->n), kBlock, 0, c->stream>>>(
-          c->n, dt, lo, hi, L, c->bc[0], c->bc[1], c->bc[2], c->x, c->y, c->z, c->vx, c->vy, c->vz,
-          c->ax, c->ay, c->az, c->aox, c->aoy, c->aoz, c->flags, c->snap);
-      timer_end(c, c->t_int);
-      CAV_HIP(hipGetLastError());
-      const bool side = c->overlap && c->ek_on && c->n > 0;
-      if (side) CAV_TRY(ewald_k_fork(c));
-      CAV_TRY(launch_ghosts(c));
-      CAV_TRY(neighbor_phase(c, false));
-      CAV_TRY(forces(c, !side));
-      if (side && (c->dipole || c->elc_on)) {
-        // a = ((a_sr + a_k) + a_dip) + a_elc, as in order: add, dipole, slab
-        // correction, then the kick
-        CAV_TRY(ewald_k_join(c));
-        k_add3<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->ax, c->ay, c->az, c->ekx,
-                                                         c->eky, c->ekz);
-        if (c->dipole) CAV_TRY(launch_dipole(c));
-        if (c->elc_on) CAV_TRY(launch_elc(c));
-        k_kick<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, 0.5 * dt, c->vx, c->vy, c->vz,
-                                                         c->ax, c->ay, c->az, c->aox, c->aoy,
-                                                         c->aoz);
-      } else if (side) {
-        CAV_TRY(ewald_k_join(c));
-        k_kick_join<<<grid_for(c->n), kBlock, 0, c->stream>>>(
-            c->n, 0.5 * dt, c->vx, c->vy, c->vz, c->ax, c->ay, c->az, c->ekx, c->eky, c->ekz,
-            c->aox, c->aoy, c->aoz);
-      } else {
-        k_kick<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, 0.5 * dt, c->vx, c->vy, c->vz,
-                                                         c->ax, c->ay, c->az, c->aox, c->aoy,
-                                                         c->aoz);
-      }
-      CAV_HIP(hipGetLastError());
-      CAV_TRY(thermo_end_of_step(c, c->step_index));
+      k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, 0);
+      CAV_TRY(issue_step(c, dt, c->step_index, false));
       CAV_TRY(sync_flags(c));
       harvest_timers(c);
       if (c->h_flags[F_NAN]) {
-        CAV_TRY(snapshot(c, false));
-        CAV_TRY(elc_rewind(c));
+        CAV_TRY(step_back(c));
         CAV_HIP(hipStreamSynchronize(c->stream));
         return fail(c, CAV_ERR_NAN, "NaN acceleration before the drift");
       }
       CAV_TRY(check_capacity(c, &redo));
       if (redo) {
-        CAV_TRY(snapshot(c, false));
-        CAV_TRY(elc_rewind(c));
+        CAV_TRY(step_back(c));
         k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_FORCE, 1);
       }
     }
@@ -1236,15 +1228,12 @@ int cav_recalculate(cav_ctx *c, int force_rebuild)
   if (!c->setup_done) return fail(c, CAV_ERR_STATE, "cav_setup must run first");
   (void)hipSetDevice(c->device);
   CAV_TRY(refresh_params(c));
-  k_begin_step<<<1, 1, 0, c->stream>>>(c->flags);
-  CAV_TRY(wrap_and_ghosts(c));
-  CAV_TRY(neighbor_phase(c, force_rebuild != 0));
-  CAV_TRY(forces(c));
+  CAV_TRY(evaluate(c, force_rebuild != 0));
   CAV_TRY(sync_flags(c));
   bool redo = false;
   CAV_TRY(check_capacity(c, &redo));
   if (redo) {
-    CAV_TRY(neighbor_phase(c, true));
+    CAV_TRY(neighbor_phase(c, Rebuild::forced, false));
     CAV_TRY(elc_rewind(c));
     CAV_TRY(forces(c));
     CAV_TRY(sync_flags(c));
@@ -1258,7 +1247,7 @@ int cav_neighbor_build(cav_ctx *c, int update, int *rebuilt)
   if (!c) return CAV_ERR_ARG;
   if (!c->setup_done) return fail(c, CAV_ERR_STATE, "cav_setup must run first");
   k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_REBUILD, 0);
-  CAV_TRY(neighbor_phase(c, update != 0));
+  CAV_TRY(neighbor_phase(c, update ? Rebuild::forced : Rebuild::test, false));
   CAV_TRY(sync_flags(c));
   if (rebuilt) *rebuilt = c->h_flags[F_REBUILD];
   return CAV_OK;
@@ -1270,7 +1259,8 @@ int cav_exchange(cav_ctx *c, int *wrapped)
   if (!c->setup_done) return fail(c, CAV_ERR_STATE, "cav_setup must run first");
   (void)hipSetDevice(c->device);
   k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_WRAPPED, 0);
-  CAV_TRY(wrap_and_ghosts(c));
+  CAV_TRY(launch_move(c, false, 0, false));
+  CAV_TRY(launch_ghosts(c, false));
   CAV_TRY(sync_flags(c));
   if (wrapped) *wrapped = c->h_flags[F_WRAPPED] != 0;
   return CAV_OK;

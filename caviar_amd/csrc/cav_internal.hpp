@@ -32,6 +32,8 @@ enum Flag : int {
   F_GOVER = 8,     // batched replicas: ghosts exceeded the replica's ghost capacity
   F_MAXST = 9,     // largest cell stencil (candidate atoms) the cell-staged pair kernel met
   F_NL_STALE = 10, // the last list build wrote bin-order slots only: index rows are filled on demand
+  F_STOP = 11,     // a step failed (NaN or overflow): the steps queued after it leave the state alone
+  F_STEPS = 12,    // steps completed since the flags were last cleared
   F_COUNT = 16
 };
 
@@ -199,6 +201,11 @@ struct cav_ctx {
   int *lstart = nullptr, *litems = nullptr;  // cells of the last list build
   double4 *xqs = nullptr;  // (x, y, z, q) in bin order, refreshed every step
   int2 *tids = nullptr;    // (type, id) in bin order
+  // list build on the ghost-layer grid: per cell counts (owned in the high
+  // word) and the slots met in any order, bucket_cap each
+  unsigned long long *cell_cnt = nullptr;
+  int *bucket = nullptr;
+  int bucket_cap = 0;
   unsigned short *nll = nullptr;  // Verlet entries as positions in the row's cell staging order
   int *nlb = nullptr;             // Verlet entries as bin-order slots of the list build
   int *ord_blk = nullptr;  // scan block sums for the compaction
@@ -374,7 +381,11 @@ int refresh_params(cav_ctx *c);  // parameter values set after setup -> device
 void timer_end(cav_ctx *c, Timer &t);
 
 // launchers (defined in the .hip files)
-int launch_ghosts(cav_ctx *c);
+int launch_move(cav_ctx *c, bool drift, double dt, bool decide);  // drift / wrap, image counts
+int launch_ghosts(cav_ctx *c, bool decide);  // images, rebuild decision, cell counts
+bool fused_cells(const cav_ctx *c);  // whether launch_cells follows, instead of launch_bins
+int cells_alloc(cav_ctx *c);
+int launch_cells(cav_ctx *c);
 int launch_rebuild_check(cav_ctx *c);
 // for_list: the binning of a list build, which also keeps the bin order the
 // list refers to (litems, binpos)
@@ -391,8 +402,10 @@ inline bool list_on_ghost_grid(const cav_ctx *c)
   return !c->lj_cellwalk && c->pair_kind != CAV_PAIRS_CELLS && !c->all_atom_test;
 }
 int launch_nl_fill(cav_ctx *c);
-int launch_pairs(cav_ctx *c, bool lj, bool er, bool accumulate);
+// packed: the copies are current (launch_cells); reduce: virial partials summed here
+int launch_pairs(cav_ctx *c, bool lj, bool er, bool accumulate, bool packed = false, bool reduce = true);
 int launch_pack(cav_ctx *c);
+int pair_blocks(const cav_ctx *c);  // workgroups (virial partials) of the row pair kernel
 int launch_pairs_list(cav_ctx *c, bool ljl, bool sr, bool accumulate, bool pack);  // packed (x, y, z, q), (type, id) of owned + ghost slots
 int launch_lj_cellwalk(cav_ctx *c);
 int launch_zero_acc(cav_ctx *c);
@@ -408,9 +421,6 @@ int elc_rewind(cav_ctx *c);       // ELC dipole state back before a re-evaluatio
 int energy_elc(cav_ctx *c, double *e);
 int point_field_elc(cav_ctx *c, int np, const double *pts, double *field, double *pot);
 int forces_all(cav_ctx *c);
-int launch_drift(cav_ctx *c, double dt);
-int launch_kick(cav_ctx *c, double dt);
-int launch_begin_step(cav_ctx *c);
 int ewald_k_plan(cav_ctx *c);
 const char *plan_k_lattice(EwaldKPlan &p, int kx, int ky, int kz, int precision, double alpha,
                            double lx, double ly, double lz);

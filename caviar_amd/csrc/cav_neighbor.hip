@@ -73,62 +73,32 @@ struct GhostRule {
   const double *x, *y, *z;
   double xl, xu, yl, yu, zl, zu;
   int bx, by, bz;
-  __device__ __forceinline__ void sides(long i, int &sx, int &sy, int &sz) const
+  __device__ __forceinline__ void sides(double px, double py, double pz, int &sx, int &sy,
+                                        int &sz) const
   {
     // exchange_ghost_single_md_domain.cpp:70-101: strict tests, times the bc flag
-    sx = (x[i] < xl ? -1 : (x[i] > xu ? 1 : 0)) * bx;
-    sy = (y[i] < yl ? -1 : (y[i] > yu ? 1 : 0)) * by;
-    sz = (z[i] < zl ? -1 : (z[i] > zu ? 1 : 0)) * bz;
+    sx = (px < xl ? -1 : (px > xu ? 1 : 0)) * bx;
+    sy = (py < yl ? -1 : (py > yu ? 1 : 0)) * by;
+    sz = (pz < zl ? -1 : (pz > zu ? 1 : 0)) * bz;
+  }
+  __device__ __forceinline__ void sides(long i, int &sx, int &sy, int &sz) const
+  {
+    sides(x[i], y[i], z[i], sx, sy, sz);
+  }
+  static __device__ __forceinline__ int images(int sx, int sy, int sz)
+  {
+    const int a = sx != 0, b = sy != 0, c = sz != 0;
+    return a + b + c + (a & b) + (a & c) + (b & c) + (a & b & c);
   }
   __device__ __forceinline__ int operator()(long i) const
   {
     int sx, sy, sz;
     sides(i, sx, sy, sz);
-    const int a = sx != 0, b = sy != 0, c = sz != 0;
-    return a + b + c + (a & b) + (a & c) + (b & c) + (a & b & c);
+    return images(sx, sy, sz);
   }
 };
 
-// Writes the images of owned atom i at ghost slots [off, off+count): order x,
-// y, z, xy, xz, yz, xyz (exchange_ghost_single_md_domain.cpp:167-215); ghost g
-// lives at index n+g of every per-atom array.
-__global__ void k_ghost_scatter(int n, GhostRule rule, double Lx, double Ly, double Lz,
-                                const int *blk, double *x, double *y, double *z, int *type,
-                                int *id, int *mol, double *q, int *gsrc)
-{
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  const int cnt = i < n ? rule(i) : 0;
-  const int off = block_exclusive_scan(cnt, nullptr) + blk[blockIdx.x];
-  if (i >= n || cnt == 0) return;
-  int sx, sy, sz;
-  rule.sides(i, sx, sy, sz);
-  const double px = x[i], py = y[i], pz = z[i];
-  const double gx = px - sx * Lx, gy = py - sy * Ly, gz = pz - sz * Lz;
-  const int t = type[i], d = id[i], m = mol[i];
-  const double qq = q[i];
-  int g = off;
-  auto put = [&](double a, double b, double c) {
-    const long s = (long)n + g;
-    x[s] = a;
-    y[s] = b;
-    z[s] = c;
-    type[s] = t;
-    id[s] = d;
-    mol[s] = m;
-    q[s] = qq;
-    gsrc[g] = (int)i;
-    ++g;
-  };
-  if (sx) put(gx, py, pz);
-  if (sy) put(px, gy, pz);
-  if (sz) put(px, py, gz);
-  if (sx && sy) put(gx, gy, pz);
-  if (sx && sz) put(gx, py, gz);
-  if (sy && sz) put(px, gy, gz);
-  if (sx && sy && sz) put(gx, gy, gz);
-}
-
-int launch_ghosts(cav_ctx *c)
+static GhostRule ghost_rule(const cav_ctx *c)
 {
   GhostRule r;
   r.x = c->x;
@@ -143,14 +113,7 @@ int launch_ghosts(cav_ctx *c)
   r.bx = c->bc[0];
   r.by = c->bc[1];
   r.bz = c->bc[2];
-  const int nb = grid_for(c->n);
-  k_block_sums<<<nb, kBlock, 0, c->stream>>>(c->n, r, c->blk, nullptr);
-  k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
-  k_ghost_scatter<<<nb, kBlock, 0, c->stream>>>(c->n, r, c->L[0], c->L[1], c->L[2], c->blk, c->x,
-                                                c->y, c->z, c->type, c->id, c->mol, c->q,
-                                                c->gsrc);
-  CAV_HIP(hipGetLastError());
-  return CAV_OK;
+  return r;
 }
 
 // ------------------------------------------------------------ rebuild test --
@@ -487,6 +450,491 @@ int launch_bins(cav_ctx *c, bool conditional, bool for_list)
   k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nbo, c->ord_blk, c->flags + F_COUNT - 2, cond);
   k_order_scatter<<<nbo, kBlock, 0, c->stream>>>(tot, c->n, c->bin_items, c->ord_blk, c->order,
                                                  c->flags, cond);
+  CAV_HIP(hipGetLastError());
+  return CAV_OK;
+}
+
+// ------------------------------------------------------ a step's exchange --
+//
+// A step's short-range part up to the Verlet rows is four launches, whatever
+// the size: k_move (drift or wrap, per-block ghost counts, displacement test of
+// the owned atoms), k_ghosts (images, rebuild decision, cell counts and
+// buckets), k_cells (cell starts, sorted cells and everything in bin order) and
+// the list build.  As one kernel per scan, fill, sort and copy it was eighteen,
+// of 2-4 us each plus the gap before it: a step of 256 LJ atoms took 141 us,
+// now 72; of 8000 ions (FP64, kmax 8) 209, now 119; at N = 262144, where the
+// gaps hide beside Ewald_k, 0.82 ms before and now.
+
+typedef unsigned long long u64t;
+
+// Sums of two values over the 256 threads of a block, in every thread.
+__device__ __forceinline__ void block_sum2(int &a, int &b)
+{
+  __shared__ int s[2][kBlock / 64];
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o, 64);
+    b += __shfl_xor(b, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s[0][threadIdx.x >> 6] = a;
+    s[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  a = (s[0][0] + s[0][1]) + (s[0][2] + s[0][3]);
+  b = (s[1][0] + s[1][1]) + (s[1][2] + s[1][3]);
+}
+
+struct MoveArgs {
+  int n;
+  double dt;
+  double lo[3], hi[3], L[3];
+  int bc[3];
+  double *x, *y, *z;
+  const double *vx, *vy, *vz, *ax, *ay, *az;
+  double *aox, *aoy, *aoz, *snap;
+  const double *xo, *yo, *zo;  // positions at the last list build, or nullptr
+  double thr_sq;
+  int *flags, *blk;
+  u64t *cnt;  // cell counters to clear, or nullptr
+  int nbins;
+};
+
+// DRIFT: integrate_velocity_verlet's drift (md_simulator.cpp:584-594), every
+// operation rounded as the reference's expression is: r += (v*dt +
+// ((0.5*a)*dt)*dt); the step snapshot of positions, velocities and
+// accelerations ([x | y | z | vx | vy | vz | ax | ay | az], n each) is written
+// from the values it reads.  Then, for setup and recalculate too, the wrap of
+// exchange_owned (domain.cpp:418-468) and the number of the block's images.
+// Once F_STOP is set (a step before this one failed) nothing moves and the
+// snapshot stays.  HBM bound: 216 B an atom.
+template <bool DRIFT>
+__global__ __launch_bounds__(kBlock) void k_move(MoveArgs a, GhostRule rule)
+{
+  if (DRIFT && a.flags[F_STOP]) return;
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (a.cnt)
+    for (int k = i; k < a.nbins; k += gridDim.x * kBlock) a.cnt[k] = 0;
+  int cnt = 0, moved = 0;
+  if (i < a.n) {
+    double *p[3] = {a.x + i, a.y + i, a.z + i};
+    double r[3];
+    if constexpr (DRIFT) {
+      const double acc[3] = {a.ax[i], a.ay[i], a.az[i]};
+      const double v[3] = {a.vx[i], a.vy[i], a.vz[i]};
+      if (isnan(acc[0]) || isnan(acc[1]) || isnan(acc[2])) a.flags[F_NAN] = 1;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        r[d] = *p[d];
+        a.snap[(long)d * a.n + i] = r[d];
+        a.snap[(long)(3 + d) * a.n + i] = v[d];
+        a.snap[(long)(6 + d) * a.n + i] = acc[d];
+        const double h = xmul(xmul(xmul(0.5, acc[d]), a.dt), a.dt);
+        r[d] = xadd(r[d], xadd(xmul(v[d], a.dt), h));
+      }
+      a.aox[i] = acc[0];
+      a.aoy[i] = acc[1];
+      a.aoz[i] = acc[2];
+    } else {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) r[d] = *p[d];
+    }
+    bool wrapped = false;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if (a.bc[d] == 1) {
+        if (r[d] < a.lo[d]) {
+          r[d] = xadd(r[d], a.L[d]);
+          wrapped = true;
+        } else if (r[d] > a.hi[d]) {
+          r[d] = xsub(r[d], a.L[d]);
+          wrapped = true;
+        }
+      }
+      *p[d] = r[d];
+    }
+    if (wrapped) {
+      a.flags[F_WRAPPED] = 1;
+      a.flags[F_REBUILD] = 1;
+    }
+    int sx, sy, sz;
+    rule.sides(r[0], r[1], r[2], sx, sy, sz);
+    cnt = GhostRule::images(sx, sy, sz);
+    if (a.xo) {
+      const double dx = xsub(r[0], a.xo[i]), dy = xsub(r[1], a.yo[i]), dz = xsub(r[2], a.zo[i]);
+      moved = dot_rn(dx, dy, dz) > a.thr_sq;
+    }
+  }
+  if (moved) a.flags[F_REBUILD] = 1;
+  int none = 0;
+  block_sum2(cnt, none);
+  if (threadIdx.x == 0) a.blk[blockIdx.x] = cnt;
+}
+
+struct GhostArgs {
+  int n, nblk, scanned;  // scanned: blk already holds exclusive sums, F_NGHOST the total
+  double L[3];
+  const int *blk;
+  double *x, *y, *z;
+  int *type, *id, *mol, *gsrc;
+  double *q;
+  const double *xo, *yo, *zo;  // or nullptr: no rebuild decision
+  double thr_sq;
+  int rebuild_test;
+  int *flags;
+  double4 *xq;  // packed copies, or nullptr
+  int2 *tid;
+  u64t *cnt;    // cells (owned count in the high word), or nullptr
+  int *bucket, *bin_of;
+  int cap;
+};
+
+// The images of owned atom i at ghost slots n + g, g ascending with i, in the
+// order x, y, z, xy, xz, yz, xyz (exchange_ghost_single_md_domain.cpp:167-215).
+// Each block adds up the counts of the blocks before it itself (no scan
+// launch).  With the total known, the rest of Neighborlist::update_is_needed
+// (neighborlist.cpp:91-139; the owned displacements were tested by the move):
+// the number of ghosts, and each ghost's displacement.  Every slot is also
+// packed for the gathers and put into its cell's bucket, whether the list is
+// rebuilt or not: the decision is not known yet, and the counting is cheaper
+// than a launch of its own.
+__global__ __launch_bounds__(kBlock) void k_ghosts(GhostArgs a, GhostRule rule, BinRule bins)
+{
+  if (a.flags[F_STOP]) return;
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  int before, total;
+  if (a.scanned) {
+    before = a.blk[blockIdx.x];
+    total = a.flags[F_NGHOST];
+  } else {
+    before = total = 0;
+    for (int k = threadIdx.x; k < a.nblk; k += kBlock) {
+      const int v = a.blk[k];
+      total += v;
+      if (k < (int)blockIdx.x) before += v;
+    }
+    block_sum2(before, total);
+  }
+  double px = 0, py = 0, pz = 0;
+  int sx = 0, sy = 0, sz = 0, cnt = 0;
+  if (i < a.n) {
+    px = a.x[i];
+    py = a.y[i];
+    pz = a.z[i];
+    rule.sides(px, py, pz, sx, sy, sz);
+    cnt = GhostRule::images(sx, sy, sz);
+  }
+  const int off = before + block_exclusive_scan(cnt, nullptr);
+  bool test = false;
+  if (a.xo) {
+    const bool differs = a.rebuild_test || total != a.flags[F_NGHOST_OLD];
+    test = !differs;
+    if (differs && i == 0) a.flags[F_REBUILD] = 1;
+  }
+  if (i == 0 && !a.scanned) a.flags[F_NGHOST] = total;
+  if (i >= a.n) return;
+  const int t = a.type[i], d = a.id[i], m = a.mol[i];
+  const double qq = a.q[i];
+  auto slot = [&](long s, double u, double v, double w, bool owned) {
+    if (a.xq) {
+      a.xq[s] = make_double4(u, v, w, qq);
+      a.tid[s] = make_int2(t, d);
+    }
+    if (a.cnt) {
+      const int b = bins(u, v, w);
+      const int rank = (int)atomicAdd(a.cnt + b, owned ? (1ull << 32 | 1ull) : 1ull);
+      a.bin_of[s] = b;
+      if (rank < a.cap) a.bucket[(long)b * a.cap + rank] = (int)s;
+    }
+  };
+  slot(i, px, py, pz, true);
+  if (cnt == 0) return;
+  const double gx = px - sx * a.L[0], gy = py - sy * a.L[1], gz = pz - sz * a.L[2];
+  int g = off;
+  auto put = [&](double u, double v, double w) {
+    const long s = (long)a.n + g;
+    if (test) {
+      const double dx = xsub(u, a.xo[s]), dy = xsub(v, a.yo[s]), dz = xsub(w, a.zo[s]);
+      if (dot_rn(dx, dy, dz) > a.thr_sq) a.flags[F_REBUILD] = 1;
+    }
+    a.x[s] = u;
+    a.y[s] = v;
+    a.z[s] = w;
+    a.type[s] = t;
+    a.id[s] = d;
+    a.mol[s] = m;
+    a.q[s] = qq;
+    a.gsrc[g] = i;
+    slot(s, u, v, w, false);
+    ++g;
+  };
+  if (sx) put(gx, py, pz);
+  if (sy) put(px, gy, pz);
+  if (sz) put(px, py, gz);
+  if (sx && sy) put(gx, gy, pz);
+  if (sx && sz) put(gx, py, gz);
+  if (sy && sz) put(px, gy, gz);
+  if (sx && sy && sz) put(gx, gy, gz);
+}
+
+struct CellBuild {
+  int n, nbins, bpb, cap;
+  const u64t *cnt;
+  const int *bucket, *bin_of;
+  const double4 *xq;
+  const int2 *tid;
+  int *start, *items, *order, *binpos, *litems;
+  double4 *cpos, *xqs;
+  int2 *tids;
+  double *xo, *yo, *zo;
+  int *flags;
+};
+
+constexpr int kCellBlock = 1024;
+
+// Cells of a list build, one wave per cell, bpb cells per workgroup: cell
+// starts (a workgroup adds up the counters of the cells before its own),
+// the cell's slots sorted by index (update_cell_list's insertion order is
+// owned ascending, then ghosts ascending, neighborlist.cpp:457-471), and in
+// that order the slot -> atom and atom -> slot maps, the owned atoms, the list
+// build's candidates and the packed copies; pos_old as well
+// (neighborlist.cpp:302-303).  Without a rebuild only the packed copies are
+// refreshed, in the order of the last one.
+__global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
+{
+  if (a.flags[F_STOP]) return;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = a.flags[F_NGHOST];
+  const long tot = (long)a.n + G;
+  if (!a.flags[F_REBUILD]) {
+    for (long t = (long)blockIdx.x * kCellBlock + threadIdx.x; t < tot;
+         t += (long)gridDim.x * kCellBlock) {
+      const int j = a.litems[t];
+      a.xqs[t] = a.xq[j];
+      a.tids[t] = a.tid[j];
+    }
+    return;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.flags[F_NGHOST_OLD] = G;
+  __shared__ u64t part[kCellBlock / 64];
+  __shared__ u64t first[65];  // per cell: slots before it, owned atoms before it
+  const int b0 = blockIdx.x * a.bpb;
+  u64t s = 0;
+#pragma unroll 4
+  for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) part[wv] = s;
+  __syncthreads();
+  if (wv == 0) {
+    u64t base = lane < kCellBlock / 64 ? part[lane] : 0;
+    for (int o = 8; o > 0; o >>= 1) base += __shfl_xor(base, o, 16);
+    base = __shfl(base, 0, 64);
+    const u64t v = lane < a.bpb && b0 + lane < a.nbins ? a.cnt[b0 + lane] : 0;
+    u64t inc = v;
+    for (int o = 1; o < 64; o <<= 1) {
+      const u64t u = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += u;
+    }
+    first[lane] = base + inc - v;
+    if (lane == 63) first[64] = base + inc;
+    if (lane < a.bpb && b0 + lane < a.nbins) a.start[b0 + lane] = (int)(base + inc - v);
+    if (lane < a.bpb && b0 + lane == a.nbins - 1) a.start[a.nbins] = (int)(base + inc);
+  }
+  __syncthreads();
+  for (int w = wv; w < a.bpb && b0 + w < a.nbins; w += kCellBlock / 64) {
+    const int b = b0 + w;
+    const long s0 = (long)(unsigned)first[w];
+    const int o0 = (int)(first[w] >> 32);
+    const int m = (int)((unsigned)first[w + 1] - (unsigned)first[w]);
+    if (m == 0) continue;
+    const int *mine = a.bucket + (long)b * a.cap;
+    int j0 = 0x7fffffff, rank = 0;
+    if (m <= 64 && m <= a.cap) {
+      // one slot per lane, ranked by the smaller indices of the others
+      if (lane < m) j0 = mine[lane];
+      for (int k = 0; k < m; ++k) rank += __builtin_amdgcn_readlane(j0, k) < j0 ? 1 : 0;
+    } else {
+      // large cells through memory: the unsorted slots (those past the bucket's
+      // capacity are found again by their cell), then each one's rank
+      if (m > a.cap) {
+        int at = 0;
+        for (long t0 = 0; t0 < tot; t0 += 64) {
+          const bool in = t0 + lane < tot && a.bin_of[t0 + lane] == b;
+          const u64t mask = __ballot(in);
+          if (in) a.items[s0 + at + __popcll(mask & ((1ull << lane) - 1ull))] = (int)(t0 + lane);
+          at += __popcll(mask);
+        }
+      } else {
+        for (int k = lane; k < m; k += 64) a.items[s0 + k] = mine[k];
+      }
+      __threadfence_block();
+      for (int k = lane; k < m; k += 64) {
+        const int j = a.items[s0 + k];
+        int r = 0;
+        for (int u = 0; u < m; ++u) r += a.items[s0 + u] < j ? 1 : 0;
+        a.litems[s0 + r] = j;
+      }
+      __threadfence_block();
+    }
+    for (int k = lane; k < m; k += 64) {
+      int j = j0, r = rank;
+      if (m > 64 || m > a.cap) {
+        r = k;
+        j = a.litems[s0 + k];
+      }
+      const long t = s0 + r;
+      const double4 v = a.xq[j];
+      const int2 u = a.tid[j];
+      a.items[t] = j;
+      a.litems[t] = j;
+      a.binpos[j] = (int)t;
+      if (j < a.n) a.order[o0 + r] = j;  // owned atoms come first in a cell
+      a.xqs[t] = v;
+      a.tids[t] = u;
+      a.cpos[t] = make_double4(v.x, v.y, v.z, cpos_tag(j, t));
+      a.xo[j] = v.x;
+      a.yo[j] = v.y;
+      a.zo[j] = v.z;
+    }
+  }
+}
+
+// The four-launch exchange covers lists built on the ghost-layer grid for the
+// bin-order pair kernel (the default).  A workgroup of k_cells reads the
+// counters of all cells before its own, so grids past 65536 cells (about a
+// million atoms at rho = 0.3) keep the scans; so do grids so empty that the
+// buckets would take more room than the atoms' slots.
+bool fused_cells(const cav_ctx *c)
+{
+  return c->nl_on && c->bucket && c->pair_kind == CAV_PAIRS_AUTO && list_on_ghost_grid(c) && c->nlb;
+}
+
+int cells_alloc(cav_ctx *c)
+{
+  if (c->bucket) (void)hipFree(c->bucket);
+  if (c->cell_cnt) (void)hipFree(c->cell_cnt);
+  c->bucket = nullptr;
+  c->cell_cnt = nullptr;
+  if (!c->nl_on || c->n == 0 || c->xnbins > 65536) return CAV_OK;
+  // twice the mean cell and some, in whole waves
+  const double cell = c->rce * c->rce * c->rce, vol = c->L[0] * c->L[1] * c->L[2];
+  const long want = (long)(2.0 * cell * (c->n / vol)) + 32;
+  const long cap = std::min(1024L, (want + 31) / 32 * 32);
+  if (cap * c->xnbins > 32L * ((long)c->n + c->gcap) + 65536) return CAV_OK;
+  CAV_HIP(hipMalloc(&c->bucket, sizeof(int) * cap * c->xnbins));
+  CAV_HIP(hipMalloc(&c->cell_cnt, sizeof(u64t) * c->xnbins));
+  c->bucket_cap = (int)cap;
+  return CAV_OK;
+}
+
+// Owned atoms moved (drift of dt, or only wrapped) and the images counted;
+// `decide`: with the rebuild test.
+int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
+{
+  MoveArgs a;
+  a.n = c->n;
+  a.dt = dt;
+  for (int d = 0; d < 3; ++d) {
+    a.lo[d] = c->lo[d];
+    a.hi[d] = c->hi[d];
+    a.L[d] = c->L[d];
+    a.bc[d] = c->bc[d];
+  }
+  a.x = c->x;
+  a.y = c->y;
+  a.z = c->z;
+  a.vx = c->vx;
+  a.vy = c->vy;
+  a.vz = c->vz;
+  a.ax = c->ax;
+  a.ay = c->ay;
+  a.az = c->az;
+  a.aox = c->aox;
+  a.aoy = c->aoy;
+  a.aoz = c->aoz;
+  a.snap = c->snap;
+  a.xo = decide && c->nl_on ? c->xo : nullptr;
+  a.yo = c->yo;
+  a.zo = c->zo;
+  a.thr_sq = c->thr_sq;
+  a.flags = c->flags;
+  a.blk = c->blk;
+  a.cnt = fused_cells(c) ? c->cell_cnt : nullptr;
+  a.nbins = c->xnbins;
+  if (drift)
+    k_move<true><<<grid_for(c->n), kBlock, 0, c->stream>>>(a, ghost_rule(c));
+  else
+    k_move<false><<<grid_for(c->n), kBlock, 0, c->stream>>>(a, ghost_rule(c));
+  CAV_HIP(hipGetLastError());
+  return CAV_OK;
+}
+
+// Images of the moved atoms, and the rebuild decision; after launch_move.
+int launch_ghosts(cav_ctx *c, bool decide)
+{
+  const int nb = grid_for(c->n);
+  GhostArgs a;
+  a.n = c->n;
+  a.nblk = nb;
+  // each block reads every block's count: past a million atoms one scan does
+  a.scanned = nb > 4096;
+  for (int d = 0; d < 3; ++d) a.L[d] = c->L[d];
+  a.blk = c->blk;
+  a.x = c->x;
+  a.y = c->y;
+  a.z = c->z;
+  a.type = c->type;
+  a.id = c->id;
+  a.mol = c->mol;
+  a.gsrc = c->gsrc;
+  a.q = c->q;
+  a.xo = decide && c->nl_on ? c->xo : nullptr;
+  a.yo = c->yo;
+  a.zo = c->zo;
+  a.thr_sq = c->thr_sq;
+  a.rebuild_test = c->rebuild_test;
+  a.flags = c->flags;
+  const bool fused = fused_cells(c);
+  a.xq = fused ? c->xq : nullptr;
+  a.tid = c->tid;
+  a.cnt = fused ? c->cell_cnt : nullptr;
+  a.bucket = c->bucket;
+  a.bin_of = c->bin_of;
+  a.cap = c->bucket_cap;
+  if (a.scanned)
+    k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
+  k_ghosts<<<nb, kBlock, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
+  CAV_HIP(hipGetLastError());
+  return CAV_OK;
+}
+
+// Cells and bin-order copies of the images launch_ghosts made.
+int launch_cells(cav_ctx *c)
+{
+  CellBuild a;
+  a.n = c->n;
+  a.nbins = c->xnbins;
+  // one cell per wave where the chip has room, else four (fewer workgroups
+  // that add up the counters before theirs)
+  a.bpb = c->xnbins <= 4096 ? 16 : 64;
+  a.cap = c->bucket_cap;
+  a.cnt = c->cell_cnt;
+  a.bucket = c->bucket;
+  a.bin_of = c->bin_of;
+  a.xq = c->xq;
+  a.tid = c->tid;
+  a.start = c->bin_start;
+  a.items = c->bin_items;
+  a.order = c->order;
+  a.binpos = c->binpos;
+  a.litems = c->litems;
+  a.cpos = c->cpos;
+  a.xqs = c->xqs;
+  a.tids = c->tids;
+  a.xo = c->xo;
+  a.yo = c->yo;
+  a.zo = c->zo;
+  a.flags = c->flags;
+  k_cells<<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }

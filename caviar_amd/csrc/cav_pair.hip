@@ -719,6 +719,7 @@ static PairArgs pair_args(cav_ctx *c)
 }
 
 static int pair_grid(const cav_ctx *c) { return (grid_for((long)c->n * kLPA) + 7) / 8 * 8; }
+int pair_blocks(const cav_ctx *c) { return pair_grid(c); }
 
 template <typename T, bool BINS>
 static void launch_pairs_tb(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
@@ -853,7 +854,7 @@ int launch_pack(cav_ctx *c)
   return CAV_OK;
 }
 
-int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate)
+int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate, bool packed, bool reduce)
 {
   const bool lj = want_lj && c->lj_on && !c->lj_cellwalk, er = want_er && c->er_on;
   if (!lj && !er) return CAV_OK;
@@ -873,7 +874,8 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate)
   } else {
     CAV_TRY(launch_nl_fill(c));
   }
-  k_pack<<<grid_for(tot), kBlock, 0, c->stream>>>(c->n, tot, c->x, c->y, c->z, c->q, c->type,
+  if (!packed || !bins)
+    k_pack<<<grid_for(tot), kBlock, 0, c->stream>>>(c->n, tot, c->x, c->y, c->z, c->q, c->type,
                                                  c->id, c->flags, c->xq, c->tid,
                                                  cells || bins ? c->binpos : nullptr, c->xqs,
                                                  c->tids);
@@ -890,6 +892,7 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate)
   }
   timer_end(c, c->t_pair);
   CAV_HIP(hipGetLastError());
+  if (!reduce) return CAV_OK;
   return reduce_partials(c, cells ? cell_grid(c) : pair_grid(c), 0, accumulate);
 }
 

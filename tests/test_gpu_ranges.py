@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import fixtures as F
-from caviar_amd import Engine, configs
+from caviar_amd import Engine, NaNAccelerationError, configs
 from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +67,86 @@ def test_force_pass_row_splits(gpu, n, k, precision):
     fo, po = o.point_k(pts)
     assert F.rel_err(f, fo) <= tol
     assert F.rel_err(p, po) <= tol
+
+
+def _free_pair_system(n, box, pos, vel, rce=2.0):
+    """Neutral atoms with an LJ reach of 0.2: they fly straight until two meet."""
+    from caviar_amd import LJSettings, NeighborSettings, System
+    return System(lower=[0, 0, 0], upper=[box] * 3, bc=[1, 1, 1], ghost_cutoff=rce + 0.1, mass=[1.0],
+                  charge=[0.0], pos=pos, vel=vel, types=np.zeros(n, dtype=np.int32),
+                  neighbor=NeighborSettings(cutoff=rce / 1.25, cutoff_extra_coef=1.25),
+                  lj=LJSettings(cutoff=0.2, epsilon=np.ones((1, 1)), sigma=np.full((1, 1), 0.1)))
+
+
+@pytest.mark.parametrize("steps", [5, 20, 70])
+def test_nan_among_queued_steps(gpu, steps):
+    """Two atoms meet exactly in step 4: the NaN shows at the start of step 5,
+    and the state is that before it however many steps were asked for."""
+    print(f"[case] queued NaN steps={steps}", flush=True)
+    pos = np.array([[4.0, 5.0, 5.0], [6.0, 5.0, 5.0], [1.0, 1.0, 1.0]])
+    vel = np.array([[2.0, 0.0, 0.0], [-2.0, 0.0, 0.0], [0.25, 0.5, 0.0]])
+    s = _free_pair_system(3, 16.0, pos, vel)
+    e = Engine(s)
+    e.setup()
+    with pytest.raises(NaNAccelerationError):
+        e.step(0.125, steps)
+    want = pos + 4 * 0.125 * vel
+    assert np.array_equal(e.get("pos"), want)
+    assert np.isnan(e.get("acc")[:2]).all() and not np.isnan(e.get("acc")[2]).any()
+    # the atoms moved apart again: the run goes on
+    want[1, 1] += 1.0
+    e.set("pos", want)
+    e.set("vel", vel)
+    e.recalculate()
+    e.step(0.125, 3)
+    assert np.array_equal(e.get("pos"), want + 3 * 0.125 * vel)
+
+
+@pytest.mark.parametrize("steps", [1, 7, 80])
+def test_list_overflow_among_queued_steps(gpu, steps):
+    """Atoms flying together outgrow the list rows (sized for the mean density)
+    and the cell buckets in the middle of a run; the trajectory is the
+    oracle's, the pairs the exact set."""
+    print(f"[case] queued overflow, {steps} steps a call", flush=True)
+    rng = np.random.default_rng(11)
+    n, box = 400, 40.0
+    end = np.array([20.5, 20.5, 20.5]) + rng.uniform(-0.9, 0.9, (n, 3))
+    pos = rng.uniform(0.5, box - 0.5, (n, 3))
+    dt, total = 1.0 / 128, 80
+    vel = (end - pos) / (dt * 76)
+    s = _free_pair_system(n, box, pos, vel)
+    s.lj.epsilon[:] = 0.0
+    o = Oracle(s)
+    o.setup()
+    assert o.run(dt, total) == 0
+    e = Engine(s)
+    e.setup()
+    left = total
+    while left:
+        k = min(steps, left)
+        e.step(dt, k)
+        left -= k
+    assert F.rel_err(e.get("pos"), o.get("pos")) <= 1e-12
+    assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs()))
+
+
+@pytest.mark.parametrize("clump", [1, 60, 66, 130, 700])
+def test_crowded_cells(gpu, clump):
+    """Cells from empty to far past their buckets (sorted through memory):
+    ghosts and pairs bit-exact, forces against the oracle."""
+    print(f"[case] crowded cell {clump}", flush=True)
+    rng = np.random.default_rng(clump)
+    n, box = clump + 150, 30.0
+    pos = rng.uniform(0, box, (n, 3))
+    pos[rng.permutation(n)[:clump]] = rng.uniform(13.0, 14.9, (clump, 3))
+    s = configs.ions(n=n, rho=n / box ** 3, kmax=1, seed=1, dmin=0.0, with_lj=False, with_k=False)
+    s.pos = np.ascontiguousarray(pos)
+    o = Oracle(s)
+    o.setup()
+    e = Engine(s)
+    e.setup()
+    gp, gs = e.ghosts()
+    og, os_ = o.ghost_data()
+    assert np.array_equal(gp, og) and np.array_equal(gs, os_)
+    assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs()))
+    assert F.rel_err(e.get("acc"), o.get("acc")) <= 1e-11  # close pairs cancel more
