@@ -944,7 +944,7 @@ int cav_upload_atoms(cav_ctx *c, int n, const int *id, const int *type, const in
   CAV_TRY(dmalloc(c, &c->xq, tot));
   CAV_TRY(dmalloc(c, &c->tid, tot));
   CAV_TRY(dmalloc(c, &c->ord_blk, grid_for((long)tot) + 1));
-  c->nblk = grid_for(n) + 1;
+  c->nblk = grid_for(n, 64) + 1;
   CAV_TRY(dmalloc(c, &c->blk, c->nblk));
   std::vector<double> soa(3 * (size_t)n), qv(n);
   for (int i = 0; i < n; ++i) {
@@ -1049,7 +1049,8 @@ int cav_setup(cav_ctx *c)
   const long cells = (c->nbins + 7) / 8 * 8;  // one partial per cell of the cell-staged kernel
   // one partial per block of the row-gather pair kernel (kLPA lanes per atom,
   // grid rounded up to a multiple of 8), per cell of the cell-staged kernel
-  const long pair_blocks = (grid_for((long)kLPA * c->n) + 7) / 8 * 8;
+  // (up to 32 lanes for few atoms)
+  const long pair_blocks = (grid_for((long)(c->n <= 16384 ? 32 : kLPA) * c->n) + 7) / 8 * 8;
   const int npart = (int)std::max<long>(std::max<long>(3L * grid_for(std::max<long>((long)c->n, 1L << 16)),
                                                        pair_blocks),
                                         cells) + 64;

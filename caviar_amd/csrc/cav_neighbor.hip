@@ -9,11 +9,12 @@ namespace cav {
 
 // ------------------------------------------------------------------ scans --
 
-// Exclusive scan of one value per thread over a 256-thread block: wave64
-// prefix sums with DPP-backed shuffles, then the 4 wave totals through LDS.
+// Exclusive scan of one value per thread over a block of BS threads: wave64
+// prefix sums with DPP-backed shuffles, then the wave totals through LDS.
+template <int BS = kBlock>
 __device__ __forceinline__ int block_exclusive_scan(int v, int *total)
 {
-  __shared__ int wsum[kBlock / 64];
+  __shared__ int wsum[BS / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int inc = v;
 #pragma unroll
@@ -25,7 +26,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *total)
   __syncthreads();
   int base = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < kBlock / 64; ++w) {
+  for (int w = 0; w < BS / 64; ++w) {
     if (w < wave) base += wsum[w];
     tot += wsum[w];
   }
@@ -467,10 +468,11 @@ int launch_bins(cav_ctx *c, bool conditional, bool for_list)
 
 typedef unsigned long long u64t;
 
-// Sums of two values over the 256 threads of a block, in every thread.
+// Sums of two values over the BS threads of a block, in every thread.
+template <int BS>
 __device__ __forceinline__ void block_sum2(int &a, int &b)
 {
-  __shared__ int s[2][kBlock / 64];
+  __shared__ int s[2][BS / 64];
   for (int o = 32; o > 0; o >>= 1) {
     a += __shfl_xor(a, o, 64);
     b += __shfl_xor(b, o, 64);
@@ -480,8 +482,12 @@ __device__ __forceinline__ void block_sum2(int &a, int &b)
     s[1][threadIdx.x >> 6] = b;
   }
   __syncthreads();
-  a = (s[0][0] + s[0][1]) + (s[0][2] + s[0][3]);
-  b = (s[1][0] + s[1][1]) + (s[1][2] + s[1][3]);
+  a = b = 0;
+#pragma unroll
+  for (int w = 0; w < BS / 64; ++w) {
+    a += s[0][w];
+    b += s[1][w];
+  }
 }
 
 struct MoveArgs {
@@ -507,24 +513,30 @@ struct MoveArgs {
 // exchange_owned (domain.cpp:418-468) and the number of the block's images.
 // Once F_STOP is set (a step before this one failed) nothing moves and the
 // snapshot stays.  HBM bound: 216 B an atom.
-template <bool DRIFT>
-__global__ __launch_bounds__(kBlock) void k_move(MoveArgs a, GhostRule rule)
+template <bool DRIFT, int BS>
+__global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
 {
-  if (DRIFT && a.flags[F_STOP]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int i = blockIdx.x * BS + threadIdx.x;
+  const int at = i < a.n ? i : 0;
+  const int stop = a.flags[F_STOP];
+  const double old[3] = {a.x[at], a.y[at], a.z[at]};
+  double acc[3], v[3], last[3];
+  if constexpr (DRIFT) {
+    acc[0] = a.ax[at], acc[1] = a.ay[at], acc[2] = a.az[at];
+    v[0] = a.vx[at], v[1] = a.vy[at], v[2] = a.vz[at];
+  }
+  if (a.xo) last[0] = a.xo[at], last[1] = a.yo[at], last[2] = a.zo[at];
+  if (DRIFT && stop) return;
   if (a.cnt)
-    for (int k = i; k < a.nbins; k += gridDim.x * kBlock) a.cnt[k] = 0;
+    for (int k = i; k < a.nbins; k += gridDim.x * BS) a.cnt[k] = 0;
   int cnt = 0, moved = 0;
   if (i < a.n) {
     double *p[3] = {a.x + i, a.y + i, a.z + i};
-    double r[3];
+    double r[3] = {old[0], old[1], old[2]};
     if constexpr (DRIFT) {
-      const double acc[3] = {a.ax[i], a.ay[i], a.az[i]};
-      const double v[3] = {a.vx[i], a.vy[i], a.vz[i]};
       if (isnan(acc[0]) || isnan(acc[1]) || isnan(acc[2])) a.flags[F_NAN] = 1;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        r[d] = *p[d];
         a.snap[(long)d * a.n + i] = r[d];
         a.snap[(long)(3 + d) * a.n + i] = v[d];
         a.snap[(long)(6 + d) * a.n + i] = acc[d];
@@ -534,9 +546,6 @@ __global__ __launch_bounds__(kBlock) void k_move(MoveArgs a, GhostRule rule)
       a.aox[i] = acc[0];
       a.aoy[i] = acc[1];
       a.aoz[i] = acc[2];
-    } else {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) r[d] = *p[d];
     }
     bool wrapped = false;
 #pragma unroll
@@ -560,13 +569,13 @@ __global__ __launch_bounds__(kBlock) void k_move(MoveArgs a, GhostRule rule)
     rule.sides(r[0], r[1], r[2], sx, sy, sz);
     cnt = GhostRule::images(sx, sy, sz);
     if (a.xo) {
-      const double dx = xsub(r[0], a.xo[i]), dy = xsub(r[1], a.yo[i]), dz = xsub(r[2], a.zo[i]);
+      const double dx = xsub(r[0], last[0]), dy = xsub(r[1], last[1]), dz = xsub(r[2], last[2]);
       moved = dot_rn(dx, dy, dz) > a.thr_sq;
     }
   }
   if (moved) a.flags[F_REBUILD] = 1;
   int none = 0;
-  block_sum2(cnt, none);
+  block_sum2<BS>(cnt, none);
   if (threadIdx.x == 0) a.blk[blockIdx.x] = cnt;
 }
 
@@ -584,7 +593,7 @@ struct GhostArgs {
   double4 *xq;  // packed copies, or nullptr
   int2 *tid;
   u64t *cnt;    // cells (owned count in the high word), or nullptr
-  int *bucket, *bin_of;
+  int *bucket;
   int cap;
 };
 
@@ -597,89 +606,117 @@ struct GhostArgs {
 // packed for the gathers and put into its cell's bucket, whether the list is
 // rebuilt or not: the decision is not known yet, and the counting is cheaper
 // than a launch of its own.
-__global__ __launch_bounds__(kBlock) void k_ghosts(GhostArgs a, GhostRule rule, BinRule bins)
+template <int BS>
+__global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinRule bins)
 {
-  if (a.flags[F_STOP]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  // every load that depends on nothing first: at small sizes the kernel is a
+  // chain of such latencies
+  const int i = blockIdx.x * BS + threadIdx.x;
+  const bool live = i < a.n;
+  const int at = live ? i : 0;
+  const double px = a.x[at], py = a.y[at], pz = a.z[at], qq = a.q[at];
+  const int t = a.type[at], d = a.id[at], m = a.mol[at];
+  const int stop = a.flags[F_STOP], old = a.flags[F_NGHOST_OLD];
   int before, total;
   if (a.scanned) {
     before = a.blk[blockIdx.x];
     total = a.flags[F_NGHOST];
   } else {
     before = total = 0;
-    for (int k = threadIdx.x; k < a.nblk; k += kBlock) {
+    for (int k = threadIdx.x; k < a.nblk; k += BS) {
       const int v = a.blk[k];
       total += v;
       if (k < (int)blockIdx.x) before += v;
     }
-    block_sum2(before, total);
+    block_sum2<BS>(before, total);
   }
-  double px = 0, py = 0, pz = 0;
+  if (stop) return;
   int sx = 0, sy = 0, sz = 0, cnt = 0;
-  if (i < a.n) {
-    px = a.x[i];
-    py = a.y[i];
-    pz = a.z[i];
+  if (live) {
     rule.sides(px, py, pz, sx, sy, sz);
     cnt = GhostRule::images(sx, sy, sz);
   }
-  const int off = before + block_exclusive_scan(cnt, nullptr);
+  const int off = before + block_exclusive_scan<BS>(cnt, nullptr);
   bool test = false;
   if (a.xo) {
-    const bool differs = a.rebuild_test || total != a.flags[F_NGHOST_OLD];
+    const bool differs = a.rebuild_test || total != old;
     test = !differs;
     if (differs && i == 0) a.flags[F_REBUILD] = 1;
   }
   if (i == 0 && !a.scanned) a.flags[F_NGHOST] = total;
-  if (i >= a.n) return;
-  const int t = a.type[i], d = a.id[i], m = a.mol[i];
-  const double qq = a.q[i];
-  auto slot = [&](long s, double u, double v, double w, bool owned) {
+  if (!live) return;
+  const double gx = px - sx * a.L[0], gy = py - sy * a.L[1], gz = pz - sz * a.L[2];
+  // slot 0 is the atom itself, 1..7 its images in order (the axes they shift as
+  // bits: x, y, z, xy, xz, yz, xyz).  The counters' answers are asked for
+  // first, in variables of their own (an array's elements are copied together,
+  // which waits for each), so that up to eight atomics are in flight at once:
+  // one after the other they were most of this kernel's time at small sizes.
+  const int sides = (sx ? 1 : 0) | (sy ? 2 : 0) | (sz ? 4 : 0);
+  auto cell_of = [&](int ax) { return bins(ax & 1 ? gx : px, ax & 2 ? gy : py, ax & 4 ? gz : pz); };
+  u64t r0, r1, r2, r3, r4, r5, r6, r7;
+  if (a.cnt) {
+    r0 = atomicAdd(a.cnt + cell_of(0), 1ull << 32 | 1ull);
+    if (sides & 1) r1 = atomicAdd(a.cnt + cell_of(1), 1ull);
+    if (sides & 2) r2 = atomicAdd(a.cnt + cell_of(2), 1ull);
+    if (sides & 4) r3 = atomicAdd(a.cnt + cell_of(4), 1ull);
+    if ((sides & 3) == 3) r4 = atomicAdd(a.cnt + cell_of(3), 1ull);
+    if ((sides & 5) == 5) r5 = atomicAdd(a.cnt + cell_of(5), 1ull);
+    if ((sides & 6) == 6) r6 = atomicAdd(a.cnt + cell_of(6), 1ull);
+    if (sides == 7) r7 = atomicAdd(a.cnt + cell_of(7), 1ull);
+  }
+  int g = off;
+  auto put = [&](int ax) {
+    const double u = ax & 1 ? gx : px, v = ax & 2 ? gy : py, w = ax & 4 ? gz : pz;
+    long s = i;
+    if (ax > 0) {
+      s = (long)a.n + g;
+      if (test) {
+        const double dx = xsub(u, a.xo[s]), dy = xsub(v, a.yo[s]), dz = xsub(w, a.zo[s]);
+        if (dot_rn(dx, dy, dz) > a.thr_sq) a.flags[F_REBUILD] = 1;
+      }
+      a.x[s] = u;
+      a.y[s] = v;
+      a.z[s] = w;
+      a.type[s] = t;
+      a.id[s] = d;
+      a.mol[s] = m;
+      a.q[s] = qq;
+      a.gsrc[g] = i;
+      ++g;
+    }
     if (a.xq) {
       a.xq[s] = make_double4(u, v, w, qq);
       a.tid[s] = make_int2(t, d);
     }
-    if (a.cnt) {
-      const int b = bins(u, v, w);
-      const int rank = (int)atomicAdd(a.cnt + b, owned ? (1ull << 32 | 1ull) : 1ull);
-      a.bin_of[s] = b;
-      if (rank < a.cap) a.bucket[(long)b * a.cap + rank] = (int)s;
-    }
   };
-  slot(i, px, py, pz, true);
-  if (cnt == 0) return;
-  const double gx = px - sx * a.L[0], gy = py - sy * a.L[1], gz = pz - sz * a.L[2];
-  int g = off;
-  auto put = [&](double u, double v, double w) {
-    const long s = (long)a.n + g;
-    if (test) {
-      const double dx = xsub(u, a.xo[s]), dy = xsub(v, a.yo[s]), dz = xsub(w, a.zo[s]);
-      if (dot_rn(dx, dy, dz) > a.thr_sq) a.flags[F_REBUILD] = 1;
-    }
-    a.x[s] = u;
-    a.y[s] = v;
-    a.z[s] = w;
-    a.type[s] = t;
-    a.id[s] = d;
-    a.mol[s] = m;
-    a.q[s] = qq;
-    a.gsrc[g] = i;
-    slot(s, u, v, w, false);
-    ++g;
+  put(0);
+  if (sides & 1) put(1);
+  if (sides & 2) put(2);
+  if (sides & 4) put(4);
+  if ((sides & 3) == 3) put(3);
+  if ((sides & 5) == 5) put(5);
+  if ((sides & 6) == 6) put(6);
+  if (sides == 7) put(7);
+  if (!a.cnt) return;
+  auto keep = [&](long s, int ax, u64t r) {
+    const int b = cell_of(ax), rank = (int)(unsigned)r;
+    if (rank < a.cap) a.bucket[(long)b * a.cap + rank] = (int)s;
   };
-  if (sx) put(gx, py, pz);
-  if (sy) put(px, gy, pz);
-  if (sz) put(px, py, gz);
-  if (sx && sy) put(gx, gy, pz);
-  if (sx && sz) put(gx, py, gz);
-  if (sy && sz) put(px, gy, gz);
-  if (sx && sy && sz) put(gx, gy, gz);
+  long s = (long)a.n + off;
+  keep(i, 0, r0);
+  if (sides & 1) keep(s++, 1, r1);
+  if (sides & 2) keep(s++, 2, r2);
+  if (sides & 4) keep(s++, 4, r3);
+  if ((sides & 3) == 3) keep(s++, 3, r4);
+  if ((sides & 5) == 5) keep(s++, 5, r5);
+  if ((sides & 6) == 6) keep(s++, 6, r6);
+  if (sides == 7) keep(s++, 7, r7);
 }
 
 struct CellBuild {
   int n, nbins, bpb, cap;
   const u64t *cnt;
-  const int *bucket, *bin_of;
+  const int *bucket;
   const double4 *xq;
   const int2 *tid;
   int *start, *items, *order, *binpos, *litems;
@@ -699,13 +736,23 @@ constexpr int kCellBlock = 1024;
 // build's candidates and the packed copies; pos_old as well
 // (neighborlist.cpp:302-303).  Without a rebuild only the packed copies are
 // refreshed, in the order of the last one.
-__global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
+__global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
 {
-  if (a.flags[F_STOP]) return;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = a.flags[F_NGHOST];
+  const int G = a.flags[F_NGHOST], stop = a.flags[F_STOP], rebuild = a.flags[F_REBUILD];
+  const int b0 = blockIdx.x * a.bpb;
+  // counters before the workgroup's cells, its own, and the slots of each
+  // wave's first cell (whatever the bucket holds past its count): asked for
+  // together, before the flags are known
+  u64t s = 0;
+#pragma unroll 4
+  for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
+  const u64t own = lane < a.bpb && b0 + lane < a.nbins ? a.cnt[b0 + lane] : 0;
+  const int early = lane < a.cap && wv < a.bpb && b0 + wv < a.nbins
+                        ? a.bucket[(long)(b0 + wv) * a.cap + lane] : 0;
   const long tot = (long)a.n + G;
-  if (!a.flags[F_REBUILD]) {
+  if (stop) return;
+  if (!rebuild) {
     for (long t = (long)blockIdx.x * kCellBlock + threadIdx.x; t < tot;
          t += (long)gridDim.x * kCellBlock) {
       const int j = a.litems[t];
@@ -717,10 +764,6 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
   if (blockIdx.x == 0 && threadIdx.x == 0) a.flags[F_NGHOST_OLD] = G;
   __shared__ u64t part[kCellBlock / 64];
   __shared__ u64t first[65];  // per cell: slots before it, owned atoms before it
-  const int b0 = blockIdx.x * a.bpb;
-  u64t s = 0;
-#pragma unroll 4
-  for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   if (lane == 0) part[wv] = s;
   __syncthreads();
@@ -728,7 +771,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
     u64t base = lane < kCellBlock / 64 ? part[lane] : 0;
     for (int o = 8; o > 0; o >>= 1) base += __shfl_xor(base, o, 16);
     base = __shfl(base, 0, 64);
-    const u64t v = lane < a.bpb && b0 + lane < a.nbins ? a.cnt[b0 + lane] : 0;
+    const u64t v = own;
     u64t inc = v;
     for (int o = 1; o < 64; o <<= 1) {
       const u64t u = __shfl_up(inc, o, 64);
@@ -750,7 +793,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
     int j0 = 0x7fffffff, rank = 0;
     if (m <= 64 && m <= a.cap) {
       // one slot per lane, ranked by the smaller indices of the others
-      if (lane < m) j0 = mine[lane];
+      if (lane < m) j0 = w == wv ? early : mine[lane];
       for (int k = 0; k < m; ++k) rank += __builtin_amdgcn_readlane(j0, k) < j0 ? 1 : 0;
     } else {
       // large cells through memory: the unsorted slots (those past the bucket's
@@ -758,7 +801,11 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a)
       if (m > a.cap) {
         int at = 0;
         for (long t0 = 0; t0 < tot; t0 += 64) {
-          const bool in = t0 + lane < tot && a.bin_of[t0 + lane] == b;
+          bool in = false;
+          if (t0 + lane < tot) {
+            const double4 v = a.xq[t0 + lane];
+            in = bins(v.x, v.y, v.z) == b;
+          }
           const u64t mask = __ballot(in);
           if (in) a.items[s0 + at + __popcll(mask & ((1ull << lane) - 1ull))] = (int)(t0 + lane);
           at += __popcll(mask);
@@ -826,6 +873,13 @@ int cells_alloc(cav_ctx *c)
   return CAV_OK;
 }
 
+// Threads per workgroup of the move and the ghosts (the image counts are per
+// workgroup of both): one wave for few atoms, so that the images' scattered
+// stores (up to eighty an atom) spread over more CUs.  The ghosts
+// of 256 atoms 14.2 -> 8.5 us, of 4000 11.5 -> 9.3, of 8000 12.2 -> 10.2; 30011
+// 12.3 -> 13.3, which keeps 256.
+static int move_block(const cav_ctx *c) { return c->n <= 16384 ? 64 : kBlock; }
+
 // Owned atoms moved (drift of dt, or only wrapped) and the images counted;
 // `decide`: with the rebuild test.
 int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
@@ -860,10 +914,10 @@ int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
   a.blk = c->blk;
   a.cnt = fused_cells(c) ? c->cell_cnt : nullptr;
   a.nbins = c->xnbins;
-  if (drift)
-    k_move<true><<<grid_for(c->n), kBlock, 0, c->stream>>>(a, ghost_rule(c));
-  else
-    k_move<false><<<grid_for(c->n), kBlock, 0, c->stream>>>(a, ghost_rule(c));
+  const int bs = move_block(c), nb = grid_for(c->n, bs);
+  const auto kern = bs == 64 ? (drift ? k_move<true, 64> : k_move<false, 64>)
+                             : (drift ? k_move<true, kBlock> : k_move<false, kBlock>);
+  kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -871,7 +925,7 @@ int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
 // Images of the moved atoms, and the rebuild decision; after launch_move.
 int launch_ghosts(cav_ctx *c, bool decide)
 {
-  const int nb = grid_for(c->n);
+  const int bs = move_block(c), nb = grid_for(c->n, bs);
   GhostArgs a;
   a.n = c->n;
   a.nblk = nb;
@@ -898,11 +952,11 @@ int launch_ghosts(cav_ctx *c, bool decide)
   a.tid = c->tid;
   a.cnt = fused ? c->cell_cnt : nullptr;
   a.bucket = c->bucket;
-  a.bin_of = c->bin_of;
   a.cap = c->bucket_cap;
   if (a.scanned)
     k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
-  k_ghosts<<<nb, kBlock, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
+  const auto kern = bs == 64 ? k_ghosts<64> : k_ghosts<kBlock>;
+  kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -919,7 +973,6 @@ int launch_cells(cav_ctx *c)
   a.cap = c->bucket_cap;
   a.cnt = c->cell_cnt;
   a.bucket = c->bucket;
-  a.bin_of = c->bin_of;
   a.xq = c->xq;
   a.tid = c->tid;
   a.start = c->bin_start;
@@ -934,7 +987,7 @@ int launch_cells(cav_ctx *c)
   a.yo = c->yo;
   a.zo = c->zo;
   a.flags = c->flags;
-  k_cells<<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a);
+  k_cells<<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -994,7 +1047,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
                                                   const int *items, int *nl, int *nn, int *flags,
                                                   const int *cond, const RepDev *rep,
                                                   const int *cell_rep, unsigned short *nll,
-                                                  int *nlb)
+                                                  int *nlb, int split)
 {
   // Each wave builds the rows of one cell on its own (wave-local LDS, no
   // block barrier).  The wave index is read as a scalar so that everything
@@ -1015,7 +1068,10 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
     start += r;  // every replica's cell starts carry one closing entry
   }
   if (cond && !*cond) return;
-  if (!rep && b == 0 && threadIdx.x == 0) flags[F_NL_STALE] = NL ? 0 : 1;
+  // with `split` waves per cell (blockIdx.y), this one takes every split-th
+  // group of kAPI owned atoms
+  const int part = blockIdx.y;
+  if (!rep && b == 0 && part == 0 && threadIdx.x == 0) flags[F_NL_STALE] = NL ? 0 : 1;
   // staged candidates (x, y, z, index and slot) in the cell's stencil order; a stage is
   // padded to a multiple of 64 with far-away entries so every lane tests one
   __shared__ double4 sc_[kListWaves][kCand];
@@ -1028,7 +1084,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
     const int v = (t + lane < e0) ? items[t + lane] - base : n;
     no += __popcll(__ballot(v < n));
   }
-  if (no == 0) return;
+  if (no <= kAPI * part) return;
   const int sb = st_off[b], ns = st_off[b + 1] - sb;  // <= 27 stencil cells
   // padding and empty owned slots sit at +-1e300: their squared distance to
   // anything is +inf, so they never pass the cutoff test
@@ -1079,7 +1135,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
       const int mpad = (m + 63) & ~63;
       if (m + lane < mpad) sc[m + lane] = far_cand;
       __syncwarp();
-      for (int o0 = 0; o0 < gsize; o0 += kAPI) {
+      for (int o0 = kAPI * part; o0 < gsize; o0 += kAPI * split) {
         // the kAPI owned atoms are the same for every lane: positions, slots,
         // row offsets and row counters in scalar registers (empty slots of
         // the group carry the far sentinel and never pass)
@@ -1136,7 +1192,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
       }
       __syncwarp();
     }
-    if (lane < gsize) {
+    if (lane < gsize && lane / kAPI % split == part) {
       const int i = cpos_index(mine.w) - base + obase;
       nn[i] = cnt < cap ? cnt : cap;
       // the longest row is needed only to regrow the list after an overflow:
@@ -1158,10 +1214,16 @@ static void launch_list_wave(hipStream_t st, int n, int nbins, int cap, double r
                              const int *cond, const RepDev *rep, const int *cell_rep,
                              unsigned short *nll, int *nlb)
 {
-  const dim3 g(list_grid(nbins)), blk(64 * kListWaves);
+  // Waves per cell: small grids leave CUs idle, and a wave's chain over its
+  // atoms' groups is then the kernel's time; every wave stages the candidates
+  // for itself, so a full chip keeps one.  Measured with 1 / 2 / 3 / 6 waves
+  // (us): 125 cells 24 / 16 / 13 / 11, 1000 cells 34 / 23 / 20 / 17, 2744 cells
+  // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
+  const int split = std::max(1, std::min(6, 8192 / nbins));
+  const dim3 g(list_grid(nbins), split), blk(64 * kListWaves);
 #define CAV_LISTW(A, B, C)                                                                      \
   k_list_wave<A, B, C><<<g, blk, 0, st>>>(n, nbins, cap, rce2, cpos, st_off, stc, start, items, \
-                                          nl, nn, flags, cond, rep, cell_rep, nll, nlb)
+                                          nl, nn, flags, cond, rep, cell_rep, nll, nlb, split)
   if (nlb && !nl)
     CAV_LISTW(false, false, true);
   else if (nlb)

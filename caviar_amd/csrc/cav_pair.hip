@@ -170,19 +170,17 @@ __device__ __forceinline__ void block_virial(double vir, double *part)
   }
 }
 
-// Row-gather pair kernel: kLPA lanes share one atom's row (coalesced row
+// Row-gather pair kernel: LPA lanes share one atom's row (coalesced row
 // reads, balanced work); each lane fetches pair_u<T>() indices, then their (x, y,
 // z, q) and (type, id), before computing, so the gathers overlap.  The
 // partial forces of an atom's lanes are summed with a fixed shuffle tree, so
 // FP64 results stay reproducible.
-template <typename T, bool LJ, bool ER, bool LAM, bool BINS>
+template <typename T, bool LJ, bool ER, bool LAM, bool BINS, int LPA = kLPA>
 __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
 {
   extern __shared__ double dyn_pair[];
   T *tab = reinterpret_cast<T *>(dyn_pair);
   const int nt2 = LJ ? a.nt * a.nt : 0;
-  stage_lj_tables(a, nt2, tab);
-  __syncthreads();
   if (a.rep) {  // one replica per grid row: shift every array to it
     const RepDev &r = a.rep[blockIdx.y];
     const int base = r.base, obase = r.obase;
@@ -212,28 +210,35 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
     blk = (long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
   }
   const long gid = blk * kBlock + threadIdx.x;
-  const int t = (int)(gid / kLPA), sub = (int)(gid % kLPA);
+  const int t = (int)(gid / LPA), sub = (int)(gid % LPA);
   double vir = 0.0;
   T fx = 0, fy = 0, fz = 0;
-  int i = 0, ti = 0;
+  int i = 0, ti = 0, cnt = 0, moli = 0;
+  double4 pi4 = make_double4(0, 0, 0, 0);
+  int2 tii = make_int2(0, 0);
   if (t < a.n) {
     i = a.order ? a.order[t] : t;
-    const double4 pi4 = a.xq[i];
-    const int2 tii = a.tid[i];
+    pi4 = a.xq[i];
+    tii = a.tid[i];
+    moli = LAM ? a.mol[i] : 0;
+    cnt = a.nn[i];
+  }
+  // (staged while the atom's own loads are under way)
+  stage_lj_tables(a, nt2, tab);
+  __syncthreads();
+  if (t < a.n) {
     ti = tii.x;
-    const int moli = LAM ? a.mol[i] : 0;
     const T qi = (T)pi4.w;
     const T keqi = (T)(a.ke) * qi;
-    const int cnt = a.nn[i];
     const int *row = (BINS ? a.nlb : a.nl) + (long)i * a.cap;
     constexpr int U = pair_u<T>();
-    for (int k0 = sub; k0 < cnt; k0 += U * kLPA) {
+    for (int k0 = sub; k0 < cnt; k0 += U * LPA) {
       int jj[U];
       double4 pj[U];
       int2 tj[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int k = k0 + u * kLPA;
+        const int k = k0 + u * LPA;
         jj[u] = k < cnt ? row[k] : -1;
       }
       if constexpr (BINS) {
@@ -266,7 +271,7 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
     }
   }
 #pragma unroll
-  for (int o = 1; o < kLPA; o <<= 1) {
+  for (int o = 1; o < LPA; o <<= 1) {
     fx += __shfl_xor(fx, o, 64);
     fy += __shfl_xor(fy, o, 64);
     fz += __shfl_xor(fz, o, 64);
@@ -718,34 +723,50 @@ static PairArgs pair_args(cav_ctx *c)
   return a;
 }
 
-static int pair_grid(const cav_ctx *c) { return (grid_for((long)c->n * kLPA) + 7) / 8 * 8; }
-int pair_blocks(const cav_ctx *c) { return pair_grid(c); }
+static int pair_grid(const cav_ctx *c, int lpa = kLPA)
+{
+  return (grid_for((long)c->n * lpa) + 7) / 8 * 8;
+}
 
-template <typename T, bool BINS>
+// Lanes per atom of the row pair kernel (through slots and through indices
+// alike, so that both sum in one order): more where the chip has room, since a
+// lane's serial groups of gathers are then its time.  Measured with 8 / 16 / 32 lanes (us): 256 LJ atoms 8.5 / 6.2 / 5.1, 4000 9.1 /
+// 6.5 / 6.0, 8000 ions (FP64) 14.0 / 13.5 / 11.8, 30011 (mixed) 19.3 / 19.4 /
+// 24.0, 65536 (FP64) 101 / 112 / 118.
+static int pair_lanes(const cav_ctx *c) { return c->n <= 16384 ? 32 : kLPA; }
+
+int pair_blocks(const cav_ctx *c) { return pair_grid(c, pair_lanes(c)); }
+
+template <typename T, bool BINS, int LPA>
 static void launch_pairs_tb(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
 {
-  const int g = pair_grid(c);
+  const int g = pair_grid(c, LPA);
   const size_t lds = 3 * sizeof(T) * a.nt * a.nt;  // LJ tables
   if (lj && er && lam)
-    k_pairs<T, true, true, true, BINS><<<g, kBlock, lds, c->stream>>>(a);
+    k_pairs<T, true, true, true, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
   else if (lj && er)
-    k_pairs<T, true, true, false, BINS><<<g, kBlock, lds, c->stream>>>(a);
+    k_pairs<T, true, true, false, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
   else if (lj)
-    k_pairs<T, true, false, false, BINS><<<g, kBlock, lds, c->stream>>>(a);
+    k_pairs<T, true, false, false, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
   else if (er && lam)
-    k_pairs<T, false, true, true, BINS><<<g, kBlock, 0, c->stream>>>(a);
+    k_pairs<T, false, true, true, BINS, LPA><<<g, kBlock, 0, c->stream>>>(a);
   else
-    k_pairs<T, false, true, false, BINS><<<g, kBlock, 0, c->stream>>>(a);
+    k_pairs<T, false, true, false, BINS, LPA><<<g, kBlock, 0, c->stream>>>(a);
 }
 
 // rows as bin-order slots (a.nlb) or as atom indices, each its own kernel
 template <typename T>
 static void launch_pairs_t(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
 {
-  if (a.nlb)
-    launch_pairs_tb<T, true>(c, a, lj, er, lam);
+  const bool wide = pair_lanes(c) == 32;
+  if (a.nlb && wide)
+    launch_pairs_tb<T, true, 32>(c, a, lj, er, lam);
+  else if (a.nlb)
+    launch_pairs_tb<T, true, kLPA>(c, a, lj, er, lam);
+  else if (wide)
+    launch_pairs_tb<T, false, 32>(c, a, lj, er, lam);
   else
-    launch_pairs_tb<T, false>(c, a, lj, er, lam);
+    launch_pairs_tb<T, false, kLPA>(c, a, lj, er, lam);
 }
 
 // The cell-staged kernel runs on request (CAV_PAIRS_CELLS) where it applies:
@@ -863,7 +884,7 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate, bool p
   const long tot = (long)c->n + c->gcap;
   const bool cells = cell_staged(c);
   // every block writes one virial partial: the buffer must cover the grid
-  if ((cells ? cell_grid(c) : pair_grid(c)) > c->npart)
+  if ((cells ? cell_grid(c) : pair_blocks(c)) > c->npart)
     return fail(c, CAV_ERR_STATE, "partial-sum buffer smaller than the pair grid");
   const bool bins = !cells && sorted_rows(c);
   if (bins) {
@@ -893,7 +914,7 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate, bool p
   timer_end(c, c->t_pair);
   CAV_HIP(hipGetLastError());
   if (!reduce) return CAV_OK;
-  return reduce_partials(c, cells ? cell_grid(c) : pair_grid(c), 0, accumulate);
+  return reduce_partials(c, cells ? cell_grid(c) : pair_blocks(c), 0, accumulate);
 }
 
 __global__ void k_zero_acc(int n, double *ax, double *ay, double *az)

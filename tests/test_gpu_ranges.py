@@ -150,3 +150,26 @@ def test_crowded_cells(gpu, clump):
     assert np.array_equal(gp, og) and np.array_equal(gs, os_)
     assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs()))
     assert F.rel_err(e.get("acc"), o.get("acc")) <= 1e-11  # close pairs cancel more
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 257, 16383, 16385])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_steps_at_workgroup_edges(gpu, n, precision):
+    """Atom counts about the sizes where workgroups, lanes per atom and waves
+    per cell change: 12 steps, list kept and rebuilt, against the oracle
+    (1e-9 after the steps; mixed 1e-5), ghosts and pairs exactly."""
+    print(f"[case] steps n={n} {precision}", flush=True)
+    s = configs.ions(n=n, rho=0.3, kmax=2, seed=n)
+    o = Oracle(s, threads=8)
+    o.setup()
+    assert o.run(0.002, 12) == 0
+    e = Engine(s, precision=precision)
+    e.setup()
+    e.step(0.002, 5)
+    e.step(0.002, 7)
+    tol = 1e-9 if precision == "fp64" else 1e-5
+    for what in ("pos", "vel", "acc"):
+        assert F.rel_err(e.get(what), o.get(what)) <= tol, what
+    if precision == "fp64":
+        assert abs(e.virial() - o.virial()) <= 1e-9 * abs(o.virial())
+        assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs()))
