@@ -154,6 +154,113 @@ __global__ void k_ghost_charge_of_type(int n, int gcap, const int *flags, const 
   if (g < ng) q[n + g] = charge[type[n + g]];
 }
 
+// ----------------------------------------------------------- host exchanges --
+
+bool stage_room(Stage &s, size_t count)
+{
+  if (count <= s.cap) return true;
+  if (count * sizeof(double) > kStageMax) return false;
+  stage_free(s);
+  const size_t want = std::max(count, (size_t)4096);
+  if (hipHostMalloc((void **)&s.host, sizeof(double) * want) != hipSuccess ||
+      hipHostGetDevicePointer((void **)&s.dev, s.host, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    stage_free(s);
+    return false;
+  }
+  for (hipEvent_t &e : s.ev)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      stage_free(s);
+      return false;
+    }
+  s.cap = want;
+  return true;
+}
+
+void stage_free(Stage &s)
+{
+  if (s.host) (void)hipHostFree(s.host);
+  for (hipEvent_t &e : s.ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+  s.host = s.dev = nullptr;
+  s.cap = 0;
+}
+
+// Elements e0 .. e1 of the AoS triples, written to (or read from) host memory
+// in order: whole cache lines over the link, whose rate bounds both.
+__global__ void k_to_host3(long e0, long e1, const double *a, const double *b, const double *c,
+                           double *out)
+{
+  const long e = e0 + (long)blockIdx.x * kBlock + threadIdx.x;
+  if (e >= e1) return;
+  const long i = e / 3;
+  const int k = (int)(e - 3 * i);
+  out[e] = k == 0 ? a[i] : (k == 1 ? b[i] : c[i]);
+}
+
+__global__ void k_from_host3(long count, const double *in, double *a, double *b, double *c)
+{
+  const long e = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (e >= count) return;
+  const long i = e / 3;
+  const int k = (int)(e - 3 * i);
+  (k == 0 ? a : (k == 1 ? b : c))[i] = in[e];
+}
+
+__global__ void k_copy_d(long count, const double *in, double *out)
+{
+  const long e = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (e < count) out[e] = in[e];
+}
+
+// Downloads above 1 MB go in pieces: the host copies one out of the pinned
+// memory while the next ones cross the link.
+hipError_t stage_get3(Stage &s, hipStream_t st, long n, const double *a, const double *b,
+                      const double *c, double *out)
+{
+  const long count = 3 * n;
+  const int parts = count > 131072 ? kStageParts : 1;
+  const long per = (count + parts - 1) / parts;
+  for (int p = 0; p < parts; ++p) {
+    const long e0 = p * per, e1 = std::min(count, e0 + per);
+    if (e0 < e1) k_to_host3<<<grid_for(e1 - e0), kBlock, 0, st>>>(e0, e1, a, b, c, s.dev);
+    if (hipError_t e = hipEventRecord(s.ev[p], st)) return e;
+  }
+  for (int p = 0; p < parts; ++p) {
+    const long e0 = p * per, e1 = std::min(count, e0 + per);
+    if (hipError_t e = hipEventSynchronize(s.ev[p])) return e;
+    if (e0 < e1) std::memcpy(out + e0, s.host + e0, sizeof(double) * (e1 - e0));
+  }
+  return hipGetLastError();
+}
+
+hipError_t stage_put3(Stage &s, hipStream_t st, long n, const double *in, double *a, double *b,
+                      double *c)
+{
+  std::memcpy(s.host, in, sizeof(double) * 3 * n);
+  if (n > 0) k_from_host3<<<grid_for(3 * n), kBlock, 0, st>>>(3 * n, s.dev, a, b, c);
+  return hipStreamSynchronize(st);  // the staging memory is free again
+}
+
+hipError_t stage_get(Stage &s, hipStream_t st, size_t count, const double *src, double *out)
+{
+  if (count) k_copy_d<<<grid_for((long)count), kBlock, 0, st>>>((long)count, src, s.dev);
+  if (hipError_t e = hipStreamSynchronize(st)) return e;
+  std::memcpy(out, s.host, sizeof(double) * count);
+  return hipGetLastError();
+}
+
+// (the staging memory is in use until the stream has passed this point)
+hipError_t stage_put(Stage &s, hipStream_t st, size_t count, const double *in, double *dst)
+{
+  std::memcpy(s.host, in, sizeof(double) * count);
+  if (count) k_copy_d<<<grid_for((long)count), kBlock, 0, st>>>((long)count, s.dev, dst);
+  return hipGetLastError();
+}
+
 }  // namespace cav
 
 using namespace cav;
@@ -187,10 +294,11 @@ static void free_all(cav_ctx *c)
                   c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos, c->sk_sum,
                   c->binpos,  c->xqs,    c->tids,       c->nll,    c->nlb,    c->lstart, c->litems,
                   c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part,
-                  c->cell_cnt, c->bucket};
+                  c->cell_cnt, c->bucket, c->pt_dev, c->pt_tab};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_flags) (void)hipHostFree(c->h_flags);
+  stage_free(c->stage);
 }
 
 static int upload_params(cav_ctx *c)
@@ -498,6 +606,14 @@ static int neighbor_phase(cav_ctx *c, Rebuild how, bool fused)
   }
   if (!fused) CAV_TRY(launch_save_old(c, true));
   timer_end(c, c->t_list);
+  return CAV_OK;
+}
+
+// The first `count` device scalars.
+static int read_scal(cav_ctx *c, int count, double *v)
+{
+  if (!stage_room(c->stage, count)) return fail(c, CAV_ERR_HIP, "no pinned host memory");
+  CAV_HIP(stage_get(c->stage, c->stream, count, c->scal, v));
   return CAV_OK;
 }
 
@@ -991,6 +1107,11 @@ int cav_download(cav_ctx *c, int which, double *out)
 {
   if (!c || !out || which < 0 || which > 3) return fail(c, CAV_ERR_ARG, "bad download request");
   (void)hipSetDevice(c->device);
+  if (stage_room(c->stage, 3 * (size_t)c->n)) {
+    CAV_HIP(stage_get3(c->stage, c->stream, c->n, soa_of(c, which, 0), soa_of(c, which, 1),
+                       soa_of(c, which, 2), out));
+    return CAV_OK;
+  }
   std::vector<double> soa(3 * (size_t)c->n);
   for (int k = 0; k < 3; ++k)
     CAV_HIP(hipMemcpyAsync(soa.data() + (size_t)k * c->n, soa_of(c, which, k), sizeof(double) * c->n,
@@ -1005,6 +1126,11 @@ int cav_upload(cav_ctx *c, int which, const double *in)
 {
   if (!c || !in || which < 0 || which > 3) return fail(c, CAV_ERR_ARG, "bad upload request");
   (void)hipSetDevice(c->device);
+  if (stage_room(c->stage, 3 * (size_t)c->n)) {
+    CAV_HIP(stage_put3(c->stage, c->stream, c->n, in, soa_of(c, which, 0), soa_of(c, which, 1),
+                       soa_of(c, which, 2)));
+    return CAV_OK;
+  }
   std::vector<double> soa(3 * (size_t)c->n);
   for (int i = 0; i < c->n; ++i)
     for (int k = 0; k < 3; ++k) soa[(size_t)k * c->n + i] = in[3 * i + k];
@@ -1481,9 +1607,7 @@ int cav_list_stats(cav_ctx *c, double *ppa, double *lj_ppa)
 int cav_virial(cav_ctx *c, double *v)
 {
   if (!c || !v) return CAV_ERR_ARG;
-  CAV_HIP(hipMemcpyAsync(v, c->scal, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
-  return CAV_OK;
+  return read_scal(c, 1, v);
 }
 
 int cav_num_kvectors(cav_ctx *c, int *nk)
@@ -1533,8 +1657,7 @@ int cav_energy(cav_ctx *c, double *e_lj, double *e_r, double *e_k)
   }
   // one read-back for every term: [1] LJ, [2] real space, [3] lattice, [8..10] dipole
   double v[12];
-  CAV_HIP(hipMemcpyAsync(v, c->scal, sizeof(v), hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
+  CAV_TRY(read_scal(c, 12, v));
   if (e_k) *e_k = energy_k(c, v);
   if (e_r) *e_r = 0.5 * v[2] * c->er_ke;  // energy.cpp:50 and potential.cpp:85
   if (e_lj) *e_lj = v[1];

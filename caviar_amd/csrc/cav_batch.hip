@@ -167,6 +167,7 @@ static void batch_free(cav_batch *b)
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->h_flags) (void)hipHostFree(b->h_flags);
+  stage_free(b->stage);
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
 }
@@ -721,6 +722,11 @@ int cav_batch_download(cav_batch *b, int replica, int which, double *out)
   default: return CAV_ERR_ARG;
   }
   const long off = slot ? d.base : d.obase;
+  (void)hipSetDevice(b->device);
+  if (stage_room(b->stage, 3 * (size_t)d.n)) {
+    BAT_HIP(stage_get3(b->stage, b->stream, d.n, src[0] + off, src[1] + off, src[2] + off, out));
+    return CAV_OK;
+  }
   for (int k = 0; k < 3; ++k) {
     a[k].resize(d.n);
     BAT_HIP(hipMemcpyAsync(a[k].data(), src[k] + off, sizeof(double) * d.n, hipMemcpyDeviceToHost, b->stream));

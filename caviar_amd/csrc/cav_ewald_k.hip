@@ -2104,6 +2104,27 @@ double energy_k(const cav_ctx *c, const double *v)
   return ek;
 }
 
+// Room for a point query: doubles for coordinates and results, bytes of phase
+// tables; kept for the next one.
+int point_room(cav_ctx *c, size_t doubles, size_t table_bytes)
+{
+  if (doubles > c->pt_cap) {
+    if (c->pt_dev) (void)hipFree(c->pt_dev);
+    c->pt_dev = nullptr;
+    c->pt_cap = 0;
+    CAV_HIP(hipMalloc(&c->pt_dev, sizeof(double) * doubles));
+    c->pt_cap = doubles;
+  }
+  if (table_bytes > c->pt_tab_cap) {
+    if (c->pt_tab) (void)hipFree(c->pt_tab);
+    c->pt_tab = nullptr;
+    c->pt_tab_cap = 0;
+    CAV_HIP(hipMalloc(&c->pt_tab, table_bytes));
+    c->pt_tab_cap = table_bytes;
+  }
+  return CAV_OK;
+}
+
 // Point queries: tables for the points, then the force pass with q = 1 into a
 // per-point (field, potential) buffer; the dipole field is added on the host.
 int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *pot)
@@ -2111,42 +2132,50 @@ int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *
   const EwaldKPlan &p = c->ek;
   const int TS = p.nX + p.nY + p.nZ;
   const size_t tsz = c->precision == CAV_FP64 ? sizeof(double) : sizeof(float);
-  double *d;
-  void *tab;
-  CAV_HIP(hipMalloc(&d, sizeof(double) * 7 * (size_t)(np > 0 ? np : 1)));
-  CAV_HIP(hipMalloc(&tab, (size_t)(np > 0 ? np : 1) * TS * 2 * tsz));
-  std::vector<double> soa(3 * (size_t)np);
-  for (int i = 0; i < np; ++i)
-    for (int k = 0; k < 3; ++k) soa[(size_t)k * np + i] = pts[3 * i + k];
-  CAV_HIP(hipMemcpyAsync(d, soa.data(), sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
+  const size_t cnt = std::max(np, 1);
+  CAV_TRY(point_room(c, 7 * cnt + 3, cnt * TS * 2 * tsz));
+  double *d = c->pt_dev;
+  void *tab = c->pt_tab;
+  const bool staged = stage_room(c->stage, 4 * cnt + 3);
+  if (staged) {
+    CAV_HIP(stage_put3(c->stage, c->stream, np, pts, d, d + np, d + 2 * (size_t)np));
+  } else {
+    std::vector<double> soa(3 * (size_t)np);
+    for (int i = 0; i < np; ++i)
+      for (int k = 0; k < 3; ++k) soa[(size_t)k * np + i] = pts[3 * (size_t)i + k];
+    CAV_HIP(hipMemcpyAsync(d, soa.data(), sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
+    CAV_HIP(hipStreamSynchronize(c->stream));
+  }
+  double *d4 = d + 3 * (size_t)np;  // [4 np] results, then the dipole sum
   if (c->precision == CAV_FP64) {
     k_tables<double><<<grid_for((long)np * TS), kBlock, 0, c->stream>>>(
-        np, TS, p.kx, p.ky, p.kz, 1.0 / p.lx, 1.0 / p.ly, 1.0 / p.lz, d, d + np, d + 2 * np,
+        np, TS, p.kx, p.ky, p.kz, 1.0 / p.lx, 1.0 / p.ly, 1.0 / p.lz, d, d + np, d + 2 * (size_t)np,
         (Cx<double> *)tab);
-    CAV_TRY(kforce<double>(c, np, tab, d + 3 * np));
+    CAV_TRY(kforce<double>(c, np, tab, d4));
   } else {
     k_tables<float><<<grid_for((long)np * TS), kBlock, 0, c->stream>>>(
-        np, TS, p.kx, p.ky, p.kz, 1.0 / p.lx, 1.0 / p.ly, 1.0 / p.lz, d, d + np, d + 2 * np,
+        np, TS, p.kx, p.ky, p.kz, 1.0 / p.lx, 1.0 / p.ly, 1.0 / p.lz, d, d + np, d + 2 * (size_t)np,
         (Cx<float> *)tab);
-    CAV_TRY(kforce<float>(c, np, tab, d + 3 * np));
+    CAV_TRY(kforce<float>(c, np, tab, d4));
   }
-  std::vector<double> o4(4 * (size_t)np);
-  CAV_HIP(hipMemcpyAsync(o4.data(), d + 3 * np, sizeof(double) * 4 * np, hipMemcpyDeviceToHost,
-                         c->stream));
-  double dsum[3] = {0, 0, 0};
-  if (c->dipole)
-    CAV_HIP(hipMemcpyAsync(dsum, c->scal + 8, sizeof(double) * 3, hipMemcpyDeviceToHost, c->stream));
-  CAV_HIP(hipStreamSynchronize(c->stream));
+  CAV_HIP(hipMemcpyAsync(d4 + 4 * (size_t)np, c->scal + 8, sizeof(double) * 3,
+                         hipMemcpyDeviceToDevice, c->stream));
+  std::vector<double> o4(4 * (size_t)np + 3);
+  if (staged) {
+    CAV_HIP(stage_get(c->stage, c->stream, o4.size(), d4, o4.data()));
+  } else {
+    CAV_HIP(hipMemcpyAsync(o4.data(), d4, sizeof(double) * o4.size(), hipMemcpyDeviceToHost, c->stream));
+    CAV_HIP(hipStreamSynchronize(c->stream));
+  }
+  const double *dsum = o4.data() + 4 * (size_t)np;
   for (int i = 0; i < np; ++i) {
     for (int k = 0; k < 3; ++k) {
       double f = o4[4 * (size_t)i + k];
       if (c->dipole) f += -dsum[k] * p.dip_coef;
-      if (field) field[3 * i + k] = f;
+      if (field) field[3 * (size_t)i + k] = f;
     }
     if (pot) pot[i] = o4[4 * (size_t)i + 3];
   }
-  CAV_HIP(hipFree(d));
-  CAV_HIP(hipFree(tab));
   return CAV_OK;
 }
 

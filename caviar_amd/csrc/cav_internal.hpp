@@ -84,6 +84,21 @@ struct EwaldKPlan {
   std::vector<int> ref_r, ref_c, ref_conj;  // reference k order -> (row, col, conjugate?)
 };
 
+// Pinned host memory that kernels read and write in place: an exchange of a
+// few kilobytes is then one launch and one wait, where a copy to or from
+// pageable memory goes through the runtime's own staging (about 15 us each),
+// and megabytes need no copy engine start.  Grown as needed up to kStageMax,
+// given back with its owner; one exchange at a time (the owner's calls are
+// not concurrent).
+constexpr size_t kStageMax = size_t(64) << 20;  // bytes; larger exchanges use plain copies
+constexpr int kStageParts = 8;                  // pieces a large download overlaps
+
+struct Stage {
+  double *host = nullptr, *dev = nullptr;
+  size_t cap = 0;  // doubles
+  hipEvent_t ev[kStageParts] = {};
+};
+
 // One replica of a batch as the device kernels see it (see cav_batch.hip).
 // Slot arrays hold each replica's owned atoms then its ghosts from `base`;
 // owned-indexed arrays (velocities, accelerations, Verlet rows, FP64 phase
@@ -234,8 +249,12 @@ struct cav_ctx {
   // the side stream's Ewald_k leaves the dipole term to the main stream, which
   // adds it after the k-space sum (the in-order rounding: (a_sr + a_k) + a_dip)
   bool defer_dipole = false;
+  cav::Stage stage;
+  double *pt_dev = nullptr;  // point queries: coordinates and results
+  size_t pt_cap = 0;
+  void *pt_tab = nullptr;    // and their phase tables
+  size_t pt_tab_cap = 0;
   double *scal = nullptr;  // [0] virial, [1] e_lj, [2] e_r, [3] e_k, [4..] scratch
-  double *h_scal = nullptr;
 
   // Ewald_k device buffers
   void *tab = nullptr;       // phase tables (T): X[nX][n], Y[nY][n], Z[nZ][n] complex
@@ -296,6 +315,8 @@ struct cav_batch {
   double er_alpha = 1, er_ke = 1;
   double ek_alpha = 0, ek_ke = 1;
   int kx = 1, ky = 1, kz = 1;
+
+  cav::Stage stage;
 
   // replicas as given (host)
   struct HostRep {
@@ -380,6 +401,18 @@ int tuning_phase(cav_ctx *c);
 int refresh_params(cav_ctx *c);  // parameter values set after setup -> device
 void timer_end(cav_ctx *c, Timer &t);
 
+// host exchanges through a Stage (cav_api.hip): room for `count` doubles (false
+// where plain copies are to be used); three arrays of n to AoS host memory and
+// back, and plain arrays
+bool stage_room(Stage &s, size_t count);
+void stage_free(Stage &s);
+hipError_t stage_get3(Stage &s, hipStream_t st, long n, const double *a, const double *b,
+                      const double *c, double *out);
+hipError_t stage_put3(Stage &s, hipStream_t st, long n, const double *in, double *a, double *b,
+                      double *c);
+hipError_t stage_get(Stage &s, hipStream_t st, size_t count, const double *src, double *out);
+hipError_t stage_put(Stage &s, hipStream_t st, size_t count, const double *in, double *dst);
+
 // launchers (defined in the .hip files)
 int launch_move(cav_ctx *c, bool drift, double dt, bool decide);  // drift / wrap, image counts
 int launch_ghosts(cav_ctx *c, bool decide);  // images, rebuild decision, cell counts
@@ -431,6 +464,7 @@ int launch_energy_r(cav_ctx *c);   // into scal[2]
 int launch_energy_lj(cav_ctx *c);  // into scal[1]
 double energy_k(const cav_ctx *c, const double *scal);  // from the scalars of the last evaluation
 int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot);
+int point_room(cav_ctx *c, size_t doubles, size_t table_bytes);
 int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *pot);
 int reduce_partials(cav_ctx *c, int count, int slot, bool add = false);
 int bfail(cav_batch *b, int code, const std::string &msg);

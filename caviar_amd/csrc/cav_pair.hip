@@ -4,6 +4,7 @@
 // every atom gathers its own row, so FP64 results are reproducible run to run.
 // No MFMA: the pair loop is a gather over irregular rows, not a contraction.
 #include <algorithm>
+#include <cstring>
 
 #include "cav_internal.hpp"
 
@@ -1127,20 +1128,29 @@ __global__ __launch_bounds__(kBlock) void k_point_r(CellArgs c, int np, const do
 
 int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot)
 {
-  double *d;
-  CAV_HIP(hipMalloc(&d, sizeof(double) * 7 * (size_t)(np > 0 ? np : 1)));
-  CAV_HIP(hipMemcpyAsync(d, pts, sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
+  // the points are read from pinned host memory and the sums written there,
+  // both once per point
+  const bool staged = stage_room(c->stage, 7 * (size_t)np);
+  double *d = c->stage.dev;
+  if (staged)
+    std::memcpy(c->stage.host, pts, sizeof(double) * 3 * np);
+  else {
+    CAV_TRY(point_room(c, 7 * (size_t)np, 0));
+    d = c->pt_dev;
+    CAV_HIP(hipMemcpyAsync(d, pts, sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
+  }
+  double *df = d + 3 * (size_t)np, *dp = d + 6 * (size_t)np;
   if (np > 0)
     k_point_r<<<(np + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, c->stream>>>(
-        cell_args(c), np, d, c->er_alpha, c->er_ke, d + 3 * np, d + 6 * np);
+        cell_args(c), np, d, c->er_alpha, c->er_ke, df, dp);
   CAV_HIP(hipGetLastError());
-  if (field)
-    CAV_HIP(hipMemcpyAsync(field, d + 3 * np, sizeof(double) * 3 * np, hipMemcpyDeviceToHost,
-                           c->stream));
-  if (pot)
-    CAV_HIP(hipMemcpyAsync(pot, d + 6 * np, sizeof(double) * np, hipMemcpyDeviceToHost, c->stream));
+  if (!staged && field)
+    CAV_HIP(hipMemcpyAsync(field, df, sizeof(double) * 3 * np, hipMemcpyDeviceToHost, c->stream));
+  if (!staged && pot)
+    CAV_HIP(hipMemcpyAsync(pot, dp, sizeof(double) * np, hipMemcpyDeviceToHost, c->stream));
   CAV_HIP(hipStreamSynchronize(c->stream));
-  CAV_HIP(hipFree(d));
+  if (staged && field) std::memcpy(field, c->stage.host + 3 * (size_t)np, sizeof(double) * 3 * np);
+  if (staged && pot) std::memcpy(pot, c->stage.host + 6 * (size_t)np, sizeof(double) * np);
   return CAV_OK;
 }
 
