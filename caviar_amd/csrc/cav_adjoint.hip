@@ -20,7 +20,7 @@
 namespace cav {
 
 // Ewald_k pieces exposed by cav_ewald_k.hip
-int ewald_k_weighted_sk(cav_ctx *c, const double *weights, double *sk_out);
+int ewald_k_weight_sets(cav_ctx *c, const double *w, double *ss, double *sw);
 int ewald_k_field(cav_ctx *c, double *out4);
 
 constexpr int kLPAa = 16;
@@ -32,6 +32,7 @@ struct AdjArgs {
   const double4 *xq;
   const int2 *tid;
   const int *mol, *nl, *nn;
+  const int *items;       // rows hold bin-order slots to look up here, or nullptr
   const double *w;        // 3n residual weights (AoS)
   const double *eps, *sig;
   double lj_rc, lj_rc2;
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_pairs(AdjArgs a)
     const int cnt = a.nn[i];
     const int *row = a.nl + (long)i * a.cap;
     for (int k = sub; k < cnt; k += kLPAa) {
-      const int j = row[k];
+      const int j = a.items ? a.items[row[k]] : row[k];
       const double4 pj = a.xq[j];
       const double dx = pj.x - pi4.x, dy = pj.y - pi4.y, dz = pj.z - pi4.z;
       const double r2 = dx * dx + dy * dy + dz * dz;
@@ -182,13 +183,32 @@ static void launch_adjoint_pairs(int nt, dim3 grid, size_t sh, hipStream_t st, c
   }
 }
 
-__global__ void k_reduce_cols(int rows, int cols, const double *part, double *out)
+// Column sums of up to three tables of partials ([rows][cols] each), one per
+// workgroup: 16 waves take every 16th row, a lane per column, and are added in
+// order.  (One wave walking all rows took 10-17 us.)  Batched: grid row =
+// replica, its tables and outputs one after another.
+struct ColSums {
+  const double *part[3];
+  double *out[3];
+  int rows[3], cols[3];
+};
+
+__global__ __launch_bounds__(1024) void k_reduce_cols(ColSums s)
 {
-  const int v = threadIdx.x;
-  if (v >= cols) return;
+  __shared__ double red[16][64];
+  const int k = blockIdx.x, v = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int rows = s.rows[k], cols = s.cols[k];
+  const double *p = s.part[k] + (long)blockIdx.y * rows * cols;
   double x = 0;
-  for (int r = 0; r < rows; ++r) x += part[(long)r * cols + v];
-  out[v] = x;
+  if (v < cols)
+#pragma unroll 4
+    for (int r = g; r < rows; r += 16) x += p[(long)r * cols + v];
+  red[g][v] = x;
+  __syncthreads();
+  if (g != 0 || v >= cols) return;
+  x = 0;
+  for (int w = 0; w < 16; ++w) x += red[w][v];
+  s.out[k][(long)blockIdx.y * cols + v] = x;
 }
 
 // k-space term of dL/dq_s through S: C sum_H W Im(conj(S^(s)) T), with
@@ -247,26 +267,8 @@ __global__ void k_adjoint_field(int n, int nt, const double *w, const double *f4
   }
 }
 
-__global__ void k_fill_weights(int n, int mode, int s, const int *type, const double *q,
-                               const double *w, double *u)
-{
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  u[i] = mode < 0 ? (type[i] == s ? 1.0 : 0.0) : q[i] * w[3 * i + mode];
-}
-
 
 // ---------------------------------------------------------- batched replicas --
-
-__global__ void kb_reduce_cols(int rows, int cols, const double *part, double *out)
-{
-  const int v = threadIdx.x;
-  if (v >= cols) return;
-  const double *p = part + (long)blockIdx.x * rows * cols;
-  double x = 0;
-  for (int r = 0; r < rows; ++r) x += p[(long)r * cols + v];
-  out[(long)blockIdx.x * cols + v] = x;
-}
 
 // k_adjoint_kspace for every replica (grid row): planes [B][Rpad][SC]
 __global__ void kb_adjoint_kspace(const RepDev *rep, int R, int Rpad, int SC, int nY, int nZ, int ky,
@@ -331,27 +333,35 @@ __global__ void kb_adjoint_field(const RepDev *rep, int nt, const double *w, con
   }
 }
 
-__global__ void kb_fill_weights(long nown, int mode, int s, const int *type_o, const double *q_o,
-                                const double *w, double *u)
-{
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nown) return;
-  u[i] = mode < 0 ? (type_o[i] == s ? 1.0 : 0.0) : q_o[i] * w[3 * i + mode];
-}
 }  // namespace cav
 
 using namespace cav;
 
 // Device buffers of one adjoint call, in doubles: residual weights, per-block
-// partials, reduced outputs, and for Ewald_k the per-atom weights, the species
-// and residual-weighted structure factors and the per-atom k-space field.
+// partials, reduced outputs, and for Ewald_k the species and
+// residual-weighted structure factors and the per-atom k-space field.
 struct AdjWork {
-  double *w = nullptr, *part = nullptr, *out = nullptr, *u = nullptr, *ss = nullptr,
-         *sw = nullptr, *f4 = nullptr;
+  double *w = nullptr, *part = nullptr, *out = nullptr, *ss = nullptr, *sw = nullptr,
+         *f4 = nullptr;
 };
 
+// (u: room once taken by per-atom weights; it still counts towards the fixed
+// scratch, whose limit callers know)
 struct AdjSizes {
   size_t w = 0, part = 0, out = 0, u = 0, ss = 0, sw = 0, f4 = 0;
+  static size_t up(size_t v) { return (v + 31) / 32 * 32; }  // 256-byte boundaries
+  size_t total() const { return up(w) + up(part) + up(out) + up(u) + up(ss) + up(sw) + up(f4); }
+  AdjWork carve(double *q) const
+  {
+    AdjWork k;
+    k.w = q;
+    k.part = k.w + up(w);
+    k.out = k.part + up(part);
+    k.ss = k.out + up(out);
+    k.sw = k.ss + up(ss);
+    k.f4 = k.sw + up(sw);
+    return k;
+  }
 };
 
 static AdjSizes adjoint_sizes(const cav_ctx *c)
@@ -391,10 +401,28 @@ static int adjoint_run(cav_ctx *c, const double *w_host, const AdjWork &k, doubl
 {
   const int n = c->n, nt = c->nt, nt2 = nt * nt, nv = 2 * nt2 + nt;
   const int nblk = grid_for((long)n * kLPAa);
-  CAV_HIP(hipMemcpyAsync(k.w, w_host, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
-  for (int v = 0; v < nv + 2 * nt; ++v) hout[v] = 0.0;
-  if (c->lj_on || c->er_on) {
-    CAV_TRY(launch_nl_fill(c));  // the index rows, if the last build wrote slots only
+  const bool pairs = c->lj_on || c->er_on;
+  // through pinned memory where it is there (this call allocates nothing)
+  const bool staged = c->stage.cap >= std::max(3 * (size_t)n, (size_t)(nv + 2 * nt));
+  if (staged)
+    CAV_HIP(stage_put(c->stage, c->stream, 3 * (size_t)n, w_host, k.w));
+  else
+    CAV_HIP(hipMemcpyAsync(k.w, w_host, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
+  // partial sums: the pair kernel's, then the lattice's and the field's
+  const EwaldKPlan &p = c->ek;
+  const int nb = c->ek_on ? grid_for((long)p.R * p.nZ) : 0, nb2 = grid_for(n);
+  double *part1 = k.part + (size_t)nblk * nv, *part2 = part1 + (size_t)nb * nt + 16;
+  ColSums cs;
+  int tables = 0;
+  auto sum = [&](const double *part, int rows, int cols, double *out) {
+    cs.part[tables] = part;
+    cs.rows[tables] = rows;
+    cs.cols[tables] = cols;
+    cs.out[tables++] = out;
+  };
+  if (pairs) {
+    const bool slots = sorted_rows(c);
+    if (!slots) CAV_TRY(launch_nl_fill(c));  // index rows, if the last build wrote slots only
     AdjArgs a;
     a.n = n;
     a.nt = nt;
@@ -402,7 +430,8 @@ static int adjoint_run(cav_ctx *c, const double *w_host, const AdjWork &k, doubl
     a.xq = c->xq;
     a.tid = c->tid;
     a.mol = c->mol;
-    a.nl = c->nl;
+    a.nl = slots ? c->nlb : c->nl;
+    a.items = slots ? c->litems : nullptr;
     a.nn = c->nn;
     a.w = k.w;
     a.eps = c->d_raw_eps;
@@ -422,37 +451,29 @@ static int adjoint_run(cav_ctx *c, const double *w_host, const AdjWork &k, doubl
     a.rep = nullptr;
     const size_t sh = sizeof(double) * (kBlock / kLPAa) * nv;
     launch_adjoint_pairs(c->nt, dim3(nblk), sh, c->stream, a);
-    k_reduce_cols<<<1, 64, 0, c->stream>>>(nblk, nv, k.part, k.out);
-    CAV_HIP(hipGetLastError());
-    CAV_HIP(hipMemcpyAsync(hout, k.out, sizeof(double) * nv, hipMemcpyDeviceToHost, c->stream));
-    CAV_HIP(hipStreamSynchronize(c->stream));
+    sum(k.part, nblk, nv, k.out);
   }
   if (c->ek_on) {
-    const EwaldKPlan &p = c->ek;
-    const size_t plane = (size_t)p.Rpad * 2 * p.nZ;
     // per-atom k-space field G_i (uses the operand of the last force evaluation)
     CAV_TRY(ewald_k_field(c, k.f4));
-    for (int s = 0; s < nt; ++s) {
-      k_fill_weights<<<grid_for(n), kBlock, 0, c->stream>>>(n, -1, s, c->type, c->q, k.w, k.u);
-      CAV_TRY(ewald_k_weighted_sk(c, k.u, k.ss + s * plane));
-    }
-    for (int d = 0; d < 3; ++d) {
-      k_fill_weights<<<grid_for(n), kBlock, 0, c->stream>>>(n, d, 0, c->type, c->q, k.w, k.u);
-      CAV_TRY(ewald_k_weighted_sk(c, k.u, k.sw + d * plane));
-    }
-    const int nb = grid_for((long)p.R * p.nZ);
+    CAV_TRY(ewald_k_weight_sets(c, k.w, k.ss, k.sw));
     k_adjoint_kspace<<<nb, kBlock, 0, c->stream>>>(p.R, p.Rpad, p.nY, p.nZ, p.ky, p.kz, nt,
                                                    CAV_2PI / p.lx, CAV_2PI / p.ly, CAV_2PI / p.lz,
-                                                   c->d_W, k.ss, k.sw, k.part);
-    k_reduce_cols<<<1, 64, 0, c->stream>>>(nb, nt, k.part, k.out + nv);
-    const int nb2 = grid_for(n);
-    double *part2 = k.part + (size_t)nb * nt + 16;
+                                                   c->d_W, k.ss, k.sw, part1);
     k_adjoint_field<<<nb2, kBlock, 0, c->stream>>>(n, nt, k.w, k.f4, c->type, part2);
-    k_reduce_cols<<<1, 64, 0, c->stream>>>(nb2, nt, part2, k.out + nv + nt);
-    CAV_HIP(hipGetLastError());
-    CAV_HIP(hipMemcpyAsync(hout + nv, k.out + nv, sizeof(double) * 2 * nt,
-                           hipMemcpyDeviceToHost, c->stream));
+    sum(part1, nb, nt, k.out + nv);
+    sum(part2, nb2, nt, k.out + nv + nt);
+  }
+  if (tables) k_reduce_cols<<<tables, 1024, 0, c->stream>>>(cs);
+  CAV_HIP(hipGetLastError());
+  if (staged) {
+    CAV_HIP(stage_get(c->stage, c->stream, nv + 2 * (size_t)nt, k.out, hout));
+  } else {
+    CAV_HIP(hipMemcpyAsync(hout, k.out, sizeof(double) * (nv + 2 * nt), hipMemcpyDeviceToHost, c->stream));
     CAV_HIP(hipStreamSynchronize(c->stream));
+  }
+  if (!pairs) std::fill(hout, hout + nv, 0.0);
+  if (c->ek_on) {
     const double C = CAV_4PI * c->ek_ke * p.lxyz_inv;
     for (int s = 0; s < nt; ++s) hout[2 * nt2 + s] += C * hout[nv + s] + hout[nv + nt + s];
   }
@@ -482,28 +503,19 @@ extern "C" int cav_adjoint(cav_ctx *c, const double *w_host, double *g_eps, doub
   const bool dirty = c->params_dirty;
   CAV_TRY(refresh_params(c));
   if (dirty && (c->lj_on || c->er_on)) CAV_TRY(launch_pack(c));
-  // the workspace of this call, allocated here and released on every exit
-  struct Owned {
-    AdjWork k;
-    ~Owned()
-    {
-      double *ps[] = {k.w, k.part, k.out, k.u, k.ss, k.sw, k.f4};
-      for (double *q : ps)
-        if (q) (void)hipFree(q);
-    }
-  } own;
+  // the workspace is kept for the next call (a fit makes thousands): its
+  // allocation and release cost more than the kernels of a 2000-atom frame
   const AdjSizes z = adjoint_sizes(c);
-  CAV_HIP(hipMalloc(&own.k.w, sizeof(double) * z.w));
-  CAV_HIP(hipMalloc(&own.k.part, sizeof(double) * z.part));
-  CAV_HIP(hipMalloc(&own.k.out, sizeof(double) * z.out));
-  if (c->ek_on) {
-    CAV_HIP(hipMalloc(&own.k.u, sizeof(double) * z.u));
-    CAV_HIP(hipMalloc(&own.k.ss, sizeof(double) * z.ss));
-    CAV_HIP(hipMalloc(&own.k.sw, sizeof(double) * z.sw));
-    CAV_HIP(hipMalloc(&own.k.f4, sizeof(double) * z.f4));
+  if (z.total() > c->adj_cap) {
+    if (c->adj_ws) (void)hipFree(c->adj_ws);
+    c->adj_ws = nullptr;
+    c->adj_cap = 0;
+    CAV_HIP(hipMalloc(&c->adj_ws, sizeof(double) * z.total()));
+    c->adj_cap = z.total();
   }
+  (void)stage_room(c->stage, 3 * (size_t)c->n);
   std::vector<double> hout(z.out, 0.0);
-  CAV_TRY(adjoint_run(c, w_host, own.k, hout.data()));
+  CAV_TRY(adjoint_run(c, w_host, z.carve(c->adj_ws), hout.data()));
   adjoint_outputs(c, hout.data(), g_eps, g_sigma, g_charge);
   return CAV_OK;
 }
@@ -550,9 +562,7 @@ extern "C" int cav_adjoint_noalloc(cav_ctx *c, const double *w_host, double *g_e
                 "parameter values changed since the last force evaluation: cav_adjoint_noalloc "
                 "allocates nothing, so call cav_recalculate, cav_forces or cav_adjoint first");
   const AdjSizes z = adjoint_sizes(c);
-  // each buffer starts on a 256-byte boundary (32 doubles)
-  auto up = [](size_t v) { return (v + 31) / 32 * 32; };
-  const size_t need = up(z.w) + up(z.part) + up(z.out) + up(z.u) + up(z.ss) + up(z.sw) + up(z.f4);
+  const size_t need = z.total();
   if (need * sizeof(double) > kAdjScratchBytes)
     return fail(c, CAV_ERR_CAPACITY,
                 "cav_adjoint_noalloc needs " + std::to_string(need * sizeof(double)) +
@@ -561,25 +571,8 @@ extern "C" int cav_adjoint_noalloc(cav_ctx *c, const double *w_host, double *g_e
   (void)hipSetDevice(c->device);
   double *base = nullptr;
   CAV_TRY(adj_scratch(c, &base));
-  AdjWork k;
-  double *q = base;
-  k.w = q;
-  q += up(z.w);
-  k.part = q;
-  q += up(z.part);
-  k.out = q;
-  q += up(z.out);
-  if (c->ek_on) {
-    k.u = q;
-    q += up(z.u);
-    k.ss = q;
-    q += up(z.ss);
-    k.sw = q;
-    q += up(z.sw);
-    k.f4 = q;
-  }
   double hout[2 * 16 + 4 + 8];  // nv + 2 nt for nt <= 4
-  CAV_TRY(adjoint_run(c, w_host, k, hout));
+  CAV_TRY(adjoint_run(c, w_host, z.carve(base), hout));
   adjoint_outputs(c, hout, g_eps, g_sigma, g_charge);
   return CAV_OK;
 }
@@ -600,13 +593,43 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
   const EwaldKPlan &p = b->ek;
   const long plane = b->ek_on ? (long)p.Rpad * roundup16(2 * p.nZ) : 1;
   const int kb = b->ek_on ? grid_for((long)p.R * p.nZ) : 1, fb = grid_for(b->maxn);
-  double *dw = nullptr, *dpart = nullptr, *dout = nullptr, *u = nullptr, *ss = nullptr, *f4 = nullptr;
-  const size_t npart = (size_t)B * std::max<long>((long)pb * nv, (long)(kb + fb) * nt) + 64;
-  BAT_HIP(hipMalloc(&dw, sizeof(double) * 3 * nown));
-  BAT_HIP(hipMalloc(&dpart, sizeof(double) * npart));
-  BAT_HIP(hipMalloc(&dout, sizeof(double) * (size_t)B * (nv + 2 * nt)));
-  BAT_HIP(hipMemcpyAsync(dw, w_host, sizeof(double) * 3 * nown, hipMemcpyHostToDevice, b->stream));
-  std::vector<double> hpair((size_t)B * nv, 0.0), hk((size_t)B * nt, 0.0), hf((size_t)B * nt, 0.0);
+  // one kept workspace: residual weights, partials, outputs, the weight sets'
+  // chunk partials (of as many sets at once as stay within 256 MB) and
+  // structure factors, the per-atom field
+  const int sets = nt + 3;
+  const long cplane = std::max(1L, (long)b->n_chunks) * plane;
+  const long at_once = b->ek_on ? std::max(1L, std::min((long)sets, (32L << 20) / cplane)) : 0;
+  const size_t szw = 3 * (size_t)nown, szp = (size_t)B * ((size_t)pb * nv + (size_t)(kb + fb) * nt) + 64,
+               szo = (size_t)B * (nv + 2 * nt), szc = b->ek_on ? (size_t)(at_once * cplane) : 0,
+               szs = b->ek_on ? (size_t)plane * B * sets : 0, szf = b->ek_on ? 4 * (size_t)nown : 0;
+  auto up = [](size_t v) { return (v + 31) / 32 * 32; };
+  const size_t need = up(szw) + up(szp) + up(szo) + up(szc) + up(szs) + up(szf);
+  if (need > b->adj_cap) {
+    if (b->adj_ws) (void)hipFree(b->adj_ws);
+    b->adj_ws = nullptr;
+    b->adj_cap = 0;
+    BAT_HIP(hipMalloc(&b->adj_ws, sizeof(double) * need));
+    b->adj_cap = need;
+  }
+  double *dw = b->adj_ws, *dpart = dw + up(szw), *dout = dpart + up(szp), *cpart = dout + up(szo),
+         *ss = cpart + up(szc), *f4 = ss + up(szs);
+  const bool staged = stage_room(b->stage, std::max(szw, szo));
+  if (staged)
+    BAT_HIP(stage_put(b->stage, b->stream, szw, w_host, dw));
+  else
+    BAT_HIP(hipMemcpyAsync(dw, w_host, sizeof(double) * szw, hipMemcpyHostToDevice, b->stream));
+  std::vector<double> hout(szo, 0.0);
+  const bool pairs = b->lj_on || b->er_on;
+  double *part1 = dpart + (size_t)B * pb * nv, *part2 = part1 + (size_t)B * kb * nt;
+  double *out1 = dout + (size_t)B * nv, *out2 = out1 + (size_t)B * nt;
+  ColSums cs;
+  int tables = 0;
+  auto sum = [&](const double *part, int rows, int cols, double *out) {
+    cs.part[tables] = part;
+    cs.rows[tables] = rows;
+    cs.cols[tables] = cols;
+    cs.out[tables++] = out;
+  };
   if (b->lj_on || b->er_on) {
     AdjArgs a;
     a.n = 0;
@@ -616,6 +639,7 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
     a.tid = b->tid;
     a.mol = nullptr;
     a.nl = b->nl;
+    a.items = nullptr;
     a.nn = b->nn;
     a.w = dw;
     a.eps = b->d_raw_eps;
@@ -635,38 +659,29 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
     a.rep = b->d_rep;
     const size_t sh = sizeof(double) * (kBlock / kLPAa) * nv;
     launch_adjoint_pairs(b->nt, dim3(pb, B), sh, b->stream, a);
-    kb_reduce_cols<<<B, 64, 0, b->stream>>>(pb, nv, dpart, dout);
-    BAT_HIP(hipGetLastError());
-    BAT_HIP(hipMemcpyAsync(hpair.data(), dout, sizeof(double) * B * nv, hipMemcpyDeviceToHost, b->stream));
-    BAT_HIP(hipStreamSynchronize(b->stream));
+    sum(dpart, pb, nv, dout);
   }
   if (b->ek_on) {
-    BAT_HIP(hipMalloc(&u, sizeof(double) * nown));
-    BAT_HIP(hipMalloc(&ss, sizeof(double) * plane * B * (nt + 3)));
-    BAT_HIP(hipMalloc(&f4, sizeof(double) * 4 * nown));
     CAV_TRY(batch_ewald_k_field(b, f4));
-    for (int s = 0; s < nt; ++s) {
-      kb_fill_weights<<<grid_for(nown), kBlock, 0, b->stream>>>(nown, -1, s, b->type_o, b->q_o, dw, u);
-      CAV_TRY(batch_weighted_sk(b, u, ss + (size_t)s * B * plane));
-    }
-    double *sw = ss + (size_t)nt * B * plane;
-    for (int d = 0; d < 3; ++d) {
-      kb_fill_weights<<<grid_for(nown), kBlock, 0, b->stream>>>(nown, d, 0, b->type_o, b->q_o, dw, u);
-      CAV_TRY(batch_weighted_sk(b, u, sw + (size_t)d * B * plane));
-    }
-    kb_adjoint_kspace<<<dim3(kb, B), kBlock, 0, b->stream>>>(b->d_rep, p.R, p.Rpad, roundup16(2 * p.nZ),
-                                                             p.nY, p.nZ, p.ky, p.kz, nt, b->d_W, ss,
-                                                             sw, dpart);
-    kb_reduce_cols<<<B, 64, 0, b->stream>>>(kb, nt, dpart, dout + (size_t)B * nv);
-    double *dpart2 = dpart + (size_t)B * kb * nt;
-    kb_adjoint_field<<<dim3(fb, B), kBlock, 0, b->stream>>>(b->d_rep, nt, dw, f4, b->type_o, dpart2);
-    kb_reduce_cols<<<B, 64, 0, b->stream>>>(fb, nt, dpart2, dout + (size_t)B * (nv + nt));
-    BAT_HIP(hipGetLastError());
-    BAT_HIP(hipMemcpyAsync(hk.data(), dout + (size_t)B * nv, sizeof(double) * B * nt, hipMemcpyDeviceToHost, b->stream));
-    BAT_HIP(hipMemcpyAsync(hf.data(), dout + (size_t)B * (nv + nt), sizeof(double) * B * nt,
-                           hipMemcpyDeviceToHost, b->stream));
+    CAV_TRY(batch_weight_sets(b, dw, cpart, at_once * std::max(1, b->n_chunks), ss));
+    kb_adjoint_kspace<<<dim3(kb, B), kBlock, 0, b->stream>>>(
+        b->d_rep, p.R, p.Rpad, roundup16(2 * p.nZ), p.nY, p.nZ, p.ky, p.kz, nt, b->d_W, ss,
+        ss + (size_t)nt * B * plane, part1);
+    kb_adjoint_field<<<dim3(fb, B), kBlock, 0, b->stream>>>(b->d_rep, nt, dw, f4, b->type_o, part2);
+    sum(part1, kb, nt, out1);
+    sum(part2, fb, nt, out2);
+  }
+  if (tables) k_reduce_cols<<<dim3(tables, B), 1024, 0, b->stream>>>(cs);
+  BAT_HIP(hipGetLastError());
+  if (staged) {
+    BAT_HIP(stage_get(b->stage, b->stream, szo, dout, hout.data()));
+  } else {
+    BAT_HIP(hipMemcpyAsync(hout.data(), dout, sizeof(double) * szo, hipMemcpyDeviceToHost, b->stream));
     BAT_HIP(hipStreamSynchronize(b->stream));
   }
+  if (!pairs) std::fill(hout.begin(), hout.begin() + (size_t)B * nv, 0.0);
+  if (!b->ek_on) std::fill(hout.begin() + (size_t)B * nv, hout.end(), 0.0);
+  const double *hpair = hout.data(), *hk = hpair + (size_t)B * nv, *hf = hk + (size_t)B * nt;
   for (int r = 0; r < B; ++r) {
     const double C = b->ek_on ? b->reps[r].c0 : 0.0;  // 4 pi ke / V of this replica
     for (int q = 0; q < nt2; ++q) {
@@ -678,8 +693,5 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
         g_charge[(size_t)r * nt + s] = hpair[(size_t)r * nv + 2 * nt2 + s] + C * hk[(size_t)r * nt + s] +
                                        hf[(size_t)r * nt + s];
   }
-  void *fr[] = {dw, dpart, dout, u, ss, f4};
-  for (void *q : fr)
-    if (q) (void)hipFree(q);
   return CAV_OK;
 }

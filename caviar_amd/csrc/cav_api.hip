@@ -294,7 +294,7 @@ static void free_all(cav_ctx *c)
                   c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos, c->sk_sum,
                   c->binpos,  c->xqs,    c->tids,       c->nll,    c->nlb,    c->lstart, c->litems,
                   c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part,
-                  c->cell_cnt, c->bucket, c->pt_dev, c->pt_tab};
+                  c->cell_cnt, c->bucket, c->pt_dev, c->pt_tab, c->adj_ws};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_flags) (void)hipHostFree(c->h_flags);

@@ -160,7 +160,7 @@ static void batch_free(cav_batch *b)
                   b->type, b->id, b->q, b->xq, b->tid, b->vx, b->vy, b->vz, b->ax, b->ay, b->az,
                   b->aox, b->aoy, b->aoz, b->type_o, b->q_o, b->snap, b->bin_of, b->bin_cnt,
                   b->bin_start, b->bin_items, b->gblk, b->nl, b->nn, b->flags, b->d_minv, b->d_lj,
-                  b->part, b->vir, b->d_W, b->tab, b->ztab, b->bmat, b->bmat_h, b->sk_part, b->sk,
+                  b->adj_ws, b->part, b->vir, b->d_W, b->tab, b->ztab, b->bmat, b->bmat_h, b->sk_part, b->sk,
                   b->epart, b->s_items, b->s_items_o, b->f_items, b->rchunks, b->cpos, b->d_raw_eps,
                   b->d_raw_sig, b->d_charge, b->nlb, b->xqs, b->tids, b->litems, b->binpos,
                   b->order, b->ocnt, b->ostart};

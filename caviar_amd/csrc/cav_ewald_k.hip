@@ -147,7 +147,22 @@ struct SArgs {
   const int4 *items;  // batched: per workgroup column (first atom, end atom, chunk slot, replica)
   int ncols, groups;  // logical grid: atom chunks (or items) x row-tile groups
   int ct0;            // first column tile of this launch (launches cover 8 tiles each)
+  // the adjoint's weight sets, one per grid row, in place of q: set v < nt is
+  // the atoms of type v, set nt + d is q times the residual weights along d;
+  // each writes its own chunk partials
+  int sets = 0, set0 = 0, nt = 0;
+  long set_stride = 0;
+  const int *type = nullptr;
+  const double *w = nullptr;
 };
+
+// Per-atom weight of an S pass: the charge, or the launch's weight set.
+__device__ __forceinline__ double s_weight(const SArgs &a, long i)
+{
+  if (a.sets == 0) return a.q[i];
+  const int v = a.set0 + blockIdx.y;
+  return v < a.nt ? (a.type[i] == v ? 1.0 : 0.0) : a.q[i] * a.w[3 * i + v - a.nt];
+}
 
 // Issue the asynchronous copy of `bytes` contiguous bytes (a multiple of 16,
 // source padded) from global memory straight into LDS, 16 bytes per lane.
@@ -242,7 +257,7 @@ __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
                       bytes, wave, nwaves, lane);
     if (threadIdx.x < stage)
       reinterpret_cast<T *>(smem_raw + 2 * stage_bytes)[b * stage + threadIdx.x] =
-          threadIdx.x < cnt ? (T)a.q[base + threadIdx.x] : (T)0;
+          threadIdx.x < cnt ? (T)s_weight(a, base + threadIdx.x) : (T)0;
   };
 
   int b = 0;
@@ -296,7 +311,7 @@ __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
         const int row = (rt0 + r) * 16 + mfma_row<T>(lk, e);
         const int col = (a.ct0 + s) * 16 + lr;
         const double v = (double)acc[r][s][e];
-        a.part[((long)chunk * a.Rpad + row) * a.SC + col] = v;
+        a.part[blockIdx.y * a.set_stride + ((long)chunk * a.Rpad + row) * a.SC + col] = v;
       }
   }
 }
@@ -1590,10 +1605,14 @@ int ewald_k_alloc(cav_ctx *c)
   c->sk_chunks = (c->n + chunk - 1) / chunk;
   if (c->sk_chunks < 1) c->sk_chunks = 1;
   const int SC = roundup(2 * p.nZ, 16);
+  // chunk partials of one S pass, and of several of the adjoint's weight sets
+  // at once while they stay small (64 MB)
+  const size_t plane_bytes = sizeof(double) * (size_t)p.Rpad * SC;
+  c->sk_planes = std::max((long)c->sk_chunks,
+                          std::min(7L * c->sk_chunks, (64L << 20) / (long)plane_bytes));
   if (c->sk_part) (void)hipFree(c->sk_part);
-  CAV_HIP(hipMalloc(&c->sk_part, sizeof(double) * (size_t)c->sk_chunks * p.Rpad * SC));
-  CAV_HIP(hipMemsetAsync(c->sk_part, 0, sizeof(double) * (size_t)c->sk_chunks * p.Rpad * SC,
-                         c->stream));
+  CAV_HIP(hipMalloc(&c->sk_part, plane_bytes * c->sk_planes));
+  CAV_HIP(hipMemsetAsync(c->sk_part, 0, plane_bytes * c->sk_planes, c->stream));
   if (c->sk) (void)hipFree(c->sk);
   CAV_HIP(hipMalloc(&c->sk, sizeof(double) * (size_t)p.Rpad * 2 * p.nZ));
   if (c->sk_sum) (void)hipFree(c->sk_sum);
@@ -1641,27 +1660,19 @@ static void launch_sk_rt(hipStream_t st, SArgs a, dim3 lgrid, size_t smem, int S
 {
   a.ncols = (int)lgrid.x;
   a.groups = (int)lgrid.y;
-  const dim3 grid((lgrid.x + 7) / 8 * 8 * lgrid.y);
+  const dim3 grid((lgrid.x + 7) / 8 * 8 * lgrid.y, std::max(a.sets, 1));
   const int block = 64 * waves;
-  allow_smem(k_sk<T, RT, 1>, smem);
-  allow_smem(k_sk<T, RT, 2>, smem);
-  allow_smem(k_sk<T, RT, 3>, smem);
-  allow_smem(k_sk<T, RT, 4>, smem);
-  allow_smem(k_sk<T, RT, 5>, smem);
-  allow_smem(k_sk<T, RT, 6>, smem);
-  allow_smem(k_sk<T, RT, 7>, smem);
-  allow_smem(k_sk<T, RT, 8>, smem);
   // one launch per 8 column tiles; each writes its own columns of the partials
   for (a.ct0 = 0; a.ct0 < SCT; a.ct0 += 8) {
     switch (std::min(8, SCT - a.ct0)) {
-    case 1: k_sk<T, RT, 1><<<grid, block, smem, st>>>(a); break;
-    case 2: k_sk<T, RT, 2><<<grid, block, smem, st>>>(a); break;
-    case 3: k_sk<T, RT, 3><<<grid, block, smem, st>>>(a); break;
-    case 4: k_sk<T, RT, 4><<<grid, block, smem, st>>>(a); break;
-    case 5: k_sk<T, RT, 5><<<grid, block, smem, st>>>(a); break;
-    case 6: k_sk<T, RT, 6><<<grid, block, smem, st>>>(a); break;
-    case 7: k_sk<T, RT, 7><<<grid, block, smem, st>>>(a); break;
-    default: k_sk<T, RT, 8><<<grid, block, smem, st>>>(a); break;
+    case 1: allow_smem(k_sk<T, RT, 1>, smem); k_sk<T, RT, 1><<<grid, block, smem, st>>>(a); break;
+    case 2: allow_smem(k_sk<T, RT, 2>, smem); k_sk<T, RT, 2><<<grid, block, smem, st>>>(a); break;
+    case 3: allow_smem(k_sk<T, RT, 3>, smem); k_sk<T, RT, 3><<<grid, block, smem, st>>>(a); break;
+    case 4: allow_smem(k_sk<T, RT, 4>, smem); k_sk<T, RT, 4><<<grid, block, smem, st>>>(a); break;
+    case 5: allow_smem(k_sk<T, RT, 5>, smem); k_sk<T, RT, 5><<<grid, block, smem, st>>>(a); break;
+    case 6: allow_smem(k_sk<T, RT, 6>, smem); k_sk<T, RT, 6><<<grid, block, smem, st>>>(a); break;
+    case 7: allow_smem(k_sk<T, RT, 7>, smem); k_sk<T, RT, 7><<<grid, block, smem, st>>>(a); break;
+    default: allow_smem(k_sk<T, RT, 8>, smem); k_sk<T, RT, 8><<<grid, block, smem, st>>>(a); break;
     }
   }
 }
@@ -2010,26 +2021,38 @@ int launch_dipole(cav_ctx *c)
   return CAV_OK;
 }
 
-// S over the half lattice with arbitrary real per-atom weights u_j in place
-// of the charges (the adjoint's species and residual-weighted structure
-// factors); written as [Rpad][nZ] complex FP64.
-__global__ void k_sk_sum(int nchunks, int Rpad, int SC, int nZ, const double *part, double *out)
+// Sums over chunks of the weight sets' partials (grid row = set), in
+// k_chunk_sum's order, without the padding columns: set v to ss (v < nt) or sw,
+// [Rpad][nZ] complex each.
+__global__ void k_sets_sum(int nchunks, int Rpad, int SC, int nZ, int set0, int nt,
+                           const double *part, double *ss, double *sw)
 {
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= Rpad * nZ) return;
-  const int r = t / nZ, c = t - r * nZ;
-  double sr = 0, si = 0;
-  for (int k = 0; k < nchunks; ++k) {
-    const double *p = part + ((long)k * Rpad + r) * SC + 2 * c;
-    sr += p[0];
-    si += p[1];
-  }
-  out[(long)r * 2 * nZ + 2 * c] = sr;
-  out[(long)r * 2 * nZ + 2 * c + 1] = si;
+  __shared__ double red[4][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long plane = (long)Rpad * SC, e = (long)blockIdx.x * 64 + lane;
+  part += blockIdx.y * nchunks * plane;
+  double s = 0;
+  if (e < plane)
+#pragma unroll 4
+    for (int k = wave; k < nchunks; k += 4) s += part[(long)k * plane + e];
+  red[wave][lane] = s;
+  __syncthreads();
+  const long r = e / SC, c = e - r * SC;
+  if (wave != 0 || e >= plane || c >= 2 * nZ) return;
+  const int v = set0 + blockIdx.y;
+  double *out = v < nt ? ss + (long)v * Rpad * 2 * nZ : sw + (long)(v - nt) * Rpad * 2 * nZ;
+  out[r * 2 * nZ + c] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
+// S over the half lattice with the adjoint's real per-atom weights in place of
+// the charges: the atoms of each type (into ss), and q times the residual
+// weights w along each axis (into sw), at the current positions.  All sets of
+// one launch share the phase tables; as one table build, S pass and two sums
+// per set this was 4 (nt + 3) launches, each of them too small to fill the
+// chip: 2000 atoms, kmax 6, two types 26 + 5 us a set, now 16 + 3 us for all five;
+// 64 replicas (135000 atoms), three types 282 us a set, now 540 for all six.
 template <typename T>
-static int weighted_sk_t(cav_ctx *c, const double *weights, double *out)
+static int weight_sets_t(cav_ctx *c, const double *w, double *ss, double *sw)
 {
   const EwaldKPlan &p = c->ek;
   const int TS = p.nX + p.nY + p.nZ;
@@ -2048,7 +2071,10 @@ static int weighted_sk_t(cav_ctx *c, const double *weights, double *out)
   a.chunk = (c->n + c->sk_chunks - 1) / c->sk_chunks;
   a.chunk = (a.chunk + 31) / 32 * 32;
   a.stage = s_stage(c, sizeof(T));
-  a.q = weights;
+  a.q = c->q;
+  a.type = c->type;
+  a.w = w;
+  a.nt = c->nt;
   a.tab = c->tab;
   a.part = c->sk_part;
   a.items = nullptr;
@@ -2058,19 +2084,23 @@ static int weighted_sk_t(cav_ctx *c, const double *weights, double *out)
   s_layout(c, &groups, &a.tiles_per_group, &waves);
   const int nch = (c->n + a.chunk - 1) / a.chunk;
   const size_t smem = 2 * (size_t)a.stage * TS * sizeof(Cx<T>) + 2 * (size_t)a.stage * sizeof(T);
-  launch_sk_rt<T, kRT>(c->stream, a, dim3(nch, groups), smem, a.SC / 16, waves);
   const long plane = (long)p.Rpad * a.SC;
-  k_chunk_sum<double><<<(plane + 63) / 64, kBlock, 0, c->stream>>>(c->sk_part, nch, plane, c->sk_sum);
-  k_sk_sum<<<grid_for((long)p.Rpad * p.nZ), kBlock, 0, c->stream>>>(1, p.Rpad, a.SC, p.nZ,
-                                                                    c->sk_sum, out);
+  a.set_stride = (long)nch * plane;
+  const int total = c->nt + 3, most = (int)std::max(1L, c->sk_planes / nch);
+  for (a.set0 = 0; a.set0 < total; a.set0 += most) {
+    a.sets = std::min(most, total - a.set0);
+    launch_sk_rt<T, kRT>(c->stream, a, dim3(nch, groups), smem, a.SC / 16, waves);
+    k_sets_sum<<<dim3((plane + 63) / 64, a.sets), kBlock, 0, c->stream>>>(
+        nch, p.Rpad, a.SC, p.nZ, a.set0, c->nt, c->sk_part, ss, sw);
+  }
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
 
-int ewald_k_weighted_sk(cav_ctx *c, const double *weights, double *out)
+int ewald_k_weight_sets(cav_ctx *c, const double *w, double *ss, double *sw)
 {
-  if (c->precision == CAV_FP64) return weighted_sk_t<double>(c, weights, out);
-  return weighted_sk_t<float>(c, weights, out);
+  if (c->precision == CAV_FP64) return weight_sets_t<double>(c, w, ss, sw);
+  return weight_sets_t<float>(c, w, ss, sw);
 }
 
 // Per-atom k-space field (C sum k Im(g e^{ik.r}), and the potential) with the
@@ -2539,14 +2569,19 @@ static int batch_ewald_k_t(cav_batch *b)
 
 
 // Per replica, fixed-order sum of its S-pass chunk partials into [B][plane].
-__global__ void kb_chunk_sum(const int2 *rchunks, const double *part, long plane, double *out)
+// Grid z = weight set: each has its own nchunks planes and its own output.
+__global__ void kb_chunk_sum(const int2 *rchunks, int nchunks, const double *part, long plane,
+                             double *out)
 {
+  part += (long)blockIdx.z * nchunks * plane;
+  out += (long)blockIdx.z * gridDim.y * plane;
   __shared__ double red[4][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long e = (long)blockIdx.x * 64 + lane;
   const int2 rc = rchunks[blockIdx.y];
   double s = 0;
   if (e < plane)
+#pragma unroll 4
     for (int k = wave; k < rc.y; k += 4) s += part[(long)(rc.x + k) * plane + e];
   red[wave][lane] = s;
   __syncthreads();
@@ -2599,11 +2634,12 @@ int batch_ewald_k_field(cav_batch *b, double *out4)
   return batch_field_t<float>(b, out4);
 }
 
-// S over the half lattice with per-atom weights u (owned-indexed) for every
-// replica, into out[B][Rpad][SC] (re, im at columns 2c, 2c+1).  Uses the full
-// phase tables of batch_ewald_k_field.
+// S over the half lattice with the adjoint's weight sets (as weight_sets_t;
+// w: residual weights, owned-indexed) for every replica, into
+// out[set][B][Rpad][SC] (re, im at columns 2c, 2c+1); part holds `planes` chunk
+// planes.  Uses the full phase tables of batch_ewald_k_field.
 template <typename T>
-static int batch_wsk_t(cav_batch *b, const double *u, double *out)
+static int batch_sets_t(cav_batch *b, const double *w, double *part, long planes, double *out)
 {
   const EwaldKPlan &p = b->ek;
   const int TS = p.nX + p.nY + p.nZ;
@@ -2622,24 +2658,33 @@ static int batch_wsk_t(cav_batch *b, const double *u, double *out)
   a.chunk = b->s_chunk;
   a.stage = s_stage_for(TS, sizeof(T));
   a.tiles_per_group = tpg;
-  a.q = u;
+  a.q = b->q_o;
+  a.type = b->type_o;
+  a.w = w;
+  a.nt = b->nt;
   a.tab = b->tab;
-  a.part = b->sk_part;
+  a.part = part;
   a.Rpad = p.Rpad;
   a.SC = SC;
   a.items = b->s_items_o;
   const size_t smem = 2 * (size_t)a.stage * TS * sizeof(Cx<T>) + 2 * (size_t)a.stage * sizeof(T);
-  launch_sk_rt<T, kRT>(b->stream, a, dim3(b->n_sitems, groups), smem, SC / 16, waves);
   const long plane = (long)p.Rpad * SC;
-  kb_chunk_sum<<<dim3((plane + 63) / 64, b->B), kBlock, 0, b->stream>>>(b->rchunks, b->sk_part, plane, out);
+  a.set_stride = (long)b->n_chunks * plane;
+  const int total = b->nt + 3, most = (int)std::max(1L, planes / std::max(1, b->n_chunks));
+  for (a.set0 = 0; a.set0 < total; a.set0 += most) {
+    a.sets = std::min(most, total - a.set0);
+    launch_sk_rt<T, kRT>(b->stream, a, dim3(b->n_sitems, groups), smem, SC / 16, waves);
+    kb_chunk_sum<<<dim3((plane + 63) / 64, b->B, a.sets), kBlock, 0, b->stream>>>(
+        b->rchunks, b->n_chunks, part, plane, out + (long)a.set0 * b->B * plane);
+  }
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }
 
-int batch_weighted_sk(cav_batch *b, const double *u, double *out)
+int batch_weight_sets(cav_batch *b, const double *w, double *part, long planes, double *out)
 {
-  if (b->precision == CAV_FP64) return batch_wsk_t<double>(b, u, out);
-  return batch_wsk_t<float>(b, u, out);
+  if (b->precision == CAV_FP64) return batch_sets_t<double>(b, w, part, planes, out);
+  return batch_sets_t<float>(b, w, part, planes, out);
 }
 
 // ------------------------------------------------------------------ autotuner --

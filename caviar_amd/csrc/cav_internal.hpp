@@ -262,6 +262,7 @@ struct cav_ctx {
   int tab_cap = 0;           // atoms the tables hold
   double *sk_part = nullptr; // [chunks][Rpad][2nZ]
   int sk_chunks = 0;
+  long sk_planes = 0;        // chunk planes sk_part holds
   double *sk = nullptr;      // [Rpad][2nZ] FP64
   double *sk_sum = nullptr;  // [Rpad][SC] chunk partials summed (fixed order)
   void *bmat = nullptr;      // [KZ][4*Rpad] (T) force-pass operand
@@ -285,6 +286,8 @@ struct cav_ctx {
   double *d_W = nullptr;     // [Rpad][nZ]
   double *kf_part = nullptr; // row splits' sums of the force pass
   size_t kf_cap = 0;
+  double *adj_ws = nullptr;  // workspace of cav_adjoint, kept between calls
+  size_t adj_cap = 0;
   double *kacc = nullptr;    // per-atom k-space (fx, fy, fz, phi) scratch for point queries
 
   bool setup_done = false;
@@ -317,6 +320,8 @@ struct cav_batch {
   int kx = 1, ky = 1, kz = 1;
 
   cav::Stage stage;
+  double *adj_ws = nullptr;  // workspace of cav_batch_adjoint, kept between calls
+  size_t adj_cap = 0;
 
   // replicas as given (host)
   struct HostRep {
@@ -475,7 +480,7 @@ int batch_ewald_k_plan(cav_batch *b);
 int batch_ewald_k_alloc(cav_batch *b);
 int batch_ewald_k(cav_batch *b);
 int batch_ewald_k_field(cav_batch *b, double *out4);
-int batch_weighted_sk(cav_batch *b, const double *u, double *out);
+int batch_weight_sets(cav_batch *b, const double *w, double *part, long planes, double *out);
 
 inline int grid_for(long n, int block = kBlock) { return (int)((n + block - 1) / block); }
 

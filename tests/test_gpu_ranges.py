@@ -173,3 +173,27 @@ def test_steps_at_workgroup_edges(gpu, n, precision):
     if precision == "fp64":
         assert abs(e.virial() - o.virial()) <= 1e-9 * abs(o.virial())
         assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs()))
+
+
+@pytest.mark.parametrize("n,kmax,types", [(2, 1, 2), (33, 3, 1), (700, 7, 3), (3000, 16, 4), (9000, 4, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_adjoint_weight_sets(gpu, n, kmax, types, precision):
+    """The adjoint's structure factors, all weight sets of a launch at once (and
+    in several launches where their partials are large), against the oracle's:
+    1e-10 (FP64; the gradient cancels sums 100 times its size), mixed 1e-4."""
+    print(f"[case] weight sets n={n} kmax={kmax} types={types} {precision}", flush=True)
+    s = configs.ions(n=n, rho=0.3 if n > 2 else 0.02, kmax=kmax, seed=n)
+    rng = np.random.default_rng(n)
+    s.mass = np.ones(types)
+    s.charge = rng.uniform(-1, 1, types)
+    s.types = rng.integers(0, types, n).astype(np.int32)
+    s.lj.epsilon = np.ones((types, types))
+    s.lj.sigma = rng.uniform(0.8, 1.1, (types, types))
+    o = Oracle(s, threads=8)
+    o.setup()
+    e = Engine(s, precision=precision)
+    e.setup()
+    w = rng.normal(size=(n, 3))
+    tol = 1e-10 if precision == "fp64" else 1e-4
+    for a, b in zip(e.adjoint(w), o.adjoint(w)):
+        assert F.rel_err(np.ravel(a), np.ravel(b)) <= tol
