@@ -291,7 +291,7 @@ static void free_all(cav_ctx *c)
                   c->d_thermo, c->d_mass,
                   c->part,    c->scal,   c->tab,       c->sk_part,  c->sk,       c->bmat,
                   c->d_W,     c->kacc,      c->order,    c->ord_blk,  c->xq,
-                  c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos, c->sk_sum,
+                  c->tid,     c->d_raw_eps, c->d_raw_sig, c->ztab, c->bmat_h, c->cpos,
                   c->binpos,  c->xqs,    c->tids,       c->nll,    c->nlb,    c->lstart, c->litems,
                   c->ekx,     c->eky,    c->ekz,        c->part_k, c->kf_part,
                   c->cell_cnt, c->bucket, c->pt_dev, c->pt_tab, c->adj_ws};
@@ -507,7 +507,7 @@ int cav::refresh_params(cav_ctx *c)
 
 // Starts the step's Ewald_k on the second stream once the drift has run: the
 // passes read only the owned positions and charges, and write their own
-// accelerations (zeroed first) and partial sums, so they run concurrently
+// accelerations and partial sums, so they run concurrently
 // with the ghost exchange, neighbour build and pair kernel of the main stream.
 static int ewald_k_fork(cav_ctx *c)
 {
@@ -526,11 +526,9 @@ static int ewald_k_fork(cav_ctx *c)
       std::swap(c->part, c->part_k);
     }
   } side(c);
-  k_zero3<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->ax, c->ay, c->az);
-  CAV_HIP(hipGetLastError());
-  c->defer_dipole = true;
+  c->defer_dipole = c->ek_set = true;
   const int st = launch_ewald_k(c);
-  c->defer_dipole = false;
+  c->defer_dipole = c->ek_set = false;
   CAV_TRY(st);
   CAV_HIP(hipEventRecord(c->ev_join, c->stream));
   return CAV_OK;
@@ -1184,7 +1182,8 @@ int cav_setup(cav_ctx *c)
   c->npart = npart;
   if (c->ek_on) {
     CAV_TRY(ewald_k_plan(c));
-    const int need = 3 * grid_for((long)c->ek.Rpad * c->ek.nZ) + 64;
+    // one partial per workgroup of the S reduction (64 of the padded columns)
+    const int need = c->ek.Rpad / 16 * ((2 * c->ek.nZ + 15) / 16 * 4) + 64;
     if (need > c->npart) {
       CAV_TRY(dmalloc(c, &c->part, need));
       c->npart = need;

@@ -177,12 +177,21 @@ __device__ __forceinline__ void copy_to_lds_async(const unsigned char *src, unsi
   }
 }
 
-// One workgroup: an atom chunk x a group of row tiles; wave w owns RT row
-// tiles and the SCT column tiles from ct0 (wider nz axes take one launch per
-// 8 column tiles).  A (rows x (atom,re/im)) is generated from
-// the staged X, Y tables and charges, B ((atom,re/im) x (nz,re/im)) from Z.
-// Stages of atom records are double-buffered in LDS: the next stage streams
-// in from HBM (direct-to-LDS loads) while the current one feeds the MFMAs.
+// One workgroup: an atom chunk x a group of row tiles; compute wave w owns RT
+// row tiles and the SCT column tiles from ct0 (wider nz axes take one launch
+// per 8 column tiles).  A K-step is four atoms: lane l holds q X Y of row l%16
+// and atom l/16 and, for its column (nz, re or im), Z of that atom, and the
+// product is taken as two MFMAs, Re(q X Y) times (Zr | Zi) and Im(q X Y) times
+// (-Zi | Zr).  Every complex product and every LDS read is then made by one
+// lane only; with (atom, re/im) as the four k of a step two lanes formed each
+// product and used half of it.  The last wave is the producer: it streams the
+// next stage of atom records into the other LDS buffer (direct-to-LDS loads)
+// while the compute waves multiply; a wave that issues such copies itself
+// waits for them before every LDS read.  FP64 MFMA and the A operand's VALU
+// work bound it.  N = 65536, kmax 12 (FP64):
+// 174 -> 135 us beside the short-range passes (60 us of products at the rate a large FP64 matrix
+// product reaches);
+// six weight sets of 135000 atoms in 64 replicas, kmax 6: 540 -> 365 us.
 // In the mixed form the MFMAs accumulate in FP32 over one chunk (<= 4096
 // atoms) and the chunk partials are summed in FP64.
 template <typename T, int RT, int SCT>
@@ -220,87 +229,96 @@ __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
     chunk = it.z;
   }
 
+  // the three loops below pass the same barriers: producer, waves without a
+  // row tile in this group, compute waves
+  if (wave == nwaves - 1) {
+    auto issue = [&](long base, int b) {
+      const int cnt = (int)((a1 - base) < stage ? (a1 - base) : stage);
+      const int bytes = (int)(((size_t)cnt * a.TS * sizeof(Cx<T>) + 15) / 16 * 16);
+      copy_to_lds_async(tab + (size_t)base * a.TS * sizeof(Cx<T>), smem_raw + b * stage_bytes,
+                        bytes, 0, 1, lane);
+      if (lane < stage)
+        reinterpret_cast<T *>(smem_raw + 2 * stage_bytes)[b * stage + lane] =
+            lane < cnt ? (T)s_weight(a, base + lane) : (T)0;
+      __builtin_amdgcn_s_waitcnt(0);
+    };
+    int b = 0;
+    if (a0 < a1) issue(a0, 0);
+    __syncthreads();
+    for (long base = a0; base < a1; base += stage) {
+      if (base + stage < a1) issue(base + stage, b ^ 1);
+      __syncthreads();
+      b ^= 1;
+    }
+    return;
+  }
+  if (rt0 >= rt_end) {
+    __syncthreads();
+    for (long base = a0; base < a1; base += stage) __syncthreads();
+    return;
+  }
+
   V acc[RT][SCT];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int s = 0; s < SCT; ++s) acc[r][s] = V{0, 0, 0, 0};
 
-  // lane roles inside a 16x16x4 tile: A[row=l%16][k=l/16], B[k=l/16][col=l%16]
+  // lane roles inside a 16x16x4 tile: A[row=l%16][k=l/16], B[k=l/16][col=l%16];
+  // rows past the lattice and columns past nz read entry 0 (finite) and are
+  // cleared on output
   const int lr = lane & 15, lk = lane >> 4;
-  const int jj = lk >> 1, part = lk & 1;  // atom within the K-step, re/im half
+  const int offY = a.nX, offZ = a.nX + a.nY;
   int rnx[RT], rny[RT];
-  bool rvalid[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int row = (rt0 + r) * 16 + lr;
-    rvalid[r] = (rt0 + r) < rt_end && row < a.nX * a.nY;
-    rnx[r] = rvalid[r] ? row / a.nY : 0;
-    rny[r] = rvalid[r] ? row % a.nY : 0;  // index into Y (ny + ky)
+    const bool ok = (rt0 + r) < rt_end && row < a.nX * a.nY;
+    rnx[r] = ok ? row / a.nY : 0;
+    rny[r] = offY + (ok ? row % a.nY : 0);
   }
-  int zc[SCT], zt[SCT];
-  bool zvalid[SCT];
+  const int zt = lr & 1;  // this column's half of (re, im)
+  int zc[SCT];
 #pragma unroll
   for (int s = 0; s < SCT; ++s) {
-    const int col = (a.ct0 + s) * 16 + lr;
-    zc[s] = col >> 1;
-    zt[s] = col & 1;
-    zvalid[s] = zc[s] < a.nZ;
+    const int c = ((a.ct0 + s) * 16 + lr) >> 1;
+    zc[s] = offZ + (c < a.nZ ? c : 0);
   }
-  const int offY = a.nX, offZ = a.nX + a.nY;
-  const bool active = rt0 < rt_end;
-
-  auto issue = [&](long base, int b) {
-    const int cnt = (int)((a1 - base) < stage ? (a1 - base) : stage);
-    const int bytes = (int)(((size_t)cnt * a.TS * sizeof(Cx<T>) + 15) / 16 * 16);
-    copy_to_lds_async(tab + (size_t)base * a.TS * sizeof(Cx<T>), smem_raw + b * stage_bytes,
-                      bytes, wave, nwaves, lane);
-    if (threadIdx.x < stage)
-      reinterpret_cast<T *>(smem_raw + 2 * stage_bytes)[b * stage + threadIdx.x] =
-          threadIdx.x < cnt ? (T)s_weight(a, base + threadIdx.x) : (T)0;
-  };
 
   int b = 0;
-  if (a0 < a1) issue(a0, 0);
-  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   for (long base = a0; base < a1; base += stage) {
-    if (base + stage < a1) issue(base + stage, b ^ 1);  // streams in during the MFMAs below
     const int cnt = (int)((a1 - base) < stage ? (a1 - base) : stage);
     const Cx<T> *st = reinterpret_cast<const Cx<T> *>(smem_raw + b * stage_bytes);
     const T *sq = reinterpret_cast<const T *>(smem_raw + 2 * stage_bytes) + b * stage;
-    if (active) {
 #pragma unroll 2
-      for (int ks = 0; ks < stage / 2; ++ks) {
-        const int j = 2 * ks + jj;
-        const bool jv = j < cnt;
-        const Cx<T> *rec = st + (jv ? j : 0) * a.TS;
-        const T qj = jv ? sq[j] : (T)0;
-        T av[RT];
+    for (int k0 = 0; k0 < cnt; k0 += 4) {
+      // atoms past the stage's end weigh nothing and read its first record
+      const int j = k0 + lk < cnt ? k0 + lk : 0;
+      const Cx<T> *rec = st + j * a.TS;
+      const T qj = k0 + lk < cnt ? sq[j] : (T)0;
+      T pr[RT], pi[RT];
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const Cx<T> X = rec[rnx[r]], Y = rec[offY + rny[r]];
-          const T pr = X.re * Y.re - X.im * Y.im;
-          const T pi = X.re * Y.im + X.im * Y.re;
-          av[r] = rvalid[r] ? qj * (part ? pi : pr) : (T)0;
-        }
+      for (int r = 0; r < RT; ++r) {
+        const Cx<T> X = rec[rnx[r]], Y = rec[rny[r]];
+        pr[r] = qj * (X.re * Y.re - X.im * Y.im);
+        pi[r] = qj * (X.re * Y.im + X.im * Y.re);
+      }
 #pragma unroll
-        for (int s = 0; s < SCT; ++s) {
-          const Cx<T> Z = rec[offZ + (zvalid[s] ? zc[s] : 0)];
-          // re column: (Zr, -Zi); im column: (Zi, Zr) along (re, im) of A
-          T bv = zt[s] == 0 ? (part ? -Z.im : Z.re) : (part ? Z.re : Z.im);
-          bv = (zvalid[s] && jv) ? bv : (T)0;
+      for (int s = 0; s < SCT; ++s) {
+        const Cx<T> Z = rec[zc[s]];
+        const T b0 = zt ? Z.im : Z.re, b1 = zt ? Z.re : -Z.im;
 #pragma unroll
-          for (int r = 0; r < RT; ++r) acc[r][s] = Mfma<T>::op(av[r], bv, acc[r][s]);
-        }
+        for (int r = 0; r < RT; ++r) acc[r][s] = Mfma<T>::op(pr[r], b0, acc[r][s]);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r][s] = Mfma<T>::op(pi[r], b1, acc[r][s]);
       }
     }
-    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     b ^= 1;
   }
-  if (!active) return;
   // D[row = mfma_row(l/16, e)][col = l%16]
+  const int nrow = a.nX * a.nY;
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     if (rt0 + r >= rt_end) break;
@@ -310,7 +328,7 @@ __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
       for (int e = 0; e < 4; ++e) {
         const int row = (rt0 + r) * 16 + mfma_row<T>(lk, e);
         const int col = (a.ct0 + s) * 16 + lr;
-        const double v = (double)acc[r][s][e];
+        const double v = row < nrow && col < 2 * a.nZ ? (double)acc[r][s][e] : 0.0;
         a.part[blockIdx.y * a.set_stride + ((long)chunk * a.Rpad + row) * a.SC + col] = v;
       }
   }
@@ -331,69 +349,89 @@ __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
 // 2 (nZ - 1) other kappa (kappa' = 2 c' + re/im, c' = nz below kz, nz - 1 above).
 __host__ __device__ constexpr int split_blk_bytes(int nkh) { return 4 * nkh * 2 * 64 * 16 + 128; }
 
-template <typename T, typename P>
-__global__ void k_sk_reduce(int nchunks, int Rpad, int SC, int R, int nZ, int kz, int KSS, int KSP,
-                            const P *part, const double *W, double *sk, T *bm,
-                            double *epart, double inv_sa, _Float16 *bmh, int nkh, double sb,
-                            const int2 *rchunks, long bm_stride, long bmh_stride)
+struct SReduce {
+  int nchunks, Rpad, SC, R, nZ, kz, KSS, KSP;
+  const void *part;
+  const double *W;
+  double *sk;
+  void *bm;
+  double *epart;
+  double inv_sa;
+  _Float16 *bmh;  // split form's operand, or nullptr
+  int nkh;
+  double sb;
+};
+
+// One lattice point (row r, column c) with its S: S itself, the force-pass
+// operands and the energy term W |S|^2.
+template <typename T>
+__device__ __forceinline__ double put_operand(const SReduce &a, int r, int c, double sr, double si)
 {
-  if (rchunks) {  // batched: grid row b reduces replica b's chunks into its own S and operands
-    const int b = blockIdx.y;
-    part += (long)rchunks[b].x * Rpad * SC;
-    nchunks = rchunks[b].y;
-    W += (long)b * R * nZ;
-    sk += (long)b * Rpad * 2 * nZ;
-    bm += b * bm_stride;
-    if (bmh) bmh += b * bmh_stride;
-    epart += (long)b * gridDim.x;
-  }
+  sr *= a.inv_sa;
+  si *= a.inv_sa;
+  a.sk[(long)r * 2 * a.nZ + 2 * c] = sr;
+  a.sk[(long)r * 2 * a.nZ + 2 * c + 1] = si;
+  const double w = r < a.R ? a.W[(long)r * a.nZ + c] : 0.0;
+  const double gr = w * sr, gi = -w * si, nz = (double)(c - a.kz);
+  const int rb = r >> 4, rr = r & 15;
+  T *bm = reinterpret_cast<T *>(a.bm);
+  // values for kappa = 2c (s=0) and 2c+1 (s=1) of the four components
+  const double v[4][2] = {{gr, -gi}, {gi, gr}, {nz * gr, -nz * gi}, {nz * gi, nz * gr}};
+#pragma unroll
+  for (int comp = 0; comp < 4; ++comp)
+#pragma unroll
+    for (int sidx = 0; sidx < 2; ++sidx) {
+      const int kap = 2 * c + sidx;
+      const int lanef = (kap & 3) * 16 + rr;
+      const int ks = kap >> 2, sl = ks / a.KSS;  // K-step and its slab
+      bm[((((long)sl * (a.Rpad >> 4) + rb) * 4 + comp) * 64 + lanef) * a.KSP + (ks - sl * a.KSS)] =
+          (T)v[comp][sidx];
+      if (a.bmh) {
+        // split form: K-step kap'/32, lane (kap'%32/8)*16 + rr, element
+        // kap'%8; 64 lanes x 8 hi halves, then 64 lanes x 8 lo halves
+        _Float16 *blk = a.bmh + (long)rb * (split_blk_bytes(a.nkh) / 2);
+        const float vf = (float)(v[comp][sidx] * a.sb);
+        if (c == a.kz) {
+          if (comp < 2 && sidx == 0)
+            reinterpret_cast<float *>(blk + 4 * a.nkh * 2 * 64 * 8)[comp * 16 + rr] = vf;
+        } else {
+          const int kq = 2 * (c < a.kz ? c : c - 1) + sidx;
+          const int unit = (comp * a.nkh + (kq >> 5)) * 2;
+          const int ln = ((kq & 31) >> 3) * 16 + rr, el = kq & 7;
+          const _Float16 h = (_Float16)vf;
+          blk[(unit * 64 + ln) * 8 + el] = h;
+          blk[((unit + 1) * 64 + ln) * 8 + el] = (_Float16)(vf - (float)h);
+        }
+      }
+    }
+  return w * (sr * sr + si * si);
+}
+
+// Batched: grid row b reduces replica b's (few) chunks into its own S and
+// operands, one thread per lattice point.
+template <typename T, typename P>
+__global__ void k_sk_reduce(SReduce a, const int2 *rchunks, long bm_stride, long bmh_stride)
+{
+  const int b = blockIdx.y;
+  const P *part = reinterpret_cast<const P *>(a.part) + (long)rchunks[b].x * a.Rpad * a.SC;
+  a.nchunks = rchunks[b].y;
+  a.W += (long)b * a.R * a.nZ;
+  a.sk += (long)b * a.Rpad * 2 * a.nZ;
+  a.bm = reinterpret_cast<T *>(a.bm) + b * bm_stride;
+  if (a.bmh) a.bmh += b * bmh_stride;
+  a.epart += (long)b * gridDim.x;
   const int t = blockIdx.x * kBlock + threadIdx.x;
   double e = 0;
-  if (t < Rpad * nZ) {
-    const int r = t / nZ, c = t - r * nZ;
+  if (t < a.Rpad * a.nZ) {
+    const int r = t / a.nZ, c = t - r * a.nZ;
     double sr = 0, si = 0;
-    for (int k = 0; k < nchunks; ++k) {
-      const P *p = part + ((long)k * Rpad + r) * SC + 2 * c;
+#pragma unroll 4
+    for (int k = 0; k < a.nchunks; ++k) {
+      const P *p = part + ((long)k * a.Rpad + r) * a.SC + 2 * c;
       sr += (double)p[0];
       si += (double)p[1];
     }
-    sr *= inv_sa;
-    si *= inv_sa;
-    sk[(long)r * 2 * nZ + 2 * c] = sr;
-    sk[(long)r * 2 * nZ + 2 * c + 1] = si;
-    const double w = r < R ? W[(long)r * nZ + c] : 0.0;
-    e = w * (sr * sr + si * si);
-    const double gr = w * sr, gi = -w * si, nz = (double)(c - kz);
-    const int rb = r >> 4, rr = r & 15;
-    // values for kappa = 2c (s=0) and 2c+1 (s=1) of the four components
-    const double v[4][2] = {{gr, -gi}, {gi, gr}, {nz * gr, -nz * gi}, {nz * gi, nz * gr}};
-#pragma unroll
-    for (int comp = 0; comp < 4; ++comp)
-#pragma unroll
-      for (int sidx = 0; sidx < 2; ++sidx) {
-        const int kap = 2 * c + sidx;
-        const int lanef = (kap & 3) * 16 + rr;
-        const int ks = kap >> 2, sl = ks / KSS;  // K-step and its slab
-        bm[((((long)sl * (Rpad >> 4) + rb) * 4 + comp) * 64 + lanef) * KSP + (ks - sl * KSS)] =
-            (T)v[comp][sidx];
-        if (bmh) {
-          // split form: K-step kap'/32, lane (kap'%32/8)*16 + rr, element
-          // kap'%8; 64 lanes x 8 hi halves, then 64 lanes x 8 lo halves
-          _Float16 *blk = bmh + (long)rb * (split_blk_bytes(nkh) / 2);
-          const float vf = (float)(v[comp][sidx] * sb);
-          if (c == kz) {
-            if (comp < 2 && sidx == 0)
-              reinterpret_cast<float *>(blk + 4 * nkh * 2 * 64 * 8)[comp * 16 + rr] = vf;
-          } else {
-            const int kq = 2 * (c < kz ? c : c - 1) + sidx;
-            const int unit = (comp * nkh + (kq >> 5)) * 2;
-            const int ln = ((kq & 31) >> 3) * 16 + rr, el = kq & 7;
-            const _Float16 h = (_Float16)vf;
-            blk[(unit * 64 + ln) * 8 + el] = h;
-            blk[((unit + 1) * 64 + ln) * 8 + el] = (_Float16)(vf - (float)h);
-          }
-        }
-      }
+    e = put_operand<T>(a, r, c, sr, si);
   }
   __shared__ double red[kBlock];
   red[threadIdx.x] = e;
@@ -402,51 +440,57 @@ __global__ void k_sk_reduce(int nchunks, int Rpad, int SC, int R, int nZ, int kz
     if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) epart[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) a.epart[blockIdx.x] = red[0];
 }
 
-// Fixed-order sum of the S-pass chunk partials ([chunk][plane] -> [plane]):
-// 64 entries per block, wave w sums chunks w, w+4, ..., then the four wave sums
-// are combined in one fixed order (coalesced, and 4x the parallelism of one
-// thread per entry walking every chunk).
-template <typename P>
-__global__ void k_chunk_sum(const P *part, int nchunks, long plane, double *out)
+// The same for one system, whose chunks are many: a workgroup sums 64 columns
+// of a row tile's partials, its 16 waves every 16th chunk each (then in wave
+// order), and 32 of its threads write the operands of its 32 lattice points.
+// Reading the partials bounds it.  As a sum of 4 waves a workgroup and a
+// second launch it took 35 + 5 us at N = 30011, kmax 10 (469 chunks), 20 + 5 us at
+// N = 8000, kmax 8; now 8 and 7 us.
+constexpr int kReduceBlock = 1024;
+
+template <typename T, typename P>
+__global__ __launch_bounds__(kReduceBlock) void k_sk_finish(SReduce a)
 {
-  __shared__ double red[4][64];
+  __shared__ double red[kReduceBlock / 64][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long e = (long)blockIdx.x * 64 + lane;
+  const long plane = (long)a.Rpad * a.SC, e = (long)blockIdx.x * 64 + lane;  // plane: multiple of 64
+  const P *part = reinterpret_cast<const P *>(a.part);
   double s = 0;
-  if (e < plane)
-    for (int k = wave; k < nchunks; k += 4) s += (double)part[(long)k * plane + e];
+#pragma unroll 8
+  for (int k = wave; k < a.nchunks; k += kReduceBlock / 64) s += (double)part[(long)k * plane + e];
   red[wave][lane] = s;
   __syncthreads();
-  if (wave == 0 && e < plane) out[e] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+  if (wave != 0) return;
+  s = 0;
+#pragma unroll
+  for (int w = 0; w < kReduceBlock / 64; ++w) s += red[w][lane];
+  // even lanes hold Re S of a point, their neighbours Im S
+  const double si = __shfl_xor(s, 1, 64);
+  const int r = (int)(e / a.SC), c = (int)(e - (long)r * a.SC) >> 1;
+  double en = 0;
+  if (!(lane & 1) && c < a.nZ) en = put_operand<T>(a, r, c, s, si);
+  for (int o = 32; o > 0; o >>= 1) en += __shfl_xor(en, o, 64);
+  if (lane == 0) a.epart[blockIdx.x] = en;
 }
 
-// The same sums for FP32 partials, four adjacent entries per lane (16-byte
-// loads; plane is a multiple of 4); per entry the summation order is
-// k_chunk_sum's.
-__global__ void k_chunk_sum4(const float *part, int nchunks, long plane, double *out)
+// The lattice energy's partials, summed by the force pass's first workgroup.
+__device__ __forceinline__ void sum_energy(const double *epart, int count, double *out)
 {
-  __shared__ double red[4][4][64];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long e = ((long)blockIdx.x * 64 + lane) * 4;
-  double s[4] = {0, 0, 0, 0};
-  if (e < plane)
-    for (int k = wave; k < nchunks; k += 4) {
-      const float4 v = *reinterpret_cast<const float4 *>(part + (long)k * plane + e);
-      s[0] += (double)v.x;
-      s[1] += (double)v.y;
-      s[2] += (double)v.z;
-      s[3] += (double)v.w;
-    }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) red[wave][i][lane] = s[i];
+  __shared__ double ered[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  double s = 0;
+  for (int k = threadIdx.x; k < count; k += blockDim.x) s += epart[k];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) ered[wave] = s;
   __syncthreads();
-  if (wave == 0 && e < plane)
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      out[e + i] = (red[0][i][lane] + red[1][i][lane]) + (red[2][i][lane] + red[3][i][lane]);
+  if (threadIdx.x == 0) {
+    s = 0;
+    for (int w = 0; w < nw; ++w) s += ered[w];
+    *out = s;
+  }
 }
 
 // zero the padding rows of the operand (kappa >= 2 nZ)
@@ -475,6 +519,10 @@ struct FArgs {
   double *part;  // row splits: [slab * splits + split][4][n] sums, or nullptr
   int rb_per;    // row blocks per split (blockIdx.y)
   int slab;      // K slab of this launch
+  int set;       // write the accelerations instead of adding to them
+  const double *epart;  // lattice energy partials to sum into *eout, or nullptr
+  int ecount;
+  double *eout;
   // batched: per workgroup (first atom, end atom, -, replica), the replicas'
   // constants, and the operand stride (bytes) between replicas
   const int4 *items;
@@ -516,6 +564,7 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
     a.kzs = r.kzs;
   }
   const int offY = a.nX, offZ = a.nX + a.nY;
+  if (a.epart && blockIdx.x == 0 && blockIdx.y == 0) sum_energy(a.epart, a.ecount, a.eout);
 
   // A fragments: A[atom = l%16][kappa = 4 (s0 + s) + l/16] = (Zr, Zi)(c = kappa/2)
   T am[NT][KS];
@@ -674,9 +723,10 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
           a.out4[4 * atom + 3] = a.c0 * vp;
         } else {
           const double qm = a.q[atom] * a.minv[a.type[atom]];
-          a.ax[atom] += gx * qm;
-          a.ay[atom] += gy * qm;
-          a.az[atom] += gz * qm;
+          const bool add = !a.set || a.slab > 0;
+          a.ax[atom] = (add ? a.ax[atom] : 0.0) + gx * qm;
+          a.ay[atom] = (add ? a.ay[atom] : 0.0) + gy * qm;
+          a.az[atom] = (add ? a.az[atom] : 0.0) + gz * qm;
         }
       }
     }
@@ -688,7 +738,7 @@ __global__ __launch_bounds__(64 * kWavesF) void k_kforce(FArgs a)
 // the charge) and 1/m.
 __global__ void k_kforce_sum(int n, int nparts, const double *part, const double *q,
                              const double *minv, const int *type, double *ax, double *ay,
-                             double *az, double *out4)
+                             double *az, double *out4, int set)
 {
   const int i = blockIdx.x * kBlock + threadIdx.x, d = blockIdx.y;
   if (i >= n) return;
@@ -700,7 +750,7 @@ __global__ void k_kforce_sum(int n, int nparts, const double *part, const double
     out4[4L * i + d] = v;
   } else {
     double *a = d == 0 ? ax : (d == 1 ? ay : az);
-    a[i] += v * (q ? q[i] * minv[type[i]] : minv[type[i]]);
+    a[i] = (set ? 0.0 : a[i]) + v * (q ? q[i] * minv[type[i]] : minv[type[i]]);
   }
 }
 
@@ -1083,7 +1133,10 @@ struct FArgsH {
   double c0, kxs, kys, kzs;  // c0 includes 1/(sA sB): X carries q sA, the operand sB
   double *ax, *ay, *az;
   double *part;       // row splits, as FArgs (without the potential)
-  int rb_per;
+  int rb_per, set;
+  const double *epart;
+  int ecount;
+  double *eout;
   const int4 *items;  // batched, as FArgs
   const RepDev *rep;
   long bm_stride;
@@ -1130,6 +1183,7 @@ __global__ __launch_bounds__(64 * W) void k_kforce_h(FArgsH a)
   }
   const long base = wg_base + (long)wave * (16 * NT);
   const int offY = a.nX;
+  if (a.epart && blockIdx.x == 0 && blockIdx.y == 0) sum_energy(a.epart, a.ecount, a.eout);
   {
     // the workgroup's table blocks (its first atom starts a block)
     const long cnt = min((long)wg_atoms, a.n - wg_base);
@@ -1318,9 +1372,9 @@ __global__ __launch_bounds__(64 * W) void k_kforce_h(FArgsH a)
         }
         // the phase factors carry the atom's charge (times sA, removed in c0)
         const double m = a.minv[a.type[atom]];
-        a.ax[atom] += gx * m;
-        a.ay[atom] += gy * m;
-        a.az[atom] += gz * m;
+        a.ax[atom] = (a.set ? 0.0 : a.ax[atom]) + gx * m;
+        a.ay[atom] = (a.set ? 0.0 : a.ay[atom]) + gy * m;
+        a.az[atom] = (a.set ? 0.0 : a.az[atom]) + gz * m;
       }
     }
 }
@@ -1506,12 +1560,12 @@ int ewald_k_plan(cav_ctx *c)
 
 constexpr int kRT = 3;  // row tiles per S-pass wave
 
-// Row-tile groups of the S pass: as few groups as the 8-wave limit allows,
-// split evenly so that no wave of a group idles.
+// Row-tile groups of the S pass: as few groups as seven compute waves allow (the
+// eighth is the producer), split evenly so that no wave of a group idles.
 static void s_layout(const cav_ctx *c, int *groups, int *tiles_per_group, int *waves)
 {
   const int tiles = c->ek.Rpad / 16;
-  const int per_max = kWavesMax * kRT;
+  const int per_max = (kWavesMax - 1) * kRT;
   const int g = (tiles + per_max - 1) / per_max;
   int tpg = (tiles + g - 1) / g;
   tpg = (tpg + kRT - 1) / kRT * kRT;
@@ -1537,7 +1591,7 @@ static void s_layout_h(int Rpad, int RT, int *groups, int *tiles_per_group, int 
 static void s_layout_rt(int Rpad, int RT, int *groups, int *tiles_per_group, int *waves)
 {
   const int tiles = Rpad / 16;
-  const int per_max = kWavesMax * RT;
+  const int per_max = (kWavesMax - 1) * RT;
   const int g = (tiles + per_max - 1) / per_max;
   int tpg = (tiles + g - 1) / g;
   tpg = (tpg + RT - 1) / RT * RT;
@@ -1556,6 +1610,9 @@ static int s_chunk(const cav_ctx *c, int ntarget)
   // aim for >= ntarget workgroups over the whole grid; chunk multiple of 32
   int groups, tpg, waves;
   s_layout(c, &groups, &tpg, &waves);
+  // FP64: a workgroup of four to seven compute waves has a CU to itself, and
+  // one round of them leaves half the partials of two
+  if (c->precision == CAV_FP64 && waves >= 4) ntarget /= 2;
   long per = ((long)c->n * groups + ntarget - 1) / ntarget;
   per = (per + 31) / 32 * 32;
   if (per < 32) per = 32;
@@ -1615,8 +1672,6 @@ int ewald_k_alloc(cav_ctx *c)
   CAV_HIP(hipMemsetAsync(c->sk_part, 0, plane_bytes * c->sk_planes, c->stream));
   if (c->sk) (void)hipFree(c->sk);
   CAV_HIP(hipMalloc(&c->sk, sizeof(double) * (size_t)p.Rpad * 2 * p.nZ));
-  if (c->sk_sum) (void)hipFree(c->sk_sum);
-  CAV_HIP(hipMalloc(&c->sk_sum, sizeof(double) * (size_t)p.Rpad * SC));
   if (c->bmat) (void)hipFree(c->bmat);
   const size_t bm_elems = p.nslab * slab_elems(p);
   CAV_HIP(hipMalloc(&c->bmat, bm_elems * tsz));
@@ -1661,7 +1716,7 @@ static void launch_sk_rt(hipStream_t st, SArgs a, dim3 lgrid, size_t smem, int S
   a.ncols = (int)lgrid.x;
   a.groups = (int)lgrid.y;
   const dim3 grid((lgrid.x + 7) / 8 * 8 * lgrid.y, std::max(a.sets, 1));
-  const int block = 64 * waves;
+  const int block = 64 * (waves + 1);  // compute waves + the producer wave
   // one launch per 8 column tiles; each writes its own columns of the partials
   for (a.ct0 = 0; a.ct0 < SCT; a.ct0 += 8) {
     switch (std::min(8, SCT - a.ct0)) {
@@ -1692,6 +1747,7 @@ static void launch_kforce_t(hipStream_t st, FArgs a, const EwaldKPlan &p, int gr
     a.nks = std::min(p.KSS, nks - a.s0);
     a.out4_add = sl > 0;
     a.slab = sl;
+    if (sl > 0) a.epart = nullptr;
     a.bm = bm0 + sl * slab_elems(p) * sizeof(T);
     if (KS <= 8) {
       allow_smem(k_kforce<T, 8, NT>, smem);
@@ -1712,8 +1768,34 @@ static void launch_kforce_t(hipStream_t st, FArgs a, const EwaldKPlan &p, int gr
   }
 }
 
-// Phase tables + S pass + reduction for npts points (the owned atoms, or query
-// points when tab/positions are the caller's).
+// Workgroups of k_sk_finish, one lattice-energy partial each.
+static int energy_blocks(const EwaldKPlan &p) { return p.Rpad / 16 * (roundup(2 * p.nZ, 16) / 4); }
+
+static SReduce sk_reduce_args(cav_ctx *c, int nchunks, int SC, double inv_sa, _Float16 *bmh)
+{
+  const EwaldKPlan &p = c->ek;
+  SReduce a;
+  a.nchunks = nchunks;
+  a.Rpad = p.Rpad;
+  a.SC = SC;
+  a.R = p.R;
+  a.nZ = p.nZ;
+  a.kz = p.kz;
+  a.KSS = p.KSS;
+  a.KSP = p.KSP;
+  a.part = c->sk_part;
+  a.W = c->d_W;
+  a.sk = c->sk;
+  a.bm = c->bmat;
+  a.epart = c->part;
+  a.inv_sa = inv_sa;
+  a.bmh = bmh;
+  a.nkh = c->nkh;
+  a.sb = c->sB;
+  return a;
+}
+
+// Phase tables + S pass + reduction of the owned atoms.
 template <typename T>
 static int sk_pipeline(cav_ctx *c)
 {
@@ -1750,14 +1832,10 @@ static int sk_pipeline(cav_ctx *c)
   timer_begin(c, c->t_sk);
   launch_sk_rt<T, kRT>(c->stream, a, grid, smem, a.SC / 16, waves);
   timer_end(c, c->t_sk);
-  const int nthr = p.Rpad * p.nZ;
-  const long plane = (long)p.Rpad * a.SC;
-  k_chunk_sum<double><<<(plane + 63) / 64, kBlock, 0, c->stream>>>(c->sk_part, nch, plane, c->sk_sum);
-  k_sk_reduce<T, double><<<grid_for(nthr), kBlock, 0, c->stream>>>(
-      1, p.Rpad, a.SC, p.R, p.nZ, p.kz, p.KSS, p.KSP, c->sk_sum, c->d_W, c->sk, (T *)c->bmat, c->part,
-      1.0, nullptr, 0, 1.0, nullptr, 0, 0);
+  k_sk_finish<T, double><<<energy_blocks(p), kReduceBlock, 0, c->stream>>>(
+      sk_reduce_args(c, nch, a.SC, 1.0, nullptr));
   CAV_HIP(hipGetLastError());
-  return reduce_partials(c, grid_for(nthr), 3);
+  return CAV_OK;
 }
 
 template <typename T>
@@ -1765,6 +1843,11 @@ static int kforce(cav_ctx *c, int npts, const void *tab, double *out4)
 {
   const EwaldKPlan &p = c->ek;
   FArgs f;
+  // the force pass after an S pass sums its energy partials
+  f.set = c->ek_set;
+  f.epart = out4 ? nullptr : c->part;
+  f.ecount = energy_blocks(p);
+  f.eout = c->scal + 3;
   f.n = npts;
   f.TS = p.nX + p.nY + p.nZ;
   f.nX = p.nX;
@@ -1803,7 +1886,7 @@ static int kforce(cav_ctx *c, int npts, const void *tab, double *out4)
   launch_kforce_t<T>(c->stream, f, p, g, used);
   if (used > 1)
     k_kforce_sum<<<dim3(grid_for(npts), out4 ? 4 : 3), kBlock, 0, c->stream>>>(
-        npts, p.nslab * used, f.part, f.q, f.minv, f.type, f.ax, f.ay, f.az, out4);
+        npts, p.nslab * used, f.part, f.q, f.minv, f.type, f.ax, f.ay, f.az, out4, f.set);
   timer_end(c, c->t_force);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -1887,15 +1970,10 @@ static int sk_pipeline_h(cav_ctx *c)
   else
     launch_sk_h<3>(c->stream, a, lg, smem, split_sct(p), waves);
   timer_end(c, c->t_sk);
-  const int nthr = p.Rpad * p.nZ;
-  const long plane = (long)p.Rpad * a.SC;
-  k_chunk_sum4<<<(plane / 4 + 63) / 64, kBlock, 0, c->stream>>>(
-      reinterpret_cast<const float *>(c->sk_part), nch, plane, c->sk_sum);
-  k_sk_reduce<float, double><<<grid_for(nthr), kBlock, 0, c->stream>>>(
-      1, p.Rpad, a.SC, p.R, p.nZ, p.kz, p.KSS, p.KSP, c->sk_sum, c->d_W, c->sk, (float *)c->bmat,
-      c->part, 1.0 / c->sA, (_Float16 *)c->bmat_h, c->nkh, c->sB, nullptr, 0, 0);
+  k_sk_finish<float, float><<<energy_blocks(p), kReduceBlock, 0, c->stream>>>(
+      sk_reduce_args(c, nch, a.SC, 1.0 / c->sA, (_Float16 *)c->bmat_h));
   CAV_HIP(hipGetLastError());
-  return reduce_partials(c, grid_for(nthr), 3);
+  return CAV_OK;
 }
 
 // LDS of a split force-pass workgroup: two operand blocks plus the blocked X
@@ -1937,6 +2015,10 @@ static int kforce_h(cav_ctx *c)
 {
   const EwaldKPlan &p = c->ek;
   FArgsH f;
+  f.set = c->ek_set;
+  f.epart = c->part;
+  f.ecount = energy_blocks(p);
+  f.eout = c->scal + 3;
   f.n = c->n;
   f.TS = p.nX + p.nY;
   f.nX = p.nX;
@@ -1985,7 +2067,7 @@ static int kforce_h(cav_ctx *c)
   }
   if (used > 1)
     k_kforce_sum<<<dim3(grid_for(c->n), 3), kBlock, 0, c->stream>>>(
-        c->n, used, f.part, nullptr, f.minv, f.type, f.ax, f.ay, f.az, nullptr);
+        c->n, used, f.part, nullptr, f.minv, f.type, f.ax, f.ay, f.az, nullptr, f.set);
   timer_end(c, c->t_force);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -2492,17 +2574,30 @@ static int batch_ewald_k_t(cav_batch *b)
     else
       batch_sk_h<3>(b, a, groups, smem, split_sct(p), waves);
   }
-  const int nthr = p.Rpad * p.nZ;
+  SReduce sr;
+  sr.nchunks = 0;
+  sr.Rpad = p.Rpad;
+  sr.SC = SC;
+  sr.R = p.R;
+  sr.nZ = p.nZ;
+  sr.kz = p.kz;
+  sr.KSS = p.KSS;
+  sr.KSP = p.KSP;
+  sr.part = b->sk_part;
+  sr.W = b->d_W;
+  sr.sk = b->sk;
+  sr.bm = b->bmat;
+  sr.epart = b->epart;
+  sr.inv_sa = split ? 1.0 / b->sA : 1.0;
+  sr.bmh = split ? (_Float16 *)b->bmat_h : nullptr;
+  sr.nkh = b->nkh;
+  sr.sb = split ? b->sB : 1.0;
+  const dim3 rgrid(grid_for((long)p.Rpad * p.nZ), b->B);
   // partials: FP32 from the split S pass, FP64 from the FP32 / FP64 tiles
   if (split)
-    k_sk_reduce<T, float><<<dim3(grid_for(nthr), b->B), kBlock, 0, b->stream>>>(
-        0, p.Rpad, SC, p.R, p.nZ, p.kz, p.KSS, p.KSP, reinterpret_cast<const float *>(b->sk_part),
-        b->d_W, b->sk, (T *)b->bmat, b->epart, 1.0 / b->sA, (_Float16 *)b->bmat_h, b->nkh, b->sB,
-        b->rchunks, b->bm_stride, b->bmh_stride);
+    k_sk_reduce<T, float><<<rgrid, kBlock, 0, b->stream>>>(sr, b->rchunks, b->bm_stride, b->bmh_stride);
   else
-    k_sk_reduce<T, double><<<dim3(grid_for(nthr), b->B), kBlock, 0, b->stream>>>(
-        0, p.Rpad, SC, p.R, p.nZ, p.kz, p.KSS, p.KSP, b->sk_part, b->d_W, b->sk, (T *)b->bmat,
-        b->epart, 1.0, nullptr, b->nkh, 1.0, b->rchunks, b->bm_stride, b->bmh_stride);
+    k_sk_reduce<T, double><<<rgrid, kBlock, 0, b->stream>>>(sr, b->rchunks, b->bm_stride, b->bmh_stride);
   if (!split) {
     FArgs f;
     f.n = 0;
@@ -2529,6 +2624,8 @@ static int batch_ewald_k_t(cav_batch *b)
     f.rep = b->d_rep;
     f.bm_stride = b->bm_stride * (long)sizeof(T);
     f.part = nullptr;
+    f.epart = nullptr;
+    f.set = 0;
     f.rb_per = p.Rpad / 16;
     launch_kforce_t<T>(b->stream, f, p, b->n_fitems, 1);
   } else {
@@ -2557,6 +2654,8 @@ static int batch_ewald_k_t(cav_batch *b)
     f.bm_stride = b->bmh_stride * (long)sizeof(_Float16);
     f.inv_sb = 1.0 / b->sB / b->sA;
     f.part = nullptr;
+    f.epart = nullptr;
+    f.set = 0;
     f.rb_per = p.Rpad / 16;
     if (b->f_nt == 1)
       launch_kforce_h<1, kWavesF>(b->stream, f, b->nkh, b->n_fitems, 1, split_force_lds_p(p, b->nkh, 1));
@@ -2622,6 +2721,8 @@ static int batch_field_t(cav_batch *b, double *out4)
   f.rep = b->d_rep;
   f.bm_stride = b->bm_stride * (long)sizeof(T);
   f.part = nullptr;
+  f.epart = nullptr;
+  f.set = 0;
   f.rb_per = p.Rpad / 16;
   launch_kforce_t<T>(b->stream, f, p, b->n_fitems, 1);
   BAT_HIP(hipGetLastError());

@@ -249,6 +249,7 @@ struct cav_ctx {
   // the side stream's Ewald_k leaves the dipole term to the main stream, which
   // adds it after the k-space sum (the in-order rounding: (a_sr + a_k) + a_dip)
   bool defer_dipole = false;
+  bool ek_set = false;  // Ewald_k writes its accelerations instead of adding them
   cav::Stage stage;
   double *pt_dev = nullptr;  // point queries: coordinates and results
   size_t pt_cap = 0;
@@ -264,7 +265,6 @@ struct cav_ctx {
   int sk_chunks = 0;
   long sk_planes = 0;        // chunk planes sk_part holds
   double *sk = nullptr;      // [Rpad][2nZ] FP64
-  double *sk_sum = nullptr;  // [Rpad][SC] chunk partials summed (fixed order)
   void *bmat = nullptr;      // [KZ][4*Rpad] (T) force-pass operand
   // mixed form: split-FP16 Z records and force-pass operand (hi + lo halves)
   void *ztab = nullptr;      // [n][nZ] x 16 B: (Zr,-Zi) hi, (Zr,-Zi) lo, (Zi,Zr) hi, (Zi,Zr) lo
