@@ -37,7 +37,8 @@ struct AdjArgs {
   const double *eps, *sig;
   double lj_rc, lj_rc2;
   int lj_on, er_on, lambda_set;
-  double alpha, a2, ke, two_a_rpi;
+  EwaldAlpha al;
+  double ke, two_a_rpi;
   const double *lambda, *charge;
   double *part;  // [block][nvals]: g_eps[nt2] | g_sig[nt2] | g_q[nt]
   const RepDev *rep;  // batched replicas (blockIdx.y) or nullptr
@@ -123,8 +124,9 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_pairs(AdjArgs a)
           if (lam == 0.0) skip = true;
         }
         if (!skip) {
-          const double rn = sqrt(r2);
-          const double sr = (a.two_a_rpi * exp(-a.a2 * r2) + erfc(a.alpha * rn) / rn) / r2;
+          double e, ec, ri2;
+          ewald_real(r2, a.al, e, ec, ri2);
+          const double sr = fma(a.two_a_rpi, e, ec) * ri2;
           // coef = -lam ke q_a q_b sr: d/dq_a = -lam ke q_b sr, d/dq_b = -lam ke q_a sr
           const double base = -lam * a.ke * sr * wr;
           double qtj = 0;
@@ -441,8 +443,7 @@ static int adjoint_run(cav_ctx *c, const double *w_host, const AdjWork &k, doubl
     a.lj_on = c->lj_on;
     a.er_on = c->er_on;
     a.lambda_set = c->lambda_set;
-    a.alpha = c->er_alpha;
-    a.a2 = c->er_alpha * c->er_alpha;
+    a.al = ewald_alpha(c->er_alpha);
     a.ke = c->er_ke;
     a.two_a_rpi = 2 * c->er_alpha * CAV_PIS_INV;
     a.lambda = c->d_lambda;
@@ -649,8 +650,7 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
     a.lj_on = b->lj_on;
     a.er_on = b->er_on;
     a.lambda_set = 0;
-    a.alpha = b->er_alpha;
-    a.a2 = b->er_alpha * b->er_alpha;
+    a.al = ewald_alpha(b->er_alpha);
     a.ke = b->er_ke;
     a.two_a_rpi = 2 * b->er_alpha * CAV_PIS_INV;
     a.lambda = nullptr;

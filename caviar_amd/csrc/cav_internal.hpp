@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/caviar_amd.h"
+#include "cav_math.hpp"
 
 #define CAV_PI 3.14159265358979323846
 #define CAV_2PI 6.28318530717958647692     // macro_constants.h:22

@@ -49,7 +49,8 @@ struct PairArgs {
   const double *c12, *c6, *cshift;
   double lj_rc2;
   // Ewald real space
-  double alpha, a2, ke, two_a_rpi;
+  EwaldAlpha al;
+  double ke, two_a_rpi;
   const double *lambda;
   double *ax, *ay, *az;
   double *part;
@@ -136,14 +137,15 @@ __device__ __forceinline__ T pair_coef(const PairArgs &a, const T *tab, int nt2,
         const T qj = (T)pj.w;
         T ce;
         if constexpr (sizeof(T) == 8) {
-          const double rn = sqrt(r2);
-          const double s = (a.two_a_rpi * exp(-a.a2 * r2) + erfc(a.alpha * rn) / rn) * (1.0 / r2);
+          double e, ec, ri2;
+          ewald_real(r2, a.al, e, ec, ri2);
+          const double s = fma(a.two_a_rpi, e, ec) * ri2;
           ce = -lam * a.ke * (double)qi * qj * s;
         } else {
           const float rinv = __frsqrt_rn(r2);
           const float rn = r2 * rinv;
-          const float e = __expf(-(float)a.a2 * r2);
-          const float ec = erfc_hastings((float)a.alpha * rn, e);
+          const float e = __expf(-(float)a.al.a2 * r2);
+          const float ec = erfc_hastings((float)a.al.alpha * rn, e);
           const float s = fmaf((float)a.two_a_rpi, e, ec * rinv) * (rinv * rinv);
           ce = -lam * keqi * qj * s;
         }
@@ -708,8 +710,7 @@ static PairArgs pair_args(cav_ctx *c)
   a.c6 = c->d_eps + nt2;
   a.cshift = c->d_eps + 2 * nt2;
   a.lj_rc2 = c->lj_rc * c->lj_rc;
-  a.alpha = c->er_alpha;
-  a.a2 = c->er_alpha * c->er_alpha;
+  a.al = ewald_alpha(c->er_alpha);
   a.ke = c->er_ke;
   a.two_a_rpi = 2 * c->er_alpha * CAV_PIS_INV;
   a.lambda = c->d_lambda;
@@ -1086,7 +1087,7 @@ __device__ __forceinline__ double4 walk_cand(const CellArgs &c, const int *s_bas
 // all of its candidates by itself and a launch held np / 64 waves: 1000 points
 // among 100 ions took 818 us, now 14 us.
 __global__ __launch_bounds__(kBlock) void k_point_r(CellArgs c, int np, const double *pts,
-                                                    double alpha, double ke, double *field,
+                                                    EwaldAlpha al, double ke, double *field,
                                                     double *pot)
 {
   __shared__ int s_base_[kBlock / 64][32], s_off_[kBlock / 64][33];
@@ -1097,17 +1098,19 @@ __global__ __launch_bounds__(kBlock) void k_point_r(CellArgs c, int np, const do
   int *s_base = s_base_[wv], *s_off = s_off_[wv];
   const int total = walk_ranges(c, cell_of(c, px, py, pz), s_base, s_off);
   __syncwarp();
-  const double a2 = alpha * alpha;
+  const double two_a_rpi = 2 * al.alpha * CAV_PIS_INV;
   double phi = 0, ex = 0, ey = 0, ez = 0;
   int cell = 0;
   for (int g = lane; g < total; g += 64) {
     const double4 v = walk_cand(c, s_base, s_off, g, cell);
     const double dx = px - v.x, dy = py - v.y, dz = pz - v.z;
     if (dx == 0 && dy == 0 && dz == 0) continue;
-    const double d2 = dx * dx + dy * dy + dz * dz, dn = sqrt(d2);
-    const double ec = erfc(alpha * dn) / dn;
-    phi += v.w * ec;
-    const double sr = (2 * alpha * CAV_PIS_INV * exp(-a2 * d2) + ec) / d2;
+    const double d2 = dx * dx + dy * dy + dz * dz;
+    double e, ec, ri2;
+    ewald_real(d2, al, e, ec, ri2);
+    const bool none = d2 >= 1e290;  // infinitely far: both terms vanish
+    phi += none ? 0.0 : v.w * ec;
+    const double sr = none ? 0.0 : fma(two_a_rpi, e, ec) * ri2;
     ex += v.w * sr * dx;
     ey += v.w * sr * dy;
     ez += v.w * sr * dz;
@@ -1142,7 +1145,7 @@ int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *
   double *df = d + 3 * (size_t)np, *dp = d + 6 * (size_t)np;
   if (np > 0)
     k_point_r<<<(np + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, c->stream>>>(
-        cell_args(c), np, d, c->er_alpha, c->er_ke, df, dp);
+        cell_args(c), np, d, ewald_alpha(c->er_alpha), c->er_ke, df, dp);
   CAV_HIP(hipGetLastError());
   if (!staged && field)
     CAV_HIP(hipMemcpyAsync(field, df, sizeof(double) * 3 * np, hipMemcpyDeviceToHost, c->stream));
@@ -1164,7 +1167,7 @@ constexpr int kWalkCand = 512;
 // over the candidates.  The FP64 erfc of every (atom, candidate) bounds it
 // (about 500 an atom at rho = 0.3); one lane per atom, each walking its
 // stencil through scattered loads, took 3395 us at N = 100003, now 395 us.
-__global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, double alpha, double *part)
+__global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, EwaldAlpha al, double *part)
 {
   __shared__ double4 cand[kWalkCand];
   __shared__ int s_base[32], s_off[33];
@@ -1194,8 +1197,10 @@ __global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, double alpha, d
           const double4 v = cand[t];
           const double dx = xi - v.x, dy = yi - v.y, dz = zi - v.z;
           if (dx == 0 && dy == 0 && dz == 0) continue;
-          const double dn = sqrt(dx * dx + dy * dy + dz * dz);
-          phi += v.w * (erfc(alpha * dn) / dn);
+          const double d2 = dx * dx + dy * dy + dz * dz;
+          double e, ec, ri2;
+          ewald_real(d2, al, e, ec, ri2);
+          phi += d2 >= 1e290 ? 0.0 : v.w * ec;  // infinitely far: nothing
         }
         e += c.q[i] * phi;
       }
@@ -1213,7 +1218,7 @@ __global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, double alpha, d
 int launch_energy_r(cav_ctx *c)
 {
   if (c->nbins > c->npart) return fail(c, CAV_ERR_STATE, "partial-sum buffer smaller than the cell grid");
-  k_energy_r<<<c->nbins, kBlock, 0, c->stream>>>(cell_args(c), c->er_alpha, c->part);
+  k_energy_r<<<c->nbins, kBlock, 0, c->stream>>>(cell_args(c), ewald_alpha(c->er_alpha), c->part);
   CAV_HIP(hipGetLastError());
   return reduce_partials(c, c->nbins, 2);
 }
@@ -1374,8 +1379,7 @@ int batch_pairs(cav_batch *b)
     a.c6 = b->d_lj + nt2;
     a.cshift = b->d_lj + 2 * nt2;
     a.lj_rc2 = b->lj_rc * b->lj_rc;
-    a.alpha = b->er_alpha;
-    a.a2 = b->er_alpha * b->er_alpha;
+    a.al = ewald_alpha(b->er_alpha);
     a.ke = b->er_ke;
     a.two_a_rpi = 2 * b->er_alpha * CAV_PIS_INV;
     a.lambda = nullptr;

@@ -197,3 +197,36 @@ def test_adjoint_weight_sets(gpu, n, kmax, types, precision):
     tol = 1e-10 if precision == "fp64" else 1e-4
     for a, b in zip(e.adjoint(w), o.adjoint(w)):
         assert F.rel_err(np.ravel(a), np.ravel(b)) <= tol
+
+
+@pytest.mark.parametrize("alpha", [0.9, 2.5, 0.0])
+def test_real_space_terms_accuracy(gpu, alpha):
+    """Potential and field of one ion at distances from 1e-3 to 1.4 cells
+    (alpha r from 0 to 10), against 40-digit erfc and exp: 4e-15 relative, i.e.
+    8 ulp for the fit at large alpha r and 10 for the distance, the products and
+    the exponential's last bit."""
+    mp = pytest.importorskip("mpmath")
+    mp.mp.dps = 40
+    print(f"[case] real-space terms alpha={alpha}", flush=True)
+    s = configs.ions(n=1, rho=1e-3, kmax=1, seed=1, with_lj=False, with_k=False)
+    s.lower, s.upper = np.zeros(3), np.full(3, 64.0)
+    s.bc = np.zeros(3, dtype=np.int32)
+    s.pos = np.array([[32.0, 32.0, 32.0]])
+    s.ewald_r.alpha, s.ewald_r.k_electrostatic = alpha, 1.0
+    e = Engine(s)
+    e.setup()
+    # distances exact in FP64 differences: multiples of 2^-20
+    r = np.unique(np.round(np.geomspace(1e-3, 4.0, 400) * 2 ** 20) / 2 ** 20)
+    pts = np.repeat(s.pos, len(r), axis=0)
+    pts[:, 0] += r
+    f, p = e.point_field("r", pts)
+    q = float(s.charge[s.types[0]])
+    al = mp.mpf(alpha)
+    for k in range(len(r)):
+        x = mp.mpf(float(r[k]))
+        ec = mp.erfc(al * x) / x
+        g = (2 * al / mp.sqrt(mp.pi) * mp.exp(-(al * x) ** 2) + ec) / x
+        if ec < mp.mpf(10) ** -290:
+            continue
+        assert abs(mp.mpf(float(p[k])) - q * ec) <= 4e-15 * abs(ec), (r[k], alpha)
+        assert abs(mp.mpf(float(f[k, 0])) - q * g) <= 4e-15 * abs(g), (r[k], alpha)
