@@ -67,8 +67,8 @@ __device__ __forceinline__ double exp_neg(double x, double lo)
 // exp and the library's erfc, whose ranges all run in a wave of mixed
 // distances, take half as many instructions again.  FP64 issue bounds the
 // kernels that are not bound by their gathers: real-space energy at N = 100003
-// 395 -> 249 us, adjoint pairs of 64 replicas 327 -> 265; the pair kernel at
-// N = 65536 (gathers) 101 -> 97 alone.
+// 395 -> 249 us, adjoint pairs of 64 replicas 327 -> 265, the pair kernel at
+// N = 65536 56 -> 37 (in order).
 __device__ __forceinline__ void ewald_real(double r2, const EwaldAlpha &al, double &e, double &ec,
                                            double &ri2)
 {
