@@ -230,3 +230,31 @@ def test_real_space_terms_accuracy(gpu, alpha):
             continue
         assert abs(mp.mpf(float(p[k])) - q * ec) <= 4e-15 * abs(ec), (r[k], alpha)
         assert abs(mp.mpf(float(f[k, 0])) - q * g) <= 4e-15 * abs(g), (r[k], alpha)
+
+
+@pytest.mark.parametrize("n", [255, 256, 700])
+@pytest.mark.parametrize("n_r_df,which", [(d, w) for d in (0, 3) for w in
+                                          ("temp", "berendsen", "nve", "both", "both_no_temp")]
+                         + [(5, "temp")])   # the kinetic energy is 0 there: no finite factors
+def test_constraints_end_of_step(gpu, n, n_r_df, which):
+    """A step's end with every combination of temperature, Berendsen, NVE and
+    pressure, against the oracle after 6 steps (1e-9), with atom counts about a
+    block of partial sums."""
+    from caviar_amd import BerendsenSettings, NVESettings, ThermoSettings
+    print(f"[case] constraints n={n} n_r_df={n_r_df} {which}", flush=True)
+    s = configs.ions(n=n, rho=0.3, kmax=2, seed=n)
+    s.thermo = ThermoSettings(k_b=1.3, n_r_df=n_r_df, temperature_process=which != "both_no_temp",
+                              pressure_process=True)
+    if which in ("berendsen", "both", "both_no_temp"):
+        s.berendsen = BerendsenSettings(temperature=0.9, coupling=0.05, dt=0.002, step=2)
+    if which in ("nve", "both", "both_no_temp"):
+        s.nve = NVESettings(kbt=1.1, step=3)
+    o = Oracle(s)
+    o.setup()
+    assert o.run(0.002, 6) == 0
+    e = Engine(s)
+    e.setup()
+    e.step(0.002, 6)
+    assert F.rel_err(e.get("vel"), o.get("vel")) <= 1e-9
+    for got, want in zip(e.thermo(), o.thermo()):
+        assert abs(got - want) <= 1e-9 * abs(want)
