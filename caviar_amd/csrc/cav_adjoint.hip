@@ -64,6 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_pairs(AdjArgs a)
     a.xq += r.base;
     a.tid += r.base;
     a.nl += (long)r.obase * a.cap;
+    a.items += r.base;  // (a batch keeps its rows as slots)
     a.nn += r.obase;
     a.w += 3L * r.obase;
     a.part += (long)blockIdx.y * gridDim.x * NV;
@@ -639,8 +640,8 @@ extern "C" int cav_batch_adjoint(cav_batch *b, const double *w_host, double *g_e
     a.xq = b->xq;
     a.tid = b->tid;
     a.mol = nullptr;
-    a.nl = b->nl;
-    a.items = nullptr;
+    a.nl = b->nlb;
+    a.items = b->litems;
     a.nn = b->nn;
     a.w = dw;
     a.eps = b->d_raw_eps;

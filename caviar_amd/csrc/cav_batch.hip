@@ -33,14 +33,14 @@ int bhip_check(cav_batch *b, hipError_t e, const char *what)
 
 // ----------------------------------------------------------------- kernels --
 
-__global__ void kb_begin(int B, int *flags)
+// rebuild: every replica's list is built whatever the displacements
+__global__ void kb_begin(int B, int *flags, int rebuild)
 {
   const int r = blockIdx.x * kBlock + threadIdx.x;
   if (r >= B) return;
   int *f = flags + 16 * r;
   f[F_WRAPPED] = 0;
-  f[F_REBUILD] = f[F_FORCE];
-  f[F_FORCE] = 0;
+  f[F_REBUILD] = rebuild;
   f[F_NAN] = 0;
   f[F_OVERFLOW] = 0;
   f[F_MAXNB] = 0;
@@ -53,85 +53,60 @@ __global__ void kb_set_all(int B, int *flags, int idx, int v)
   if (r < B) flags[16 * r + idx] = v;
 }
 
-// exchange_owned for every replica (setup)
-__global__ void kb_wrap(const RepDev *rep, double *x, double *y, double *z, int *flags)
+// Sum of a replica's pair virial partials in a fixed order, by one workgroup.
+__device__ __forceinline__ void replica_virial(int nper, const double *part, double *out)
+{
+  __shared__ double red[kBlock];
+  double s = 0;
+  for (int i = threadIdx.x; i < nper; i += kBlock) s += part[i];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = kBlock / 2; w > 0; w >>= 1) {
+    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = red[0];
+}
+
+__global__ __launch_bounds__(kBlock) void kb_virial(int nper, const double *part, double *vir)
+{
+  replica_virial(nper, part + (long)blockIdx.x * nper, vir + blockIdx.x);
+}
+
+// The end of a step: v += (0.5*dt) * (a + a_old) per replica (grid row), its
+// virial, and its flags, written straight to the host's (pinned) copy and
+// cleared for the next step: a copy and two small launches less a step.
+__global__ __launch_bounds__(kBlock) void kb_kick(const RepDev *rep, double hdt, double *vx,
+                                                  double *vy, double *vz, const double *ax,
+                                                  const double *ay, const double *az,
+                                                  const double *aox, const double *aoy,
+                                                  const double *aoz, int nper, const double *part,
+                                                  double *vir, int *flags, int *host_flags)
 {
   const RepDev &r = rep[blockIdx.y];
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= r.n) return;
-  double *p[3] = {x + r.base + i, y + r.base + i, z + r.base + i};
-  bool wrapped = false;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double v = *p[d];
-    if (v < r.lo[d]) {
-      v = xadd(v, r.L[d]);
-      wrapped = true;
-    } else if (v > r.hi[d]) {
-      v = xsub(v, r.L[d]);
-      wrapped = true;
-    }
-    *p[d] = v;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < r.n) {
+    const long i = (long)r.obase + t;
+    vx[i] = xadd(vx[i], xmul(hdt, xadd(ax[i], aox[i])));
+    vy[i] = xadd(vy[i], xmul(hdt, xadd(ay[i], aoy[i])));
+    vz[i] = xadd(vz[i], xmul(hdt, xadd(az[i], aoz[i])));
   }
-  if (wrapped) {
-    flags[16 * blockIdx.y + F_WRAPPED] = 1;
-    flags[16 * blockIdx.y + F_REBUILD] = 1;
+  if (blockIdx.x != 0) return;
+  replica_virial(nper, part + (long)blockIdx.y * nper, vir + blockIdx.y);
+  if (threadIdx.x < 16) {
+    const int k = threadIdx.x;
+    int *f = flags + 16 * blockIdx.y + k;
+    host_flags[16 * blockIdx.y + k] = *f;
+    if (k == F_WRAPPED || k == F_REBUILD || k == F_NAN || k == F_OVERFLOW || k == F_MAXNB ||
+        k == F_GOVER)
+      *f = 0;
   }
 }
 
-// drift + wrap + NaN check, as the single-system k_drift (md_simulator.cpp:555-590)
-__global__ void kb_drift(const RepDev *rep, double dt, double *x, double *y, double *z,
-                         const double *vx, const double *vy, const double *vz, const double *ax,
-                         const double *ay, const double *az, double *aox, double *aoy, double *aoz,
-                         int *flags)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= r.n) return;
-  int *f = flags + 16 * blockIdx.y;
-  const long o = r.obase + i, s = r.base + i;
-  const double a[3] = {ax[o], ay[o], az[o]};
-  if (isnan(a[0]) || isnan(a[1]) || isnan(a[2])) f[F_NAN] = 1;
-  const double v[3] = {vx[o], vy[o], vz[o]};
-  double *p[3] = {x + s, y + s, z + s};
-  bool wrapped = false;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double h = xmul(xmul(xmul(0.5, a[d]), dt), dt);
-    double q = xadd(*p[d], xadd(xmul(v[d], dt), h));
-    if (q < r.lo[d]) {
-      q = xadd(q, r.L[d]);
-      wrapped = true;
-    } else if (q > r.hi[d]) {
-      q = xsub(q, r.L[d]);
-      wrapped = true;
-    }
-    *p[d] = q;
-  }
-  aox[o] = a[0];
-  aoy[o] = a[1];
-  aoz[o] = a[2];
-  if (wrapped) {
-    f[F_WRAPPED] = 1;
-    f[F_REBUILD] = 1;
-  }
-}
-
-__global__ void kb_kick(long nown, double hdt, double *vx, double *vy, double *vz, const double *ax,
-                        const double *ay, const double *az, const double *aox, const double *aoy,
-                        const double *aoz)
-{
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nown) return;
-  vx[i] = xadd(vx[i], xmul(hdt, xadd(ax[i], aox[i])));
-  vy[i] = xadd(vy[i], xmul(hdt, xadd(ay[i], aoy[i])));
-  vz[i] = xadd(vz[i], xmul(hdt, xadd(az[i], aoz[i])));
-}
-
-// positions (slots) and velocities/accelerations (owned) <-> the snapshot
-__global__ void kb_snapshot(const RepDev *rep, long nown, int save, double *x, double *y, double *z,
-                            double *vx, double *vy, double *vz, double *ax, double *ay, double *az,
-                            double *snap)
+// positions (slots) and velocities/accelerations (owned) back from the snapshot
+__global__ void kb_restore(const RepDev *rep, long nown, double *x, double *y, double *z,
+                           double *vx, double *vy, double *vz, double *ax, double *ay, double *az,
+                           const double *snap)
 {
   const RepDev &r = rep[blockIdx.y];
   const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -139,13 +114,7 @@ __global__ void kb_snapshot(const RepDev *rep, long nown, int save, double *x, d
   const long o = r.obase + i, s = r.base + i;
   double *a[9] = {x + s, y + s, z + s, vx + o, vy + o, vz + o, ax + o, ay + o, az + o};
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    double *sv = snap + k * nown + o;
-    if (save)
-      *sv = *a[k];
-    else
-      *a[k] = *sv;
-  }
+  for (int k = 0; k < 9; ++k) *a[k] = snap[k * nown + o];
 }
 
 }  // namespace cav
@@ -156,14 +125,13 @@ using namespace cav;
 
 static void batch_free(cav_batch *b)
 {
-  void *ptrs[] = {b->d_rep, b->cell_rep, b->st_off, b->st, b->x, b->y, b->z, b->xo, b->yo, b->zo,
+  void *ptrs[] = {b->d_rep, b->waves, b->st_off, b->st, b->x, b->y, b->z, b->xo, b->yo, b->zo,
                   b->type, b->id, b->q, b->xq, b->tid, b->vx, b->vy, b->vz, b->ax, b->ay, b->az,
-                  b->aox, b->aoy, b->aoz, b->type_o, b->q_o, b->snap, b->bin_of, b->bin_cnt,
-                  b->bin_start, b->bin_items, b->gblk, b->nl, b->nn, b->flags, b->d_minv, b->d_lj,
-                  b->adj_ws, b->part, b->vir, b->d_W, b->tab, b->ztab, b->bmat, b->bmat_h, b->sk_part, b->sk,
-                  b->epart, b->s_items, b->s_items_o, b->f_items, b->rchunks, b->cpos, b->d_raw_eps,
-                  b->d_raw_sig, b->d_charge, b->nlb, b->xqs, b->tids, b->litems, b->binpos,
-                  b->order, b->ocnt, b->ostart};
+                  b->type_o, b->q_o, b->snap, b->cell_cnt, b->cell_first, b->bucket, b->bin_start,
+                  b->bin_items, b->gblk, b->nn, b->flags, b->d_minv, b->d_lj, b->adj_ws, b->part,
+                  b->vir, b->d_W, b->tab, b->ztab, b->bmat, b->bmat_h, b->sk_part, b->sk, b->epart,
+                  b->s_items, b->s_items_o, b->f_items, b->rchunks, b->cpos, b->d_raw_eps,
+                  b->d_raw_sig, b->d_charge, b->nlb, b->xqs, b->tids, b->litems, b->order};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->h_flags) (void)hipHostFree(b->h_flags);
@@ -200,7 +168,7 @@ static int batch_layout(cav_batch *b)
   b->cinv = 1.0 / b->rce;
   long slots = 0, own = 0, tabs = 0;
   int cells = 0, maxn = 0;
-  b->h_cell_rep.clear();
+  b->h_waves.clear();
   b->h_st_off.clear();
   b->h_st.clear();
   size_t list_need = 16;
@@ -251,9 +219,11 @@ static int batch_layout(cav_batch *b)
         for (int c = cy - 1; c <= cy + 1; ++c)
           for (int e = cz - 1; e <= cz + 1; ++e)
             if (a >= 0 && a < nbx && c >= 0 && c < nby && e >= 0 && e < nbz)
-              b->h_st.push_back(cells + a + nbx * c + nbx * nby * e);
-      b->h_cell_rep.push_back(r);
+              b->h_st.push_back(a + nbx * c + nbx * nby * e);
+      if (cx > 0 && cx < nbx - 1 && cy > 0 && cy < nby - 1 && cz > 0 && cz < nbz - 1)
+        b->h_waves.push_back(make_int2(k, r));
     }
+    for (int k = 0; k < nbins; k += 64) b->h_waves.push_back(make_int2(-1 - k, r));
     cells += nbins;
     const double vol = d.L[0] * d.L[1] * d.L[2];
     const double expect = 4.18879020478639 * b->rce2 * b->rce * (h.n / vol);
@@ -265,7 +235,6 @@ static int batch_layout(cav_batch *b)
   b->ntab = tabs;
   b->ncells = cells;
   b->maxn = maxn;
-  b->scan_blocks = grid_for(maxn);
   b->pair_blocks = grid_for((long)maxn * kLPA);
   for (int r = 0; r < b->B; ++r) b->reps[r].pbase = r * b->pair_blocks;
   if (b->cap < (int)list_need) b->cap = (int)((list_need + 3) / 4 * 4);
@@ -273,7 +242,9 @@ static int batch_layout(cav_batch *b)
 
   // device buffers
   CAV_TRY(balloc(b, &b->d_rep, b->B));
-  CAV_TRY(balloc(b, &b->cell_rep, b->ncells));
+  b->nwaves = (int)b->h_waves.size();
+  CAV_TRY(balloc(b, &b->waves, b->nwaves));
+  CAV_TRY(batch_cells_alloc(b));
   CAV_TRY(balloc(b, &b->st_off, b->h_st_off.size()));
   CAV_TRY(balloc(b, &b->st, b->h_st.size()));
   double **sd[] = {&b->x, &b->y, &b->z, &b->xo, &b->yo, &b->zo, &b->q};
@@ -282,37 +253,35 @@ static int batch_layout(cav_batch *b)
   CAV_TRY(balloc(b, &b->id, slots));
   CAV_TRY(balloc(b, &b->xq, slots));
   CAV_TRY(balloc(b, &b->tid, slots));
-  CAV_TRY(balloc(b, &b->bin_of, slots));
   CAV_TRY(balloc(b, &b->bin_items, slots));
   CAV_TRY(balloc(b, &b->cpos, slots));
-  double **od[] = {&b->vx, &b->vy, &b->vz, &b->ax, &b->ay, &b->az, &b->aox, &b->aoy, &b->aoz, &b->q_o};
+  double **od[] = {&b->vx, &b->vy, &b->vz, &b->ax, &b->ay, &b->az, &b->q_o};
   for (double **p : od) CAV_TRY(balloc(b, p, own));
   CAV_TRY(balloc(b, &b->type_o, own));
   CAV_TRY(balloc(b, &b->snap, 9 * (size_t)own));
-  CAV_TRY(balloc(b, &b->bin_cnt, 2 * (size_t)b->ncells));
+  b->aox = b->snap + 6 * (size_t)own;
+  b->aoy = b->snap + 7 * (size_t)own;
+  b->aoz = b->snap + 8 * (size_t)own;
   CAV_TRY(balloc(b, &b->bin_start, (size_t)b->ncells + b->B));
-  CAV_TRY(balloc(b, &b->gblk, (size_t)b->B * b->scan_blocks));
-  CAV_TRY(balloc(b, &b->nl, (size_t)own * b->cap));
   CAV_TRY(balloc(b, &b->nlb, (size_t)own * b->cap));
   CAV_TRY(balloc(b, &b->nn, own));
   CAV_TRY(balloc(b, &b->xqs, slots));
   CAV_TRY(balloc(b, &b->tids, slots));
   CAV_TRY(balloc(b, &b->litems, slots));
-  CAV_TRY(balloc(b, &b->binpos, slots));
   CAV_TRY(balloc(b, &b->order, own));
-  CAV_TRY(balloc(b, &b->ocnt, b->ncells));
-  CAV_TRY(balloc(b, &b->ostart, b->ncells));
   CAV_TRY(balloc(b, &b->flags, 16 * (size_t)b->B));
   CAV_TRY(balloc(b, &b->part, (size_t)b->B * b->pair_blocks));
   CAV_TRY(balloc(b, &b->vir, b->B));
   if (b->h_flags) (void)hipHostFree(b->h_flags);
+  b->h_flags = nullptr;
   BAT_HIP(hipHostMalloc((void **)&b->h_flags, sizeof(int) * 16 * b->B));
+  BAT_HIP(hipHostGetDevicePointer((void **)&b->hd_flags, b->h_flags, 0));
   BAT_HIP(hipMemset(b->flags, 0, sizeof(int) * 16 * b->B));
   BAT_HIP(hipMemset(b->xo, 0, sizeof(double) * slots));
   BAT_HIP(hipMemset(b->yo, 0, sizeof(double) * slots));
   BAT_HIP(hipMemset(b->zo, 0, sizeof(double) * slots));
   BAT_HIP(hipMemcpy(b->d_rep, b->reps.data(), sizeof(RepDev) * b->B, hipMemcpyHostToDevice));
-  BAT_HIP(hipMemcpy(b->cell_rep, b->h_cell_rep.data(), sizeof(int) * b->ncells, hipMemcpyHostToDevice));
+  BAT_HIP(hipMemcpy(b->waves, b->h_waves.data(), sizeof(int2) * b->nwaves, hipMemcpyHostToDevice));
   BAT_HIP(hipMemcpy(b->st_off, b->h_st_off.data(), sizeof(int) * b->h_st_off.size(), hipMemcpyHostToDevice));
   BAT_HIP(hipMemcpy(b->st, b->h_st.data(), sizeof(int) * b->h_st.size(), hipMemcpyHostToDevice));
 
@@ -399,17 +368,11 @@ static int batch_sync_flags(cav_batch *b)
 // One step of every replica (graph-capturable: no host decisions inside).
 static int batch_step_body(cav_batch *b, double dt)
 {
-  const dim3 own_grid(grid_for(b->maxn), b->B);
-  kb_snapshot<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->nown, 1, b->x, b->y, b->z, b->vx, b->vy,
-                                                   b->vz, b->ax, b->ay, b->az, b->snap);
-  kb_begin<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags);
-  kb_drift<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, dt, b->x, b->y, b->z, b->vx, b->vy, b->vz,
-                                                b->ax, b->ay, b->az, b->aox, b->aoy, b->aoz, b->flags);
-  CAV_TRY(batch_neighbor(b, false));
+  CAV_TRY(batch_neighbor(b, true, dt));
   CAV_TRY(batch_forces(b));
-  kb_kick<<<grid_for(b->nown), kBlock, 0, b->stream>>>(b->nown, 0.5 * dt, b->vx, b->vy, b->vz, b->ax,
-                                                        b->ay, b->az, b->aox, b->aoy, b->aoz);
-  BAT_HIP(hipMemcpyAsync(b->h_flags, b->flags, sizeof(int) * 16 * b->B, hipMemcpyDeviceToHost, b->stream));
+  kb_kick<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(
+      b->d_rep, 0.5 * dt, b->vx, b->vy, b->vz, b->ax, b->ay, b->az, b->aox, b->aoy, b->aoz,
+      b->pair_blocks, b->part, b->vir, b->flags, b->hd_flags);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -455,8 +418,8 @@ static int batch_grow(cav_batch *b, bool *relaid)
   if (!gover && !need) return CAV_OK;
   // back to the state before the step, on the host
   const dim3 own_grid(grid_for(b->maxn), b->B);
-  kb_snapshot<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->nown, 0, b->x, b->y, b->z, b->vx, b->vy,
-                                                   b->vz, b->ax, b->ay, b->az, b->snap);
+  kb_restore<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->nown, b->x, b->y, b->z, b->vx, b->vy,
+                                                  b->vz, b->ax, b->ay, b->az, b->snap);
   std::vector<double> hx(b->nslots), hy(b->nslots), hz(b->nslots), hv[3];
   BAT_HIP(hipMemcpyAsync(hx.data(), b->x, sizeof(double) * b->nslots, hipMemcpyDeviceToHost, b->stream));
   BAT_HIP(hipMemcpyAsync(hy.data(), b->y, sizeof(double) * b->nslots, hipMemcpyDeviceToHost, b->stream));
@@ -489,11 +452,12 @@ static int batch_setup_impl(cav_batch *b)
   for (int attempt = 0; attempt < 6; ++attempt) {
     CAV_TRY(batch_layout(b));
     kb_set_all<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags, F_NGHOST_OLD, -1);
-    kb_begin<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags);
-    kb_wrap<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(b->d_rep, b->x, b->y, b->z, b->flags);
-    CAV_TRY(batch_neighbor(b, true));
+    kb_begin<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags, 1);
+    CAV_TRY(batch_neighbor(b, false, 0));
     CAV_TRY(batch_forces(b));
+    kb_virial<<<b->B, kBlock, 0, b->stream>>>(b->pair_blocks, b->part, b->vir);
     CAV_TRY(batch_sync_flags(b));
+    kb_begin<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags, 0);
     bool grow = false;
     for (int r = 0; r < b->B; ++r) {
       const int *f = b->h_flags + 16 * r;
@@ -530,8 +494,8 @@ static int batch_run(cav_batch *b, double dt, int nsteps, bool graph)
       for (int r = 0; r < b->B; ++r) nan |= b->h_flags[16 * r + F_NAN] != 0;
       if (nan) {
         const dim3 own_grid(grid_for(b->maxn), b->B);
-        kb_snapshot<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->nown, 0, b->x, b->y, b->z, b->vx,
-                                                         b->vy, b->vz, b->ax, b->ay, b->az, b->snap);
+        kb_restore<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->nown, b->x, b->y, b->z, b->vx,
+                                                        b->vy, b->vz, b->ax, b->ay, b->az, b->snap);
         BAT_HIP(hipStreamSynchronize(b->stream));
         return bfail(b, CAV_ERR_NAN, "NaN acceleration before the drift");
       }
@@ -753,15 +717,18 @@ int cav_batch_get_pairs(cav_batch *b, int replica, int *ij, long capacity, long 
   if (!b || !npairs || replica < 0 || replica >= b->B) return CAV_ERR_ARG;
   if (!b->setup_done) return bfail(b, CAV_ERR_STATE, "cav_batch_setup must run first");
   const RepDev &d = b->reps[replica];
-  std::vector<int> nl((size_t)d.n * b->cap), nn(d.n);
-  BAT_HIP(hipMemcpyAsync(nl.data(), b->nl + (size_t)d.obase * b->cap, sizeof(int) * nl.size(),
+  // rows of bin-order slots, and the atom or ghost in each slot
+  std::vector<int> nl((size_t)d.n * b->cap), nn(d.n), items((size_t)d.n + d.gcap);
+  BAT_HIP(hipMemcpyAsync(nl.data(), b->nlb + (size_t)d.obase * b->cap, sizeof(int) * nl.size(),
+                         hipMemcpyDeviceToHost, b->stream));
+  BAT_HIP(hipMemcpyAsync(items.data(), b->litems + d.base, sizeof(int) * items.size(),
                          hipMemcpyDeviceToHost, b->stream));
   BAT_HIP(hipMemcpyAsync(nn.data(), b->nn + d.obase, sizeof(int) * d.n, hipMemcpyDeviceToHost, b->stream));
   BAT_HIP(hipStreamSynchronize(b->stream));
   long k = 0;
   for (int i = 0; i < d.n; ++i)
     for (int e = 0; e < nn[i]; ++e) {
-      const int j = nl[(size_t)i * b->cap + e];
+      const int j = items[nl[(size_t)i * b->cap + e]];
       if (j < d.n && j <= i) continue;
       if (ij && k < capacity) {
         ij[2 * k] = i;

@@ -335,12 +335,17 @@ struct cav_batch {
   std::vector<cav::RepDev> reps;
   int B = 0;
   long nslots = 0, nown = 0, ntab = 0;
-  int ncells = 0, maxn = 0, pair_blocks = 0, scan_blocks = 0;
-  std::vector<int> h_cell_rep, h_st_off, h_st;
+  int ncells = 0, maxcells = 0, maxn = 0, pair_blocks = 0, scan_blocks = 0;
+  std::vector<int> h_st_off, h_st;
+  std::vector<int2> h_waves;
 
   // device
   cav::RepDev *d_rep = nullptr;
-  int *cell_rep = nullptr, *st_off = nullptr, *st = nullptr;
+  int *st_off = nullptr, *st = nullptr;  // stencils, as cells of the replica
+  // the list build's waves: (cell, replica) of every inner cell, and (-1 -
+  // first cell, replica) of every 64 cells for owned atoms in the outer layer
+  int2 *waves = nullptr;
+  int nwaves = 0;
   double *x = nullptr, *y = nullptr, *z = nullptr;     // slots
   double *xo = nullptr, *yo = nullptr, *zo = nullptr;  // slots at the last list build
   int *type = nullptr;                                 // slots
@@ -350,24 +355,24 @@ struct cav_batch {
   int2 *tid = nullptr;
   double *vx = nullptr, *vy = nullptr, *vz = nullptr;  // owned
   double *ax = nullptr, *ay = nullptr, *az = nullptr;
-  double *aox = nullptr, *aoy = nullptr, *aoz = nullptr;
+  double *aox = nullptr, *aoy = nullptr, *aoz = nullptr;  // the snapshot's accelerations
   int *type_o = nullptr;                               // owned
   double *q_o = nullptr;
   double *snap = nullptr;  // [9][nown]: positions, velocities, accelerations
-  int *bin_of = nullptr, *bin_cnt = nullptr, *bin_start = nullptr, *bin_items = nullptr;
+  int *bin_start = nullptr, *bin_items = nullptr;
+  unsigned long long *cell_cnt = nullptr, *cell_first = nullptr;
+  int *bucket = nullptr, bucket_cap = 0;  // unsorted slots of every cell
   double4 *cpos = nullptr; // slots: (x, y, z, slot) in bin order
   int *gblk = nullptr;     // [B][scan_blocks] ghost-count block sums
-  int *nl = nullptr, *nn = nullptr;
-  // the pair kernel's bin-order gathers: rows as replica-local bin slots
-  // (beside nl), bin-ordered copies of (x, y, z, q) and (type, id), slot ->
-  // local atom, local atom -> slot, owned atoms in cell order, and per cell
-  // the owned count and its offset within the replica
+  int *nn = nullptr;
+  // Verlet rows as replica-local bin slots, bin-ordered copies of (x, y, z, q)
+  // and (type, id), slot -> local atom, owned atoms in cell order
   int *nlb = nullptr;
   double4 *xqs = nullptr;
   int2 *tids = nullptr;
-  int *litems = nullptr, *binpos = nullptr, *order = nullptr, *ocnt = nullptr, *ostart = nullptr;
+  int *litems = nullptr, *order = nullptr;
   int cap = 0;
-  int *flags = nullptr, *h_flags = nullptr;  // [B][F_COUNT]
+  int *flags = nullptr, *h_flags = nullptr, *hd_flags = nullptr;  // [B][16]; hd_flags: h_flags for the device
   double *d_minv = nullptr, *d_lj = nullptr;
   double *d_raw_eps = nullptr, *d_raw_sig = nullptr, *d_charge = nullptr;  // for the adjoint
   double *part = nullptr;  // [B][pair_blocks] virial partials
@@ -475,8 +480,10 @@ int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *
 int reduce_partials(cav_ctx *c, int count, int slot, bool add = false);
 int bfail(cav_batch *b, int code, const std::string &msg);
 int bhip_check(cav_batch *b, hipError_t e, const char *what);
-int batch_neighbor(cav_batch *b, bool forced);   // ghosts, rebuild test, cells, list
-int batch_pairs(cav_batch *b);                   // pack + LJ/Ewald_r + virial
+int batch_cells_alloc(cav_batch *b);
+// move or wrap, ghosts, rebuild test (drift), cells, packed copies, list
+int batch_neighbor(cav_batch *b, bool drift, double dt);
+int batch_pairs(cav_batch *b);  // LJ/Ewald_r, virial partials
 int batch_ewald_k_plan(cav_batch *b);
 int batch_ewald_k_alloc(cav_batch *b);
 int batch_ewald_k(cav_batch *b);

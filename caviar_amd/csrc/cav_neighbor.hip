@@ -490,6 +490,38 @@ __device__ __forceinline__ void block_sum2(int &a, int &b)
   }
 }
 
+// Batched replicas run the kernels of the exchange with grid row blockIdx.y =
+// replica: each shifts its arrays to the replica's slots (base), owned atoms
+// (obase) and cells (cbase) and takes the box, ghost and cell rules from it.
+__device__ __forceinline__ GhostRule ghost_rule_of(const RepDev &r, double gc)
+{
+  GhostRule g;
+  g.x = g.y = g.z = nullptr;
+  g.xl = r.lo[0] + gc;
+  g.xu = r.hi[0] - gc;
+  g.yl = r.lo[1] + gc;
+  g.yu = r.hi[1] - gc;
+  g.zl = r.lo[2] + gc;
+  g.zu = r.hi[2] - gc;
+  g.bx = g.by = g.bz = 1;
+  return g;
+}
+
+// A replica's cells: the grid with the ghost layer (r.nb counts it).
+__device__ __forceinline__ BinRule bin_rule_of(const RepDev &r, double cinv)
+{
+  BinRule b;
+  b.lox = r.lo[0];
+  b.loy = r.lo[1];
+  b.loz = r.lo[2];
+  b.cinv = cinv;
+  b.shift = 1;
+  b.nbx = r.nb[0];
+  b.nby = r.nb[1];
+  b.nbz = r.nb[2];
+  return b;
+}
+
 struct MoveArgs {
   int n;
   double dt;
@@ -503,6 +535,9 @@ struct MoveArgs {
   int *flags, *blk;
   u64t *cnt;  // cell counters to clear, or nullptr
   int nbins;
+  long stride;  // of the snapshot's planes
+  const RepDev *rep;  // REP: the replicas, and their ghost cutoff
+  double gc;
 };
 
 // DRIFT: integrate_velocity_verlet's drift (md_simulator.cpp:584-594), every
@@ -513,9 +548,33 @@ struct MoveArgs {
 // exchange_owned (domain.cpp:418-468) and the number of the block's images.
 // Once F_STOP is set (a step before this one failed) nothing moves and the
 // snapshot stays.  HBM bound: 216 B an atom.
-template <bool DRIFT, int BS>
+template <bool DRIFT, int BS, bool REP>
 __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
 {
+  if constexpr (REP) {
+    const RepDev &r = a.rep[blockIdx.y];
+    if ((int)blockIdx.x >= (r.n + BS - 1) / BS) return;
+    a.n = r.n;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      a.lo[d] = r.lo[d];
+      a.hi[d] = r.hi[d];
+      a.L[d] = r.L[d];
+      a.bc[d] = 1;
+    }
+    a.x += r.base, a.y += r.base, a.z += r.base;
+    if (a.xo) a.xo += r.base, a.yo += r.base, a.zo += r.base;
+    if constexpr (DRIFT) {
+      a.vx += r.obase, a.vy += r.obase, a.vz += r.obase;
+      a.ax += r.obase, a.ay += r.obase, a.az += r.obase;
+      a.snap += r.obase;
+    }
+    a.flags += 16 * blockIdx.y;
+    a.blk += (long)blockIdx.y * gridDim.x;
+    a.cnt += r.cbase;
+    a.nbins = r.nbins;
+    rule = ghost_rule_of(r, a.gc);
+  }
   const int i = blockIdx.x * BS + threadIdx.x;
   const int at = i < a.n ? i : 0;
   const int stop = a.flags[F_STOP];
@@ -528,7 +587,7 @@ __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
   if (a.xo) last[0] = a.xo[at], last[1] = a.yo[at], last[2] = a.zo[at];
   if (DRIFT && stop) return;
   if (a.cnt)
-    for (int k = i; k < a.nbins; k += gridDim.x * BS) a.cnt[k] = 0;
+    for (int k = i; k < a.nbins; k += (REP ? (a.n + BS - 1) / BS : (int)gridDim.x) * BS) a.cnt[k] = 0;
   int cnt = 0, moved = 0;
   if (i < a.n) {
     double *p[3] = {a.x + i, a.y + i, a.z + i};
@@ -537,15 +596,17 @@ __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
       if (isnan(acc[0]) || isnan(acc[1]) || isnan(acc[2])) a.flags[F_NAN] = 1;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        a.snap[(long)d * a.n + i] = r[d];
-        a.snap[(long)(3 + d) * a.n + i] = v[d];
-        a.snap[(long)(6 + d) * a.n + i] = acc[d];
+        a.snap[d * a.stride + i] = r[d];
+        a.snap[(3 + d) * a.stride + i] = v[d];
+        a.snap[(6 + d) * a.stride + i] = acc[d];
         const double h = xmul(xmul(xmul(0.5, acc[d]), a.dt), a.dt);
         r[d] = xadd(r[d], xadd(xmul(v[d], a.dt), h));
       }
-      a.aox[i] = acc[0];
-      a.aoy[i] = acc[1];
-      a.aoz[i] = acc[2];
+      if constexpr (!REP) {  // a batch reads the snapshot's planes
+        a.aox[i] = acc[0];
+        a.aoy[i] = acc[1];
+        a.aoz[i] = acc[2];
+      }
     }
     bool wrapped = false;
 #pragma unroll
@@ -595,6 +656,8 @@ struct GhostArgs {
   u64t *cnt;    // cells (owned count in the high word), or nullptr
   int *bucket;
   int cap;
+  const RepDev *rep;  // REP: the replicas, their ghost cutoff and cell width
+  double gc, cinv;
 };
 
 // The images of owned atom i at ghost slots n + g, g ascending with i, in the
@@ -606,16 +669,38 @@ struct GhostArgs {
 // packed for the gathers and put into its cell's bucket, whether the list is
 // rebuilt or not: the decision is not known yet, and the counting is cheaper
 // than a launch of its own.
-template <int BS>
+template <int BS, bool REP>
 __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinRule bins)
 {
+  int gcap = 0;
+  if constexpr (REP) {
+    const RepDev &r = a.rep[blockIdx.y];
+    a.n = r.n;
+    a.nblk = (r.n + BS - 1) / BS;
+    if ((int)blockIdx.x >= a.nblk) return;
+    gcap = r.gcap;
+    a.L[0] = r.L[0], a.L[1] = r.L[1], a.L[2] = r.L[2];
+    a.blk += (long)blockIdx.y * gridDim.x;
+    a.x += r.base, a.y += r.base, a.z += r.base;
+    a.type += r.base;
+    a.id += r.base;
+    a.q += r.base;
+    if (a.xo) a.xo += r.base, a.yo += r.base, a.zo += r.base;
+    a.flags += 16 * blockIdx.y;
+    a.xq += r.base;
+    a.tid += r.base;
+    a.cnt += r.cbase;
+    a.bucket += (long)r.cbase * a.cap;
+    rule = ghost_rule_of(r, a.gc);
+    bins = bin_rule_of(r, a.cinv);
+  }
   // every load that depends on nothing first: at small sizes the kernel is a
   // chain of such latencies
   const int i = blockIdx.x * BS + threadIdx.x;
   const bool live = i < a.n;
   const int at = live ? i : 0;
   const double px = a.x[at], py = a.y[at], pz = a.z[at], qq = a.q[at];
-  const int t = a.type[at], d = a.id[at], m = a.mol[at];
+  const int t = a.type[at], d = a.id[at], m = REP ? 0 : a.mol[at];
   const int stop = a.flags[F_STOP], old = a.flags[F_NGHOST_OLD];
   int before, total;
   if (a.scanned) {
@@ -637,6 +722,13 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
     cnt = GhostRule::images(sx, sy, sz);
   }
   const int off = before + block_exclusive_scan<BS>(cnt, nullptr);
+  // a batch gives each replica the ghost slots it expects: images past them
+  // are left out and the step is taken again with more
+  const bool over = REP && total > gcap;
+  if (over) {
+    total = gcap;
+    if (i == 0) a.flags[F_GOVER] = 1;
+  }
   bool test = false;
   if (a.xo) {
     const bool differs = a.rebuild_test || total != old;
@@ -651,18 +743,22 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
   // first, in variables of their own (an array's elements are copied together,
   // which waits for each), so that up to eight atomics are in flight at once:
   // one after the other they were most of this kernel's time at small sizes.
-  const int sides = (sx ? 1 : 0) | (sy ? 2 : 0) | (sz ? 4 : 0);
+  const bool mx = sx != 0, my = sy != 0, mz = sz != 0;
+  int img = (mx ? 1 : 0) | (my ? 2 : 0) | (mz ? 4 : 0) | (mx && my ? 8 : 0) | (mx && mz ? 16 : 0) |
+            (my && mz ? 32 : 0) | (mx && my && mz ? 64 : 0);
+  if (over)
+    while (img && off + __popc(img) > gcap) img &= ~(1 << (31 - __clz(img)));
   auto cell_of = [&](int ax) { return bins(ax & 1 ? gx : px, ax & 2 ? gy : py, ax & 4 ? gz : pz); };
   u64t r0, r1, r2, r3, r4, r5, r6, r7;
   if (a.cnt) {
     r0 = atomicAdd(a.cnt + cell_of(0), 1ull << 32 | 1ull);
-    if (sides & 1) r1 = atomicAdd(a.cnt + cell_of(1), 1ull);
-    if (sides & 2) r2 = atomicAdd(a.cnt + cell_of(2), 1ull);
-    if (sides & 4) r3 = atomicAdd(a.cnt + cell_of(4), 1ull);
-    if ((sides & 3) == 3) r4 = atomicAdd(a.cnt + cell_of(3), 1ull);
-    if ((sides & 5) == 5) r5 = atomicAdd(a.cnt + cell_of(5), 1ull);
-    if ((sides & 6) == 6) r6 = atomicAdd(a.cnt + cell_of(6), 1ull);
-    if (sides == 7) r7 = atomicAdd(a.cnt + cell_of(7), 1ull);
+    if (img & 1) r1 = atomicAdd(a.cnt + cell_of(1), 1ull);
+    if (img & 2) r2 = atomicAdd(a.cnt + cell_of(2), 1ull);
+    if (img & 4) r3 = atomicAdd(a.cnt + cell_of(4), 1ull);
+    if (img & 8) r4 = atomicAdd(a.cnt + cell_of(3), 1ull);
+    if (img & 16) r5 = atomicAdd(a.cnt + cell_of(5), 1ull);
+    if (img & 32) r6 = atomicAdd(a.cnt + cell_of(6), 1ull);
+    if (img & 64) r7 = atomicAdd(a.cnt + cell_of(7), 1ull);
   }
   int g = off;
   auto put = [&](int ax) {
@@ -679,9 +775,11 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
       a.z[s] = w;
       a.type[s] = t;
       a.id[s] = d;
-      a.mol[s] = m;
       a.q[s] = qq;
-      a.gsrc[g] = i;
+      if constexpr (!REP) {
+        a.mol[s] = m;
+        a.gsrc[g] = i;
+      }
       ++g;
     }
     if (a.xq) {
@@ -690,13 +788,13 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
     }
   };
   put(0);
-  if (sides & 1) put(1);
-  if (sides & 2) put(2);
-  if (sides & 4) put(4);
-  if ((sides & 3) == 3) put(3);
-  if ((sides & 5) == 5) put(5);
-  if ((sides & 6) == 6) put(6);
-  if (sides == 7) put(7);
+  if (img & 1) put(1);
+  if (img & 2) put(2);
+  if (img & 4) put(4);
+  if (img & 8) put(3);
+  if (img & 16) put(5);
+  if (img & 32) put(6);
+  if (img & 64) put(7);
   if (!a.cnt) return;
   auto keep = [&](long s, int ax, u64t r) {
     const int b = cell_of(ax), rank = (int)(unsigned)r;
@@ -704,13 +802,13 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
   };
   long s = (long)a.n + off;
   keep(i, 0, r0);
-  if (sides & 1) keep(s++, 1, r1);
-  if (sides & 2) keep(s++, 2, r2);
-  if (sides & 4) keep(s++, 4, r3);
-  if ((sides & 3) == 3) keep(s++, 3, r4);
-  if ((sides & 5) == 5) keep(s++, 5, r5);
-  if ((sides & 6) == 6) keep(s++, 6, r6);
-  if (sides == 7) keep(s++, 7, r7);
+  if (img & 1) keep(s++, 1, r1);
+  if (img & 2) keep(s++, 2, r2);
+  if (img & 4) keep(s++, 4, r3);
+  if (img & 8) keep(s++, 3, r4);
+  if (img & 16) keep(s++, 5, r5);
+  if (img & 32) keep(s++, 6, r6);
+  if (img & 64) keep(s++, 7, r7);
 }
 
 struct CellBuild {
@@ -724,6 +822,9 @@ struct CellBuild {
   int2 *tids;
   double *xo, *yo, *zo;
   int *flags;
+  const RepDev *rep;  // REP: the replicas, their cell width
+  double cinv;
+  const u64t *first;  // counters before each workgroup's cells, or nullptr: added up here
 };
 
 constexpr int kCellBlock = 1024;
@@ -736,8 +837,28 @@ constexpr int kCellBlock = 1024;
 // build's candidates and the packed copies; pos_old as well
 // (neighborlist.cpp:302-303).  Without a rebuild only the packed copies are
 // refreshed, in the order of the last one.
+template <bool REP>
 __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
 {
+  int blocks = gridDim.x;
+  if constexpr (REP) {
+    const RepDev &r = a.rep[blockIdx.y];
+    a.n = r.n;
+    a.nbins = r.nbins;
+    blocks = (r.nbins + a.bpb - 1) / a.bpb;
+    if ((int)blockIdx.x >= blocks) return;
+    if (a.first) a.first += (long)blockIdx.y * gridDim.x;
+    a.cnt += r.cbase;
+    a.bucket += (long)r.cbase * a.cap;
+    a.xq += r.base, a.tid += r.base;
+    a.start += r.cbase + blockIdx.y;  // one closing entry a replica
+    a.items += r.base, a.litems += r.base;
+    a.order += r.obase;
+    a.cpos += r.base, a.xqs += r.base, a.tids += r.base;
+    a.xo += r.base, a.yo += r.base, a.zo += r.base;
+    a.flags += 16 * blockIdx.y;
+    bins = bin_rule_of(r, a.cinv);
+  }
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.flags[F_NGHOST], stop = a.flags[F_STOP], rebuild = a.flags[F_REBUILD];
   const int b0 = blockIdx.x * a.bpb;
@@ -745,8 +866,12 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
   // wave's first cell (whatever the bucket holds past its count): asked for
   // together, before the flags are known
   u64t s = 0;
+  if (REP && a.first) {
+    if (threadIdx.x == 0) s = a.first[blockIdx.x];
+  } else {
 #pragma unroll 4
-  for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
+    for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
+  }
   const u64t own = lane < a.bpb && b0 + lane < a.nbins ? a.cnt[b0 + lane] : 0;
   const int early = lane < a.cap && wv < a.bpb && b0 + wv < a.nbins
                         ? a.bucket[(long)(b0 + wv) * a.cap + lane] : 0;
@@ -754,7 +879,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
   if (stop) return;
   if (!rebuild) {
     for (long t = (long)blockIdx.x * kCellBlock + threadIdx.x; t < tot;
-         t += (long)gridDim.x * kCellBlock) {
+         t += (long)blocks * kCellBlock) {
       const int j = a.litems[t];
       a.xqs[t] = a.xq[j];
       a.tids[t] = a.tid[j];
@@ -833,7 +958,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
       const int2 u = a.tid[j];
       a.items[t] = j;
       a.litems[t] = j;
-      a.binpos[j] = (int)t;
+      if constexpr (!REP) a.binpos[j] = (int)t;
       if (j < a.n) a.order[o0 + r] = j;  // owned atoms come first in a cell
       a.xqs[t] = v;
       a.tids[t] = u;
@@ -915,8 +1040,10 @@ int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
   a.cnt = fused_cells(c) ? c->cell_cnt : nullptr;
   a.nbins = c->xnbins;
   const int bs = move_block(c), nb = grid_for(c->n, bs);
-  const auto kern = bs == 64 ? (drift ? k_move<true, 64> : k_move<false, 64>)
-                             : (drift ? k_move<true, kBlock> : k_move<false, kBlock>);
+  a.stride = c->n;
+  a.rep = nullptr;
+  const auto kern = bs == 64 ? (drift ? k_move<true, 64, false> : k_move<false, 64, false>)
+                             : (drift ? k_move<true, kBlock, false> : k_move<false, kBlock, false>);
   kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -955,7 +1082,8 @@ int launch_ghosts(cav_ctx *c, bool decide)
   a.cap = c->bucket_cap;
   if (a.scanned)
     k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
-  const auto kern = bs == 64 ? k_ghosts<64> : k_ghosts<kBlock>;
+  a.rep = nullptr;
+  const auto kern = bs == 64 ? k_ghosts<64, false> : k_ghosts<kBlock, false>;
   kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
@@ -987,7 +1115,9 @@ int launch_cells(cav_ctx *c)
   a.yo = c->yo;
   a.zo = c->zo;
   a.flags = c->flags;
-  k_cells<<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
+  a.rep = nullptr;
+  a.first = nullptr;
+  k_cells<false><<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -1041,165 +1171,190 @@ static int list_grid(long cells) { return (int)((cells + kListWaves - 1) / kList
 // bin-order slots nlb) are template flags, so the append path of the inner
 // loop carries only the stores the launch needs.
 template <bool NL, bool NLL, bool NLB>
-__global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins, int cap, double rce2,
-                                                  const double4 *cpos, const int *st_off,
-                                                  const int *st, const int *start,
-                                                  const int *items, int *nl, int *nn, int *flags,
-                                                  const int *cond, const RepDev *rep,
-                                                  const int *cell_rep, unsigned short *nll,
-                                                  int *nlb, int split)
+__global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves, int nbx, int nby, int nbz,
+                                                  int cap, double rce2, const double4 *cpos,
+                                                  const int *st_off, const int *st,
+                                                  const int *start, const int *items, int *nl,
+                                                  int *nn, int *flags, const int *cond,
+                                                  const RepDev *rep, const int2 *waves,
+                                                  unsigned short *nll, int *nlb, int split)
 {
   // Each wave builds the rows of one cell on its own (wave-local LDS, no
   // block barrier).  The wave index is read as a scalar so that everything
   // derived from the cell stays in scalar registers.
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = (int)((long)blockIdx.x * kListWaves + wv);
-  if (b >= nbins) return;
-  // batched replicas: this cell's replica decides the owned range, the row base
-  // and the flags; entries are stored replica-local (owned i, ghost n+g)
-  int base = 0, obase = 0;
-  if (rep) {
-    const int r = cell_rep[b];
-    base = rep[r].base;
-    n = rep[r].n;
-    obase = rep[r].obase;
-    flags += 16 * r;
+  const int w = (int)((long)blockIdx.x * kListWaves + wv);
+  if (w >= nwaves) return;
+  const int lane = threadIdx.x & 63;
+  int b = w;
+  bool shell = false;
+  if (waves) {  // batched replicas: arrays shifted to the wave's
+    const int2 v = waves[w];
+    const RepDev &r = rep[v.y];
+    n = r.n;
+    flags += 16 * v.y;
     cond = flags + F_REBUILD;
-    start += r;  // every replica's cell starts carry one closing entry
+    shell = v.x < 0;
+    b = shell ? -1 - v.x : v.x;
+    nbx = r.nb[0], nby = r.nb[1], nbz = r.nb[2];
+    cpos += r.base;
+    items += r.base;
+    start += r.cbase + v.y;  // every replica's cell starts carry one closing entry
+    st_off += r.cbase;
+    nn += r.obase;
+    nlb += (long)r.obase * cap;
+  } else if (nbx) {
+    const int ix = nbx - 2, iy = nby - 2, ni = ix * iy * (nbz - 2);
+    shell = w >= ni;
+    const int y = w / ix;
+    b = shell ? 64 * (w - ni) : w - y * ix + 1 + nbx * (y % iy + 1 + nby * (y / iy + 1));
   }
   if (cond && !*cond) return;
   // with `split` waves per cell (blockIdx.y), this one takes every split-th
   // group of kAPI owned atoms
   const int part = blockIdx.y;
-  if (!rep && b == 0 && part == 0 && threadIdx.x == 0) flags[F_NL_STALE] = NL ? 0 : 1;
-  // staged candidates (x, y, z, index and slot) in the cell's stencil order; a stage is
-  // padded to a multiple of 64 with far-away entries so every lane tests one
-  __shared__ double4 sc_[kListWaves][kCand];
-  double4 *sc = sc_[wv];
-  const int lane = threadIdx.x & 63;
-  const int s0 = start[b], e0 = start[b + 1];
-  // owned atoms come first in a sorted bin
-  int no = 0;
-  for (int t = s0; t < e0; t += 64) {
-    const int v = (t + lane < e0) ? items[t + lane] - base : n;
-    no += __popcll(__ballot(v < n));
+  if (!waves && w == 0 && part == 0 && threadIdx.x == 0) flags[F_NL_STALE] = NL ? 0 : 1;
+  u64t todo = 1;
+  if (shell) {  // the cells among the next 64 that are of the layer and hold an owned atom
+    const int c = b + lane, cx = c % nbx, cy = c / nbx % nby, cz = c / (nbx * nby);
+    bool has = c < nbx * nby * nbz && (cx == 0 || cx == nbx - 1 || cy == 0 || cy == nby - 1 ||
+                                       cz == 0 || cz == nbz - 1);
+    if (has) {
+      const int first = start[c];
+      has = first < start[c + 1] && items[first] < n;  // owned atoms come first in a sorted bin
+    }
+    todo = __ballot(has);
   }
-  if (no <= kAPI * part) return;
-  const int sb = st_off[b], ns = st_off[b + 1] - sb;  // <= 27 stencil cells
-  // padding and empty owned slots sit at +-1e300: their squared distance to
-  // anything is +inf, so they never pass the cutoff test
-  const double4 far_cand = make_double4(1e300, 1e300, 1e300, cpos_tag(-1, -1));
-  // the stencil's cell ranges, loaded by lanes 0..ns-1 at once, and their
-  // running offsets in staging order (stencil cells in order, each in bin order)
-  __shared__ int s_base_[kListWaves][32], s_off_[kListWaves][33];
-  int *s_base = s_base_[wv], *s_off = s_off_[wv];
-  int total;
-  {
-    int cb = 0, cn = 0;
-    if (lane < ns) {
-      const int cell = st[sb + lane];
-      cb = start[cell];
-      cn = start[cell + 1] - cb;
+  for (int b0 = b; todo; todo &= todo - 1) {
+    b = b0 + __ffsll(todo) - 1;
+    // staged candidates (x, y, z, index and slot) in the cell's stencil order; a stage is
+    // padded to a multiple of 64 with far-away entries so every lane tests one
+    __shared__ double4 sc_[kListWaves][kCand];
+    double4 *sc = sc_[wv];
+    const int s0 = start[b], e0 = start[b + 1];
+    // owned atoms come first in a sorted bin
+    int no = 0;
+    for (int t = s0; t < e0; t += 64) {
+      const int v = (t + lane < e0) ? items[t + lane] : n;
+      no += __popcll(__ballot(v < n));
     }
-    int incl = cn;
-    for (int o = 1; o < 32; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    if (lane < ns) {
-      s_base[lane] = cb;
-      s_off[lane + 1] = incl;
-    }
-    if (lane == 0) s_off[0] = 0;
-    total = __shfl(incl, ns > 0 ? ns - 1 : 0, 64);
-    if (ns == 0) total = 0;
-    __syncwarp();
-  }
-  for (int og = 0; og < no; og += 64) {
-    const int gsize = (no - og) < 64 ? (no - og) : 64;
-    // lane t holds owned atom og+t (position, slot) and its row count; the
-    // kAPI atoms of a group are read from those lanes, never from memory
-    const double4 mine = lane < gsize ? cpos[s0 + og + lane]
-                                      : make_double4(-1e300, -1e300, -1e300, cpos_tag(-1, -1));
-    int cnt = 0;
-    for (int mbase = 0; mbase < total; mbase += kCand) {
-      // stage candidates mbase .. mbase+m-1 of the flattened stencil: each
-      // lane finds its cells by walking the offsets forward, all loads at once
-      const int m = (total - mbase) < kCand ? (total - mbase) : kCand;
-      int c = 0;
-      for (int t = lane; t < m; t += 64) {
-        const int g = mbase + t;
-        while (s_off[c + 1] <= g) ++c;
-        sc[t] = cpos[s_base[c] + g - s_off[c]];
+    if (no <= kAPI * part) continue;
+    const int sb = st_off[b], ns = st_off[b + 1] - sb;  // <= 27 stencil cells
+    // padding and empty owned slots sit at +-1e300: their squared distance to
+    // anything is +inf, so they never pass the cutoff test
+    const double4 far_cand = make_double4(1e300, 1e300, 1e300, cpos_tag(-1, -1));
+    // the stencil's cell ranges, loaded by lanes 0..ns-1 at once, and their
+    // running offsets in staging order (stencil cells in order, each in bin order)
+    __shared__ int s_base_[kListWaves][32], s_off_[kListWaves][33];
+    int *s_base = s_base_[wv], *s_off = s_off_[wv];
+    int total;
+    {
+      int cb = 0, cn = 0;
+      if (lane < ns) {
+        const int cell = st[sb + lane];
+        cb = start[cell];
+        cn = start[cell + 1] - cb;
       }
-      const int mpad = (m + 63) & ~63;
-      if (m + lane < mpad) sc[m + lane] = far_cand;
+      int incl = cn;
+      for (int o = 1; o < 32; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
+      }
+      if (lane < ns) {
+        s_base[lane] = cb;
+        s_off[lane + 1] = incl;
+      }
+      if (lane == 0) s_off[0] = 0;
+      total = __shfl(incl, ns > 0 ? ns - 1 : 0, 64);
+      if (ns == 0) total = 0;
       __syncwarp();
-      for (int o0 = kAPI * part; o0 < gsize; o0 += kAPI * split) {
-        // the kAPI owned atoms are the same for every lane: positions, slots,
-        // row offsets and row counters in scalar registers (empty slots of
-        // the group carry the far sentinel and never pass)
-        int ia[kAPI], c0[kAPI];
-        long row[kAPI];
-        double px[kAPI], py[kAPI], pz[kAPI];
-#pragma unroll
-        for (int u = 0; u < kAPI; ++u) {
-          const int src = o0 + u;  // < 64: o0 is a multiple of kAPI below 64
-          ia[u] = __builtin_amdgcn_readlane(cpos_index(mine.w), src);
-          px[u] = lane_d(mine.x, src);
-          py[u] = lane_d(mine.y, src);
-          pz[u] = lane_d(mine.z, src);
-          c0[u] = __builtin_amdgcn_readlane(cnt, src);
-          row[u] = (long)(obase + ia[u] - base) * cap;
+    }
+    for (int og = 0; og < no; og += 64) {
+      const int gsize = (no - og) < 64 ? (no - og) : 64;
+      // lane t holds owned atom og+t (position, slot) and its row count; the
+      // kAPI atoms of a group are read from those lanes, never from memory
+      const double4 mine = lane < gsize ? cpos[s0 + og + lane]
+                                        : make_double4(-1e300, -1e300, -1e300, cpos_tag(-1, -1));
+      int cnt = 0;
+      for (int mbase = 0; mbase < total; mbase += kCand) {
+        // stage candidates mbase .. mbase+m-1 of the flattened stencil: each
+        // lane finds its cells by walking the offsets forward, all loads at once
+        const int m = (total - mbase) < kCand ? (total - mbase) : kCand;
+        int c = 0;
+        for (int t = lane; t < m; t += 64) {
+          const int g = mbase + t;
+          while (s_off[c + 1] <= g) ++c;
+          sc[t] = cpos[s_base[c] + g - s_off[c]];
         }
-        for (int cc = 0; cc < mpad; cc += 64) {
-          const int idx = cc + lane;
-          const double4 q = sc[idx];
-          const int j = cpos_index(q.w);
+        const int mpad = (m + 63) & ~63;
+        if (m + lane < mpad) sc[m + lane] = far_cand;
+        __syncwarp();
+        for (int o0 = kAPI * part; o0 < gsize; o0 += kAPI * split) {
+          // the kAPI owned atoms are the same for every lane: positions, slots,
+          // row offsets and row counters in scalar registers (empty slots of
+          // the group carry the far sentinel and never pass)
+          int ia[kAPI], c0[kAPI];
+          long row[kAPI];
+          double px[kAPI], py[kAPI], pz[kAPI];
 #pragma unroll
           for (int u = 0; u < kAPI; ++u) {
-            const double dx = xsub(px[u], q.x), dy = xsub(py[u], q.y), dz = xsub(pz[u], q.z);
-            const bool pass = j != ia[u] && dot_rn(dx, dy, dz) < rce2;
-            // the ballot of the compare itself (a scalar mask), the lane's
-            // rank among the passing lanes by mbcnt, and a scalar row counter
-            const unsigned long long mask = __builtin_amdgcn_ballot_w64(pass);
-            if (mask) {
-              const int cu = c0[u];
-              const unsigned pre = __builtin_amdgcn_mbcnt_hi(
-                  (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-              if (pass && cu + (int)pre < cap) {
-                // uniform row pointers plus a 32-bit lane offset
-                const long at0 = row[u] + cu;
-                if constexpr (NL) {
-                  int *rp = nl + at0;
-                  rp[pre] = j - base;
+            const int src = o0 + u;  // < 64: o0 is a multiple of kAPI below 64
+            ia[u] = __builtin_amdgcn_readlane(cpos_index(mine.w), src);
+            px[u] = lane_d(mine.x, src);
+            py[u] = lane_d(mine.y, src);
+            pz[u] = lane_d(mine.z, src);
+            c0[u] = __builtin_amdgcn_readlane(cnt, src);
+            row[u] = (long)ia[u] * cap;
+          }
+          for (int cc = 0; cc < mpad; cc += 64) {
+            const int idx = cc + lane;
+            const double4 q = sc[idx];
+            const int j = cpos_index(q.w);
+#pragma unroll
+            for (int u = 0; u < kAPI; ++u) {
+              const double dx = xsub(px[u], q.x), dy = xsub(py[u], q.y), dz = xsub(pz[u], q.z);
+              const bool pass = j != ia[u] && dot_rn(dx, dy, dz) < rce2;
+              // the ballot of the compare itself (a scalar mask), the lane's
+              // rank among the passing lanes by mbcnt, and a scalar row counter
+              const unsigned long long mask = __builtin_amdgcn_ballot_w64(pass);
+              if (mask) {
+                const int cu = c0[u];
+                const unsigned pre = __builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+                if (pass && cu + (int)pre < cap) {
+                  // uniform row pointers plus a 32-bit lane offset
+                  const long at0 = row[u] + cu;
+                  if constexpr (NL) {
+                    int *rp = nl + at0;
+                    rp[pre] = j;
+                  }
+                  if constexpr (NLL) {
+                    unsigned short *lp = nll + at0;
+                    lp[pre] = (unsigned short)(mbase + idx);  // position in the stencil staging order
+                  }
+                  if constexpr (NLB) {
+                    int *bp = nlb + at0;
+                    bp[pre] = cpos_slot(q.w);  // bin-order slot of the candidate
+                  }
                 }
-                if constexpr (NLL) {
-                  unsigned short *lp = nll + at0;
-                  lp[pre] = (unsigned short)(mbase + idx);  // position in the stencil staging order
-                }
-                if constexpr (NLB) {
-                  int *bp = nlb + at0;
-                  bp[pre] = cpos_slot(q.w) - base;  // bin-order slot of the candidate
-                }
+                c0[u] = cu + (int)__popcll(mask);
               }
-              c0[u] = cu + (int)__popcll(mask);
             }
           }
-        }
 #pragma unroll
-        for (int u = 0; u < kAPI; ++u) cnt = lane == o0 + u ? c0[u] : cnt;
+          for (int u = 0; u < kAPI; ++u) cnt = lane == o0 + u ? c0[u] : cnt;
+        }
+        __syncwarp();
       }
-      __syncwarp();
-    }
-    if (lane < gsize && lane / kAPI % split == part) {
-      const int i = cpos_index(mine.w) - base + obase;
-      nn[i] = cnt < cap ? cnt : cap;
-      // the longest row is needed only to regrow the list after an overflow:
-      // one device-wide atomic per overflowing row, none otherwise
-      if (cnt > cap) {
-        flags[F_OVERFLOW] = 1;
-        atomicMax(flags + F_MAXNB, cnt);
+      if (lane < gsize && lane / kAPI % split == part) {
+        const int i = cpos_index(mine.w);
+        nn[i] = cnt < cap ? cnt : cap;
+        // the longest row is needed only to regrow the list after an overflow:
+        // one device-wide atomic per overflowing row, none otherwise
+        if (cnt > cap) {
+          flags[F_OVERFLOW] = 1;
+          atomicMax(flags + F_MAXNB, cnt);
+        }
       }
     }
   }
@@ -1208,10 +1363,10 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nbins,
 // k_list_wave for the outputs that are not null (index rows, staging
 // positions, bin-order slots: the combinations the single system and the
 // batched replicas use)
-static void launch_list_wave(hipStream_t st, int n, int nbins, int cap, double rce2,
+static void launch_list_wave(hipStream_t st, int n, int nbins, const int *xnb, int cap, double rce2,
                              const double4 *cpos, const int *st_off, const int *stc,
                              const int *start, const int *items, int *nl, int *nn, int *flags,
-                             const int *cond, const RepDev *rep, const int *cell_rep,
+                             const int *cond, const RepDev *rep, const int2 *waves, int nwaves,
                              unsigned short *nll, int *nlb)
 {
   // Waves per cell: small grids leave CUs idle, and a wave's chain over its
@@ -1220,10 +1375,22 @@ static void launch_list_wave(hipStream_t st, int n, int nbins, int cap, double r
   // (us): 125 cells 24 / 16 / 13 / 11, 1000 cells 34 / 23 / 20 / 17, 2744 cells
   // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
   const int split = std::max(1, std::min(6, 8192 / nbins));
-  const dim3 g(list_grid(nbins), split), blk(64 * kListWaves);
-#define CAV_LISTW(A, B, C)                                                                      \
-  k_list_wave<A, B, C><<<g, blk, 0, st>>>(n, nbins, cap, rce2, cpos, st_off, stc, start, items, \
-                                          nl, nn, flags, cond, rep, cell_rep, nll, nlb, split)
+  // One wave per cell, or on a grid with a ghost layer (xnb: its cells per
+  // axis) one per inner cell and one per 64 of all cells for what owned atoms
+  // the layer holds (positions on the upper face)
+  int bx = 0, by = 0, bz = 0;
+  if (!waves) {
+    nwaves = nbins;
+    if (xnb) {
+      bx = xnb[0] + 2, by = xnb[1] + 2, bz = xnb[2] + 2;
+      nwaves = xnb[0] * xnb[1] * xnb[2] + (nbins + 63) / 64;
+    }
+  }
+  const dim3 g(list_grid(nwaves), split), blk(64 * kListWaves);
+#define CAV_LISTW(A, B, C)                                                                       \
+  k_list_wave<A, B, C><<<g, blk, 0, st>>>(n, nwaves, bx, by, bz, cap, rce2, cpos, st_off, stc,   \
+                                          start, items, nl, nn, flags, cond, rep, waves, nll,    \
+                                          nlb, split)
   if (nlb && !nl)
     CAV_LISTW(false, false, true);
   else if (nlb)
@@ -1294,10 +1461,11 @@ int launch_list(cav_ctx *c, bool conditional)
     k_list_all<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->nl_cap, c->nl, c->nn, c->flags,
                                                         cond);
   else
-    launch_list_wave(c->stream, c->n, xg ? c->xnbins : c->nbins, c->nl_cap, c->rce2, c->cpos,
+    launch_list_wave(c->stream, c->n, xg ? c->xnbins : c->nbins, xg ? c->nb : nullptr, c->nl_cap,
+                     c->rce2, c->cpos,
                      xg ? c->d_xst_off : c->d_st_off, xg ? c->d_xst : c->d_st, c->bin_start,
                      c->bin_items, with_nlb ? nullptr : c->nl, c->nn, c->flags, cond, nullptr,
-                     nullptr, with_nll ? c->nll : nullptr, with_nlb ? c->nlb : nullptr);
+                     nullptr, 0, with_nll ? c->nll : nullptr, with_nlb ? c->nlb : nullptr);
   // (the bin order itself, litems and binpos, was kept by the list build's
   // binning; the cell-staged kernel also needs the cell starts)
   if (with_nll) {
@@ -1362,329 +1530,174 @@ int launch_save_old(cav_ctx *c, bool conditional)
   return CAV_OK;
 }
 
-
 // ---------------------------------------------------------- batched replicas --
 //
-// The same steps for every replica of a cav_batch at once: grid row
-// blockIdx.y is the replica for per-atom work; per-cell work maps a global
-// cell to its replica.  Each replica's decisions (ghost count, rebuild) live
-// in its own 16 flag words.
+// The same exchange for every replica of a cav_batch at once, in the same
+// kernels: grid row blockIdx.y is the replica, whose decisions (ghost count,
+// rebuild) live in its own 16 flag words.  Before, thirteen kernels of its own
+// took a step: 256 replicas (540000 atoms, 1.5 million with their images)
+// 455 us beside the list, now 360; with the index rows no longer written the
+// list build went from 506 to 444 us.
 
-__device__ __forceinline__ GhostRule ghost_rule_of(const RepDev &r, double gc, const double *x,
-                                                   const double *y, const double *z)
+// Counters before every bpb-th cell of a replica, for grids on which each
+// workgroup of k_cells adding them up itself would read too much.
+__global__ __launch_bounds__(kCellBlock) void kb_cell_first(const RepDev *rep, int bpb, int blocks,
+                                                            const u64t *cnt, u64t *first)
 {
-  GhostRule g;
-  g.x = x + r.base;
-  g.y = y + r.base;
-  g.z = z + r.base;
-  g.xl = r.lo[0] + gc;
-  g.xu = r.hi[0] - gc;
-  g.yl = r.lo[1] + gc;
-  g.yu = r.hi[1] - gc;
-  g.zl = r.lo[2] + gc;
-  g.zu = r.hi[2] - gc;
-  g.bx = g.by = g.bz = 1;
-  return g;
-}
-
-__global__ void kb_ghost_sums(const RepDev *rep, double gc, const double *x, const double *y,
-                              const double *z, int nblk, int *gblk)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const GhostRule g = ghost_rule_of(r, gc, x, y, z);
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  int tot;
-  block_exclusive_scan(i < r.n ? g(i) : 0, &tot);
-  if (threadIdx.x == 0) gblk[(long)blockIdx.y * nblk + blockIdx.x] = tot;
-}
-
-__global__ void kb_ghost_scan(const RepDev *rep, int nblk, int *gblk, int *flags)
-{
-  const int rr = blockIdx.x;
-  int *blk = gblk + (long)rr * nblk;
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nblk; base += kBlock) {
-    const int i = base + threadIdx.x;
-    const int v = i < nblk ? blk[i] : 0;
-    int tot;
-    const int ex = block_exclusive_scan(v, &tot);
-    if (i < nblk) blk[i] = ex + carry;
-    __syncthreads();
-    if (threadIdx.x == 0) carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    int *f = flags + 16 * rr;
-    f[F_NGHOST] = carry < rep[rr].gcap ? carry : rep[rr].gcap;
-    if (carry > rep[rr].gcap) f[F_GOVER] = 1;
-  }
-}
-
-__global__ void kb_ghost_scatter(const RepDev *rep, double gc, int nblk, const int *gblk, double *x,
-                                 double *y, double *z, int *type, int *id, double *q)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const GhostRule rule = ghost_rule_of(r, gc, x, y, z);
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  const int cnt = i < r.n ? rule(i) : 0;
-  const int off = block_exclusive_scan(cnt, nullptr) + gblk[(long)blockIdx.y * nblk + blockIdx.x];
-  if (i >= r.n || cnt == 0) return;
-  int sx, sy, sz;
-  rule.sides(i, sx, sy, sz);
-  const long own = r.base + i;
-  const double px = x[own], py = y[own], pz = z[own];
-  const double gx = px - sx * r.L[0], gy = py - sy * r.L[1], gz = pz - sz * r.L[2];
-  const int t = type[own];
-  const double qq = q[own];
-  int g = off;
-  auto put = [&](double a, double b, double c) {
-    if (g < r.gcap) {
-      const long s = (long)r.base + r.n + g;
-      x[s] = a;
-      y[s] = b;
-      z[s] = c;
-      type[s] = t;
-      id[s] = (int)i;
-      q[s] = qq;
+  const RepDev &r = rep[blockIdx.x];
+  cnt += r.cbase;
+  first += (long)blockIdx.x * blocks;
+  const int nb = (r.nbins + bpb - 1) / bpb, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __shared__ u64t part[kCellBlock / 64];
+  u64t carry = 0;
+  for (int k0 = 0; k0 < nb; k0 += kCellBlock) {
+    const int k = k0 + threadIdx.x;
+    u64t v = 0;
+    if (k < nb)
+      for (int c = k * bpb; c < min(r.nbins, (k + 1) * bpb); ++c) v += cnt[c];
+    u64t inc = v;
+    for (int o = 1; o < 64; o <<= 1) {
+      const u64t u = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += u;
     }
-    ++g;
-  };
-  if (sx) put(gx, py, pz);
-  if (sy) put(px, gy, pz);
-  if (sz) put(px, py, gz);
-  if (sx && sy) put(gx, gy, pz);
-  if (sx && sz) put(gx, py, gz);
-  if (sy && sz) put(px, gy, gz);
-  if (sx && sy && sz) put(gx, gy, gz);
-}
-
-__global__ void kb_rebuild_check(const RepDev *rep, const double *x, const double *y,
-                                 const double *z, const double *xo, const double *yo,
-                                 const double *zo, double thr_sq, int *flags)
-{
-  const RepDev &r = rep[blockIdx.y];
-  int *f = flags + 16 * blockIdx.y;
-  if (f[F_REBUILD]) return;
-  const int G = f[F_NGHOST], Gold = f[F_NGHOST_OLD];
-  if (G != Gold) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) f[F_REBUILD] = 1;
-    return;
-  }
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a >= (long)r.n + G) return;
-  const long s = r.base + a;
-  const double dx = xsub(x[s], xo[s]), dy = xsub(y[s], yo[s]), dz = xsub(z[s], zo[s]);
-  if (dot_rn(dx, dy, dz) > thr_sq) f[F_REBUILD] = 1;
-}
-
-__global__ void kb_set_rebuild(int B, int *flags)
-{
-  const int r = blockIdx.x * kBlock + threadIdx.x;
-  if (r < B) flags[16 * r + F_REBUILD] = 1;
-}
-
-// A replica's cells: the grid with the ghost layer (r.nb counts it).
-__device__ __forceinline__ BinRule bin_rule_of(const RepDev &r, double cinv)
-{
-  BinRule b;
-  b.lox = r.lo[0];
-  b.loy = r.lo[1];
-  b.loz = r.lo[2];
-  b.cinv = cinv;
-  b.shift = 1;
-  b.nbx = r.nb[0];
-  b.nby = r.nb[1];
-  b.nbz = r.nb[2];
-  return b;
-}
-
-// cell counts of the rebuilding replicas (zeroed first by kb_zero_cells)
-__global__ void kb_zero_cells(const RepDev *rep, const int *flags, int *cnt, int *cur)
-{
-  const RepDev &r = rep[blockIdx.y];
-  if (!flags[16 * blockIdx.y + F_REBUILD]) return;
-  const int k = blockIdx.x * kBlock + threadIdx.x;
-  if (k < r.nbins) cnt[r.cbase + k] = cur[r.cbase + k] = 0;
-}
-
-__global__ void kb_bin_count(const RepDev *rep, double cinv, const double *x, const double *y,
-                             const double *z, const int *flags, int *bin_of, int *cnt)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const int *f = flags + 16 * blockIdx.y;
-  if (!f[F_REBUILD]) return;
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a >= (long)r.n + f[F_NGHOST]) return;
-  const long s = r.base + a;
-  const int c = r.cbase + bin_rule_of(r, cinv)(x[s], y[s], z[s]);
-  bin_of[s] = c;
-  atomicAdd(cnt + c, 1);
-}
-
-// per replica: cell starts (absolute into the item array, replica r's starts
-// at index cbase + r .. cbase + r + nbins)
-__global__ void kb_bin_start(const RepDev *rep, const int *flags, const int *cnt, int *start)
-{
-  const int rr = blockIdx.x;
-  const RepDev &r = rep[rr];
-  if (!flags[16 * rr + F_REBUILD]) return;
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = r.base;
-  __syncthreads();
-  int *st = start + r.cbase + rr;
-  for (int k0 = 0; k0 < r.nbins; k0 += kBlock) {
-    const int k = k0 + threadIdx.x;
-    const int v = k < r.nbins ? cnt[r.cbase + k] : 0;
-    int tot;
-    const int ex = block_exclusive_scan(v, &tot);
-    if (k < r.nbins) st[k] = carry + ex;
+    if (lane == 63) part[wv] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) st[r.nbins] = carry;
-}
-
-__global__ void kb_bin_fill(const RepDev *rep, const int *flags, const int *bin_of,
-                            const int *cell_rep, const int *start, int *cur, int *items)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const int *f = flags + 16 * blockIdx.y;
-  if (!f[F_REBUILD]) return;
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a >= (long)r.n + f[F_NGHOST]) return;
-  const long s = r.base + a;
-  const int c = bin_of[s];
-  items[start[c + blockIdx.y] + atomicAdd(cur + c, 1)] = (int)s;
-}
-
-// After the sort a cell lists its owned atoms first (they have the lower
-// slots); their count goes to ocnt, taken before the sort (it is order-free).
-__global__ __launch_bounds__(64 * kSortWaves) void kb_bin_sort(const RepDev *rep, int ncells,
-                                                               const int *cell_rep,
-                                                               const int *flags, const int *start,
-                                                               int *items, int *ocnt)
-{
-  __shared__ int v_[kSortWaves][kSortWaveMax];
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c = blockIdx.x * kSortWaves + wv;
-  if (c >= ncells) return;
-  const int rr = cell_rep[c];
-  if (!flags[16 * rr + F_REBUILD]) return;
-  const int s0 = start[c + rr], e0 = start[c + rr + 1];
-  const int lane = threadIdx.x & 63, own_end = rep[rr].base + rep[rr].n;
-  int no = 0;
-  for (int t = s0; t < e0; t += 64) no += __popcll(__ballot(t + lane < e0 && items[t + lane] < own_end));
-  if (lane == 0) ocnt[c] = no;
-  sort_bin_wave(s0, e0, items, v_[wv]);
-}
-
-// per replica: each cell's first owned atom in cell order (exclusive scan of
-// the owned counts over the replica's cells)
-__global__ void kb_owned_start(const RepDev *rep, const int *flags, const int *ocnt, int *ostart)
-{
-  const int rr = blockIdx.x;
-  const RepDev &r = rep[rr];
-  if (!flags[16 * rr + F_REBUILD]) return;
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int k0 = 0; k0 < r.nbins; k0 += kBlock) {
-    const int k = k0 + threadIdx.x;
-    const int v = k < r.nbins ? ocnt[r.cbase + k] : 0;
-    int tot;
-    const int ex = block_exclusive_scan(v, &tot);
-    if (k < r.nbins) ostart[r.cbase + k] = carry + ex;
-    __syncthreads();
-    if (threadIdx.x == 0) carry += tot;
+    u64t before = carry;
+    for (int q = 0; q < kCellBlock / 64; ++q) {
+      if (q < wv) before += part[q];
+      carry += part[q];
+    }
+    if (k < nb) first[k] = before + inc - v;
     __syncthreads();
   }
 }
 
-// (x, y, z, index and slot) in bin order for the list build, and the bin
-// order the pair kernel reads through: slot -> local atom (litems), local atom
-// -> slot (binpos), owned atoms in cell order (order)
-__global__ void kb_cell_pack(const RepDev *rep, const int *flags, const int *items,
-                             const int *bin_of, const int *start, const int *ostart,
-                             const double *x, const double *y, const double *z, double4 *cpos,
-                             int *litems, int *binpos, int *order)
-{
-  const int rr = blockIdx.y;
-  const RepDev &r = rep[rr];
-  const int *f = flags + 16 * rr;
-  if (!f[F_REBUILD]) return;
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a >= (long)r.n + f[F_NGHOST]) return;
-  const long t = r.base + a;
-  const int j = items[t];
-  cpos[t] = make_double4(x[j], y[j], z[j], cpos_tag(j, t));
-  const int lj = j - r.base;
-  litems[t] = lj;
-  binpos[j] = (int)a;
-  if (lj < r.n) {
-    // owned atoms come first in their sorted cell
-    const int c = bin_of[j];
-    order[r.obase + ostart[c] + (int)(t - start[c + rr])] = lj;
-  }
-}
+// Threads per workgroup, as move_block
+static int batch_block(const cav_batch *b) { return b->nown <= 16384 ? 64 : kBlock; }
 
-__global__ void kb_save_old(const RepDev *rep, const double *x, const double *y, const double *z,
-                            double *xo, double *yo, double *zo, int *flags)
-{
-  const RepDev &r = rep[blockIdx.y];
-  int *f = flags + 16 * blockIdx.y;
-  if (!f[F_REBUILD]) return;
-  const int G = f[F_NGHOST];
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a == 0) f[F_NGHOST_OLD] = G;
-  if (a >= (long)r.n + G) return;
-  const long s = r.base + a;
-  xo[s] = x[s];
-  yo[s] = y[s];
-  zo[s] = z[s];
-}
+// Cells per workgroup of k_cells, and its workgroups per replica
+static int cells_per_block(const cav_batch *b) { return b->maxcells <= 4096 ? 16 : 64; }
 
-// Ghosts, rebuild decision, cells and Verlet rows of every replica.
-int batch_neighbor(cav_batch *b, bool forced)
+int batch_cells_alloc(cav_batch *b)
 {
-  const dim3 own_grid(b->scan_blocks, b->B);
-  kb_ghost_sums<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->ghost_cutoff, b->x, b->y, b->z,
-                                                     b->scan_blocks, b->gblk);
-  kb_ghost_scan<<<b->B, kBlock, 0, b->stream>>>(b->d_rep, b->scan_blocks, b->gblk, b->flags);
-  kb_ghost_scatter<<<own_grid, kBlock, 0, b->stream>>>(b->d_rep, b->ghost_cutoff, b->scan_blocks,
-                                                        b->gblk, b->x, b->y, b->z, b->type, b->id,
-                                                        b->q);
-  if (!b->nl_on) return CAV_OK;
-  int maxslots = 0, maxcells = 0;
+  b->maxcells = 0;
+  double density = 0;
   for (const RepDev &r : b->reps) {
-    maxslots = std::max(maxslots, r.n + r.gcap);
-    maxcells = std::max(maxcells, r.nbins);
+    b->maxcells = std::max(b->maxcells, r.nbins);
+    density = std::max(density, r.n / (r.L[0] * r.L[1] * r.L[2]));
   }
-  const dim3 slot_grid(grid_for(maxslots), b->B), cell_grid(grid_for(maxcells), b->B);
-  if (forced)
-    kb_set_rebuild<<<grid_for(b->B), kBlock, 0, b->stream>>>(b->B, b->flags);
-  else
-    kb_rebuild_check<<<slot_grid, kBlock, 0, b->stream>>>(b->d_rep, b->x, b->y, b->z, b->xo, b->yo,
-                                                           b->zo, b->thr_sq, b->flags);
-  kb_zero_cells<<<cell_grid, kBlock, 0, b->stream>>>(b->d_rep, b->flags, b->bin_cnt, b->bin_cnt + b->ncells);
-  kb_bin_count<<<slot_grid, kBlock, 0, b->stream>>>(b->d_rep, b->cinv, b->x, b->y, b->z, b->flags,
-                                                     b->bin_of, b->bin_cnt);
-  kb_bin_start<<<b->B, kBlock, 0, b->stream>>>(b->d_rep, b->flags, b->bin_cnt, b->bin_start);
-  kb_bin_fill<<<slot_grid, kBlock, 0, b->stream>>>(b->d_rep, b->flags, b->bin_of, b->cell_rep,
-                                                    b->bin_start, b->bin_cnt + b->ncells, b->bin_items);
-  kb_bin_sort<<<(b->ncells + kSortWaves - 1) / kSortWaves, 64 * kSortWaves, 0, b->stream>>>(
-      b->d_rep, b->ncells, b->cell_rep, b->flags, b->bin_start, b->bin_items, b->ocnt);
-  kb_owned_start<<<b->B, kBlock, 0, b->stream>>>(b->d_rep, b->flags, b->ocnt, b->ostart);
-  kb_cell_pack<<<slot_grid, kBlock, 0, b->stream>>>(b->d_rep, b->flags, b->bin_items, b->bin_of,
-                                                     b->bin_start, b->ostart, b->x, b->y, b->z,
-                                                     b->cpos, b->litems, b->binpos, b->order);
-  launch_list_wave(b->stream, 0, b->ncells, b->cap, b->rce2, b->cpos, b->st_off, b->st,
-                   b->bin_start, b->bin_items, b->nl, b->nn, b->flags, nullptr, b->d_rep,
-                   b->cell_rep, nullptr, b->nlb);
-  kb_save_old<<<slot_grid, kBlock, 0, b->stream>>>(b->d_rep, b->x, b->y, b->z, b->xo, b->yo, b->zo,
-                                                    b->flags);
+  b->scan_blocks = grid_for(b->maxn, batch_block(b));
+  // twice the densest replica's mean cell and some, as the single system
+  const double want = 2.0 * b->rce * b->rce * b->rce * density + 32;
+  b->bucket_cap = (int)(std::min(1024.0, want + 31) / 32) * 32;
+  const int blocks = (b->maxcells + cells_per_block(b) - 1) / cells_per_block(b);
+  void **bufs[] = {(void **)&b->cell_cnt, (void **)&b->bucket, (void **)&b->cell_first,
+                   (void **)&b->gblk};
+  const size_t bytes[] = {sizeof(u64t) * b->ncells, sizeof(int) * (size_t)b->bucket_cap * b->ncells,
+                          b->maxcells > 65536 ? sizeof(u64t) * (size_t)blocks * b->B : 0,
+                          sizeof(int) * (size_t)b->B * b->scan_blocks};
+  for (int k = 0; k < 4; ++k) {
+    if (*bufs[k]) (void)hipFree(*bufs[k]);
+    *bufs[k] = nullptr;
+    if (bytes[k]) BAT_HIP(hipMalloc(bufs[k], bytes[k]));
+  }
+  return CAV_OK;
+}
+
+// Owned atoms of every replica drifted (or only wrapped), images, the rebuild
+// decision (`drift` false: every list is rebuilt, F_REBUILD is already set),
+// cells, packed copies and Verlet rows.
+int batch_neighbor(cav_batch *b, bool drift, double dt)
+{
+  const int bs = batch_block(b);
+  const dim3 own_grid(b->scan_blocks, b->B);
+  MoveArgs m;
+  m.n = 0;
+  m.dt = dt;
+  m.x = b->x;
+  m.y = b->y;
+  m.z = b->z;
+  m.vx = b->vx;
+  m.vy = b->vy;
+  m.vz = b->vz;
+  m.ax = b->ax;
+  m.ay = b->ay;
+  m.az = b->az;
+  m.aox = m.aoy = m.aoz = nullptr;
+  m.snap = b->snap;
+  m.xo = drift ? b->xo : nullptr;
+  m.yo = b->yo;
+  m.zo = b->zo;
+  m.thr_sq = b->thr_sq;
+  m.flags = b->flags;
+  m.blk = b->gblk;
+  m.cnt = b->cell_cnt;
+  m.nbins = 0;
+  m.stride = b->nown;
+  m.rep = b->d_rep;
+  m.gc = b->ghost_cutoff;
+  const auto move = bs == 64 ? (drift ? k_move<true, 64, true> : k_move<false, 64, true>)
+                             : (drift ? k_move<true, kBlock, true> : k_move<false, kBlock, true>);
+  move<<<own_grid, bs, 0, b->stream>>>(m, GhostRule{});
+  BAT_HIP(hipGetLastError());
+  GhostArgs g;
+  g.n = g.nblk = 0;
+  g.scanned = 0;
+  g.blk = b->gblk;
+  g.x = b->x;
+  g.y = b->y;
+  g.z = b->z;
+  g.type = b->type;
+  g.id = b->id;
+  g.mol = g.gsrc = nullptr;
+  g.q = b->q;
+  g.xo = drift ? b->xo : nullptr;
+  g.yo = b->yo;
+  g.zo = b->zo;
+  g.thr_sq = b->thr_sq;
+  g.rebuild_test = 0;
+  g.flags = b->flags;
+  g.xq = b->xq;
+  g.tid = b->tid;
+  g.cnt = b->cell_cnt;
+  g.bucket = b->bucket;
+  g.cap = b->bucket_cap;
+  g.rep = b->d_rep;
+  g.gc = b->ghost_cutoff;
+  g.cinv = b->cinv;
+  const auto ghosts = bs == 64 ? k_ghosts<64, true> : k_ghosts<kBlock, true>;
+  ghosts<<<own_grid, bs, 0, b->stream>>>(g, GhostRule{}, BinRule{});
+  CellBuild a;
+  a.n = a.nbins = 0;
+  a.bpb = cells_per_block(b);
+  a.cap = b->bucket_cap;
+  a.cnt = b->cell_cnt;
+  a.bucket = b->bucket;
+  a.xq = b->xq;
+  a.tid = b->tid;
+  a.start = b->bin_start;
+  a.items = b->bin_items;
+  a.order = b->order;
+  a.binpos = nullptr;
+  a.litems = b->litems;
+  a.cpos = b->cpos;
+  a.xqs = b->xqs;
+  a.tids = b->tids;
+  a.xo = b->xo;
+  a.yo = b->yo;
+  a.zo = b->zo;
+  a.flags = b->flags;
+  a.rep = b->d_rep;
+  a.cinv = b->cinv;
+  a.first = b->cell_first;
+  const int blocks = (b->maxcells + a.bpb - 1) / a.bpb;
+  if (a.first)
+    kb_cell_first<<<b->B, kCellBlock, 0, b->stream>>>(b->d_rep, a.bpb, blocks, b->cell_cnt,
+                                                      b->cell_first);
+  k_cells<true><<<dim3(blocks, b->B), kCellBlock, 0, b->stream>>>(a, BinRule{});
+  launch_list_wave(b->stream, 0, b->ncells, nullptr, b->cap, b->rce2, b->cpos, b->st_off, b->st,
+                   b->bin_start, b->litems, nullptr, b->nn, b->flags, nullptr, b->d_rep, b->waves,
+                   b->nwaves, nullptr, b->nlb);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }

@@ -190,7 +190,6 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
     a.n = r.n;
     a.xq += base;
     a.tid += base;
-    a.nl += (long)obase * a.cap;
     a.nn += obase;
     if (a.order) a.order += obase;
     if constexpr (BINS) {
@@ -1295,46 +1294,6 @@ int launch_energy_lj(cav_ctx *c)
 
 // ---------------------------------------------------------- batched replicas --
 
-// Packed copies of every replica's slots, by index and in the last list
-// build's bin order (binpos: slot -> replica-local bin position; a changed
-// ghost count forces a rebuild first, so every slot has one).
-__global__ void kb_pack(const RepDev *rep, const int *flags, const double *x, const double *y,
-                        const double *z, const double *q, const int *type, const int *id,
-                        double4 *xq, int2 *tid, const int *binpos, double4 *xqs, int2 *tids)
-{
-  const RepDev &r = rep[blockIdx.y];
-  const long a = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (a >= (long)r.n + flags[16 * blockIdx.y + F_NGHOST]) return;
-  const long s = r.base + a;
-  const double4 v = make_double4(x[s], y[s], z[s], q[s]);
-  const int2 w = make_int2(type[s], id[s]);
-  xq[s] = v;
-  tid[s] = w;
-  if (binpos) {
-    const long t = r.base + binpos[s];
-    xqs[t] = v;
-    tids[t] = w;
-  }
-}
-
-// per replica: sum of its per-block partials in a fixed order
-__global__ void kb_reduce_rows(int nper, const double *part, double *out)
-{
-  __shared__ double red[kBlock];
-  const double *p = part + (long)blockIdx.x * nper;
-  double s = 0;
-  for (int i = threadIdx.x; i < nper; i += kBlock) s += p[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-
-// every replica's rows are written both as indices and as bin-order slots:
-// the pair kernel reads the slots, the downloads and the adjoint the indices
 template <typename T>
 static void batch_pairs_t(cav_batch *b, const PairArgs &a, dim3 g)
 {
@@ -1347,14 +1306,10 @@ static void batch_pairs_t(cav_batch *b, const PairArgs &a, dim3 g)
     k_pairs<T, false, true, false, true><<<g, kBlock, 0, b->stream>>>(a);
 }
 
-// LJ + Ewald_r accelerations of every replica (overwriting), virial per replica.
+// LJ + Ewald_r accelerations of every replica (overwriting), virial partials
+// per replica; the packed copies are those of batch_neighbor.
 int batch_pairs(cav_batch *b)
 {
-  int maxslots = 0;
-  for (const RepDev &r : b->reps) maxslots = std::max(maxslots, r.n + r.gcap);
-  kb_pack<<<dim3(grid_for(maxslots), b->B), kBlock, 0, b->stream>>>(
-      b->d_rep, b->flags, b->x, b->y, b->z, b->q, b->type, b->id, b->xq, b->tid,
-      b->nl_on ? b->binpos : nullptr, b->xqs, b->tids);
   const dim3 g(b->pair_blocks, b->B);
   if (!b->lj_on && !b->er_on) {
     kb_zero_own<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(b->d_rep, b->ax, b->ay,
@@ -1369,7 +1324,7 @@ int batch_pairs(cav_batch *b)
     a.x = a.y = a.z = a.q = nullptr;
     a.minv = b->d_minv;
     a.type = a.id = a.mol = nullptr;
-    a.nl = b->nl;
+    a.nl = nullptr;
     a.nn = b->nn;
     a.order = b->order;
     a.xq = b->xq;
@@ -1398,7 +1353,6 @@ int batch_pairs(cav_batch *b)
     else
       batch_pairs_t<float>(b, a, g);
   }
-  kb_reduce_rows<<<b->B, kBlock, 0, b->stream>>>(b->pair_blocks, b->part, b->vir);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import fixtures as F
-from caviar_amd import Engine, NaNAccelerationError, configs
+from caviar_amd import Batch, Engine, NaNAccelerationError, configs
 from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -258,3 +258,57 @@ def test_constraints_end_of_step(gpu, n, n_r_df, which):
     assert F.rel_err(e.get("vel"), o.get("vel")) <= 1e-9
     for got, want in zip(e.thermo(), o.thermo()):
         assert abs(got - want) <= 1e-9 * abs(want)
+
+
+def _exchange_replicas():
+    rng = np.random.default_rng(8)
+
+    def free(n, box, pos):
+        return _free_pair_system(n, box, np.ascontiguousarray(pos), rng.normal(scale=3.0, size=(n, 3)))
+
+    face = rng.uniform(0, 6.0, (41, 3))       # the box is three cells: the upper faces
+    face[:7, 0] = 6.0                         # lie in the layer past the inner cells
+    face[5:12, 1] = 6.0
+    face[6] = 6.0
+    crowd = rng.uniform(0, 12.0, (700, 3))
+    # 600 atoms in one cell, 0.21 apart: beyond the LJ reach at the start and
+    # hardly into it after 12 steps (0.07 each), so that no collision amplifies
+    # the order of the sums
+    g = np.stack(np.meshgrid(*[np.arange(9) * 0.211 + 4.1] * 3, indexing="ij"), -1).reshape(-1, 3)
+    crowd[:600] = g[rng.permutation(len(g))[:600]]
+    out = [free(41, 6.0, face), free(700, 12.0, crowd), free(40, 90.0, rng.uniform(0, 90.0, (40, 3))),
+           free(1, 4.5, [[4.4, 0.1, 2.0]])]
+    out += [free(n, 9.0, rng.uniform(0, 9.0, (n, 3))) for n in (255, 256, 257)]
+    # atoms that leave the middle of their box: images beyond the slots set aside
+    g = np.stack(np.meshgrid(*[np.arange(7) * 0.5 + 6.5] * 3, indexing="ij"), -1).reshape(-1, 3)
+    s = free(len(g), 16.0, g)
+    s.vel = np.ascontiguousarray((g - 8.0) * 150.0)
+    return out + [s]
+
+
+@pytest.mark.parametrize("which", ["all", "fixed", "face"])
+def test_batch_exchange_edges(gpu, which):
+    """Images, cells and rows of a batch: atoms on the upper faces, cells past
+    their buckets, more cells than a workgroup adds up itself, one atom, counts
+    about the workgroup, ghosts outgrowing their slots.  Pairs exactly as the
+    oracle's, positions within 1e-12 after 12 steps."""
+    print(f"[case] batch exchange {which}", flush=True)
+    systems = _exchange_replicas()
+    systems = {"all": systems, "fixed": systems[:-1], "face": systems[:1]}[which]
+    b = Batch(systems)
+    b.setup()
+    for r, s in enumerate(systems):
+        o = Oracle(s.copy())
+        o.setup()
+        assert np.array_equal(F.sorted_pairs(b.pairs(r)), F.sorted_pairs(o.pairs())), r
+        e = Engine(s.copy())
+        e.setup()
+        assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(o.pairs())), r
+    b.step(0.002, 12)
+    for r, s in enumerate(systems):
+        o = Oracle(s.copy())
+        o.setup()
+        assert o.run(0.002, 12) == 0
+        assert F.rel_err(b.get(r, "pos"), o.get("pos")) <= 1e-12, r
+        if which != "all":  # (a replica outgrowing its slots has every list rebuilt)
+            assert np.array_equal(F.sorted_pairs(b.pairs(r)), F.sorted_pairs(o.pairs())), r
