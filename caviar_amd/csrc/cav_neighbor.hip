@@ -1124,10 +1124,10 @@ int launch_cells(cav_ctx *c)
 
 // ------------------------------------------------------------- Verlet list --
 
-// Stencil candidates staged in LDS per pass (8 KB of a wave's LDS at 256).
-// Measured at N=262144, rho=0.3 (list build, ms): 128 -> 0.218, 192 -> 0.208,
-// 256 -> 0.204, 512 -> 0.257, 1024 -> 0.470: fewer candidates per pass, more
-// waves per CU; the 512 batched replicas step 4.72 ms at 256 against 5.27 at 512.
+// Stencil candidates staged in LDS per pass (8 KB of a wave's LDS at 256):
+// fewer candidates per pass, more waves per CU, but more passes over the owned
+// atoms.  Measured with 128 / 192 / 256 / 384 (us): 262144 ions 226 / 225 / 219
+// / 253 beside Ewald_k, 256 replicas 434 / 395 / 384 / 418.
 #ifndef CAV_LIST_CAND
 #define CAV_LIST_CAND 256
 #endif
@@ -1150,10 +1150,16 @@ constexpr int kCand = CAV_LIST_CAND;
 // bin sort, so staging reads are contiguous per stencil cell; passing
 // lanes append in lane order through a ballot and a prefix popcount, so rows
 // are written coalesced and in a deterministic order.
-#ifndef CAV_LIST_API
-#define CAV_LIST_API 4
-#endif
-constexpr int kAPI = CAV_LIST_API;  // owned atoms tested per staged candidate
+//
+// Instruction issue bounds it, vector and scalar alike (counters: 15 vector
+// and 18 scalar instructions for each test of 64 pairs, of which the exact
+// FP64 distance needs nine).  So the owned atoms come by scalar loads, the
+// bounds check of a buffer store stands for the tests of a full row and of an
+// idle lane, the atom itself is looked for only in the pass that holds it, and
+// a stage's cells are found by bisection with all its loads in flight.
+// In order: N=262144 144 -> 121 us, 256 replicas (540000 atoms at rho 0.2 to
+// 0.8) 444 -> 332 us.
+constexpr int kAPI = 4;  // owned atoms tested per staged candidate
 
 // Cells per workgroup, one wave each (measured at N=262144: 1 -> 0.307 ms,
 // 2 -> 0.318, 4 -> 0.323, 8 -> 0.374; the build is not occupancy bound).
@@ -1166,6 +1172,50 @@ constexpr int kAPI = CAV_LIST_API;  // owned atoms tested per staged candidate
 constexpr int kListWaves = CAV_LIST_WPB;
 
 static int list_grid(long cells) { return (int)((cells + kListWaves - 1) / kListWaves); }
+
+// One atom's row as buffers of cap entries: a store past the end is dropped by
+// the bounds check, so neither a full row nor a lane with nothing to store
+// (offset -1) needs a branch of its own.
+template <bool NL, bool NLL, bool NLB>
+struct Rows {
+  __amdgpu_buffer_rsrc_t nl, nll, nlb;
+  __device__ __forceinline__ void set(int *pl, unsigned short *pll, int *plb, long at, int cap)
+  {
+    constexpr int raw = 0x00027000;  // untyped 32-bit data
+    if constexpr (NL) nl = __builtin_amdgcn_make_buffer_rsrc(pl + at, 0, 4 * cap, raw);
+    if constexpr (NLL) nll = __builtin_amdgcn_make_buffer_rsrc(pll + at, 0, 2 * cap, raw);
+    if constexpr (NLB) nlb = __builtin_amdgcn_make_buffer_rsrc(plb + at, 0, 4 * cap, raw);
+  }
+  // entry e4 / 4 of the row: candidate (tag) at staging position pos
+  __device__ __forceinline__ void put(int e4, double tag, int pos) const
+  {
+    if constexpr (NL) __builtin_amdgcn_raw_buffer_store_b32(cpos_index(tag), nl, e4, 0, 0);
+    if constexpr (NLL)
+      __builtin_amdgcn_raw_buffer_store_b16((unsigned short)pos, nll, e4 >> 1, 0, 0);
+    if constexpr (NLB) __builtin_amdgcn_raw_buffer_store_b32(cpos_slot(tag), nlb, e4, 0, 0);
+  }
+};
+
+// An owned atom against one candidate per lane; SELF: lane `self`, if there is
+// one, holds the atom itself, which is left out.  c4: 4 per entry of the row.
+template <bool SELF, class R>
+__device__ __forceinline__ void list_test(double px, double py, double pz, const double4 &q,
+                                          double rce2, int lane, int self, int pos, const R &row,
+                                          int &c4)
+{
+  const double dx = xsub(px, q.x), dy = xsub(py, q.y), dz = xsub(pz, q.z);
+  bool pass = dot_rn(dx, dy, dz) < rce2;
+  if constexpr (SELF) pass = pass && lane != self;
+  // the compare's lanes as a scalar mask
+  const u64t mask = __builtin_amdgcn_ballot_w64(pass);
+  if (mask) {
+    // the lane's rank among the passing lanes, after the row's entries so far
+    const unsigned pre = __builtin_amdgcn_mbcnt_hi(
+        (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+    row.put(pass ? c4 + 4 * (int)pre : -1, q.w, pos);
+    c4 += 4 * (int)__popcll(mask);
+  }
+}
 
 // The row outputs a build writes (index rows nl, staging positions nll,
 // bin-order slots nlb) are template flags, so the append path of the inner
@@ -1214,6 +1264,12 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves
   // group of kAPI owned atoms
   const int part = blockIdx.y;
   if (!waves && w == 0 && part == 0 && threadIdx.x == 0) flags[F_NL_STALE] = NL ? 0 : 1;
+  // staged candidates (x, y, z, index and slot) in the cell's stencil order; a stage is
+  // padded to a multiple of 64 with far-away entries so every lane tests one
+  __shared__ double4 sc_[kListWaves][kCand];
+  double4 *sc = sc_[wv];
+  __shared__ int s_off_[kListWaves][32], s_shift_[kListWaves][32];
+  int *s_off = s_off_[wv], *s_shift = s_shift_[wv];
   u64t todo = 1;
   if (shell) {  // the cells among the next 64 that are of the layer and hold an owned atom
     const int c = b + lane, cx = c % nbx, cy = c / nbx % nby, cz = c / (nbx * nby);
@@ -1227,127 +1283,115 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves
   }
   for (int b0 = b; todo; todo &= todo - 1) {
     b = b0 + __ffsll(todo) - 1;
-    // staged candidates (x, y, z, index and slot) in the cell's stencil order; a stage is
-    // padded to a multiple of 64 with far-away entries so every lane tests one
-    __shared__ double4 sc_[kListWaves][kCand];
-    double4 *sc = sc_[wv];
+    // the stencil's cell ranges, loaded by lanes 0..ns-1 at once, and the
+    // cell's own atoms: two chains of loads, side by side
     const int s0 = start[b], e0 = start[b + 1];
-    // owned atoms come first in a sorted bin
-    int no = 0;
+    const int sb = st_off[b], ns = st_off[b + 1] - sb;  // <= 27 stencil cells
+    int cell = -1, cb = 0, cn = 0;
+    if (lane < ns) {
+      cell = st[sb + lane];
+      cb = start[cell];
+      cn = start[cell + 1] - cb;
+    }
+    int no = 0;  // owned atoms come first in a sorted bin
     for (int t = s0; t < e0; t += 64) {
       const int v = (t + lane < e0) ? items[t + lane] : n;
       no += __popcll(__ballot(v < n));
     }
     if (no <= kAPI * part) continue;
-    const int sb = st_off[b], ns = st_off[b + 1] - sb;  // <= 27 stencil cells
-    // padding and empty owned slots sit at +-1e300: their squared distance to
-    // anything is +inf, so they never pass the cutoff test
-    const double4 far_cand = make_double4(1e300, 1e300, 1e300, cpos_tag(-1, -1));
-    // the stencil's cell ranges, loaded by lanes 0..ns-1 at once, and their
-    // running offsets in staging order (stencil cells in order, each in bin order)
-    __shared__ int s_base_[kListWaves][32], s_off_[kListWaves][33];
-    int *s_base = s_base_[wv], *s_off = s_off_[wv];
-    int total;
-    {
-      int cb = 0, cn = 0;
-      if (lane < ns) {
-        const int cell = st[sb + lane];
-        cb = start[cell];
-        cn = start[cell + 1] - cb;
-      }
-      int incl = cn;
-      for (int o = 1; o < 32; o <<= 1) {
-        const int v = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += v;
-      }
-      if (lane < ns) {
-        s_base[lane] = cb;
-        s_off[lane + 1] = incl;
-      }
-      if (lane == 0) s_off[0] = 0;
-      total = __shfl(incl, ns > 0 ? ns - 1 : 0, 64);
-      if (ns == 0) total = 0;
-      __syncwarp();
+    // running offsets of the ranges in staging order (stencil cells in order,
+    // each in bin order), and what takes a staging position to its slot
+    int incl = cn;
+    for (int o = 1; o < 32; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
     }
+    const int total = __builtin_amdgcn_readlane(incl, 31);  // lanes past ns add nothing
+    if (lane < 32) {
+      s_off[lane] = incl - cn;
+      s_shift[lane] = cb - (incl - cn);
+    }
+    // staging position of the cell's first atom: where a row's own atom is left out
+    const int centre = __ffsll(__ballot(cell == b)) - 1;
+    const int own0 = __builtin_amdgcn_readlane(incl - cn, centre);
+    __syncwarp();
     for (int og = 0; og < no; og += 64) {
       const int gsize = (no - og) < 64 ? (no - og) : 64;
-      // lane t holds owned atom og+t (position, slot) and its row count; the
-      // kAPI atoms of a group are read from those lanes, never from memory
-      const double4 mine = lane < gsize ? cpos[s0 + og + lane]
-                                        : make_double4(-1e300, -1e300, -1e300, cpos_tag(-1, -1));
-      int cnt = 0;
+      int cnt = 0;  // lane t: the row count of owned atom og + t
       for (int mbase = 0; mbase < total; mbase += kCand) {
         // stage candidates mbase .. mbase+m-1 of the flattened stencil: each
-        // lane finds its cells by walking the offsets forward, all loads at once
+        // lane finds the cells of its kCand/64 by bisection and issues their
+        // loads together
         const int m = (total - mbase) < kCand ? (total - mbase) : kCand;
-        int c = 0;
-        for (int t = lane; t < m; t += 64) {
-          const int g = mbase + t;
-          while (s_off[c + 1] <= g) ++c;
-          sc[t] = cpos[s_base[c] + g - s_off[c]];
-        }
         const int mpad = (m + 63) & ~63;
-        if (m + lane < mpad) sc[m + lane] = far_cand;
+        int at[kCand / 64];
+        double4 cv[kCand / 64];
+#pragma unroll
+        for (int q = 0; q < kCand / 64; ++q) at[q] = 0;
+#pragma unroll
+        for (int step = 16; step > 0; step >>= 1)
+#pragma unroll
+          for (int q = 0; q < kCand / 64; ++q)
+            if (s_off[at[q] + step] <= mbase + 64 * q + lane) at[q] += step;
+#pragma unroll
+        for (int q = 0; q < kCand / 64; ++q) {
+          const int g = mbase + 64 * q + lane;
+          at[q] = g < total ? s_shift[at[q]] + g : s0;
+        }
+#pragma unroll
+        for (int q = 0; q < kCand / 64; ++q) cv[q] = cpos[at[q]];
+#pragma unroll
+        for (int q = 0; q < kCand / 64; ++q) {
+          cv[q].x = 64 * q + lane < m ? cv[q].x : 1e300;
+          sc[64 * q + lane] = cv[q];
+        }
         __syncwarp();
         for (int o0 = kAPI * part; o0 < gsize; o0 += kAPI * split) {
-          // the kAPI owned atoms are the same for every lane: positions, slots,
-          // row offsets and row counters in scalar registers (empty slots of
-          // the group carry the far sentinel and never pass)
-          int ia[kAPI], c0[kAPI];
-          long row[kAPI];
+          // the kAPI owned atoms are the same for every lane: positions (by
+          // scalar loads), rows and row lengths in scalar registers.  Empty
+          // places of the group and padding sit at x = -+1e300: their squared
+          // distance to anything is +inf, so they never pass the cutoff test
           double px[kAPI], py[kAPI], pz[kAPI];
+          Rows<NL, NLL, NLB> row[kAPI];
 #pragma unroll
           for (int u = 0; u < kAPI; ++u) {
             const int src = o0 + u;  // < 64: o0 is a multiple of kAPI below 64
-            ia[u] = __builtin_amdgcn_readlane(cpos_index(mine.w), src);
-            px[u] = lane_d(mine.x, src);
-            py[u] = lane_d(mine.y, src);
-            pz[u] = lane_d(mine.z, src);
-            c0[u] = __builtin_amdgcn_readlane(cnt, src);
-            row[u] = (long)ia[u] * cap;
+            const auto *own = (const __attribute__((address_space(4))) double *)(cpos + s0 + og +
+                                                                                min(src, gsize - 1));
+            px[u] = src < gsize ? own[0] : -1e300;
+            py[u] = own[1];
+            pz[u] = own[2];
+            row[u].set(nl, nll, nlb, (long)cpos_index(own[3]) * cap, cap);
           }
+          // the row lengths, 4 per entry (an array would be copied as a whole)
+          static_assert(kAPI == 4, "four atoms a group");
+          int c0 = 4 * __builtin_amdgcn_readlane(cnt, o0), c1 = 4 * __builtin_amdgcn_readlane(cnt, o0 + 1),
+              c2 = 4 * __builtin_amdgcn_readlane(cnt, o0 + 2), c3 = 4 * __builtin_amdgcn_readlane(cnt, o0 + 3);
+          // the group's own places in the staging order, where no lane passes
+          const int self0 = own0 + og + o0 - mbase;
           for (int cc = 0; cc < mpad; cc += 64) {
             const int idx = cc + lane;
             const double4 q = sc[idx];
-            const int j = cpos_index(q.w);
-#pragma unroll
-            for (int u = 0; u < kAPI; ++u) {
-              const double dx = xsub(px[u], q.x), dy = xsub(py[u], q.y), dz = xsub(pz[u], q.z);
-              const bool pass = j != ia[u] && dot_rn(dx, dy, dz) < rce2;
-              // the ballot of the compare itself (a scalar mask), the lane's
-              // rank among the passing lanes by mbcnt, and a scalar row counter
-              const unsigned long long mask = __builtin_amdgcn_ballot_w64(pass);
-              if (mask) {
-                const int cu = c0[u];
-                const unsigned pre = __builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-                if (pass && cu + (int)pre < cap) {
-                  // uniform row pointers plus a 32-bit lane offset
-                  const long at0 = row[u] + cu;
-                  if constexpr (NL) {
-                    int *rp = nl + at0;
-                    rp[pre] = j;
-                  }
-                  if constexpr (NLL) {
-                    unsigned short *lp = nll + at0;
-                    lp[pre] = (unsigned short)(mbase + idx);  // position in the stencil staging order
-                  }
-                  if constexpr (NLB) {
-                    int *bp = nlb + at0;
-                    bp[pre] = cpos_slot(q.w);  // bin-order slot of the candidate
-                  }
-                }
-                c0[u] = cu + (int)__popcll(mask);
-              }
+            if ((unsigned)(self0 - cc + kAPI - 1) < 64u + kAPI - 1) {
+              const int self = self0 - cc;
+              list_test<true>(px[0], py[0], pz[0], q, rce2, lane, self, mbase + idx, row[0], c0);
+              list_test<true>(px[1], py[1], pz[1], q, rce2, lane, self + 1, mbase + idx, row[1], c1);
+              list_test<true>(px[2], py[2], pz[2], q, rce2, lane, self + 2, mbase + idx, row[2], c2);
+              list_test<true>(px[3], py[3], pz[3], q, rce2, lane, self + 3, mbase + idx, row[3], c3);
+            } else {
+              list_test<false>(px[0], py[0], pz[0], q, rce2, lane, 0, mbase + idx, row[0], c0);
+              list_test<false>(px[1], py[1], pz[1], q, rce2, lane, 0, mbase + idx, row[1], c1);
+              list_test<false>(px[2], py[2], pz[2], q, rce2, lane, 0, mbase + idx, row[2], c2);
+              list_test<false>(px[3], py[3], pz[3], q, rce2, lane, 0, mbase + idx, row[3], c3);
             }
           }
-#pragma unroll
-          for (int u = 0; u < kAPI; ++u) cnt = lane == o0 + u ? c0[u] : cnt;
+          cnt = lane == o0 ? c0 >> 2 : lane == o0 + 1 ? c1 >> 2 : lane == o0 + 2 ? c2 >> 2
+              : lane == o0 + 3 ? c3 >> 2 : cnt;
         }
         __syncwarp();
       }
       if (lane < gsize && lane / kAPI % split == part) {
-        const int i = cpos_index(mine.w);
+        const int i = cpos_index(cpos[s0 + og + lane].w);
         nn[i] = cnt < cap ? cnt : cap;
         // the longest row is needed only to regrow the list after an overflow:
         // one device-wide atomic per overflowing row, none otherwise
@@ -1373,7 +1417,7 @@ static void launch_list_wave(hipStream_t st, int n, int nbins, const int *xnb, i
   // atoms' groups is then the kernel's time; every wave stages the candidates
   // for itself, so a full chip keeps one.  Measured with 1 / 2 / 3 / 6 waves
   // (us): 125 cells 24 / 16 / 13 / 11, 1000 cells 34 / 23 / 20 / 17, 2744 cells
-  // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
+    // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
   const int split = std::max(1, std::min(6, 8192 / nbins));
   // One wave per cell, or on a grid with a ghost layer (xnb: its cells per
   // axis) one per inner cell and one per 64 of all cells for what owned atoms
