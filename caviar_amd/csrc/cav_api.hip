@@ -138,10 +138,13 @@ __global__ void k_zero3(int n, double *a, double *b, double *c)
   if (i < n) a[i] = b[i] = c[i] = 0.0;
 }
 
-__global__ void k_charge_of_type(int n, const int *type, const double *charge, double *q)
+// Per-atom charges from the table per type, and a copy of that table.
+__global__ void k_charge_of_type(int n, const int *type, const double *charge, double *q, int nt,
+                                 double *qtype)
 {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i < n) q[i] = charge[type[i]];
+  if (i < nt) qtype[i] = charge[i];
 }
 
 // The same over the ghost slots n .. n + flags[F_NGHOST) of the last exchange
@@ -286,7 +289,7 @@ static void free_all(cav_ctx *c)
                   c->mol,     c->q,      c->gsrc,      c->flags,    c->blk,      c->bin_of,
                   c->bin_cnt, c->bin_start, c->bin_items, c->d_st_off, c->d_st,  c->scan_tmp,
                   c->d_xst_off, c->d_xst,
-                  c->nl,      c->nn,     c->d_minv,    c->d_charge, c->d_eps,    c->d_lambda,
+                  c->nl,      c->nn,     c->d_minv,    c->d_charge, c->d_qtype, c->d_eps,    c->d_lambda,
                   c->d_ljl,   c->d_sr_lambda, c->d_elc_k, c->d_elc_chi, c->d_elc_dip,
                   c->d_thermo, c->d_mass,
                   c->part,    c->scal,   c->tab,       c->sk_part,  c->sk,       c->bmat,
@@ -464,9 +467,9 @@ static int neighbor_init(cav_ctx *c)
 static int alloc_list(cav_ctx *c, int cap)
 {
   c->nl_cap = cap;
-  CAV_TRY(dmalloc(c, &c->nl, (size_t)cap * c->n));
+  CAV_TRY(dmalloc(c, &c->nl, (size_t)cap * c->n + kRowPad));
   CAV_TRY(dmalloc(c, &c->nll, (size_t)cap * c->n));
-  CAV_TRY(dmalloc(c, &c->nlb, (size_t)cap * c->n));
+  CAV_TRY(dmalloc(c, &c->nlb, (size_t)cap * c->n + kRowPad));
   return CAV_OK;
 }
 
@@ -491,7 +494,8 @@ int cav::refresh_params(cav_ctx *c)
 {
   if (!c->params_dirty) return CAV_OK;
   CAV_TRY(upload_params(c));
-  k_charge_of_type<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->type, c->d_charge, c->q);
+  k_charge_of_type<<<grid_for(std::max(c->n, c->nt)), kBlock, 0, c->stream>>>(
+      c->n, c->type, c->d_charge, c->q, c->nt, c->d_qtype);
   if (c->gcap > 0)
     k_ghost_charge_of_type<<<grid_for(c->gcap), kBlock, 0, c->stream>>>(c->n, c->gcap, c->flags,
                                                                           c->type, c->d_charge, c->q);
@@ -597,7 +601,7 @@ static int neighbor_phase(cav_ctx *c, Rebuild how, bool fused)
     CAV_TRY(launch_bins(c, !c->lj_cellwalk, true));
   timer_end(c, c->t_nb);
   timer_begin(c, c->t_list);
-  CAV_TRY(launch_list(c, true));
+  CAV_TRY(launch_list(c, true, fused));
   if (how == Rebuild::forced) {  // the build is known to run
     c->nll_built = c->nll_pending;
     c->nlb_built = c->nlb_pending;
@@ -1046,12 +1050,13 @@ int cav_upload_atoms(cav_ctx *c, int n, const int *id, const int *type, const in
   CAV_TRY(dmalloc(c, &c->gsrc, c->gcap));
   CAV_TRY(dmalloc(c, &c->bin_of, tot));
   CAV_TRY(dmalloc(c, &c->bin_items, tot));
-  CAV_TRY(dmalloc(c, &c->cpos, tot));
+  // (the list build reads, and ignores, up to three slots past the end)
+  CAV_TRY(dmalloc(c, &c->cpos, tot + 4));
   CAV_TRY(dmalloc(c, &c->binpos, tot));
-  CAV_TRY(dmalloc(c, &c->litems, tot));
+  CAV_TRY(dmalloc(c, &c->litems, tot + 4));
   // no list build's bin order exists for the new slot arrays yet
   k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_NGHOST_OLD, -1);
-  CAV_TRY(dmalloc(c, &c->xqs, tot));
+  CAV_TRY(dmalloc(c, &c->xqs, tot + 4));
   CAV_TRY(dmalloc(c, &c->tids, tot));
   CAV_TRY(dmalloc(c, &c->nn, n));
   CAV_TRY(dmalloc(c, &c->order, n));
@@ -1065,6 +1070,9 @@ int cav_upload_atoms(cav_ctx *c, int n, const int *id, const int *type, const in
     for (int k = 0; k < 3; ++k) soa[(size_t)k * n + i] = pos[3 * i + k];
     qv[i] = c->charge[type[i]];
   }
+  c->q_of = c->charge;
+  c->ids_ascend = true;
+  for (int i = 1; i < n; ++i) c->ids_ascend = c->ids_ascend && id[i] > id[i - 1];
   const size_t b = sizeof(double) * n;
   CAV_HIP(hipMemcpy(c->x, soa.data(), b, hipMemcpyHostToDevice));
   CAV_HIP(hipMemcpy(c->y, soa.data() + n, b, hipMemcpyHostToDevice));
@@ -1212,6 +1220,11 @@ int cav_setup(cav_ctx *c)
     cap = (cap + 3) / 4 * 4;
     CAV_TRY(alloc_list(c, cap));
   }
+  // the charges per type that the atoms' were taken from
+  std::vector<double> qt = c->charge;
+  std::copy(c->q_of.begin(), c->q_of.begin() + std::min(qt.size(), c->q_of.size()), qt.begin());
+  CAV_TRY(dmalloc(c, &c->d_qtype, qt.size()));
+  CAV_HIP(hipMemcpy(c->d_qtype, qt.data(), sizeof(double) * qt.size(), hipMemcpyHostToDevice));
   k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_NGHOST_OLD, -1);
   for (int attempt = 0; attempt < 4; ++attempt) {
     if (attempt) CAV_TRY(elc_rewind(c));  // the retried evaluation is the same one

@@ -113,6 +113,44 @@ struct RepDev {
   int pbase;                 // first per-block partial slot
 };
 
+// Which replica a workgroup of a batched kernel works on, and as which of its
+// workgroups: grid (workgroups, replicas), or with `deal` grid (8, workgroups,
+// rounds).  Workgroups go to the eight XCDs in turn, so a dealt replica stays
+// on one XCD and its gathers in that XCD's L2.
+struct RepGrid {
+  const RepDev *rep = nullptr;
+  const int *deal = nullptr;  // [rounds][8] replicas, -1: none
+};
+
+// Row entries past a row's capacity that the pair kernel may read (and ignores)
+constexpr int kRowPad = 384;
+
+// In the type word of a ghost's bin-ordered record
+constexpr int kImage = (int)0x80000000u;
+
+#ifdef __HIPCC__
+// The bin-ordered record that the row pair kernel gathers: x, y, z and, in the
+// fourth word, the type (with kImage) and the id.
+__device__ __forceinline__ double4 slot_record(const double4 &v, const int2 &w, bool image)
+{
+  const int2 m = make_int2(image ? w.x | kImage : w.x, w.y);
+  return make_double4(v.x, v.y, v.z, __hiloint2double(m.y, m.x));
+}
+
+// The workgroup's replica (negative: none) and its place among the replica's.
+__device__ __forceinline__ int rep_block(const RepGrid &g, int &blk, int &blocks)
+{
+  if (g.deal) {
+    blk = blockIdx.y;
+    blocks = gridDim.y;
+    return g.deal[8 * blockIdx.z + blockIdx.x];
+  }
+  blk = blockIdx.x;
+  blocks = gridDim.x;
+  return blockIdx.y;
+}
+#endif
+
 }  // namespace cav
 
 struct cav_ctx {
@@ -215,7 +253,12 @@ struct cav_ctx {
   double4 *cpos = nullptr; // (x, y, z, index) in bin order, for the list build
   int *binpos = nullptr;   // bin-order position of every slot at the last list build
   int *lstart = nullptr, *litems = nullptr;  // cells of the last list build
-  double4 *xqs = nullptr;  // (x, y, z, q) in bin order, refreshed every step
+  // in bin order, refreshed every step: slot_record for the row kernel, or
+  // (x, y, z, q) for the cell-staged one
+  double4 *xqs = nullptr;
+  double *d_qtype = nullptr;  // charges per type that the atoms' were taken from
+  std::vector<double> q_of;   // ... at their upload
+  bool ids_ascend = false;    // the owned ids ascend with the index
   int2 *tids = nullptr;    // (type, id) in bin order
   // list build on the ghost-layer grid: per cell counts (owned in the high
   // word) and the slots met in any order, bucket_cap each
@@ -339,8 +382,10 @@ struct cav_batch {
   std::vector<int> h_st_off, h_st;
   std::vector<int2> h_waves;
 
+  std::vector<int> h_deal;  // empty: replicas are not dealt to XCDs
   // device
   cav::RepDev *d_rep = nullptr;
+  int *d_deal = nullptr;
   int *st_off = nullptr, *st = nullptr;  // stencils, as cells of the replica
   // the list build's waves: (cell, replica) of every inner cell, and (-1 -
   // first cell, replica) of every 64 cells for owned atoms in the outer layer
@@ -362,14 +407,11 @@ struct cav_batch {
   int *bin_start = nullptr, *bin_items = nullptr;
   unsigned long long *cell_cnt = nullptr, *cell_first = nullptr;
   int *bucket = nullptr, bucket_cap = 0;  // unsorted slots of every cell
-  double4 *cpos = nullptr; // slots: (x, y, z, slot) in bin order
   int *gblk = nullptr;     // [B][scan_blocks] ghost-count block sums
   int *nn = nullptr;
-  // Verlet rows as replica-local bin slots, bin-ordered copies of (x, y, z, q)
-  // and (type, id), slot -> local atom, owned atoms in cell order
+  // Verlet rows as replica-local bin slots, bin-ordered records, slot -> local atom, owned atoms in cell order
   int *nlb = nullptr;
   double4 *xqs = nullptr;
-  int2 *tids = nullptr;
   int *litems = nullptr, *order = nullptr;
   int cap = 0;
   int *flags = nullptr, *h_flags = nullptr, *hd_flags = nullptr;  // [B][16]; hd_flags: h_flags for the device
@@ -434,7 +476,8 @@ int launch_rebuild_check(cav_ctx *c);
 // for_list: the binning of a list build, which also keeps the bin order the
 // list refers to (litems, binpos)
 int launch_bins(cav_ctx *c, bool conditional, bool for_list = false);
-int launch_list(cav_ctx *c, bool conditional);
+// packed: the bin-ordered packed copies are current (launch_cells)
+int launch_list(cav_ctx *c, bool conditional, bool packed);
 int launch_save_old(cav_ctx *c, bool conditional);
 bool cell_staged(const cav_ctx *c);
 bool sorted_rows(const cav_ctx *c);
@@ -480,6 +523,9 @@ int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *
 int reduce_partials(cav_ctx *c, int count, int slot, bool add = false);
 int bfail(cav_batch *b, int code, const std::string &msg);
 int bhip_check(cav_batch *b, hipError_t e, const char *what);
+// grid of `blocks` workgroups a replica, and its kernel argument
+dim3 batch_grid(const cav_batch *b, int blocks);
+RepGrid batch_reps(const cav_batch *b);
 int batch_cells_alloc(cav_batch *b);
 // move or wrap, ghosts, rebuild test (drift), cells, packed copies, list
 int batch_neighbor(cav_batch *b, bool drift, double dt);

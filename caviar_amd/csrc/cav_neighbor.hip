@@ -490,8 +490,8 @@ __device__ __forceinline__ void block_sum2(int &a, int &b)
   }
 }
 
-// Batched replicas run the kernels of the exchange with grid row blockIdx.y =
-// replica: each shifts its arrays to the replica's slots (base), owned atoms
+// Batched replicas run the kernels of the exchange with each workgroup on one
+// replica (rep_block): it shifts its arrays to the replica's slots (base), owned atoms
 // (obase) and cells (cbase) and takes the box, ghost and cell rules from it.
 __device__ __forceinline__ GhostRule ghost_rule_of(const RepDev &r, double gc)
 {
@@ -536,7 +536,7 @@ struct MoveArgs {
   u64t *cnt;  // cell counters to clear, or nullptr
   int nbins;
   long stride;  // of the snapshot's planes
-  const RepDev *rep;  // REP: the replicas, and their ghost cutoff
+  RepGrid reps;  // REP: the replicas, and their ghost cutoff
   double gc;
 };
 
@@ -551,9 +551,14 @@ struct MoveArgs {
 template <bool DRIFT, int BS, bool REP>
 __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
 {
+  int blk = blockIdx.x, blocks = gridDim.x;
   if constexpr (REP) {
-    const RepDev &r = a.rep[blockIdx.y];
-    if ((int)blockIdx.x >= (r.n + BS - 1) / BS) return;
+    const int rr = rep_block(a.reps, blk, blocks);
+    if (rr < 0) return;
+    const RepDev &r = a.reps.rep[rr];
+    a.blk += (long)rr * blocks;
+    blocks = (r.n + BS - 1) / BS;
+    if (blk >= blocks) return;
     a.n = r.n;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -569,13 +574,12 @@ __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
       a.ax += r.obase, a.ay += r.obase, a.az += r.obase;
       a.snap += r.obase;
     }
-    a.flags += 16 * blockIdx.y;
-    a.blk += (long)blockIdx.y * gridDim.x;
+    a.flags += 16 * rr;
     a.cnt += r.cbase;
     a.nbins = r.nbins;
     rule = ghost_rule_of(r, a.gc);
   }
-  const int i = blockIdx.x * BS + threadIdx.x;
+  const int i = blk * BS + threadIdx.x;
   const int at = i < a.n ? i : 0;
   const int stop = a.flags[F_STOP];
   const double old[3] = {a.x[at], a.y[at], a.z[at]};
@@ -587,7 +591,7 @@ __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
   if (a.xo) last[0] = a.xo[at], last[1] = a.yo[at], last[2] = a.zo[at];
   if (DRIFT && stop) return;
   if (a.cnt)
-    for (int k = i; k < a.nbins; k += (REP ? (a.n + BS - 1) / BS : (int)gridDim.x) * BS) a.cnt[k] = 0;
+    for (int k = i; k < a.nbins; k += blocks * BS) a.cnt[k] = 0;
   int cnt = 0, moved = 0;
   if (i < a.n) {
     double *p[3] = {a.x + i, a.y + i, a.z + i};
@@ -637,7 +641,7 @@ __global__ __launch_bounds__(BS) void k_move(MoveArgs a, GhostRule rule)
   if (moved) a.flags[F_REBUILD] = 1;
   int none = 0;
   block_sum2<BS>(cnt, none);
-  if (threadIdx.x == 0) a.blk[blockIdx.x] = cnt;
+  if (threadIdx.x == 0) a.blk[blk] = cnt;
 }
 
 struct GhostArgs {
@@ -656,7 +660,7 @@ struct GhostArgs {
   u64t *cnt;    // cells (owned count in the high word), or nullptr
   int *bucket;
   int cap;
-  const RepDev *rep;  // REP: the replicas, their ghost cutoff and cell width
+  RepGrid reps;  // REP: the replicas, their ghost cutoff and cell width
   double gc, cinv;
 };
 
@@ -672,21 +676,24 @@ struct GhostArgs {
 template <int BS, bool REP>
 __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinRule bins)
 {
-  int gcap = 0;
+  int gcap = 0, blk = blockIdx.x;
   if constexpr (REP) {
-    const RepDev &r = a.rep[blockIdx.y];
+    int blocks;
+    const int rr = rep_block(a.reps, blk, blocks);
+    if (rr < 0) return;
+    const RepDev &r = a.reps.rep[rr];
     a.n = r.n;
     a.nblk = (r.n + BS - 1) / BS;
-    if ((int)blockIdx.x >= a.nblk) return;
+    if (blk >= a.nblk) return;
+    a.blk += (long)rr * blocks;
+    a.flags += 16 * rr;
     gcap = r.gcap;
     a.L[0] = r.L[0], a.L[1] = r.L[1], a.L[2] = r.L[2];
-    a.blk += (long)blockIdx.y * gridDim.x;
     a.x += r.base, a.y += r.base, a.z += r.base;
     a.type += r.base;
     a.id += r.base;
     a.q += r.base;
     if (a.xo) a.xo += r.base, a.yo += r.base, a.zo += r.base;
-    a.flags += 16 * blockIdx.y;
     a.xq += r.base;
     a.tid += r.base;
     a.cnt += r.cbase;
@@ -696,7 +703,7 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
   }
   // every load that depends on nothing first: at small sizes the kernel is a
   // chain of such latencies
-  const int i = blockIdx.x * BS + threadIdx.x;
+  const int i = blk * BS + threadIdx.x;
   const bool live = i < a.n;
   const int at = live ? i : 0;
   const double px = a.x[at], py = a.y[at], pz = a.z[at], qq = a.q[at];
@@ -704,14 +711,14 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
   const int stop = a.flags[F_STOP], old = a.flags[F_NGHOST_OLD];
   int before, total;
   if (a.scanned) {
-    before = a.blk[blockIdx.x];
+    before = a.blk[blk];
     total = a.flags[F_NGHOST];
   } else {
     before = total = 0;
     for (int k = threadIdx.x; k < a.nblk; k += BS) {
       const int v = a.blk[k];
       total += v;
-      if (k < (int)blockIdx.x) before += v;
+      if (k < blk) before += v;
     }
     block_sum2<BS>(before, total);
   }
@@ -770,14 +777,14 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
         const double dx = xsub(u, a.xo[s]), dy = xsub(v, a.yo[s]), dz = xsub(w, a.zo[s]);
         if (dot_rn(dx, dy, dz) > a.thr_sq) a.flags[F_REBUILD] = 1;
       }
-      a.x[s] = u;
-      a.y[s] = v;
-      a.z[s] = w;
-      a.type[s] = t;
-      a.id[s] = d;
-      a.q[s] = qq;
-      if constexpr (!REP) {
+      if constexpr (!REP) {  // (of a batch's images only the packed copies are read)
+        a.x[s] = u;
+        a.y[s] = v;
+        a.z[s] = w;
+        a.type[s] = t;
+        a.id[s] = d;
         a.mol[s] = m;
+        a.q[s] = qq;
         a.gsrc[g] = i;
       }
       ++g;
@@ -818,11 +825,10 @@ struct CellBuild {
   const double4 *xq;
   const int2 *tid;
   int *start, *items, *order, *binpos, *litems;
-  double4 *cpos, *xqs;
-  int2 *tids;
+  double4 *xqs;  // slot_record
   double *xo, *yo, *zo;
   int *flags;
-  const RepDev *rep;  // REP: the replicas, their cell width
+  RepGrid reps;  // REP: the replicas, their cell width
   double cinv;
   const u64t *first;  // counters before each workgroup's cells, or nullptr: added up here
 };
@@ -840,34 +846,36 @@ constexpr int kCellBlock = 1024;
 template <bool REP>
 __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
 {
-  int blocks = gridDim.x;
+  int blk = blockIdx.x, blocks = gridDim.x;
   if constexpr (REP) {
-    const RepDev &r = a.rep[blockIdx.y];
+    const int rr = rep_block(a.reps, blk, blocks);
+    if (rr < 0) return;
+    const RepDev &r = a.reps.rep[rr];
     a.n = r.n;
     a.nbins = r.nbins;
+    if (a.first) a.first += (long)rr * blocks;
     blocks = (r.nbins + a.bpb - 1) / a.bpb;
-    if ((int)blockIdx.x >= blocks) return;
-    if (a.first) a.first += (long)blockIdx.y * gridDim.x;
+    if (blk >= blocks) return;
     a.cnt += r.cbase;
     a.bucket += (long)r.cbase * a.cap;
     a.xq += r.base, a.tid += r.base;
-    a.start += r.cbase + blockIdx.y;  // one closing entry a replica
+    a.start += r.cbase + rr;  // one closing entry a replica
     a.items += r.base, a.litems += r.base;
     a.order += r.obase;
-    a.cpos += r.base, a.xqs += r.base, a.tids += r.base;
+    a.xqs += r.base;
     a.xo += r.base, a.yo += r.base, a.zo += r.base;
-    a.flags += 16 * blockIdx.y;
+    a.flags += 16 * rr;
     bins = bin_rule_of(r, a.cinv);
   }
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.flags[F_NGHOST], stop = a.flags[F_STOP], rebuild = a.flags[F_REBUILD];
-  const int b0 = blockIdx.x * a.bpb;
+  const int b0 = blk * a.bpb;
   // counters before the workgroup's cells, its own, and the slots of each
   // wave's first cell (whatever the bucket holds past its count): asked for
   // together, before the flags are known
   u64t s = 0;
   if (REP && a.first) {
-    if (threadIdx.x == 0) s = a.first[blockIdx.x];
+    if (threadIdx.x == 0) s = a.first[blk];
   } else {
 #pragma unroll 4
     for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
@@ -878,15 +886,14 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
   const long tot = (long)a.n + G;
   if (stop) return;
   if (!rebuild) {
-    for (long t = (long)blockIdx.x * kCellBlock + threadIdx.x; t < tot;
+    for (long t = (long)blk * kCellBlock + threadIdx.x; t < tot;
          t += (long)blocks * kCellBlock) {
       const int j = a.litems[t];
-      a.xqs[t] = a.xq[j];
-      a.tids[t] = a.tid[j];
+      a.xqs[t] = slot_record(a.xq[j], a.tid[j], j >= a.n);
     }
     return;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.flags[F_NGHOST_OLD] = G;
+  if (blk == 0 && threadIdx.x == 0) a.flags[F_NGHOST_OLD] = G;
   __shared__ u64t part[kCellBlock / 64];
   __shared__ u64t first[65];  // per cell: slots before it, owned atoms before it
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -956,13 +963,10 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
       const long t = s0 + r;
       const double4 v = a.xq[j];
       const int2 u = a.tid[j];
-      a.items[t] = j;
       a.litems[t] = j;
       if constexpr (!REP) a.binpos[j] = (int)t;
       if (j < a.n) a.order[o0 + r] = j;  // owned atoms come first in a cell
-      a.xqs[t] = v;
-      a.tids[t] = u;
-      a.cpos[t] = make_double4(v.x, v.y, v.z, cpos_tag(j, t));
+      a.xqs[t] = slot_record(v, u, j >= a.n);
       a.xo[j] = v.x;
       a.yo[j] = v.y;
       a.zo[j] = v.z;
@@ -1041,7 +1045,6 @@ int launch_move(cav_ctx *c, bool drift, double dt, bool decide)
   a.nbins = c->xnbins;
   const int bs = move_block(c), nb = grid_for(c->n, bs);
   a.stride = c->n;
-  a.rep = nullptr;
   const auto kern = bs == 64 ? (drift ? k_move<true, 64, false> : k_move<false, 64, false>)
                              : (drift ? k_move<true, kBlock, false> : k_move<false, kBlock, false>);
   kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c));
@@ -1082,7 +1085,6 @@ int launch_ghosts(cav_ctx *c, bool decide)
   a.cap = c->bucket_cap;
   if (a.scanned)
     k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
-  a.rep = nullptr;
   const auto kern = bs == 64 ? k_ghosts<64, false> : k_ghosts<kBlock, false>;
   kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
   CAV_HIP(hipGetLastError());
@@ -1108,14 +1110,11 @@ int launch_cells(cav_ctx *c)
   a.order = c->order;
   a.binpos = c->binpos;
   a.litems = c->litems;
-  a.cpos = c->cpos;
   a.xqs = c->xqs;
-  a.tids = c->tids;
   a.xo = c->xo;
   a.yo = c->yo;
   a.zo = c->zo;
   a.flags = c->flags;
-  a.rep = nullptr;
   a.first = nullptr;
   k_cells<false><<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
   CAV_HIP(hipGetLastError());
@@ -1220,7 +1219,11 @@ __device__ __forceinline__ void list_test(double px, double py, double pz, const
 // The row outputs a build writes (index rows nl, staging positions nll,
 // bin-order slots nlb) are template flags, so the append path of the inner
 // loop carries only the stores the launch needs.
-template <bool NL, bool NLL, bool NLB>
+//
+// PACKED: candidates come from the bin-ordered records that the pair kernel
+// gathers, with `items` the slots' atoms; else from a copy made for the list
+// (x, y, z, index and slot).
+template <bool NL, bool NLL, bool NLB, bool PACKED>
 __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves, int nbx, int nby, int nbz,
                                                   int cap, double rce2, const double4 *cpos,
                                                   const int *st_off, const int *st,
@@ -1343,6 +1346,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves
 #pragma unroll
         for (int q = 0; q < kCand / 64; ++q) {
           cv[q].x = 64 * q + lane < m ? cv[q].x : 1e300;
+          if constexpr (PACKED) cv[q].w = cpos_tag(-1, at[q]);
           sc[64 * q + lane] = cv[q];
         }
         __syncwarp();
@@ -1356,12 +1360,20 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves
 #pragma unroll
           for (int u = 0; u < kAPI; ++u) {
             const int src = o0 + u;  // < 64: o0 is a multiple of kAPI below 64
-            const auto *own = (const __attribute__((address_space(4))) double *)(cpos + s0 + og +
-                                                                                min(src, gsize - 1));
-            px[u] = src < gsize ? own[0] : -1e300;
+            // (past the group: some other slot's values, or the arrays' padding)
+            typedef const __attribute__((address_space(4))) double *scalar_d;
+            const long at = (long)s0 + og + src;
+            const scalar_d own = (scalar_d)(cpos + at);
+            px[u] = own[0];
             py[u] = own[1];
             pz[u] = own[2];
-            row[u].set(nl, nll, nlb, (long)cpos_index(own[3]) * cap, cap);
+            int i = PACKED ? ((const __attribute__((address_space(4))) int *)items)[at]
+                           : cpos_index(own[3]);
+            if (src >= gsize) {
+              px[u] = -1e300;
+              i = 0;
+            }
+            row[u].set(nl, nll, nlb, (long)i * cap, cap);
           }
           // the row lengths, 4 per entry (an array would be copied as a whole)
           static_assert(kAPI == 4, "four atoms a group");
@@ -1391,7 +1403,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_list_wave(int n, int nwaves
         __syncwarp();
       }
       if (lane < gsize && lane / kAPI % split == part) {
-        const int i = cpos_index(cpos[s0 + og + lane].w);
+        const int i = items[s0 + og + lane];
         nn[i] = cnt < cap ? cnt : cap;
         // the longest row is needed only to regrow the list after an overflow:
         // one device-wide atomic per overflowing row, none otherwise
@@ -1411,13 +1423,13 @@ static void launch_list_wave(hipStream_t st, int n, int nbins, const int *xnb, i
                              const double4 *cpos, const int *st_off, const int *stc,
                              const int *start, const int *items, int *nl, int *nn, int *flags,
                              const int *cond, const RepDev *rep, const int2 *waves, int nwaves,
-                             unsigned short *nll, int *nlb)
+                             unsigned short *nll, int *nlb, bool packed)
 {
   // Waves per cell: small grids leave CUs idle, and a wave's chain over its
   // atoms' groups is then the kernel's time; every wave stages the candidates
   // for itself, so a full chip keeps one.  Measured with 1 / 2 / 3 / 6 waves
   // (us): 125 cells 24 / 16 / 13 / 11, 1000 cells 34 / 23 / 20 / 17, 2744 cells
-    // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
+  // 45 / 34 / 33 / 34, 8000 cells 77 / 76 / 84 / 104.
   const int split = std::max(1, std::min(6, 8192 / nbins));
   // One wave per cell, or on a grid with a ghost layer (xnb: its cells per
   // axis) one per inner cell and one per 64 of all cells for what owned atoms
@@ -1431,18 +1443,18 @@ static void launch_list_wave(hipStream_t st, int n, int nbins, const int *xnb, i
     }
   }
   const dim3 g(list_grid(nwaves), split), blk(64 * kListWaves);
-#define CAV_LISTW(A, B, C)                                                                       \
-  k_list_wave<A, B, C><<<g, blk, 0, st>>>(n, nwaves, bx, by, bz, cap, rce2, cpos, st_off, stc,   \
-                                          start, items, nl, nn, flags, cond, rep, waves, nll,    \
-                                          nlb, split)
-  if (nlb && !nl)
-    CAV_LISTW(false, false, true);
+#define CAV_LISTW(A, B, C, D)                                                                    \
+  k_list_wave<A, B, C, D><<<g, blk, 0, st>>>(n, nwaves, bx, by, bz, cap, rce2, cpos,             \
+                                             st_off, stc, start, items, nl, nn, flags, cond, rep, \
+                                             waves, nll, nlb, split)
+  if (nlb && packed)
+    CAV_LISTW(false, false, true, true);
   else if (nlb)
-    CAV_LISTW(true, false, true);
+    CAV_LISTW(false, false, true, false);
   else if (nll)
-    CAV_LISTW(true, true, false);
+    CAV_LISTW(true, true, false, false);
   else
-    CAV_LISTW(true, false, false);
+    CAV_LISTW(true, false, false, false);
 #undef CAV_LISTW
 }
 
@@ -1484,7 +1496,7 @@ __global__ void k_list_bins(int n, int nbins, long cap_total, const int *start, 
   }
 }
 
-int launch_list(cav_ctx *c, bool conditional)
+int launch_list(cav_ctx *c, bool conditional, bool packed)
 {
   const int *cond = conditional ? c->flags + F_REBUILD : nullptr;
   // staging positions (and the cells they refer to) only for the cell-staged
@@ -1506,10 +1518,10 @@ int launch_list(cav_ctx *c, bool conditional)
                                                         cond);
   else
     launch_list_wave(c->stream, c->n, xg ? c->xnbins : c->nbins, xg ? c->nb : nullptr, c->nl_cap,
-                     c->rce2, c->cpos,
+                     c->rce2, packed ? c->xqs : c->cpos,
                      xg ? c->d_xst_off : c->d_st_off, xg ? c->d_xst : c->d_st, c->bin_start,
-                     c->bin_items, with_nlb ? nullptr : c->nl, c->nn, c->flags, cond, nullptr,
-                     nullptr, 0, with_nll ? c->nll : nullptr, with_nlb ? c->nlb : nullptr);
+                     packed ? c->litems : c->bin_items, with_nlb ? nullptr : c->nl, c->nn, c->flags, cond, nullptr,
+                     nullptr, 0, with_nll ? c->nll : nullptr, with_nlb ? c->nlb : nullptr, packed);
   // (the bin order itself, litems and binpos, was kept by the list build's
   // binning; the cell-staged kernel also needs the cell starts)
   if (with_nll) {
@@ -1654,7 +1666,7 @@ int batch_cells_alloc(cav_batch *b)
 int batch_neighbor(cav_batch *b, bool drift, double dt)
 {
   const int bs = batch_block(b);
-  const dim3 own_grid(b->scan_blocks, b->B);
+  const dim3 own_grid = batch_grid(b, b->scan_blocks);
   MoveArgs m;
   m.n = 0;
   m.dt = dt;
@@ -1678,7 +1690,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   m.cnt = b->cell_cnt;
   m.nbins = 0;
   m.stride = b->nown;
-  m.rep = b->d_rep;
+  m.reps = batch_reps(b);
   m.gc = b->ghost_cutoff;
   const auto move = bs == 64 ? (drift ? k_move<true, 64, true> : k_move<false, 64, true>)
                              : (drift ? k_move<true, kBlock, true> : k_move<false, kBlock, true>);
@@ -1706,7 +1718,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   g.cnt = b->cell_cnt;
   g.bucket = b->bucket;
   g.cap = b->bucket_cap;
-  g.rep = b->d_rep;
+  g.reps = batch_reps(b);
   g.gc = b->ghost_cutoff;
   g.cinv = b->cinv;
   const auto ghosts = bs == 64 ? k_ghosts<64, true> : k_ghosts<kBlock, true>;
@@ -1724,24 +1736,22 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   a.order = b->order;
   a.binpos = nullptr;
   a.litems = b->litems;
-  a.cpos = b->cpos;
   a.xqs = b->xqs;
-  a.tids = b->tids;
   a.xo = b->xo;
   a.yo = b->yo;
   a.zo = b->zo;
   a.flags = b->flags;
-  a.rep = b->d_rep;
+  a.reps = batch_reps(b);
   a.cinv = b->cinv;
   a.first = b->cell_first;
   const int blocks = (b->maxcells + a.bpb - 1) / a.bpb;
   if (a.first)
     kb_cell_first<<<b->B, kCellBlock, 0, b->stream>>>(b->d_rep, a.bpb, blocks, b->cell_cnt,
                                                       b->cell_first);
-  k_cells<true><<<dim3(blocks, b->B), kCellBlock, 0, b->stream>>>(a, BinRule{});
-  launch_list_wave(b->stream, 0, b->ncells, nullptr, b->cap, b->rce2, b->cpos, b->st_off, b->st,
+  k_cells<true><<<batch_grid(b, blocks), kCellBlock, 0, b->stream>>>(a, BinRule{});
+  launch_list_wave(b->stream, 0, b->ncells, nullptr, b->cap, b->rce2, b->xqs, b->st_off, b->st,
                    b->bin_start, b->litems, nullptr, b->nn, b->flags, nullptr, b->d_rep, b->waves,
-                   b->nwaves, nullptr, b->nlb);
+                   b->nwaves, nullptr, b->nlb, true);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }

@@ -55,31 +55,33 @@ struct PairArgs {
   double *ax, *ay, *az;
   double *part;
   int accumulate;  // add into the acceleration instead of overwriting it
-  const RepDev *rep;  // batched replicas (blockIdx.y) or nullptr
+  RepGrid reps;  // batched replicas, or none
   // rows as bin-order slots (or nullptr): neighbours are then read from the
   // bin-ordered copies, where the neighbours of cell-ordered atoms lie close
   // together, with the atom index from the list build's bin order
   const int *nlb;
-  const double4 *xqs;
-  const int2 *tids;
+  const double4 *xqs;  // slot_record
   const int *litems;
+  const double *qtype;  // charge per type
 };
 
-// Neighbours whose loads a lane issues together in the row-gather kernel
-// (measured at N=262144 with gathers by atom index: FP32 2/4/6/8 ->
-// 0.187/0.166/0.157/0.164 ms, FP64 0.204/0.220/0.208/0.254 ms, the FP64 pair
-// math needs the registers; from the bin-ordered copies, FP32 4/6/8/10 ->
-// 0.111/0.108/0.115/0.126 ms).
+// Neighbours whose loads a lane issues together in the row-gather kernel.
+// Measured with 4 / 5 / 6 / 8 (us): mixed, 262144 ions 104 / 101 / 104 / 114, 256
+// replicas 276 / 271 / 273 / 283; FP64 with 2 / 3 / 4: 65536 ions 36.0 / 36.0 /
+// 36.2 in order, 120 / 128 / 128 beside Ewald_k (its math needs the registers).
 template <typename T>
-constexpr int pair_u() { return sizeof(T) == 8 ? 2 : 6; }
+constexpr int pair_u() { return sizeof(T) == 8 ? 2 : 5; }
 
-// LJ per type pair (c12, c6, cshift) staged in LDS as T at kernel start:
-// 3 nt^2 values, converted once instead of per pair.
+// LJ per type pair (c12, c6, cshift) staged in LDS as T at kernel start: 3 nt^2
+// values, a pair's side by side, converted once instead of per pair.
 template <typename T>
 __device__ __forceinline__ void stage_lj_tables(const PairArgs &a, int nt2, T *tab)
 {
-  for (int t = threadIdx.x; t < 3 * nt2; t += blockDim.x)
-    tab[t] = (T)(t < nt2 ? a.c12[t] : (t < 2 * nt2 ? a.c6[t - nt2] : a.cshift[t - 2 * nt2]));
+  for (int t = threadIdx.x; t < nt2; t += blockDim.x) {
+    tab[3 * t] = (T)a.c12[t];
+    tab[3 * t + 1] = (T)a.c6[t];
+    tab[3 * t + 2] = (T)a.cshift[t];
+  }
 }
 
 template <typename T>
@@ -97,13 +99,16 @@ __device__ __forceinline__ T recip(T x)
 //   LJ: lj_cell_list.cpp:141-142 skips dr^2 > rc^2; shifted-force coefficients.
 //   ER: electrostatic_ewald_r.cpp:162-211, every listed pair, exact zero skipped,
 //       lambda of same-molecule pairs (0 skips the pair).
+// p: the type-pair entry as the reference indexes it, [lower owned index][partner]
+// (pair_entry); counted: the virial's share, once per reference list entry
+// (owned j > i or a ghost, and j > i for a ghost too) with id_i < id_j.
 template <typename T, bool LJ, bool ER, bool LAM>
-__device__ __forceinline__ T pair_coef(const PairArgs &a, const T *tab, int nt2, int i, int j,
-                                       int ti, int idi, int moli, const int2 &tj, T qi, T keqi,
-                                       const double4 &pi4, const double4 &pj, T &dx, T &dy, T &dz,
+__device__ __forceinline__ T pair_coef(const PairArgs &a, const T *tab, int p, bool counted,
+                                       bool same_mol, T qi, T keqi, T qj, const double4 &pi4,
+                                       double xj, double yj, double zj, T &dx, T &dy, T &dz,
                                        double &vir)
 {
-  const double dxd = pj.x - pi4.x, dyd = pj.y - pi4.y, dzd = pj.z - pi4.z;
+  const double dxd = xj - pi4.x, dyd = yj - pi4.y, dzd = zj - pi4.z;
   dx = (T)dxd;
   dy = (T)dyd;
   dz = (T)dzd;
@@ -113,28 +118,26 @@ __device__ __forceinline__ T pair_coef(const PairArgs &a, const T *tab, int nt2,
   else
     r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
   T coef = 0;
-  // type-pair entry as the reference indexes it: [lower owned index][partner]
-  const int p = (j < a.n && j < i) ? tj.x * a.nt + ti : ti * a.nt + tj.x;
   if constexpr (LJ) {
     if (!(r2 > (T)a.lj_rc2)) {
       const T ri2 = recip(r2);
       const T ri4 = ri2 * ri2, ri8 = ri4 * ri4;
-      coef += -tab[p] * (ri8 * ri4 * ri2) + tab[nt2 + p] * ri8 + tab[2 * nt2 + p];
+      coef += -tab[3 * p] * (ri8 * ri4 * ri2) + tab[3 * p + 1] * ri8 + tab[3 * p + 2];
     }
   }
   if constexpr (ER) {
-    if (!(dxd == 0 && dyd == 0 && dzd == 0)) {
+    // (a distance whose square is not zero is not)
+    if (r2 != 0 || !(dxd == 0 && dyd == 0 && dzd == 0)) {
       T lam = 1;
       bool skip = false;
       if constexpr (LAM) {
-        if (moli == a.mol[j]) {
+        if (same_mol) {
           const T l = (T)a.lambda[p];
           if (l == 0) skip = true;
           lam = l;
         }
       }
       if (!skip) {
-        const T qj = (T)pj.w;
         T ce;
         if constexpr (sizeof(T) == 8) {
           double e, ec, ri2;
@@ -150,12 +153,16 @@ __device__ __forceinline__ T pair_coef(const PairArgs &a, const T *tab, int nt2,
           ce = -lam * keqi * qj * s;
         }
         coef += ce;
-        // virial once per reference list entry (owned j > i or ghost), id_i < id_j
-        if ((j >= a.n || j > i) && idi < tj.y) vir += -(double)ce * (double)r2;
+        if (counted) vir += -(double)ce * (double)r2;
       }
     }
   }
   return coef;
+}
+
+__device__ __forceinline__ int pair_entry(bool lower, int ti, int tj, int nt)
+{
+  return lower ? __mul24(tj, nt) + ti : __mul24(ti, nt) + tj;
 }
 
 // Deterministic per-block sum of the virial: fixed shuffle tree per wave, then
@@ -178,24 +185,42 @@ __device__ __forceinline__ void block_virial(double vir, double *part)
 // z, q) and (type, id), before computing, so the gathers overlap.  The
 // partial forces of an atom's lanes are summed with a fixed shuffle tree, so
 // FP64 results stay reproducible.
-template <typename T, bool LJ, bool ER, bool LAM, bool BINS, int LPA = kLPA>
+//
+// Gather instructions bound it (N=262144 mixed: the address units take about 25
+// clocks for each, of whatever width, 78% of their time; the vector units are
+// half busy).  So a slot is one record of two 16-byte loads: the charge is
+// looked up by type, and with ids that ascend with the atom index
+// (ROWS_SLOTS_ASC) images and the order of a pair are told by id, without the
+// slot's atom.  The next row entries are fetched while these are used.  Before,
+// with (x, y, z, q), (type, id) and the atom gathered apart (us): mixed, 262144
+// ions 110, 256 replicas (540000 atoms, rho 0.2 to 0.8) 381; FP64, 65536 ions
+// 41; now 92, 271 and 36.  Planes x, y, z instead of records (a third fewer
+// bytes through the L1, but as many instructions) gained nothing.
+enum { ROWS_INDEX, ROWS_SLOTS, ROWS_SLOTS_ASC };
+
+template <typename T, bool LJ, bool ER, bool LAM, int ROWS, int LPA = kLPA>
 __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
 {
   extern __shared__ double dyn_pair[];
   T *tab = reinterpret_cast<T *>(dyn_pair);
   const int nt2 = LJ ? a.nt * a.nt : 0;
-  if (a.rep) {  // one replica per grid row: shift every array to it
-    const RepDev &r = a.rep[blockIdx.y];
+  T *qt = tab + 3 * nt2;
+  int part_at = blockIdx.x, blk32 = blockIdx.x;
+  if (a.reps.rep) {  // the workgroup's replica: shift every array to it
+    int blocks;
+    const int rr = rep_block(a.reps, blk32, blocks);
+    if (rr < 0) return;
+    const RepDev &r = a.reps.rep[rr];
+    part_at = blk32;
     const int base = r.base, obase = r.obase;
     a.n = r.n;
     a.xq += base;
     a.tid += base;
     a.nn += obase;
     if (a.order) a.order += obase;
-    if constexpr (BINS) {
+    if constexpr (ROWS != ROWS_INDEX) {
       a.nlb += (long)obase * a.cap;
       a.xqs += base;
-      a.tids += base;
       a.litems += base;
     }
     a.ax += obase;
@@ -203,8 +228,8 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
     a.az += obase;
     a.part += r.pbase;
   }
-  long blk = blockIdx.x;
-  if (!a.rep) {
+  long blk = blk32;
+  if (!a.reps.rep) {
     // XCD-aware order (the grid is a multiple of 8 and dispatch is round-robin
     // over the 8 XCDs): each XCD gets a contiguous run of cell-ordered atoms,
     // so neighbouring atoms' gathers share one L2
@@ -227,45 +252,67 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
   }
   // (staged while the atom's own loads are under way)
   stage_lj_tables(a, nt2, tab);
+  if constexpr (ROWS != ROWS_INDEX)
+    for (int q = threadIdx.x; q < a.nt; q += kBlock) qt[q] = (T)a.qtype[q];
   __syncthreads();
   if (t < a.n) {
     ti = tii.x;
     const T qi = (T)pi4.w;
     const T keqi = (T)(a.ke) * qi;
-    const int *row = (BINS ? a.nlb : a.nl) + (long)i * a.cap;
+    const int *row = (ROWS != ROWS_INDEX ? a.nlb : a.nl) + (long)i * a.cap;
     constexpr int U = pair_u<T>();
+    // entries past the row (read all the same, rows are padded) stand for slot 0
+    // and are skipped below; the next entries are fetched while these are used
+    int next[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) next[u] = row[sub + u * LPA];
     for (int k0 = sub; k0 < cnt; k0 += U * LPA) {
       int jj[U];
-      double4 pj[U];
+      double xj[U], yj[U], zj[U];
+      T qj[U];
       int2 tj[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = k0 + u * LPA;
-        jj[u] = k < cnt ? row[k] : -1;
-      }
-      if constexpr (BINS) {
-        // entries past the row read slot 0 and are skipped below
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int pp = jj[u] < 0 ? 0 : jj[u];
-          pj[u] = a.xqs[pp];
-          tj[u] = a.tids[pp];
-          jj[u] = jj[u] < 0 ? -1 : a.litems[pp];
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int j = jj[u] < 0 ? i : jj[u];
-          pj[u] = a.xq[j];
-          tj[u] = a.tid[j];
-        }
-      }
+      for (int u = 0; u < U; ++u) jj[u] = next[u];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (jj[u] < 0) break;
+        const unsigned k = k0 + u * LPA < cnt ? jj[u] : 0;
+        if constexpr (ROWS != ROWS_INDEX) {
+          const double4 v = a.xqs[k];
+          xj[u] = v.x;
+          yj[u] = v.y;
+          zj[u] = v.z;
+          tj[u] = make_int2(__double2loint(v.w), __double2hiint(v.w));
+          if constexpr (ROWS == ROWS_SLOTS) jj[u] = a.litems[k];
+        } else {
+          const double4 v = a.xq[k];
+          xj[u] = v.x;
+          yj[u] = v.y;
+          zj[u] = v.z;
+          qj[u] = (T)v.w;
+          tj[u] = a.tid[k];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) next[u] = row[k0 + (U + u) * LPA];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (k0 + u * LPA >= cnt) break;
+        const int type = ROWS != ROWS_INDEX ? tj[u].x & ~kImage : tj[u].x;
+        if constexpr (ROWS != ROWS_INDEX) qj[u] = qt[type];
+        bool lower, counted = tii.y < tj[u].y;
+        if constexpr (ROWS == ROWS_SLOTS_ASC) {
+          lower = !(tj[u].x & kImage) && tj[u].y < tii.y;
+        } else {
+          lower = jj[u] < i;
+          counted = counted && jj[u] > i;
+        }
+        bool same_mol = false;
+        if constexpr (LAM) same_mol = moli == a.mol[jj[u]];
         T dx, dy, dz;
-        const T coef = pair_coef<T, LJ, ER, LAM>(a, tab, nt2, i, jj[u], ti, tii.y, moli, tj[u], qi,
-                                                 keqi, pi4, pj[u], dx, dy, dz, vir);
+        const T coef = pair_coef<T, LJ, ER, LAM>(a, tab, pair_entry(lower, ti, type, a.nt), counted,
+                                                 same_mol, qi, keqi, qj[u], pi4, xj[u], yj[u], zj[u],
+                                                 dx, dy, dz, vir);
         fx = fma(coef, dx, fx);
         fy = fma(coef, dy, fy);
         fz = fma(coef, dz, fz);
@@ -290,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void k_pairs(PairArgs a)
       a.az[i] = (double)fz * mi;
     }
   }
-  block_virial(vir, a.part + blockIdx.x);
+  block_virial(vir, a.part + part_at);
 }
 
 // ------------------------------------- force_field lj and short-range kernel --
@@ -602,8 +649,9 @@ __global__ __launch_bounds__(kBlock) void k_pairs_cells(PairArgs a, CellPairArgs
                 tj = a.tid[j];
               }
               T dx, dy, dz;
-              const T coef = pair_coef<T, LJ, ER, false>(a, tab, nt2, i, j, ti, tii.y, 0, tj, qi,
-                                                         keqi, pi4, pj, dx, dy, dz, vir);
+              const T coef = pair_coef<T, LJ, ER, false>(
+                  a, tab, pair_entry(j < i, ti, tj.x, a.nt), j > i && tii.y < tj.y, false, qi, keqi,
+                  (T)pj.w, pi4, pj.x, pj.y, pj.z, dx, dy, dz, vir);
               fx = fma(coef, dx, fx);
               fy = fma(coef, dy, fy);
               fz = fma(coef, dz, fz);
@@ -642,7 +690,8 @@ __global__ __launch_bounds__(kBlock) void k_pairs_cells(PairArgs a, CellPairArgs
 // Packed copies for the pair gathers: (x, y, z, q) and (type, id).
 __global__ void k_pack(int n, long cap_total, const double *x, const double *y, const double *z,
                        const double *q, const int *type, const int *id, const int *flags,
-                       double4 *xq, int2 *tid, const int *binpos, double4 *xqs, int2 *tids)
+                       double4 *xq, int2 *tid, const int *binpos, double4 *xqs, int2 *tids,
+                       int records)
 {
   const long a = (long)blockIdx.x * kBlock + threadIdx.x;
   if (a >= (long)n + flags[F_NGHOST] || a >= cap_total) return;
@@ -650,13 +699,14 @@ __global__ void k_pack(int n, long cap_total, const double *x, const double *y, 
   const int2 w = make_int2(type[a], id[a]);
   xq[a] = v;
   tid[a] = w;
-  // the same in bin order, for the cell-staged pair kernel: only slots that
-  // existed at the last list build have a bin position
+  // the same in bin order, for the cell-staged pair kernel or as records for
+  // the row kernel: only slots that existed at the last list build
+  // have a bin position
   if (binpos && a < (long)n + flags[F_NGHOST_OLD]) {
     const int t = binpos[a];
     if (t >= 0 && t < cap_total) {
-      xqs[t] = v;
-      tids[t] = w;
+      xqs[t] = records ? slot_record(v, w, a >= n) : v;
+      if (!records) tids[t] = w;
     }
   }
 }
@@ -686,7 +736,6 @@ int reduce_partials(cav_ctx *c, int count, int slot, bool add)
 static PairArgs pair_args(cav_ctx *c)
 {
   PairArgs a;
-  a.rep = nullptr;
   a.accumulate = 0;
   a.n = c->n;
   a.nt = c->nt;
@@ -719,8 +768,8 @@ static PairArgs pair_args(cav_ctx *c)
   a.part = c->part;
   a.nlb = nullptr;
   a.xqs = nullptr;
-  a.tids = nullptr;
   a.litems = nullptr;
+  a.qtype = nullptr;
   return a;
 }
 
@@ -738,36 +787,61 @@ static int pair_lanes(const cav_ctx *c) { return c->n <= 16384 ? 32 : kLPA; }
 
 int pair_blocks(const cav_ctx *c) { return pair_grid(c, pair_lanes(c)); }
 
-template <typename T, bool BINS, int LPA>
-static void launch_pairs_tb(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
+// LDS of the row kernel: the LJ tables and the charges per type
+template <typename T>
+static size_t pair_lds(const PairArgs &a, bool lj)
+{
+  return sizeof(T) * ((lj ? 3 * a.nt * a.nt : 0) + a.nt);
+}
+
+template <typename T, int ROWS, int LPA>
+static void launch_pairs_tr(cav_ctx *c, const PairArgs &a, bool lj, bool er)
 {
   const int g = pair_grid(c, LPA);
-  const size_t lds = 3 * sizeof(T) * a.nt * a.nt;  // LJ tables
-  if (lj && er && lam)
-    k_pairs<T, true, true, true, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
-  else if (lj && er)
-    k_pairs<T, true, true, false, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
+  const size_t lds = pair_lds<T>(a, lj);
+  if (lj && er)
+    k_pairs<T, true, true, false, ROWS, LPA><<<g, kBlock, lds, c->stream>>>(a);
   else if (lj)
-    k_pairs<T, true, false, false, BINS, LPA><<<g, kBlock, lds, c->stream>>>(a);
-  else if (er && lam)
-    k_pairs<T, false, true, true, BINS, LPA><<<g, kBlock, 0, c->stream>>>(a);
+    k_pairs<T, true, false, false, ROWS, LPA><<<g, kBlock, lds, c->stream>>>(a);
   else
-    k_pairs<T, false, true, false, BINS, LPA><<<g, kBlock, 0, c->stream>>>(a);
+    k_pairs<T, false, true, false, ROWS, LPA><<<g, kBlock, lds, c->stream>>>(a);
+}
+
+// with the per-molecule lambda (of Ewald_r), which needs the neighbour's index
+template <typename T, int ROWS, int LPA>
+static void launch_pairs_tl(cav_ctx *c, const PairArgs &a, bool lj)
+{
+  const int g = pair_grid(c, LPA);
+  const size_t lds = pair_lds<T>(a, lj);
+  if (lj)
+    k_pairs<T, true, true, true, ROWS, LPA><<<g, kBlock, lds, c->stream>>>(a);
+  else
+    k_pairs<T, false, true, true, ROWS, LPA><<<g, kBlock, lds, c->stream>>>(a);
 }
 
 // rows as bin-order slots (a.nlb) or as atom indices, each its own kernel
+template <typename T, int LPA>
+static void launch_pairs_tn(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
+{
+  if (er && lam && a.nlb)
+    launch_pairs_tl<T, ROWS_SLOTS, LPA>(c, a, lj);
+  else if (er && lam)
+    launch_pairs_tl<T, ROWS_INDEX, LPA>(c, a, lj);
+  else if (!a.nlb)
+    launch_pairs_tr<T, ROWS_INDEX, LPA>(c, a, lj, er);
+  else if (c->ids_ascend)
+    launch_pairs_tr<T, ROWS_SLOTS_ASC, LPA>(c, a, lj, er);
+  else
+    launch_pairs_tr<T, ROWS_SLOTS, LPA>(c, a, lj, er);
+}
+
 template <typename T>
 static void launch_pairs_t(cav_ctx *c, const PairArgs &a, bool lj, bool er, bool lam)
 {
-  const bool wide = pair_lanes(c) == 32;
-  if (a.nlb && wide)
-    launch_pairs_tb<T, true, 32>(c, a, lj, er, lam);
-  else if (a.nlb)
-    launch_pairs_tb<T, true, kLPA>(c, a, lj, er, lam);
-  else if (wide)
-    launch_pairs_tb<T, false, 32>(c, a, lj, er, lam);
+  if (pair_lanes(c) == 32)
+    launch_pairs_tn<T, 32>(c, a, lj, er, lam);
   else
-    launch_pairs_tb<T, false, kLPA>(c, a, lj, er, lam);
+    launch_pairs_tn<T, kLPA>(c, a, lj, er, lam);
 }
 
 // The cell-staged kernel runs on request (CAV_PAIRS_CELLS) where it applies:
@@ -871,7 +945,7 @@ int launch_pack(cav_ctx *c)
   const long tot = (long)c->n + c->gcap;
   k_pack<<<grid_for(tot), kBlock, 0, c->stream>>>(c->n, tot, c->x, c->y, c->z, c->q, c->type,
                                                  c->id, c->flags, c->xq, c->tid, nullptr, nullptr,
-                                                 nullptr);
+                                                 nullptr, 0);
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -891,8 +965,8 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate, bool p
   if (bins) {
     a.nlb = c->nlb;
     a.xqs = c->xqs;
-    a.tids = c->tids;
     a.litems = c->litems;
+    a.qtype = c->d_qtype;
   } else {
     CAV_TRY(launch_nl_fill(c));
   }
@@ -900,7 +974,7 @@ int launch_pairs(cav_ctx *c, bool want_lj, bool want_er, bool accumulate, bool p
     k_pack<<<grid_for(tot), kBlock, 0, c->stream>>>(c->n, tot, c->x, c->y, c->z, c->q, c->type,
                                                  c->id, c->flags, c->xq, c->tid,
                                                  cells || bins ? c->binpos : nullptr, c->xqs,
-                                                 c->tids);
+                                                 c->tids, bins);
   timer_begin(c, c->t_pair);
   if (cells) {
     if (c->precision == CAV_FP64)
@@ -1297,20 +1371,20 @@ int launch_energy_lj(cav_ctx *c)
 template <typename T>
 static void batch_pairs_t(cav_batch *b, const PairArgs &a, dim3 g)
 {
-  const size_t lds = 3 * sizeof(T) * a.nt * a.nt;  // LJ tables
+  const size_t lds = pair_lds<T>(a, b->lj_on);
   if (b->lj_on && b->er_on)
-    k_pairs<T, true, true, false, true><<<g, kBlock, lds, b->stream>>>(a);
+    k_pairs<T, true, true, false, ROWS_SLOTS_ASC><<<g, kBlock, lds, b->stream>>>(a);
   else if (b->lj_on)
-    k_pairs<T, true, false, false, true><<<g, kBlock, lds, b->stream>>>(a);
+    k_pairs<T, true, false, false, ROWS_SLOTS_ASC><<<g, kBlock, lds, b->stream>>>(a);
   else
-    k_pairs<T, false, true, false, true><<<g, kBlock, 0, b->stream>>>(a);
+    k_pairs<T, false, true, false, ROWS_SLOTS_ASC><<<g, kBlock, lds, b->stream>>>(a);
 }
 
 // LJ + Ewald_r accelerations of every replica (overwriting), virial partials
 // per replica; the packed copies are those of batch_neighbor.
 int batch_pairs(cav_batch *b)
 {
-  const dim3 g(b->pair_blocks, b->B);
+  const dim3 g = batch_grid(b, b->pair_blocks);
   if (!b->lj_on && !b->er_on) {
     kb_zero_own<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(b->d_rep, b->ax, b->ay,
                                                                         b->az);
@@ -1343,11 +1417,11 @@ int batch_pairs(cav_batch *b)
     a.az = b->az;
     a.part = b->part;
     a.accumulate = 0;
-    a.rep = b->d_rep;
+    a.reps = batch_reps(b);
     a.nlb = b->nlb;
     a.xqs = b->xqs;
-    a.tids = b->tids;
     a.litems = b->litems;
+    a.qtype = b->d_charge;
     if (b->precision == CAV_FP64)
       batch_pairs_t<double>(b, a, g);
     else

@@ -312,3 +312,30 @@ def test_batch_exchange_edges(gpu, which):
         assert F.rel_err(b.get(r, "pos"), o.get("pos")) <= 1e-12, r
         if which != "all":  # (a replica outgrowing its slots has every list rebuilt)
             assert np.array_equal(F.sorted_pairs(b.pairs(r)), F.sorted_pairs(o.pairs())), r
+
+
+@pytest.mark.parametrize("n", [333, 17000])
+@pytest.mark.parametrize("ids", ["ascending", "gaps", "shuffled", "equal"])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_pair_rows_by_ids(gpu, n, ids, symmetric):
+    """The row kernel tells images and the order of a pair by ids that ascend
+    with the index, else by the slots' atoms: forces and virial for both, with
+    type tables that depend on which atom is the lower one."""
+    print(f"[case] ids {ids} n={n} symmetric={symmetric}", flush=True)
+    s = configs.ions(n=n, rho=0.3, kmax=1, seed=n, with_k=False)
+    rng = np.random.default_rng(n)
+    s.ids = {"ascending": np.arange(n), "gaps": np.cumsum(rng.integers(1, 5, n)),
+             "shuffled": rng.permutation(n), "equal": np.full(n, 7)}[ids].astype(np.int32)
+    if not symmetric:
+        s.lj.epsilon = np.array([[1.0, 0.7], [1.3, 0.9]])
+        s.lj.sigma = np.array([[1.0, 0.95], [1.05, 0.9]])
+    o = Oracle(s, threads=8)
+    o.setup()
+    for kernel in ("auto", "rows"):
+        e = Engine(s)
+        e.set_pair_kernel(kernel)
+        e.setup()
+        assert F.rel_err(e.get("acc"), o.get("acc")) <= 1e-12, kernel
+        # the oracle adds some 38 n terms one by one: a random walk of roundings
+        # of partial sums several times the total, 1e-16 * sqrt(650000) * 1e3 = 1e-10
+        assert abs(e.virial() - o.virial()) <= 1e-11 * max(abs(o.virial()), abs(o.energy_r())), kernel
