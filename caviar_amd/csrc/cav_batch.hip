@@ -73,12 +73,14 @@ __global__ __launch_bounds__(kBlock) void kb_virial(int nper, const double *part
   replica_virial(nper, part + (long)blockIdx.x * nper, vir + blockIdx.x);
 }
 
-// The end of a step: v += (0.5*dt) * (a + a_old) per replica (grid row), its
-// virial, and its flags, written straight to the host's (pinned) copy and
+// The end of a step: v += (0.5*dt) * (a + a_old) per replica (grid row; JOIN:
+// first a += the concurrent Ewald_k's accelerations), its virial, and its flags, written straight to the host's (pinned) copy and
 // cleared for the next step: a copy and two small launches less a step.
+template <bool JOIN>
 __global__ __launch_bounds__(kBlock) void kb_kick(const RepDev *rep, double hdt, double *vx,
-                                                  double *vy, double *vz, const double *ax,
-                                                  const double *ay, const double *az,
+                                                  double *vy, double *vz, double *ax, double *ay,
+                                                  double *az, const double *ekx,
+                                                  const double *eky, const double *ekz,
                                                   const double *aox, const double *aoy,
                                                   const double *aoz, int nper, const double *part,
                                                   double *vir, int *flags, int *host_flags)
@@ -87,9 +89,15 @@ __global__ __launch_bounds__(kBlock) void kb_kick(const RepDev *rep, double hdt,
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t < r.n) {
     const long i = (long)r.obase + t;
-    vx[i] = xadd(vx[i], xmul(hdt, xadd(ax[i], aox[i])));
-    vy[i] = xadd(vy[i], xmul(hdt, xadd(ay[i], aoy[i])));
-    vz[i] = xadd(vz[i], xmul(hdt, xadd(az[i], aoz[i])));
+    double a[3] = {ax[i], ay[i], az[i]};
+    if constexpr (JOIN) {
+      ax[i] = a[0] = xadd(a[0], ekx[i]);
+      ay[i] = a[1] = xadd(a[1], eky[i]);
+      az[i] = a[2] = xadd(a[2], ekz[i]);
+    }
+    vx[i] = xadd(vx[i], xmul(hdt, xadd(a[0], aox[i])));
+    vy[i] = xadd(vy[i], xmul(hdt, xadd(a[1], aoy[i])));
+    vz[i] = xadd(vz[i], xmul(hdt, xadd(a[2], aoz[i])));
   }
   if (blockIdx.x != 0) return;
   replica_virial(nper, part + (long)blockIdx.y * nper, vir + blockIdx.y);
@@ -131,7 +139,8 @@ static void batch_free(cav_batch *b)
                   b->bin_items, b->gblk, b->nn, b->flags, b->d_minv, b->d_lj, b->adj_ws, b->part,
                   b->vir, b->d_W, b->tab, b->ztab, b->bmat, b->bmat_h, b->sk_part, b->sk, b->epart,
                   b->s_items, b->s_items_o, b->f_items, b->rchunks, b->d_raw_eps,
-                  b->d_raw_sig, b->d_charge, b->nlb, b->xqs, b->litems, b->order};
+                  b->d_raw_sig, b->d_charge, b->nlb, b->xqs, b->litems, b->order, b->ekx,
+                  b->eky, b->ekz};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->h_flags) (void)hipHostFree(b->h_flags);
@@ -269,6 +278,14 @@ static int batch_layout(cav_batch *b)
     CAV_TRY(balloc(b, &b->d_deal, b->h_deal.size()));
     BAT_HIP(hipMemcpy(b->d_deal, b->h_deal.data(), sizeof(int) * b->h_deal.size(), hipMemcpyHostToDevice));
   }
+  if (b->ek_on) {
+    CAV_TRY(balloc(b, &b->ekx, own));
+    CAV_TRY(balloc(b, &b->eky, own));
+    CAV_TRY(balloc(b, &b->ekz, own));
+    if (!b->kstream) BAT_HIP(hipStreamCreateWithFlags(&b->kstream, hipStreamNonBlocking));
+    if (!b->ev_fork) BAT_HIP(hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
+    if (!b->ev_join) BAT_HIP(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
+  }
   b->nwaves = (int)b->h_waves.size();
   CAV_TRY(balloc(b, &b->waves, b->nwaves));
   CAV_TRY(batch_cells_alloc(b));
@@ -392,14 +409,38 @@ static int batch_sync_flags(cav_batch *b)
   return CAV_OK;
 }
 
+// The step's Ewald_k on the second stream (a parallel branch of the captured
+// step): it reads only the moved owned atoms and writes its own accelerations,
+// so it fills the waits of the exchange, list build and pair kernel.
+int cav::batch_ewald_k_fork(cav_batch *b)
+{
+  BAT_HIP(hipEventRecord(b->ev_fork, b->stream));
+  BAT_HIP(hipStreamWaitEvent(b->kstream, b->ev_fork, 0));
+  auto flip = [&] {
+    std::swap(b->stream, b->kstream);
+    std::swap(b->ax, b->ekx);
+    std::swap(b->ay, b->eky);
+    std::swap(b->az, b->ekz);
+    b->ek_set = !b->ek_set;
+  };
+  flip();
+  const int rc = batch_ewald_k(b);
+  flip();
+  CAV_TRY(rc);
+  BAT_HIP(hipEventRecord(b->ev_join, b->kstream));
+  return CAV_OK;
+}
+
 // One step of every replica (graph-capturable: no host decisions inside).
 static int batch_step_body(cav_batch *b, double dt)
 {
   CAV_TRY(batch_neighbor(b, true, dt));
-  CAV_TRY(batch_forces(b));
-  kb_kick<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(
-      b->d_rep, 0.5 * dt, b->vx, b->vy, b->vz, b->ax, b->ay, b->az, b->aox, b->aoy, b->aoz,
-      b->pair_blocks, b->part, b->vir, b->flags, b->hd_flags);
+  CAV_TRY(batch_pairs(b));
+  if (b->ek_on) BAT_HIP(hipStreamWaitEvent(b->stream, b->ev_join, 0));
+  const auto kick = b->ek_on ? kb_kick<true> : kb_kick<false>;
+  kick<<<dim3(grid_for(b->maxn), b->B), kBlock, 0, b->stream>>>(
+      b->d_rep, 0.5 * dt, b->vx, b->vy, b->vz, b->ax, b->ay, b->az, b->ekx, b->eky, b->ekz, b->aox,
+      b->aoy, b->aoz, b->pair_blocks, b->part, b->vir, b->flags, b->hd_flags);
   BAT_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -581,9 +622,12 @@ int cav_batch_destroy(cav_batch *b)
   if (!b) return CAV_ERR_ARG;
   (void)hipSetDevice(b->device);
   (void)hipStreamSynchronize(b->stream);
-  hipStream_t st = b->stream;
+  if (b->kstream) (void)hipStreamSynchronize(b->kstream);
   batch_free(b);
-  (void)hipStreamDestroy(st);
+  if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
+  if (b->ev_join) (void)hipEventDestroy(b->ev_join);
+  if (b->kstream) (void)hipStreamDestroy(b->kstream);
+  (void)hipStreamDestroy(b->stream);
   delete b;
   return CAV_OK;
 }

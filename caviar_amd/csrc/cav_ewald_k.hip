@@ -2625,7 +2625,7 @@ static int batch_ewald_k_t(cav_batch *b)
     f.bm_stride = b->bm_stride * (long)sizeof(T);
     f.part = nullptr;
     f.epart = nullptr;
-    f.set = 0;
+    f.set = b->ek_set;
     f.rb_per = p.Rpad / 16;
     launch_kforce_t<T>(b->stream, f, p, b->n_fitems, 1);
   } else {
@@ -2655,7 +2655,7 @@ static int batch_ewald_k_t(cav_batch *b)
     f.inv_sb = 1.0 / b->sB / b->sA;
     f.part = nullptr;
     f.epart = nullptr;
-    f.set = 0;
+    f.set = b->ek_set;
     f.rb_per = p.Rpad / 16;
     if (b->f_nt == 1)
       launch_kforce_h<1, kWavesF>(b->stream, f, b->nkh, b->n_fitems, 1, split_force_lds_p(p, b->nkh, 1));

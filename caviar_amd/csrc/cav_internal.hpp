@@ -401,6 +401,12 @@ struct cav_batch {
   double *vx = nullptr, *vy = nullptr, *vz = nullptr;  // owned
   double *ax = nullptr, *ay = nullptr, *az = nullptr;
   double *aox = nullptr, *aoy = nullptr, *aoz = nullptr;  // the snapshot's accelerations
+  // a step's Ewald_k beside its short-range work: stream, fork and join, its
+  // accelerations; ek_set: they are written, not added to
+  hipStream_t kstream = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  double *ekx = nullptr, *eky = nullptr, *ekz = nullptr;
+  bool ek_set = false;
   int *type_o = nullptr;                               // owned
   double *q_o = nullptr;
   double *snap = nullptr;  // [9][nown]: positions, velocities, accelerations
@@ -533,6 +539,7 @@ int batch_pairs(cav_batch *b);  // LJ/Ewald_r, virial partials
 int batch_ewald_k_plan(cav_batch *b);
 int batch_ewald_k_alloc(cav_batch *b);
 int batch_ewald_k(cav_batch *b);
+int batch_ewald_k_fork(cav_batch *b);  // on kstream, after the move
 int batch_ewald_k_field(cav_batch *b, double *out4);
 int batch_weight_sets(cav_batch *b, const double *w, double *part, long planes, double *out);
 

@@ -1660,7 +1660,8 @@ int batch_cells_alloc(cav_batch *b)
   return CAV_OK;
 }
 
-// Owned atoms of every replica drifted (or only wrapped), images, the rebuild
+// Owned atoms of every replica drifted (its Ewald_k then starts beside the
+// rest) or only wrapped, images, the rebuild
 // decision (`drift` false: every list is rebuilt, F_REBUILD is already set),
 // cells, packed copies and Verlet rows.
 int batch_neighbor(cav_batch *b, bool drift, double dt)
@@ -1696,6 +1697,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
                              : (drift ? k_move<true, kBlock, true> : k_move<false, kBlock, true>);
   move<<<own_grid, bs, 0, b->stream>>>(m, GhostRule{});
   BAT_HIP(hipGetLastError());
+  if (drift && b->ek_on) CAV_TRY(batch_ewald_k_fork(b));
   GhostArgs g;
   g.n = g.nblk = 0;
   g.scanned = 0;
