@@ -2402,6 +2402,23 @@ int batch_ewald_k_plan(cav_batch *b)
   }
   b->nkh = std::max(1, (2 * (b->ek.nZ - 1) + 31) / 32);
   split_scales(qmax, gb > 0 ? 1.0 : 0.0, gb, &b->sA, &b->sB);
+  // Atoms per S chunk of the FP32/FP64 passes: small batches take smaller chunks,
+  // so that the workgroups even out over the chip, for more partials to sum.
+  // 64 replicas (135000 atoms, FP64, kmax 6) with 1024 / 512 / 256: S pass 149 /
+  // 127 / 94 us, the adjoint's six weight sets 738 / 727 / 626, their sums 22 /
+  // 27 / 34.  The split pass keeps 1024: 256 replicas 174 us with its sum, 169
+  // at 512, 180 at 256.
+  if (!b->tuned) {
+    int groups, tpg, waves;
+    s_layout_rt(b->ek.Rpad, kRT, &groups, &tpg, &waves);
+    auto items = [&](int chunk) {
+      long k = 0;
+      for (const RepDev &d : b->reps) k += (d.n + chunk - 1) / chunk;
+      return k * groups;
+    };
+    b->s_chunk = 1024;
+    while (!batch_split(b) && b->s_chunk > 256 && items(b->s_chunk) < 4 * 256) b->s_chunk /= 2;
+  }
   return CAV_OK;
 }
 
