@@ -1147,20 +1147,37 @@ int cav_upload(cav_ctx *c, int which, const double *in)
   return CAV_OK;
 }
 
+// The concurrent Ewald_k's accelerations and the fields that follow it in
+// order: a = ((a_sr + a_k) + a_dip) + a_elc.
+static int add_side_forces(cav_ctx *c)
+{
+  CAV_TRY(ewald_k_join(c));
+  k_add3<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->ax, c->ay, c->az, c->ekx, c->eky,
+                                                   c->ekz);
+  if (c->dipole) CAV_TRY(launch_dipole(c));
+  if (c->elc_on) CAV_TRY(launch_elc(c));
+  CAV_HIP(hipGetLastError());
+  return CAV_OK;
+}
+
 // exchange_owned and exchange_ghost, the list (rebuilt or by the test), and
-// the forces of the current positions.
+// the forces of the current positions; Ewald_k beside the short-range work, as
+// in a step.
 static int evaluate(cav_ctx *c, bool rebuild)
 {
   const bool fused = fused_cells(c);
   k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, rebuild ? 1 : 0);
   CAV_TRY(launch_move(c, false, 0, true));
+  const bool side = c->overlap && c->ek_on && c->n > 0;
+  if (side) CAV_TRY(ewald_k_fork(c));
   CAV_TRY(launch_ghosts(c, true));
   CAV_TRY(neighbor_phase(c, Rebuild::decided, fused));
   if (rebuild) {  // the build is known to run
     c->nll_built = c->nll_pending;
     c->nlb_built = c->nlb_pending;
   }
-  return forces(c, true, fused);
+  CAV_TRY(forces(c, !side, fused));
+  return side ? add_side_forces(c) : CAV_OK;
 }
 
 int cav_setup(cav_ctx *c)
@@ -1262,17 +1279,11 @@ static int issue_step(cav_ctx *c, double dt, long ts, bool queued)
                     (side || !c->ek_on) && !cell_staged(c);
   CAV_TRY(forces(c, !side, fused, !late));
   bool join = side;
-  if (side) {
+  if (side && (c->dipole || c->elc_on)) {
+    CAV_TRY(add_side_forces(c));
+    join = false;
+  } else if (side) {
     CAV_TRY(ewald_k_join(c));
-    if (c->dipole || c->elc_on) {
-      // a = ((a_sr + a_k) + a_dip) + a_elc, as in order: add, dipole, slab
-      // correction, then the kick
-      k_add3<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->ax, c->ay, c->az, c->ekx, c->eky,
-                                                       c->ekz);
-      if (c->dipole) CAV_TRY(launch_dipole(c));
-      if (c->elc_on) CAV_TRY(launch_elc(c));
-      join = false;
-    }
   }
   const int nvir = late ? pair_blocks(c) : 0;
   const auto kick = join ? k_kick<true> : k_kick<false>;
