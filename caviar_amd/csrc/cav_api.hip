@@ -539,7 +539,7 @@ static int ewald_k_fork(cav_ctx *c)
 }
 
 // The main stream waits for the side Ewald_k; the kick then adds its
-// accelerations (k_kick_join): per atom the short-range sum plus the k-space
+// accelerations (k_kick<true>): per atom the short-range sum plus the k-space
 // one, as in forces().
 static int ewald_k_join(cav_ctx *c)
 {

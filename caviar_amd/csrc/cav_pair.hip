@@ -1,7 +1,8 @@
 // Fused LJ + Ewald real-space pair kernel over the full Verlet rows, plus the
 // cell-walk kernels (LJ when its cutoff exceeds the list guarantee, the
-// real-space energy and point queries).  One lane per owned atom, no atomics:
-// every atom gathers its own row, so FP64 results are reproducible run to run.
+// real-space energy and point queries).  No atomics: every atom gathers its own
+// row, its lanes' sums meet in a fixed tree, so FP64 results are reproducible run
+// to run.
 // No MFMA: the pair loop is a gather over irregular rows, not a contraction.
 #include <algorithm>
 #include <cstring>

@@ -317,7 +317,7 @@ int cav_set_tiles(cav_ctx *ctx, int s_rows, int s_chunk, int f_tiles, int f_wave
  * every pass in order on one stream (per-kernel timings without contention).
  * The accelerations are the same either way. */
 int cav_set_overlap(cav_ctx *ctx, int on);
-/* Short-range pair kernel.  CAV_PAIRS_AUTO (default): the row kernel (8 lanes
+/* Short-range pair kernel.  CAV_PAIRS_AUTO (default): the row kernel (8 or 32 lanes
  * per atom) reads each Verlet row as the bin-order slots the list build
  * recorded and gathers the neighbours from bin-ordered copies of the atoms,
  * where the neighbours of cell-ordered atoms lie close together; the atom-index
