@@ -833,7 +833,10 @@ struct CellBuild {
   const u64t *first;  // counters before each workgroup's cells, or nullptr: added up here
 };
 
-constexpr int kCellBlock = 1024;
+// Threads of a cell workgroup.  A batch, whose replicas have few cells each, takes
+// four waves: sixteen wait for a whole compute unit beside Ewald_k's passes (256
+// replicas: 208 us, four waves of two cells 116; alone 97 and 79).
+constexpr int kCellBlock = 1024, kBatchCellBlock = 256;
 
 // Cells of a list build, one wave per cell, bpb cells per workgroup: cell
 // starts (a workgroup adds up the counters of the cells before its own),
@@ -843,8 +846,8 @@ constexpr int kCellBlock = 1024;
 // build's candidates and the packed copies; pos_old as well
 // (neighborlist.cpp:302-303).  Without a rebuild only the packed copies are
 // refreshed, in the order of the last one.
-template <bool REP>
-__global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
+template <bool REP, int CB>
+__global__ __launch_bounds__(CB) void k_cells(CellBuild a, BinRule bins)
 {
   int blk = blockIdx.x, blocks = gridDim.x;
   if constexpr (REP) {
@@ -878,7 +881,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
     if (threadIdx.x == 0) s = a.first[blk];
   } else {
 #pragma unroll 4
-    for (int k = threadIdx.x; k < b0; k += kCellBlock) s += a.cnt[k];
+    for (int k = threadIdx.x; k < b0; k += CB) s += a.cnt[k];
   }
   const u64t own = lane < a.bpb && b0 + lane < a.nbins ? a.cnt[b0 + lane] : 0;
   const int early = lane < a.cap && wv < a.bpb && b0 + wv < a.nbins
@@ -886,21 +889,21 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
   const long tot = (long)a.n + G;
   if (stop) return;
   if (!rebuild) {
-    for (long t = (long)blk * kCellBlock + threadIdx.x; t < tot;
-         t += (long)blocks * kCellBlock) {
+    for (long t = (long)blk * CB + threadIdx.x; t < tot;
+         t += (long)blocks * CB) {
       const int j = a.litems[t];
       a.xqs[t] = slot_record(a.xq[j], a.tid[j], j >= a.n);
     }
     return;
   }
   if (blk == 0 && threadIdx.x == 0) a.flags[F_NGHOST_OLD] = G;
-  __shared__ u64t part[kCellBlock / 64];
+  __shared__ u64t part[CB / 64];
   __shared__ u64t first[65];  // per cell: slots before it, owned atoms before it
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   if (lane == 0) part[wv] = s;
   __syncthreads();
   if (wv == 0) {
-    u64t base = lane < kCellBlock / 64 ? part[lane] : 0;
+    u64t base = lane < CB / 64 ? part[lane] : 0;
     for (int o = 8; o > 0; o >>= 1) base += __shfl_xor(base, o, 16);
     base = __shfl(base, 0, 64);
     const u64t v = own;
@@ -915,7 +918,7 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(CellBuild a, BinRule bins)
     if (lane < a.bpb && b0 + lane == a.nbins - 1) a.start[a.nbins] = (int)(base + inc);
   }
   __syncthreads();
-  for (int w = wv; w < a.bpb && b0 + w < a.nbins; w += kCellBlock / 64) {
+  for (int w = wv; w < a.bpb && b0 + w < a.nbins; w += CB / 64) {
     const int b = b0 + w;
     const long s0 = (long)(unsigned)first[w];
     const int o0 = (int)(first[w] >> 32);
@@ -1116,7 +1119,7 @@ int launch_cells(cav_ctx *c)
   a.zo = c->zo;
   a.flags = c->flags;
   a.first = nullptr;
-  k_cells<false><<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
+  k_cells<false, kCellBlock><<<(c->xnbins + a.bpb - 1) / a.bpb, kCellBlock, 0, c->stream>>>(a, bin_rule(c, true));
   CAV_HIP(hipGetLastError());
   return CAV_OK;
 }
@@ -1634,12 +1637,9 @@ __global__ __launch_bounds__(kCellBlock) void kb_cell_first(const RepDev *rep, i
 // the counts of all of its replica's.
 static int batch_block(const cav_batch *b) { return b->maxn <= 65536 ? 64 : kBlock; }
 
-// Cells per workgroup of k_cells: one a wave where the chip has room, else two
-// (256 replicas, 100000 cells: 117 -> 97 us alone), four on large grids
-static int cells_per_block(const cav_batch *b)
-{
-  return b->maxcells > 4096 ? 64 : b->ncells >= 32768 ? 32 : 16;
-}
+// Cells per workgroup of k_cells: two a wave; on large grids sixteen (fewer
+// workgroups that add up the counters before theirs)
+static int cells_per_block(const cav_batch *b) { return b->maxcells > 4096 ? 64 : 8; }
 
 int batch_cells_alloc(cav_batch *b)
 {
@@ -1757,7 +1757,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   if (a.first)
     kb_cell_first<<<b->B, kCellBlock, 0, b->stream>>>(b->d_rep, a.bpb, blocks, b->cell_cnt,
                                                       b->cell_first);
-  k_cells<true><<<batch_grid(b, blocks), kCellBlock, 0, b->stream>>>(a, BinRule{});
+  k_cells<true, kBatchCellBlock><<<batch_grid(b, blocks), kBatchCellBlock, 0, b->stream>>>(a, BinRule{});
   launch_list_wave(b->stream, 0, b->ncells, nullptr, b->cap, b->rce2, b->xqs, b->st_off, b->st,
                    b->bin_start, b->litems, nullptr, b->nn, b->flags, nullptr, b->d_rep, b->waves,
                    b->nwaves, nullptr, b->nlb, true);
