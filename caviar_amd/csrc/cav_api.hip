@@ -496,6 +496,7 @@ int cav::refresh_params(cav_ctx *c)
   CAV_TRY(upload_params(c));
   k_charge_of_type<<<grid_for(std::max(c->n, c->nt)), kBlock, 0, c->stream>>>(
       c->n, c->type, c->d_charge, c->q, c->nt, c->d_qtype);
+  c->q_of = c->charge;  // a later setup makes d_qtype from it again
   if (c->gcap > 0)
     k_ghost_charge_of_type<<<grid_for(c->gcap), kBlock, 0, c->stream>>>(c->n, c->gcap, c->flags,
                                                                           c->type, c->d_charge, c->q);

@@ -257,7 +257,7 @@ struct cav_ctx {
   // (x, y, z, q) for the cell-staged one
   double4 *xqs = nullptr;
   double *d_qtype = nullptr;  // charges per type that the atoms' were taken from
-  std::vector<double> q_of;   // ... at their upload
+  std::vector<double> q_of;   // ... at their upload or the last refresh_params
   bool ids_ascend = false;    // the owned ids ascend with the index
   int2 *tids = nullptr;    // (type, id) in bin order
   // list build on the ghost-layer grid: per cell counts (owned in the high

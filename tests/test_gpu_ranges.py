@@ -339,3 +339,29 @@ def test_pair_rows_by_ids(gpu, n, ids, symmetric):
         # the oracle adds some 38 n terms one by one: a random walk of roundings
         # of partial sums several times the total, 1e-16 * sqrt(650000) * 1e3 = 1e-10
         assert abs(e.virial() - o.virial()) <= 1e-11 * max(abs(o.virial()), abs(o.energy_r())), kernel
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kernel", ["auto", "rows"])
+def test_setup_after_charge_change(gpu, precision, kernel):
+    """Charges changed after setup hold through a second setup: both ends of a
+    pair carry the new ones, as in a fresh engine (the same sums in the same
+    order, so the same bits)."""
+    print(f"[case] charges over setups {precision} {kernel}", flush=True)
+    s = configs.ions(n=600, rho=0.3, kmax=3, seed=5)
+    e = Engine(s.copy(), precision=precision)
+    e.set_pair_kernel(kernel)
+    e.setup()
+    e.set_parameters(charge=[0.7, -1.3])
+    e.recalculate(force_rebuild=True)
+    first = e.get("acc"), e.virial()
+    e.setup()
+    second = e.get("acc"), e.virial()
+    s.charge = np.array([0.7, -1.3])
+    f = Engine(s, precision=precision)
+    f.set_pair_kernel(kernel)
+    f.setup()
+    want = f.get("acc"), f.virial()
+    for got in (first, second):
+        assert np.array_equal(got[0], want[0])
+        assert got[1] == want[1]
