@@ -51,9 +51,12 @@ __global__ void k_block_sums(long nitems, F count, int *blk, const int *cond)
 // thread sums a contiguous run of ceil(nblk / 256) entries, one block scan
 // combines the runs, and each thread then writes its run's prefixes: one
 // pass with two barriers instead of one block scan per 256 entries.
-__global__ void k_scan_blocks(int nblk, int *blk, int *total, const int *cond)
+// stop (or nullptr): nothing is scanned once it is set.  The sums are then
+// those of an earlier launch, scanned already.
+__global__ void k_scan_blocks(int nblk, int *blk, int *total, const int *cond, const int *stop)
 {
   if (cond && !*cond) return;
+  if (stop && *stop) return;
   const int per = (nblk + kBlock - 1) / kBlock;
   const int b0 = threadIdx.x * per, b1 = min(nblk, b0 + per);
   int s = 0;
@@ -432,7 +435,7 @@ int launch_bins(cav_ctx *c, bool conditional, bool for_list)
   const int nb = grid_for(nbins);
   CountOf cnt{c->bin_cnt};
   k_block_sums<<<nb, kBlock, 0, c->stream>>>(nbins, cnt, c->scan_tmp, cond);
-  k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->scan_tmp, c->flags + F_COUNT - 1, cond);
+  k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->scan_tmp, c->flags + F_COUNT - 1, cond, nullptr);
   k_bin_start<<<nb, kBlock, 0, c->stream>>>(nbins, c->bin_cnt, c->scan_tmp, c->bin_start, cond);
   k_zero_int<<<grid_for(nbins), kBlock, 0, c->stream>>>(c->bin_cnt, nbins, cond);
   k_bin_fill<<<grid_for(tot), kBlock, 0, c->stream>>>(c->n, tot, c->bin_of, c->bin_start,
@@ -448,7 +451,7 @@ int launch_bins(cav_ctx *c, bool conditional, bool for_list)
   const int nbo = grid_for(tot);
   OwnedFlagBounded of{c->bin_items, c->flags, c->n};
   k_block_sums<<<nbo, kBlock, 0, c->stream>>>(tot, of, c->ord_blk, cond);
-  k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nbo, c->ord_blk, c->flags + F_COUNT - 2, cond);
+  k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nbo, c->ord_blk, c->flags + F_COUNT - 2, cond, nullptr);
   k_order_scatter<<<nbo, kBlock, 0, c->stream>>>(tot, c->n, c->bin_items, c->ord_blk, c->order,
                                                  c->flags, cond);
   CAV_HIP(hipGetLastError());
@@ -1087,7 +1090,8 @@ int launch_ghosts(cav_ctx *c, bool decide)
   a.bucket = c->bucket;
   a.cap = c->bucket_cap;
   if (a.scanned)
-    k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr);
+    k_scan_blocks<<<1, kBlock, 0, c->stream>>>(nb, c->blk, c->flags + F_NGHOST, nullptr,
+                                               c->flags + F_STOP);
   const auto kern = bs == 64 ? k_ghosts<64, false> : k_ghosts<kBlock, false>;
   kern<<<nb, bs, 0, c->stream>>>(a, ghost_rule(c), bin_rule(c, true));
   CAV_HIP(hipGetLastError());

@@ -365,3 +365,43 @@ def test_setup_after_charge_change(gpu, precision, kernel):
     for got in (first, second):
         assert np.array_equal(got[0], want[0])
         assert got[1] == want[1]
+
+
+def test_image_counts_past_a_million_atoms(gpu):
+    """More than 4096 workgroups of image counts are scanned by a launch of its
+    own: the images bit for bit those of the rule, after the setup, after steps,
+    and after a step that failed with others queued behind it."""
+    m, box = 102, 76.0                       # 1061208 atoms, at most 40^3 cells
+    n = m ** 3
+    print(f"[case] scanned image counts n={n}", flush=True)
+    g = (np.arange(m) + 0.5) * (box / m)
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    rng = np.random.default_rng(6)
+    pos += rng.uniform(-0.2, 0.2, pos.shape)  # 0.345 apart at least, the LJ reach is 0.2
+    s = _free_pair_system(n, box, pos, np.zeros((n, 3)))
+
+    def check(e):
+        now = e.get("pos")
+        gp, gs = e.ghosts()
+        wp, ws = F.numpy_ghosts(s, now)
+        assert np.array_equal(gs, ws) and np.array_equal(gp, wp)
+        return now
+
+    e = Engine(s)
+    e.setup()
+    check(e)
+    e.set("vel", np.tile([0.5, -0.25, 0.125], (n, 1)))
+    e.step(0.125, 3)                          # some atoms wrap
+    e.set("vel", np.zeros((n, 3)))
+    e.recalculate()
+    before = check(e)
+    acc = e.get("acc")
+    inside = int(np.argmin(((before - box / 2) ** 2).sum(1)))   # an atom without images
+    acc[inside] = np.nan
+    e.set("acc", acc)
+    with pytest.raises(NaNAccelerationError):
+        e.step(0.125, 40)
+    assert np.array_equal(check(e), before)
+    e.set("acc", np.zeros((n, 3)))
+    e.step(0.125, 2)
+    check(e)
