@@ -1316,7 +1316,7 @@ static int run_queued(cav_ctx *c, double dt, int nsteps)
   int attempts = 0;
   for (int done = 0; done < nsteps;) {
     const int q = std::min(nsteps - done, kQueuedSteps);
-    k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, attempts > 0 ? 1 : 0);
+    k_begin_step<<<1, 1, 0, c->stream>>>(c->flags, 0);
     for (int s = 0; s < q; ++s) CAV_TRY(issue_step(c, dt, c->step_index + s, true));
     CAV_TRY(sync_flags(c));
     const int ok = c->h_flags[F_STEPS];
@@ -1335,6 +1335,9 @@ static int run_queued(cav_ctx *c, double dt, int nsteps)
     }
     bool redo = false;
     CAV_TRY(check_capacity(c, &redo));
+    // the new rows hold nothing yet: whatever step comes next builds them,
+    // also one of a later call
+    if (redo) k_set_flag<<<1, 1, 0, c->stream>>>(c->flags, F_FORCE, 1);
     if (attempts >= 4) return fail(c, CAV_ERR_CAPACITY, "Verlet list capacity could not be met");
   }
   return CAV_OK;
