@@ -225,6 +225,7 @@ hipError_t stage_get3(Stage &s, hipStream_t st, long n, const double *a, const d
                       const double *c, double *out)
 {
   const long count = 3 * n;
+  if (count == 0) return hipStreamSynchronize(st);  // (a stage without room has no events)
   const int parts = count > 131072 ? kStageParts : 1;
   const long per = (count + parts - 1) / parts;
   for (int p = 0; p < parts; ++p) {
