@@ -1635,6 +1635,7 @@ int cav_list_stats(cav_ctx *c, double *ppa, double *lj_ppa)
 int cav_virial(cav_ctx *c, double *v)
 {
   if (!c || !v) return CAV_ERR_ARG;
+  (void)hipSetDevice(c->device);  // the staging memory's events are made here
   return read_scal(c, 1, v);
 }
 

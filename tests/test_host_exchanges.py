@@ -104,3 +104,31 @@ for which in range(4):
     assert lib.cav_download(h, which, p) == 0, lib.cav_last_error(h)
     assert lib.cav_upload(h, which, p) == 0, lib.cav_last_error(h)
 """)
+
+
+SETUP = """
+def engine(device):
+    s = configs.ions(n=64, rho=0.3, kmax=2, seed=1)
+    e = Engine(s, device=device)
+    e.setup()
+    return e
+"""
+
+
+def test_staging_belongs_to_the_contexts_device(runtime):
+    """Each call that may be an engine's first exchange, while another device is
+    current, and the ones that follow it."""
+    run(runtime, SETUP + """
+first = dict(virial=lambda e: e.virial(), get=lambda e: e.get("pos"),
+             set=lambda e: e.set("pos", e.system.pos), energy=lambda e: e.energy(),
+             points=lambda e: e.point_field("r", e.system.pos),
+             adjoint=lambda e: e.adjoint(np.ones((e.n, 3))))
+for name, call in first.items():
+    a, b = engine(0), engine(1)
+    for e, other in ((a, 1), (b, 0)):
+        fake.fake_current(other)
+        call(e)
+        for later in first.values():
+            fake.fake_current(other)
+            later(e)
+""")
