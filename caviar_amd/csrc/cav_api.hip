@@ -616,8 +616,12 @@ static int neighbor_phase(cav_ctx *c, Rebuild how, bool fused)
 // The first `count` device scalars.
 static int read_scal(cav_ctx *c, int count, double *v)
 {
-  if (!stage_room(c->stage, count)) return fail(c, CAV_ERR_HIP, "no pinned host memory");
-  CAV_HIP(stage_get(c->stage, c->stream, count, c->scal, v));
+  if (stage_room(c->stage, count)) {
+    CAV_HIP(stage_get(c->stage, c->stream, count, c->scal, v));
+    return CAV_OK;
+  }
+  CAV_HIP(hipMemcpyAsync(v, c->scal, sizeof(double) * count, hipMemcpyDeviceToHost, c->stream));
+  CAV_HIP(hipStreamSynchronize(c->stream));
   return CAV_OK;
 }
 

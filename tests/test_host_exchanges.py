@@ -132,3 +132,18 @@ for name, call in first.items():
             fake.fake_current(other)
             later(e)
 """)
+
+
+def test_exchanges_without_pinned_memory(runtime):
+    """Where no pinned memory is to be had, every exchange takes plain copies."""
+    run(runtime, SETUP + """
+e = engine(0)
+fake.fake_pinned(0)
+e.virial()
+e.energy()
+e.get("pos")
+e.set("pos", e.system.pos)
+e.point_field("r", e.system.pos)
+e.point_field("k", e.system.pos)
+e.adjoint(np.ones((e.n, 3)))
+""")
