@@ -405,3 +405,30 @@ def test_image_counts_past_a_million_atoms(gpu):
     e.set("acc", np.zeros((n, 3)))
     e.step(0.125, 2)
     check(e)
+
+
+@pytest.mark.parametrize("n", [1048576, 1048577])
+def test_kinetic_energy_of_many_workgroups(gpu, n):
+    """Up to 4096 workgroups each adds up all sums of m v, past them a launch
+    does: kinetic energy, temperature and a Berendsen step of free atoms against
+    numpy.  FP64 sums of 1e6 terms of one sign: sqrt(1e6) * 1e-16 = 1e-13."""
+    from caviar_amd import BerendsenSettings, ThermoSettings
+    print(f"[case] kinetic energy n={n}", flush=True)
+    m, box = 102, 102.0
+    at = np.arange(n)
+    pos = np.stack([at % m, at // m % m, at // (m * m)], axis=1) + 0.5
+    rng = np.random.default_rng(n)
+    vel = rng.normal(size=(n, 3)) + [0.3, -0.2, 0.1]
+    s = _free_pair_system(n, box, np.ascontiguousarray(pos), vel)
+    s.mass = np.array([1.5])
+    s.thermo = ThermoSettings(k_b=1.1)
+    s.berendsen = BerendsenSettings(temperature=0.9, coupling=0.05, dt=0.001)
+    e = Engine(s)
+    e.setup()
+    ke = 0.5 * 1.5 * ((vel - vel.mean(0)) ** 2).sum()
+    temp = 2 * ke / (1.1 * (3 * n - 3))
+    got = e.thermo()
+    assert abs(got[0] - ke) <= 1e-13 * ke and abs(got[1] - temp) <= 1e-13 * temp
+    e.step(0.001, 1)
+    lam = np.sqrt(1 + 0.001 / 0.05 * (0.9 / temp - 1))
+    assert F.rel_err(e.get("vel"), vel * lam) <= 1e-13
