@@ -111,6 +111,8 @@ struct RepDev {
   int base, n, gcap, obase, tbase;
   int cbase, nbins, nb[3];
   int pbase;                 // first per-block partial slot
+  int bcap;                  // slots of a cell's bucket, and the first bucket's place
+  long bbase;
 };
 
 // Which replica a workgroup of a batched kernel works on, and as which of its
@@ -412,7 +414,7 @@ struct cav_batch {
   double *snap = nullptr;  // [9][nown]: positions, velocities, accelerations
   int *bin_start = nullptr, *bin_items = nullptr;
   unsigned long long *cell_cnt = nullptr, *cell_first = nullptr;
-  int *bucket = nullptr, bucket_cap = 0;  // unsorted slots of every cell
+  int *bucket = nullptr;  // unsorted slots of every cell, a replica's from its bbase
   int *gblk = nullptr;     // [B][scan_blocks] ghost-count block sums
   int *nn = nullptr;
   // Verlet rows as replica-local bin slots, bin-ordered records, slot -> local atom, owned atoms in cell order

@@ -700,7 +700,8 @@ __global__ __launch_bounds__(BS) void k_ghosts(GhostArgs a, GhostRule rule, BinR
     a.xq += r.base;
     a.tid += r.base;
     a.cnt += r.cbase;
-    a.bucket += (long)r.cbase * a.cap;
+    a.bucket += r.bbase;
+    a.cap = r.bcap;
     rule = ghost_rule_of(r, a.gc);
     bins = bin_rule_of(r, a.cinv);
   }
@@ -863,7 +864,8 @@ __global__ __launch_bounds__(CB) void k_cells(CellBuild a, BinRule bins)
     blocks = (r.nbins + a.bpb - 1) / a.bpb;
     if (blk >= blocks) return;
     a.cnt += r.cbase;
-    a.bucket += (long)r.cbase * a.cap;
+    a.bucket += r.bbase;
+    a.cap = r.bcap;
     a.xq += r.base, a.tid += r.base;
     a.start += r.cbase + rr;  // one closing entry a replica
     a.items += r.base, a.litems += r.base;
@@ -997,7 +999,7 @@ int cells_alloc(cav_ctx *c)
   c->bucket = nullptr;
   c->cell_cnt = nullptr;
   if (!c->nl_on || c->n == 0 || c->xnbins > 65536) return CAV_OK;
-  // twice the mean cell and some, in whole waves
+  // twice the mean cell and some, in whole half waves
   const double cell = c->rce * c->rce * c->rce, vol = c->L[0] * c->L[1] * c->L[2];
   const long want = (long)(2.0 * cell * (c->n / vol)) + 32;
   const long cap = std::min(1024L, (want + 31) / 32 * 32);
@@ -1648,19 +1650,21 @@ static int cells_per_block(const cav_batch *b) { return b->maxcells > 4096 ? 64 
 int batch_cells_alloc(cav_batch *b)
 {
   b->maxcells = 0;
-  double density = 0;
-  for (const RepDev &r : b->reps) {
+  size_t room = 0;
+  for (RepDev &r : b->reps) {
     b->maxcells = std::max(b->maxcells, r.nbins);
-    density = std::max(density, r.n / (r.L[0] * r.L[1] * r.L[2]));
+    // twice the replica's mean cell and some, in whole half waves, as the
+    // single system: the room stays in proportion to its cells and atoms
+    const double want = 2.0 * b->rce * b->rce * b->rce * r.n / (r.L[0] * r.L[1] * r.L[2]) + 32;
+    r.bcap = (int)(std::min(1024.0, want + 31) / 32) * 32;
+    r.bbase = (long)room;
+    room += (size_t)r.bcap * r.nbins;
   }
   b->scan_blocks = grid_for(b->maxn, batch_block(b));
-  // twice the densest replica's mean cell and some, as the single system
-  const double want = 2.0 * b->rce * b->rce * b->rce * density + 32;
-  b->bucket_cap = (int)(std::min(1024.0, want + 31) / 32) * 32;
   const int blocks = (b->maxcells + cells_per_block(b) - 1) / cells_per_block(b);
   void **bufs[] = {(void **)&b->cell_cnt, (void **)&b->bucket, (void **)&b->cell_first,
                    (void **)&b->gblk};
-  const size_t bytes[] = {sizeof(u64t) * b->ncells, sizeof(int) * (size_t)b->bucket_cap * b->ncells,
+  const size_t bytes[] = {sizeof(u64t) * b->ncells, sizeof(int) * room,
                           b->maxcells > 65536 ? sizeof(u64t) * (size_t)blocks * b->B : 0,
                           sizeof(int) * (size_t)b->B * b->scan_blocks};
   for (int k = 0; k < 4; ++k) {
@@ -1730,7 +1734,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   g.tid = b->tid;
   g.cnt = b->cell_cnt;
   g.bucket = b->bucket;
-  g.cap = b->bucket_cap;
+  g.cap = 0;
   g.reps = batch_reps(b);
   g.gc = b->ghost_cutoff;
   g.cinv = b->cinv;
@@ -1739,7 +1743,7 @@ int batch_neighbor(cav_batch *b, bool drift, double dt)
   CellBuild a;
   a.n = a.nbins = 0;
   a.bpb = cells_per_block(b);
-  a.cap = b->bucket_cap;
+  a.cap = 0;
   a.cnt = b->cell_cnt;
   a.bucket = b->bucket;
   a.xq = b->xq;

@@ -432,3 +432,32 @@ def test_kinetic_energy_of_many_workgroups(gpu, n):
     e.step(0.001, 1)
     lam = np.sqrt(1 + 0.001 / 0.05 * (0.9 / temp - 1))
     assert F.rel_err(e.get("vel"), vel * lam) <= 1e-13
+
+
+def test_batch_cells_take_room_by_their_own_replica(gpu):
+    """A dense replica beside a dilute one of many cells: the batch's memory is
+    that of its parts (the dilute one's 140608 cells at 128 bytes a bucket, the
+    dense one's rows of about 2100 neighbours), and the pairs are the exact set."""
+    import ctypes
+    from caviar_amd import load_library
+
+    def free_bytes():  # (from the HIP runtime the library is linked with)
+        v = [ctypes.c_size_t(), ctypes.c_size_t()]
+        assert load_library().hipMemGetInfo(*[ctypes.byref(x) for x in v]) == 0
+        return v[0].value
+
+    print("[case] batch buckets", flush=True)
+    rng = np.random.default_rng(4)
+    n, box = 5600, 4.5
+    dense = _free_pair_system(n, box, rng.uniform(0, box, (n, 3)), np.zeros((n, 3)))
+    dilute = _free_pair_system(200, 100.0, rng.uniform(0, 100.0, (200, 3)), np.zeros((200, 3)))
+    for s in (dense, dilute):
+        s.lj.epsilon[:] = 0.0
+    b = Batch([dense, dilute])
+    before = free_bytes()
+    b.setup()
+    used = before - free_bytes()
+    assert used <= 300e6, used
+    for r, s in enumerate((dense, dilute)):
+        gp, _ = F.numpy_ghosts(s, s.pos)
+        assert np.array_equal(F.sorted_pairs(b.pairs(r)), F.sorted_pairs(F.exact_pairs(s.pos, gp, 2.0))), r
