@@ -192,8 +192,8 @@ __device__ __forceinline__ void copy_to_lds_async(const unsigned char *src, unsi
 // 174 -> 135 us beside the short-range passes (60 us of products at the rate a large FP64 matrix
 // product reaches);
 // six weight sets of 135000 atoms in 64 replicas, kmax 6: 540 -> 365 us.
-// In the mixed form the MFMAs accumulate in FP32 over one chunk (<= 4096
-// atoms) and the chunk partials are summed in FP64.
+// In the mixed form the MFMAs accumulate in FP32 over one chunk (at most
+// kMixedChunk atoms) and the chunk partials are summed in FP64.
 template <typename T, int RT, int SCT>
 __global__ __launch_bounds__(64 * kWavesMax) void k_sk(SArgs a)
 {
@@ -1605,6 +1605,10 @@ static int s_stage(const cav_ctx *c, size_t tsz)
   return s_stage_for(c->ek.nX + c->ek.nY + c->ek.nZ, tsz);
 }
 
+// The longest chunk of the mixed form, whose sums over a chunk are FP32 (their
+// rounding error grows with its square root).
+constexpr int kMixedChunk = 4096;
+
 static int s_chunk(const cav_ctx *c, int ntarget)
 {
   // aim for >= ntarget workgroups over the whole grid; chunk multiple of 32
@@ -1613,9 +1617,14 @@ static int s_chunk(const cav_ctx *c, int ntarget)
   // FP64: a workgroup of four to seven compute waves has a CU to itself, and
   // one round of them leaves half the partials of two
   if (c->precision == CAV_FP64 && waves >= 4) ntarget /= 2;
+  // mixed: groups as eight compute waves would make them, so that giving one to
+  // the producer lengthens no chunk
+  const int tiles = c->ek.Rpad / 16;
+  if (c->precision == CAV_MIXED) groups = (tiles + kWavesMax * kRT - 1) / (kWavesMax * kRT);
   long per = ((long)c->n * groups + ntarget - 1) / ntarget;
   per = (per + 31) / 32 * 32;
   if (per < 32) per = 32;
+  if (c->precision == CAV_MIXED) per = std::min(per, (long)kMixedChunk);
   return (int)per;
 }
 

@@ -1,7 +1,7 @@
-"""Host logic of the exchanges with host memory, on a stand-in HIP runtime:
-memory is the host's, kernels do nothing, and every stream and event belongs to
-the device that was current when it was made.  An event recorded on another
-device's stream, or none at all, is an error, as in HIP.
+"""Host logic (exchanges with host memory, launch shapes) on a stand-in HIP
+runtime: memory is the host's, kernels only leave their name and grid, and every
+stream and event belongs to the device that was current when it was made.  An
+event recorded on another device's stream, or none at all, is an error, as in HIP.
 
 Each check is a program of its own with the stand-in preloaded.
 """
@@ -19,11 +19,21 @@ RUNTIME = r"""
 #include <cstdlib>
 #include <cstring>
 #include <cstddef>
+#include <map>
+#include <string>
 typedef struct { unsigned x, y, z; } dim3_t;
 struct Obj { int device; };
 static thread_local int current = 0;
 static int pinned_left = 1 << 30;
 static Obj none{0};
+struct Call { dim3_t grid, block; size_t shared; void *stream; };
+static thread_local Call call;
+static std::map<const void *, std::string> &names()
+{
+  static std::map<const void *, std::string> m;
+  return m;
+}
+static std::string launches;  // "name x y z" lines
 static Obj *stream(void *s) { return s ? (Obj *)s : &none; }
 extern "C" {
 void fake_current(int d) { current = d; }
@@ -57,9 +67,33 @@ int hipEventRecord(void *e, void *s)
   return e && ((Obj *)e)->device == stream(s)->device ? 0 : 400;
 }
 int hipEventSynchronize(void *e) { return e ? 0 : 400; }
-int hipLaunchKernel(const void *, dim3_t, dim3_t, void **, size_t, void *) { return 0; }
-int __hipPushCallConfiguration(dim3_t, dim3_t, size_t, void *) { return 0; }
-int __hipPopCallConfiguration(dim3_t *, dim3_t *, size_t *, void **) { return 0; }
+int hipLaunchKernel(const void *f, dim3_t g, dim3_t, void **, size_t, void *)
+{
+  launches += names()[f] + " " + std::to_string(g.x) + " " + std::to_string(g.y) + " " +
+              std::to_string(g.z) + "\n";
+  return 0;
+}
+const char *fake_launches() { return launches.c_str(); }
+void fake_forget() { launches.clear(); }
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t n, void *s)
+{
+  call = Call{g, b, n, s};
+  return 0;
+}
+int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *n, void **s)
+{
+  *g = call.grid, *b = call.block, *n = call.shared, *s = call.stream;
+  return 0;
+}
+int hipFuncSetAttribute(const void *, int, int) { return 0; }
+void **__hipRegisterFatBinary(const void *) { static void *p; return &p; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *,
+                           void *, void *, void *, int *)
+{
+  names()[host] = name;
+}
 }
 """
 
@@ -68,6 +102,7 @@ import ctypes, numpy as np
 import caviar_amd
 from caviar_amd import Engine, configs
 fake = ctypes.CDLL(None)
+fake.fake_launches.restype = ctypes.c_char_p
 lib = caviar_amd.load_library()
 """
 
@@ -146,4 +181,30 @@ e.set("pos", e.system.pos)
 e.point_field("r", e.system.pos)
 e.point_field("k", e.system.pos)
 e.adjoint(np.ones((e.n, 3)))
+""")
+
+
+def test_mixed_chunks_keep_their_length(runtime):
+    """The mixed form sums 32-bit products over one chunk of atoms, so its
+    chunks are no longer than an even deal of 512 workgroups of eight waves,
+    nor than 4096 atoms: the last few row tiles of a group, and past a million
+    atoms."""
+    run(runtime, """
+from caviar_amd import EwaldKSettings, System
+for n, kmax, longest in ((30000, 13, 64), (100003, 13, 224), (30000, 16, 128), (2000000, 16, 4096),
+                         (3000000, 6, 4096)):
+    rng = np.random.default_rng(1)
+    box = (n / 0.3) ** (1 / 3)
+    s = System(lower=[0] * 3, upper=[box] * 3, bc=[1] * 3, ghost_cutoff=4.0, mass=[1.0], charge=[1.0],
+               pos=rng.uniform(0, box, (n, 3)), vel=np.zeros((n, 3)), types=np.zeros(n, dtype=np.int32),
+               ewald_k=EwaldKSettings.cube(0.9, kmax, 2.0))
+    fake.fake_forget()
+    e = Engine(s, precision="mixed")
+    e.setup()
+    grids = [l.split() for l in fake.fake_launches().decode().splitlines() if "k_sk_h" in l]
+    assert len(grids) == 1, grids
+    tiles = -(-(kmax + 1) * (2 * kmax + 1) // 16)
+    chunks = int(grids[0][1]) // -(-tiles // 21)     # at least: the grid is rounded up by chunks of 8
+    assert n / chunks <= longest, (n, kmax, n / chunks)
+    e.close()
 """)
