@@ -484,7 +484,7 @@ static int sync_flags(cav_ctx *c)
     c->nll_built = c->nll_pending;
     c->nlb_built = c->nlb_pending;
   }
-  return CAV_OK;
+  return cells_fit(c);
 }
 
 // New parameter values (same structure) set after setup: upload them, refresh

@@ -540,10 +540,20 @@ static int batch_setup_impl(cav_batch *b)
     }
     if (!grow) {
       b->setup_done = true;
-      return CAV_OK;
+      bool grown;
+      return batch_cells_fit(b, &grown);  // (no graph yet)
     }
   }
   return bfail(b, CAV_ERR_CAPACITY, "batch capacities could not be met");
+}
+
+// Larger buckets for the replicas whose cells outgrew them (flags read back).
+static int batch_fit(cav_batch *b)
+{
+  bool grown = false;
+  CAV_TRY(batch_cells_fit(b, &grown));
+  if (grown) drop_graph(b);
+  return CAV_OK;
 }
 
 static int batch_run(cav_batch *b, double dt, int nsteps, bool graph)
@@ -571,6 +581,7 @@ static int batch_run(cav_batch *b, double dt, int nsteps, bool graph)
       CAV_TRY(batch_grow(b, &relaid));
       redo = relaid;
       if (relaid) CAV_TRY(batch_setup_impl(b));  // rebuilds from the restored state
+      CAV_TRY(batch_fit(b));
     }
     if (redo) return bfail(b, CAV_ERR_CAPACITY, "batch capacities could not be met");
   }

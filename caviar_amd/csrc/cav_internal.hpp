@@ -35,6 +35,7 @@ enum Flag : int {
   F_NL_STALE = 10, // the last list build wrote bin-order slots only: index rows are filled on demand
   F_STOP = 11,     // a step failed (NaN or overflow): the steps queued after it leave the state alone
   F_STEPS = 12,    // steps completed since the flags were last cleared
+  F_MAXCELL = 13,  // most slots of a cell met past its bucket's room
   F_COUNT = 16
 };
 
@@ -372,7 +373,7 @@ struct cav_batch {
   // replicas as given (host)
   struct HostRep {
     double lo[3], hi[3];
-    int n = 0, gcap = 0;
+    int n = 0, gcap = 0, bcap = 0;  // atoms; ghost slots; bucket slots once its cells were crowded
     std::vector<int> type;
     std::vector<double> pos, vel;  // AoS
   };
@@ -479,6 +480,7 @@ int launch_move(cav_ctx *c, bool drift, double dt, bool decide);  // drift / wra
 int launch_ghosts(cav_ctx *c, bool decide);  // images, rebuild decision, cell counts
 bool fused_cells(const cav_ctx *c);  // whether launch_cells follows, instead of launch_bins
 int cells_alloc(cav_ctx *c);
+int cells_fit(cav_ctx *c);  // larger buckets where cells outgrew them (flags read back)
 int launch_cells(cav_ctx *c);
 int launch_rebuild_check(cav_ctx *c);
 // for_list: the binning of a list build, which also keeps the bin order the
@@ -535,6 +537,7 @@ int bhip_check(cav_batch *b, hipError_t e, const char *what);
 dim3 batch_grid(const cav_batch *b, int blocks);
 RepGrid batch_reps(const cav_batch *b);
 int batch_cells_alloc(cav_batch *b);
+int batch_cells_fit(cav_batch *b, bool *grown);
 // move or wrap, ghosts, rebuild test (drift), cells, packed copies, list
 int batch_neighbor(cav_batch *b, bool drift, double dt);
 int batch_pairs(cav_batch *b);  // LJ/Ewald_r, virial partials

@@ -939,6 +939,7 @@ __global__ __launch_bounds__(CB) void k_cells(CellBuild a, BinRule bins)
       // large cells through memory: the unsorted slots (those past the bucket's
       // capacity are found again by their cell), then each one's rank
       if (m > a.cap) {
+        if (lane == 0) atomicMax(a.flags + F_MAXCELL, m);  // the host makes the buckets larger
         int at = 0;
         for (long t0 = 0; t0 < tot; t0 += 64) {
           bool in = false;
@@ -998,6 +999,7 @@ int cells_alloc(cav_ctx *c)
   if (c->cell_cnt) (void)hipFree(c->cell_cnt);
   c->bucket = nullptr;
   c->cell_cnt = nullptr;
+  k_zero_int<<<1, kBlock, 0, c->stream>>>(c->flags + F_MAXCELL, 1, nullptr);
   if (!c->nl_on || c->n == 0 || c->xnbins > 65536) return CAV_OK;
   // twice the mean cell and some, in whole half waves
   const double cell = c->rce * c->rce * c->rce, vol = c->L[0] * c->L[1] * c->L[2];
@@ -1006,6 +1008,32 @@ int cells_alloc(cav_ctx *c)
   if (cap * c->xnbins > 32L * ((long)c->n + c->gcap) + 65536) return CAV_OK;
   CAV_HIP(hipMalloc(&c->bucket, sizeof(int) * cap * c->xnbins));
   CAV_HIP(hipMalloc(&c->cell_cnt, sizeof(u64t) * c->xnbins));
+  c->bucket_cap = (int)cap;
+  return CAV_OK;
+}
+
+// A quarter more than the fullest cell, in whole half waves.
+static long crowd_cap(int most) { return ((long)most + most / 4 + 31) / 32 * 32; }
+
+// Buckets are sized for the mean cell.  A wave of k_cells whose cell has more
+// slots looks through all atoms for them: in a droplet of 30000 atoms (cutoff
+// 5, 150 a cell, the mean 9) 717 us a build, from larger buckets 180.  So once
+// cells were met past their room, with the flags read back and the stream
+// idle, the buckets grow to the fullest, as long as they stay within 64 MB or
+// what the slots themselves take.
+int cells_fit(cav_ctx *c)
+{
+  const int most = c->h_flags[F_MAXCELL];
+  if (!c->bucket || most <= c->bucket_cap) return CAV_OK;
+  const long cap = crowd_cap(most);
+  if (cap * c->xnbins > std::max(16L << 20, 32L * ((long)c->n + c->gcap))) return CAV_OK;
+  int *larger = nullptr;
+  if (hipMalloc(&larger, sizeof(int) * cap * c->xnbins) != hipSuccess) {
+    (void)hipGetLastError();  // the present ones do
+    return CAV_OK;
+  }
+  (void)hipFree(c->bucket);
+  c->bucket = larger;
   c->bucket_cap = (int)cap;
   return CAV_OK;
 }
@@ -1657,6 +1685,7 @@ int batch_cells_alloc(cav_batch *b)
     // single system: the room stays in proportion to its cells and atoms
     const double want = 2.0 * b->rce * b->rce * b->rce * r.n / (r.L[0] * r.L[1] * r.L[2]) + 32;
     r.bcap = (int)(std::min(1024.0, want + 31) / 32) * 32;
+    r.bcap = std::max(r.bcap, b->hreps[&r - b->reps.data()].bcap);
     r.bbase = (long)room;
     room += (size_t)r.bcap * r.nbins;
   }
@@ -1672,6 +1701,26 @@ int batch_cells_alloc(cav_batch *b)
     *bufs[k] = nullptr;
     if (bytes[k]) BAT_HIP(hipMalloc(bufs[k], bytes[k]));
   }
+  return CAV_OK;
+}
+
+// cells_fit for every replica of a batch, each within a megabyte or what its
+// slots take.  `grown`: kernel arguments have changed.
+int batch_cells_fit(cav_batch *b, bool *grown)
+{
+  *grown = false;
+  for (int k = 0; k < b->B; ++k) {
+    RepDev &r = b->reps[k];
+    const int most = b->h_flags[16 * k + F_MAXCELL];
+    const long cap = crowd_cap(most);
+    if (most <= r.bcap || cap * r.nbins > std::max(1L << 18, 32L * ((long)r.n + r.gcap))) continue;
+    b->hreps[k].bcap = (int)cap;  // (a new layout keeps it)
+    *grown = true;
+  }
+  if (!*grown) return CAV_OK;
+  CAV_TRY(batch_cells_alloc(b));
+  BAT_HIP(hipMemcpyAsync(b->d_rep, b->reps.data(), sizeof(RepDev) * b->B, hipMemcpyHostToDevice, b->stream));
+  BAT_HIP(hipStreamSynchronize(b->stream));
   return CAV_OK;
 }
 

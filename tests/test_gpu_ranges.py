@@ -152,6 +152,39 @@ def test_crowded_cells(gpu, clump):
     assert F.rel_err(e.get("acc"), o.get("acc")) <= 1e-11  # close pairs cancel more
 
 
+@pytest.mark.parametrize("clump", [60, 66, 130, 700, 1500])
+def test_crowded_cells_again(gpu, clump):
+    """Once crowded cells were met their buckets grow: the builds after that
+    sort them from the bucket, in an engine and in a batch (beside a replica
+    that is not crowded).  Free atoms that drift together: positions exactly,
+    pairs the exact set after every few steps."""
+    print(f"[case] crowded cells again {clump}", flush=True)
+    rng = np.random.default_rng(clump)
+    n, box, dt = clump + 150, 24.0, 0.0625
+    pos = rng.uniform(0, box, (n, 3))
+    pos[rng.permutation(n)[:clump]] = rng.uniform(12.0, 13.9, (clump, 3))
+    pos = np.round(pos * 1024) / 1024       # the drift is exact
+    s = _free_pair_system(n, box, pos, np.tile([3.0, -1.0, 0.5], (n, 1)))
+    s.lj.epsilon[:] = 0.0
+    other = _free_pair_system(50, box, np.round(rng.uniform(0, box, (50, 3)) * 1024) / 1024,
+                              np.zeros((50, 3)))
+    e, b = Engine(s.copy()), Batch([s, other])
+    e.setup()
+    b.setup()
+    now = pos
+    for steps in (1, 1, 5, 9):
+        e.step(dt, steps)
+        b.step(dt, steps)
+        for _ in range(steps):
+            now = now + s.vel * dt
+            now = np.where(now < 0, now + box, np.where(now > box, now - box, now))
+        assert np.array_equal(e.get("pos"), now) and np.array_equal(b.get(0, "pos"), now)
+        assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(b.pairs(0)))
+    e.recalculate(force_rebuild=True)
+    gp, _ = F.numpy_ghosts(s, now)
+    assert np.array_equal(F.sorted_pairs(e.pairs()), F.sorted_pairs(F.exact_pairs(now, gp, 2.0)))
+
+
 @pytest.mark.parametrize("n", [63, 64, 65, 257, 16383, 16385])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_steps_at_workgroup_edges(gpu, n, precision):
