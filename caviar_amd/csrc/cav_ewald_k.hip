@@ -2248,7 +2248,7 @@ int point_room(cav_ctx *c, size_t doubles, size_t table_bytes)
 
 // Point queries: tables for the points, then the force pass with q = 1 into a
 // per-point (field, potential) buffer; the dipole field is added on the host.
-int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *pot)
+static int point_part_k(cav_ctx *c, int np, const double *pts, double *field, double *pot)
 {
   const EwaldKPlan &p = c->ek;
   const int TS = p.nX + p.nY + p.nZ;
@@ -2297,6 +2297,21 @@ int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *
     }
     if (pot) pot[i] = o4[4 * (size_t)i + 3];
   }
+  return CAV_OK;
+}
+
+// The points in parts of at most 256 MB of phase tables (whole workgroups of
+// the force pass): the room for a part is kept for the next query, a map of
+// millions of places would keep gigabytes.
+int point_field_k(cav_ctx *c, int np, const double *pts, double *field, double *pot)
+{
+  const EwaldKPlan &p = c->ek;
+  const size_t record = (size_t)(p.nX + p.nY + p.nZ) * 2 *
+                        (c->precision == CAV_FP64 ? sizeof(double) : sizeof(float));
+  const int per = (int)std::max<size_t>(1, (size_t(256) << 20) / record / 4096) * 4096;
+  for (int p0 = 0; p0 == 0 || p0 < np; p0 += per)
+    CAV_TRY(point_part_k(c, std::min(per, np - p0), pts + 3 * (size_t)p0,
+                         field ? field + 3 * (size_t)p0 : nullptr, pot ? pot + p0 : nullptr));
   return CAV_OK;
 }
 

@@ -1203,7 +1203,7 @@ __global__ __launch_bounds__(kBlock) void k_point_r(CellArgs c, int np, const do
   }
 }
 
-int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot)
+static int point_part_r(cav_ctx *c, int np, const double *pts, double *field, double *pot)
 {
   // the points are read from pinned host memory and the sums written there,
   // both once per point
@@ -1228,6 +1228,16 @@ int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *
   CAV_HIP(hipStreamSynchronize(c->stream));
   if (staged && field) std::memcpy(field, c->stage.host + 3 * (size_t)np, sizeof(double) * 3 * np);
   if (staged && pot) std::memcpy(pot, c->stage.host + 6 * (size_t)np, sizeof(double) * np);
+  return CAV_OK;
+}
+
+// The points in parts that fit the staging memory.
+int point_field_r(cav_ctx *c, int np, const double *pts, double *field, double *pot)
+{
+  const int per = (int)(kStageMax / (7 * sizeof(double)));
+  for (int p0 = 0; p0 == 0 || p0 < np; p0 += per)
+    CAV_TRY(point_part_r(c, std::min(per, np - p0), pts + 3 * (size_t)p0,
+                         field ? field + 3 * (size_t)p0 : nullptr, pot ? pot + p0 : nullptr));
   return CAV_OK;
 }
 

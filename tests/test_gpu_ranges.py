@@ -467,18 +467,19 @@ def test_kinetic_energy_of_many_workgroups(gpu, n):
     assert F.rel_err(e.get("vel"), vel * lam) <= 1e-13
 
 
+def free_bytes():
+    """The GPU's free memory (from the HIP runtime the library is linked with)."""
+    import ctypes
+    from caviar_amd import load_library
+    v = [ctypes.c_size_t(), ctypes.c_size_t()]
+    assert load_library().hipMemGetInfo(*[ctypes.byref(x) for x in v]) == 0
+    return v[0].value
+
+
 def test_batch_cells_take_room_by_their_own_replica(gpu):
     """A dense replica beside a dilute one of many cells: the batch's memory is
     that of its parts (the dilute one's 140608 cells at 128 bytes a bucket, the
     dense one's rows of about 2100 neighbours), and the pairs are the exact set."""
-    import ctypes
-    from caviar_amd import load_library
-
-    def free_bytes():  # (from the HIP runtime the library is linked with)
-        v = [ctypes.c_size_t(), ctypes.c_size_t()]
-        assert load_library().hipMemGetInfo(*[ctypes.byref(x) for x in v]) == 0
-        return v[0].value
-
     print("[case] batch buckets", flush=True)
     rng = np.random.default_rng(4)
     n, box = 5600, 4.5
@@ -494,3 +495,25 @@ def test_batch_cells_take_room_by_their_own_replica(gpu):
     for r, s in enumerate((dense, dilute)):
         gp, _ = F.numpy_ghosts(s, s.pos)
         assert np.array_equal(F.sorted_pairs(b.pairs(r)), F.sorted_pairs(F.exact_pairs(s.pos, gp, 2.0))), r
+
+
+def test_point_maps_of_many_places(gpu):
+    """Maps that take several parts (over 256 MB of phase tables, over 64 MB of
+    points and sums): the room they leave behind is bounded, and the values are
+    those of the same places asked for in small numbers (FP64: the lattice sums
+    of few places are split, 1e-13)."""
+    print("[case] point maps", flush=True)
+    s = configs.ions(n=300, rho=0.3, kmax=16, seed=3)
+    e = Engine(s)
+    e.setup()
+    rng = np.random.default_rng(2)
+    pts = rng.uniform(s.lower, s.upper, (1300007, 3))
+    before = free_bytes()
+    got = {w: e.point_field(w, pts) for w in ("k", "r")}
+    used = before - free_bytes()
+    assert used <= 400e6, used
+    for at in (0, 200000, 1198372 - 30, 1300007 - 61):
+        for w in ("k", "r"):
+            f, p = e.point_field(w, pts[at:at + 61])
+            assert F.rel_err(got[w][0][at:at + 61], f) <= 1e-13, (w, at)
+            assert F.rel_err(got[w][1][at:at + 61], p) <= 1e-13, (w, at)
