@@ -348,12 +348,10 @@ struct AdjWork {
          *f4 = nullptr;
 };
 
-// (u: room once taken by per-atom weights; it still counts towards the fixed
-// scratch, whose limit callers know)
 struct AdjSizes {
-  size_t w = 0, part = 0, out = 0, u = 0, ss = 0, sw = 0, f4 = 0;
+  size_t w = 0, part = 0, out = 0, ss = 0, sw = 0, f4 = 0;
   static size_t up(size_t v) { return (v + 31) / 32 * 32; }  // 256-byte boundaries
-  size_t total() const { return up(w) + up(part) + up(out) + up(u) + up(ss) + up(sw) + up(f4); }
+  size_t total() const { return up(w) + up(part) + up(out) + up(ss) + up(sw) + up(f4); }
   AdjWork carve(double *q) const
   {
     AdjWork k;
@@ -378,7 +376,6 @@ static AdjSizes adjoint_sizes(const cav_ctx *c)
   z.out = nv + 2 * (size_t)nt;
   if (c->ek_on) {
     const size_t plane = (size_t)c->ek.Rpad * 2 * c->ek.nZ;
-    z.u = (size_t)n + 1;
     z.ss = plane * nt;
     z.sw = plane * 3;
     z.f4 = 4 * (size_t)(n + 1);
@@ -564,7 +561,9 @@ extern "C" int cav_adjoint_noalloc(cav_ctx *c, const double *w_host, double *g_e
                 "parameter values changed since the last force evaluation: cav_adjoint_noalloc "
                 "allocates nothing, so call cav_recalculate, cav_forces or cav_adjoint first");
   const AdjSizes z = adjoint_sizes(c);
-  const size_t need = z.total();
+  // with Ewald_k the systems served are those whose workspace leaves room for
+  // one more value per atom (which no kernel takes any longer)
+  const size_t need = z.total() + (c->ek_on ? AdjSizes::up((size_t)c->n + 1) : 0);
   if (need * sizeof(double) > kAdjScratchBytes)
     return fail(c, CAV_ERR_CAPACITY,
                 "cav_adjoint_noalloc needs " + std::to_string(need * sizeof(double)) +

@@ -234,8 +234,8 @@ int cav_adjoint(cav_ctx *ctx, const double *weights, double *g_epsilon, double *
  * per-atom k-space field) carved from one fixed device array per GPU of
  * cav_adjoint_noalloc_scratch_bytes() bytes (32 MiB, held until the process
  * ends) instead of per-call allocations; the call allocates nothing.
- * CAV_ERR_CAPACITY when this system's workspace exceeds the array (about
- * 400k atoms with two types at kmax 16: use cav_adjoint), CAV_ERR_STATE when
+ * CAV_ERR_CAPACITY when this system's workspace exceeds the array (from about
+ * 460000 atoms with two types at kmax 16: use cav_adjoint), CAV_ERR_STATE when
  * parameter values were changed after the last force evaluation (applying
  * them allocates: call cav_recalculate or cav_forces first).  Every call on
  * one GPU shares the array and leaves its contents behind: calls that
@@ -312,10 +312,10 @@ int cav_tiles(const cav_ctx *ctx, int *s_rows, int *s_stage, int *s_chunk, int *
  * cav_setup; the forces of the current state are recomputed.  FP64 uses the
  * chunk only. */
 int cav_set_tiles(cav_ctx *ctx, int s_rows, int s_chunk, int f_tiles, int f_waves);
-/* cav_step runs Ewald_k on a second HIP stream, concurrently with the ghost
- * exchange, neighbour build and pair kernel (on = 1, the default); 0 runs
- * every pass in order on one stream (per-kernel timings without contention).
- * The accelerations are the same either way. */
+/* cav_step, cav_setup and cav_recalculate run Ewald_k on a second HIP stream,
+ * concurrently with the ghost exchange, neighbour build and pair kernel (on =
+ * 1, the default); 0 runs every pass in order on one stream (per-kernel timings
+ * without contention).  The accelerations are the same either way. */
 int cav_set_overlap(cav_ctx *ctx, int on);
 /* Short-range pair kernel.  CAV_PAIRS_AUTO (default): the row kernel (8 or 32 lanes
  * per atom) reads each Verlet row as the bin-order slots the list build

@@ -43,6 +43,12 @@ int hipSetDevice(int d) { current = d; return 0; }
 int hipGetLastError() { return 0; }
 int hipMalloc(void **p, size_t n) { *p = calloc(n ? n : 1, 1); return 0; }
 int hipFree(void *p) { free(p); return 0; }
+int hipGetSymbolAddress(void **p, const void *)
+{
+  static void *scratch = calloc(64 << 20, 1);
+  *p = scratch;
+  return 0;
+}
 int hipHostMalloc(void **p, size_t n, unsigned)
 {
   if (pinned_left-- <= 0) return 2;
@@ -207,4 +213,23 @@ for n, kmax, longest in ((30000, 13, 64), (100003, 13, 224), (30000, 16, 128), (
     chunks = int(grids[0][1]) // -(-tiles // 21)     # at least: the grid is rounded up by chunks of 8
     assert n / chunks <= longest, (n, kmax, n / chunks)
     e.close()
+""")
+
+
+@pytest.mark.parametrize("kmax,most", [(3, 484263), (16, 462549)])
+def test_fixed_scratch_serves_the_same_systems(runtime, kmax, most):
+    """The largest system of two types that cav_adjoint_noalloc takes."""
+    run(runtime, f"""
+from caviar_amd import CaviarError, EwaldKSettings, System
+for n in ({most}, {most} + 1):
+    s = System(lower=[0] * 3, upper=[100.0] * 3, bc=[1] * 3, ghost_cutoff=4.0, mass=[1.0, 1.0],
+               charge=[1.0, -1.0], pos=np.zeros((n, 3)), vel=np.zeros((n, 3)),
+               types=np.zeros(n, dtype=np.int32), ewald_k=EwaldKSettings.cube(0.9, {kmax}, 2.0))
+    e = Engine(s)
+    e.setup()
+    try:
+        e.adjoint_noalloc(np.zeros((n, 3)))
+        assert n == {most}
+    except CaviarError as err:
+        assert n > {most} and err.code == 5
 """)
