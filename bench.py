@@ -36,8 +36,8 @@ HBM_PEAK_GBS = 8000.0
 FLOP_SK, FLOP_KF, FLOP_PAIR, FLOP_LJ, FLOP_INT = 16, 22, 43, 12, 20
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "pmc_traffic_ions_N262144_kmax16.json")
 TRAFFIC_SOURCE = ("read from profiles/pmc_traffic_ions_N262144_kmax16.json (rocprofv3 FETCH_SIZE and "
-                  "WRITE_SIZE of the same launch at the same tiles, scaled by a copy of known size); "
-                  "not measured in this run")
+                  "WRITE_SIZE of the same launch at the tiles pinned there, scaled by a copy of known "
+                  "size); not measured in this run")
 
 
 def log(msg):
@@ -60,7 +60,7 @@ def run_engine(system, precision, warmup, steps, dt, pair_kernel="auto", pin=Non
         log(f"{precision}: autotuned Ewald_k tiles {tiles} in {time.perf_counter() - t0:.2f}s")
     e.step(dt, warmup)
     t0 = time.perf_counter()
-    e.step(dt, steps)          # every step ends with a stream synchronisation
+    e.step(dt, steps)          # returns with the steps done (the stream synchronised)
     t = time.perf_counter() - t0
     # per-kernel launch times from HIP events, in a separate pass so that the
     # event records do not weigh on the throughput above; Ewald_k runs in line
