@@ -288,7 +288,7 @@ class Engine:
         return self.tiles()
 
     def set_overlap(self, on: bool):
-        """Ewald_k of a step concurrent with the short-range passes (default on)."""
+        """Ewald_k of a step or evaluation concurrent with the short-range passes (default on)."""
         self._check(self.lib.cav_set_overlap(self.h, int(bool(on))))
 
     PAIR_KERNELS = {"auto": 0, "rows": 1, "cells": 2}

@@ -1,5 +1,7 @@
 // C ABI of caviar_amd: context lifetime, settings, upload/download, and the
-// velocity-Verlet step driver (all device work on the context's one stream).
+// velocity-Verlet step driver.  Device work goes to the context's stream; a
+// step's or evaluation's Ewald_k to a second one beside it, joined before the
+// call's last kernels (cav_set_overlap).
 #include <algorithm>
 #include <cmath>
 #include <cstring>

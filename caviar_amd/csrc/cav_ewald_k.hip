@@ -2112,9 +2112,9 @@ int launch_dipole(cav_ctx *c)
   return CAV_OK;
 }
 
-// Sums over chunks of the weight sets' partials (grid row = set), in
-// k_chunk_sum's order, without the padding columns: set v to ss (v < nt) or sw,
-// [Rpad][nZ] complex each.
+// Sums over chunks of the weight sets' partials (grid row = set), without the
+// padding columns: set v to ss (v < nt) or sw, [Rpad][nZ] complex each.  Wave w
+// adds chunks w, w + 4, ... in order, then the waves' sums in pairs.
 __global__ void k_sets_sum(int nchunks, int Rpad, int SC, int nZ, int set0, int nt,
                            const double *part, double *ss, double *sw)
 {

@@ -465,9 +465,9 @@ int launch_bins(cav_ctx *c, bool conditional, bool for_list)
 // the owned atoms), k_ghosts (images, rebuild decision, cell counts and
 // buckets), k_cells (cell starts, sorted cells and everything in bin order) and
 // the list build.  As one kernel per scan, fill, sort and copy it was eighteen,
-// of 2-4 us each plus the gap before it: a step of 256 LJ atoms took 141 us,
-// now 72; of 8000 ions (FP64, kmax 8) 209, now 119; at N = 262144, where the
-// gaps hide beside Ewald_k, 0.82 ms before and now.
+// of 2-4 us each plus the gap before it: this alone took a step of 256 LJ atoms
+// from 141 to 72 us (now 39), of 8000 ions (FP64, kmax 8) from 209 to 119 (now
+// 90); at N = 262144, where the gaps hide beside Ewald_k, it changed nothing.
 
 typedef unsigned long long u64t;
 
@@ -1187,12 +1187,13 @@ constexpr int kCand = CAV_LIST_CAND;
 // lanes append in lane order through a ballot and a prefix popcount, so rows
 // are written coalesced and in a deterministic order.
 //
-// Instruction issue bounds it, vector and scalar alike (counters: 15 vector
-// and 18 scalar instructions for each test of 64 pairs, of which the exact
-// FP64 distance needs nine).  So the owned atoms come by scalar loads, the
-// bounds check of a buffer store stands for the tests of a full row and of an
-// idle lane, the atom itself is looked for only in the pass that holds it, and
-// a stage's cells are found by bisection with all its loads in flight.
+// Instruction issue bounds it (counters over a launch at N=262144: 20.0 vector
+// and 13.1 scalar instructions for each test of 64 pairs, of which the exact
+// FP64 distance needs nine; 22.6 and 13.0 before this form).  So the owned atoms
+// come by scalar loads, the bounds check of a buffer store stands for the tests
+// of a full row and of an idle lane, the atom itself is looked for only in the
+// pass that holds it, and a stage's cells are found by bisection with all its
+// loads in flight.
 // In order: N=262144 144 -> 121 us, 256 replicas (540000 atoms at rho 0.2 to
 // 0.8) 444 -> 332 us.
 constexpr int kAPI = 4;  // owned atoms tested per staged candidate
@@ -1626,11 +1627,10 @@ int launch_save_old(cav_ctx *c, bool conditional)
 // ---------------------------------------------------------- batched replicas --
 //
 // The same exchange for every replica of a cav_batch at once, in the same
-// kernels: grid row blockIdx.y is the replica, whose decisions (ghost count,
-// rebuild) live in its own 16 flag words.  Before, thirteen kernels of its own
-// took a step: 256 replicas (540000 atoms, 1.5 million with their images)
-// 455 us beside the list, now 360; with the index rows no longer written the
-// list build went from 506 to 444 us.
+// kernels: each workgroup works on one replica (RepGrid: the grid row, or dealt
+// to an XCD), whose decisions (ghost count, rebuild) live in its own 16 flag
+// words.  256 replicas (540000 atoms, 1.5 million with their images), a step's
+// exchange without the list: 455 us as thirteen kernels of its own, now 220.
 
 // Counters before every bpb-th cell of a replica, for grids on which each
 // workgroup of k_cells adding them up itself would read too much.

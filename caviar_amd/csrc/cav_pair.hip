@@ -187,8 +187,8 @@ __device__ __forceinline__ void block_virial(double vir, double *part)
 // partial forces of an atom's lanes are summed with a fixed shuffle tree, so
 // FP64 results stay reproducible.
 //
-// Gather instructions bound it (N=262144 mixed: the address units take about 25
-// clocks for each, of whatever width, 78% of their time; the vector units are
+// Gather instructions bound it (N=262144 mixed: the address units take about 24
+// clocks for each, of whatever width, 73% of their time; the vector units are
 // half busy).  So a slot is one record of two 16-byte loads: the charge is
 // looked up by type, and with ids that ascend with the atom index
 // (ROWS_SLOTS_ASC) images and the order of a pair are told by id, without the
@@ -1250,7 +1250,8 @@ constexpr int kWalkCand = 512;
 // once for the cell's owned atoms, which the four waves take in turn, lanes
 // over the candidates.  The FP64 erfc of every (atom, candidate) bounds it
 // (about 500 an atom at rho = 0.3); one lane per atom, each walking its
-// stencil through scattered loads, took 3395 us at N = 100003, now 395 us.
+// stencil through scattered loads, took 3395 us at N = 100003, this 395 and with
+// the terms of cav_math.hpp 249 us.
 __global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, EwaldAlpha al, double *part)
 {
   __shared__ double4 cand[kWalkCand];

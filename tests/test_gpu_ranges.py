@@ -369,8 +369,9 @@ def test_pair_rows_by_ids(gpu, n, ids, symmetric):
         e.set_pair_kernel(kernel)
         e.setup()
         assert F.rel_err(e.get("acc"), o.get("acc")) <= 1e-12, kernel
-        # the oracle adds some 38 n terms one by one: a random walk of roundings
-        # of partial sums several times the total, 1e-16 * sqrt(650000) * 1e3 = 1e-10
+        # the oracle adds some 38 n terms one by one: a random walk of the roundings
+        # of partial sums that reach 41 times the total (n = 17000, counted),
+        # 1.1e-16 * sqrt(645000) * 41 = 4e-12
         assert abs(e.virial() - o.virial()) <= 1e-11 * max(abs(o.virial()), abs(o.energy_r())), kernel
 
 
