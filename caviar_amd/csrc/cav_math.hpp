@@ -60,28 +60,39 @@ __device__ __forceinline__ double exp_neg(double x, double lo)
 // erfc(x) = exp(-x^2) erfcx(x), and erfcx is smooth on [0, inf): with
 // t = 1 / (1 + x/4) (the form of Hastings' approximations, Abramowitz & Stegun
 // 7.1.26) erfcx(x) = t P(2t - 1), P of degree 22, its Chebyshev fit in 40-digit
-// arithmetic truncated at 3e-17 relative; evaluated in FP64 it is within 2 ulp
-// up to x = 4 and 8 beyond, where the exponential has taken over.  The
-// exponential is shared with the Gaussian term of the force, 1/r comes from
-// v_rsq_f64 and two Newton steps, and no lane branches: sqrt, two divisions,
-// exp and the library's erfc, whose ranges all run in a wave of mixed
-// distances, take half as many instructions again.  FP64 issue bounds the
-// kernels that are not bound by their gathers: real-space energy at N = 100003
-// 395 -> 249 us, adjoint pairs of 64 replicas 327 -> 265, the pair kernel at
-// N = 65536 56 -> 37 (in order).
+// arithmetic truncated at 3e-17 relative.  The exponential is shared with the
+// Gaussian term of the force, 1/r comes from v_rsq_f64 and a Newton step, and
+// no lane branches; sqrt, two divisions, exp and the library's erfc, whose
+// ranges all run in a wave of mixed distances, take more instructions.  FP64
+// issue bounds the kernels that are not bound by their
+// gathers: real-space energy at N = 100003 395 -> 267 us, adjoint pairs of 64
+// replicas 327 -> 310, the pair kernel at N = 65536 56 -> 37 (in order).
+//
+// The quantities that the terms are most sensitive to (1/r, its square, 2t - 1)
+// each take a last correction from their residual.  Without these the kernels
+// took 256, 306 and 34 us, but the forces of 100 ions (alpha 0.9) were 2.7e-16
+// off 64-bit exact (2-norm) where the library's functions gave 2.4e-16; now
+// 2.3e-16, point potentials 2.1e-16 (library 3.2e-16), their fields 2.7e-16
+// (4.2e-16).  A term's own error is 1.6e-16 root mean square and 7e-16 at most.
 __device__ __forceinline__ void ewald_real(double r2, const EwaldAlpha &al, double &e, double &ec,
                                            double &ri2)
 {
   double y = __builtin_amdgcn_rsq(r2);
-  const double h = 0.5 * r2;
-#pragma unroll
-  for (int it = 0; it < 2; ++it) y = fma(y, fma(-h * y, y, 0.5), y);
-  const double x = al.alpha * (r2 * y);
-  const double d = fma(0.25, x, 1.0);
+  y = fma(y, fma(-0.5 * r2 * y, y, 0.5), y);
+  // r = r2 y and 1 / r from the residual 1 - r2 y^2 of the unrounded product
+  double rn = r2 * y;
+  const double f = fma(-fma(r2, y, -rn), y, fma(-rn, y, 1.0));
+  rn = fma(0.5 * rn, f, rn);
+  y = fma(0.5 * y, f, y);
+  // s = 2t - 1 = (1 - w) / (1 + w), w = x / 4: a rounding of 1 + w alone would
+  // count four times in x
+  const double w = 0.25 * (al.alpha * rn);
+  const double d = 1.0 + w;
   double t = __builtin_amdgcn_rcp(d);
-#pragma unroll
-  for (int it = 0; it < 2; ++it) t = fma(t, fma(-d, t, 1.0), t);
-  const double s = fma(2.0, t, -1.0);
+  t = fma(t, fma(-d, t, 1.0), t);
+  double s = fma(2.0, t, -1.0);
+  s = fma(fma(-w, s, (1.0 - s) - w), t, s);
+  t = fma(0.5, s, 0.5);
   double p = 3.01845414851638119e-10;
   p = fma_k(p, s, -6.63613627087004204e-11);
   p = fma_k(p, s, -3.81882222497661988e-09);
@@ -107,8 +118,9 @@ __device__ __forceinline__ void ewald_real(double r2, const EwaldAlpha &al, doub
   p = fma_k(p, s, 2.73998915250122765e-01);
   const double xx = al.a2 * r2;
   e = exp_neg(xx, fma(al.a2, r2, -xx) + al.a2lo * r2);
-  ec = e * (t * p) * y;
+  ec = e * ((t * p) * y);
   ri2 = y * y;
+  ri2 = fma(ri2, fma(-r2, ri2, 1.0), ri2);
 }
 
 }  // namespace cav

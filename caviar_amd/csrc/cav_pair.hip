@@ -1251,7 +1251,7 @@ constexpr int kWalkCand = 512;
 // over the candidates.  The FP64 erfc of every (atom, candidate) bounds it
 // (about 500 an atom at rho = 0.3); one lane per atom, each walking its
 // stencil through scattered loads, took 3395 us at N = 100003, this 395 and with
-// the terms of cav_math.hpp 249 us.
+// the terms of cav_math.hpp 267 us.
 __global__ __launch_bounds__(kBlock) void k_energy_r(CellArgs c, EwaldAlpha al, double *part)
 {
   __shared__ double4 cand[kWalkCand];

@@ -265,6 +265,37 @@ def test_real_space_terms_accuracy(gpu, alpha):
         assert abs(mp.mpf(float(f[k, 0])) - q * g) <= 4e-15 * abs(g), (r[k], alpha)
 
 
+def test_real_space_terms_rounding(gpu):
+    """The same terms' usual error, where alpha r is small and they are largest:
+    about ten roundings between the distance and each sum, of at most
+    2^-53 / sqrt(3) = 6.4e-17 root mean square each, so 2e-16; the distance's
+    square counts up to 1.4 times (alpha^2 r^2)."""
+    mp = pytest.importorskip("mpmath")
+    mp.mp.dps = 40
+    print("[case] real-space terms' rounding", flush=True)
+    s = configs.ions(n=1, rho=1e-3, kmax=1, seed=1, with_lj=False, with_k=False)
+    s.lower, s.upper = np.zeros(3), np.full(3, 64.0)
+    s.bc = np.zeros(3, dtype=np.int32)
+    s.pos = np.array([[32.0, 32.0, 32.0]])
+    s.ewald_r.alpha, s.ewald_r.k_electrostatic = 0.3, 1.0
+    e = Engine(s)
+    e.setup()
+    pts = np.repeat(s.pos, 1500, axis=0)
+    pts[:, 0] += np.random.default_rng(5).uniform(0.7, 4.0, len(pts))
+    f, p = e.point_field("r", pts)
+    q = float(s.charge[s.types[0]])
+    al = mp.mpf(0.3)
+    err = np.empty((2, len(pts)))
+    for k in range(len(pts)):
+        x = mp.mpf(float(pts[k, 0])) - 32
+        ec = mp.erfc(al * x) / x
+        g = (2 * al / mp.sqrt(mp.pi) * mp.exp(-(al * x) ** 2) + ec) / x
+        err[0, k] = float(mp.mpf(float(p[k])) / (q * ec) - 1)
+        err[1, k] = float(mp.mpf(float(f[k, 0])) / (q * g) - 1)
+    rms = np.sqrt((err ** 2).mean(1))
+    assert rms[0] <= 2e-16 and rms[1] <= 2e-16, rms
+
+
 @pytest.mark.parametrize("n", [255, 256, 700])
 @pytest.mark.parametrize("n_r_df,which", [(d, w) for d in (0, 3) for w in
                                           ("temp", "berendsen", "nve", "both", "both_no_temp")]
