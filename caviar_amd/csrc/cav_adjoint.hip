@@ -21,6 +21,7 @@ namespace cav {
 
 // Ewald_k pieces exposed by cav_ewald_k.hip
 int ewald_k_weight_sets(cav_ctx *c, const double *w, double *ss, double *sw);
+int ewald_k_sets_room(cav_ctx *c);
 int ewald_k_field(cav_ctx *c, double *out4);
 
 constexpr int kLPAa = 16;
@@ -512,6 +513,7 @@ extern "C" int cav_adjoint(cav_ctx *c, const double *w_host, double *g_eps, doub
     CAV_HIP(hipMalloc(&c->adj_ws, sizeof(double) * z.total()));
     c->adj_cap = z.total();
   }
+  if (c->ek_on) CAV_TRY(ewald_k_sets_room(c));
   (void)stage_room(c->stage, 3 * (size_t)c->n);
   std::vector<double> hout(z.out, 0.0);
   CAV_TRY(adjoint_run(c, w_host, z.carve(c->adj_ws), hout.data()));

@@ -549,3 +549,25 @@ def test_point_maps_of_many_places(gpu):
             f, p = e.point_field(w, pts[at:at + 61])
             assert F.rel_err(got[w][0][at:at + 61], f) <= 1e-13, (w, at)
             assert F.rel_err(got[w][1][at:at + 61], p) <= 1e-13, (w, at)
+
+
+def test_setup_takes_no_room_for_the_adjoint(gpu):
+    """What only the adjoint uses is taken at its first call, once: a setup of
+    8000 ions leaves less than 50 MB, the adjoint's partial sums come to 20."""
+    print("[case] setup room", flush=True)
+    s = configs.ions(n=8000, rho=0.3, kmax=8, seed=3)
+    e = Engine(s)
+    before = free_bytes()
+    e.setup()
+    at_setup = free_bytes()
+    w = np.random.default_rng(1).normal(size=(s.n, 3))
+    g = e.adjoint(w)
+    first = free_bytes()
+    for _ in range(3):
+        assert np.array_equal(e.adjoint(w)[2], g[2])
+    assert free_bytes() == first
+    assert before - at_setup <= 50e6, before - at_setup
+    assert np.array_equal(e.adjoint_noalloc(w)[2], g[2])
+    f = Engine(s)              # the scratch's adjoint without the room: the same bits
+    f.setup()
+    assert np.array_equal(f.adjoint_noalloc(w)[2], g[2])
