@@ -1027,6 +1027,7 @@ int cells_fit(cav_ctx *c)
   if (!c->bucket || most <= c->bucket_cap) return CAV_OK;
   const long cap = crowd_cap(most);
   if (cap * c->xnbins > std::max(16L << 20, 32L * ((long)c->n + c->gcap))) return CAV_OK;
+  (void)hipSetDevice(c->device);
   int *larger = nullptr;
   if (hipMalloc(&larger, sizeof(int) * cap * c->xnbins) != hipSuccess) {
     (void)hipGetLastError();  // the present ones do
