@@ -1330,6 +1330,8 @@ static int run_queued(cav_ctx *c, double dt, int nsteps)
     done += ok;
     c->step_index += ok;
     if (!c->h_flags[F_STOP]) {
+      // (a step neither counted nor failed has not run)
+      if (ok != q) return fail(c, CAV_ERR_HIP, "queued steps did not complete");
       attempts = 0;
       continue;
     }

@@ -130,7 +130,7 @@ def run(runtime, body):
     preload = ":".join(filter(None, [runtime, os.environ.get("LD_PRELOAD")]))
     env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=ROOT)
     p = subprocess.run([sys.executable, "-c", HEAD + body], env=env, cwd=ROOT, capture_output=True,
-                       text=True, timeout=120)
+                       text=True, timeout=60)
     assert p.returncode == 0, p.stdout + p.stderr
 
 
@@ -232,4 +232,17 @@ for n in ({most}, {most} + 1):
         assert n == {most}
     except CaviarError as err:
         assert n > {most} and err.code == 5
+""")
+
+
+def test_steps_that_do_not_run_are_an_error(runtime):
+    """Queued steps whose kernels leave no trace end the call, not an endless
+    repetition (here no kernel runs)."""
+    run(runtime, SETUP + """
+e = engine(0)
+try:
+    e.step(0.001, 3)
+    assert False
+except caviar_amd.CaviarError as err:
+    assert err.code == 2
 """)
