@@ -25,6 +25,7 @@ typedef struct { unsigned x, y, z; } dim3_t;
 struct Obj { int device; };
 static thread_local int current = 0;
 static int pinned_left = 1 << 30;
+static int crowd = 0, malloc_device = -1;
 static Obj none{0};
 struct Call { dim3_t grid, block; size_t shared; void *stream; };
 static thread_local Call call;
@@ -38,10 +39,12 @@ static Obj *stream(void *s) { return s ? (Obj *)s : &none; }
 extern "C" {
 void fake_current(int d) { current = d; }
 void fake_pinned(int left) { pinned_left = left; }
+void fake_crowd(int most) { crowd = most, malloc_device = -1; }  // F_MAXCELL of flags read back
+int fake_malloc_device() { return malloc_device; }
 int hipGetDeviceCount(int *n) { *n = 2; return 0; }
 int hipSetDevice(int d) { current = d; return 0; }
 int hipGetLastError() { return 0; }
-int hipMalloc(void **p, size_t n) { *p = calloc(n ? n : 1, 1); return 0; }
+int hipMalloc(void **p, size_t n) { malloc_device = current; *p = calloc(n ? n : 1, 1); return 0; }
 int hipFree(void *p) { free(p); return 0; }
 int hipGetSymbolAddress(void **p, const void *)
 {
@@ -59,7 +62,12 @@ int hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return 0; }
 int hipMemset(void *p, int v, size_t n) { memset(p, v, n); return 0; }
 int hipMemsetAsync(void *p, int v, size_t n, void *) { return hipMemset(p, v, n); }
 int hipMemcpy(void *d, const void *s, size_t n, int) { if (n) memcpy(d, s, n); return 0; }
-int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *) { return hipMemcpy(d, s, n, k); }
+int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *)
+{
+  hipMemcpy(d, s, n, k);
+  if (crowd && k == 2 && n == 16 * sizeof(int)) ((int *)d)[13] = crowd;
+  return 0;
+}
 int hipStreamCreate(void **s) { *s = new Obj{current}; return 0; }
 int hipStreamCreateWithFlags(void **s, unsigned) { return hipStreamCreate(s); }
 int hipStreamDestroy(void *s) { delete (Obj *)s; return 0; }
@@ -245,4 +253,17 @@ try:
     assert False
 except caviar_amd.CaviarError as err:
     assert err.code == 2
+""")
+
+
+def test_cell_buckets_grow_on_the_contexts_device(runtime):
+    """Flags read back while another device is current: larger buckets are
+    still the context's own device's."""
+    run(runtime, SETUP + """
+e = engine(0)
+fake.fake_crowd(1000)
+fake.fake_current(1)
+n = ctypes.c_int()
+assert lib.cav_num_ghosts(e.h, ctypes.byref(n)) == 0
+assert fake.fake_malloc_device() == 0
 """)
